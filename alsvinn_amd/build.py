@@ -25,6 +25,10 @@ SOURCES = [
     "avh_stage_euler1.hip",
     "avh_stage_euler2.hip",
     "avh_stage_euler3.hip",
+    "avh_stage_euler3_none.hip",
+    "avh_stage_euler3_weno2.hip",
+    "avh_stage_euler3_eno2.hip",
+    "avh_stage_euler3_eno3.hip",
 ]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -57,7 +61,7 @@ def build(verbose=False):
     os.makedirs(BUILD, exist_ok=True)
     jobs = min(len(SOURCES), max(1, min(8, os.cpu_count() or 1)))
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as ex:
-        objs = list(ex.map(_compile, SOURCES))
+        objs = list(ex.map(_compile, reversed(SOURCES)))  # the longest first
     tmp = LIB + ".tmp"
     cmd = [HIPCC, "--offload-arch=" + ARCH, "-shared", "-fPIC", "-o", tmp] + objs
     r = subprocess.run(cmd, capture_output=True, text=True)

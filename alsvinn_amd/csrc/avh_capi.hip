@@ -116,7 +116,7 @@ __device__ __forceinline__ double draw_double(unsigned long long r, int elo, int
     return __longlong_as_double((long long)(((unsigned long long)(e + 1023) << 52) | mant));
 }
 
-enum { ARITH_SQRT = 0, ARITH_DIV_RHO = 1, ARITH_DIV_WENO = 2, ARITH_DIV_ROE = 3, ARITH_FREXP = 4 };
+enum { ARITH_SQRT = 0, ARITH_DIV_RHO = 1, ARITH_DIV_WENO = 2, ARITH_DIV_ROE = 3, ARITH_FREXP = 4, ARITH_DIV_STAR = 5, ARITH_DIV_ONE = 6 };
 
 // frexp exponent of a finite double from its bits: 0 for +-0; for normal x
 // the biased exponent - 1022; for subnormal x = mant * 2^-1074 the position
@@ -172,6 +172,21 @@ __global__ __launch_bounds__(256) void arith_selftest_kernel(int kind, unsigned 
             if (r1 & (1ull << 63)) a = -a;
             got = (double)frexp_exp(a);
             want = (double)frexp_exp_bits(a);
+        } else if (kind == ARITH_DIV_STAR) {
+            // HLL3's star quotients: denominators +-[2^-150, 2^150], nonzero
+            // numerators +-[2^-840, 2^600], each quotient within [2^-1000, 2^750]
+            b = draw_double(r1, -150, 150);
+            a = draw_double(r0, -840, 600);
+            if (r1 & (1ull << 62)) a = -a;
+            if (r1 & (1ull << 63)) b = -b;
+            got = div_shared(a, b, div_recip(b));
+            want = a / b;
+        } else if (kind == ARITH_DIV_ONE) {
+            // reciprocals of WENO2's smoothness terms, d in [2^-53, 2^348]
+            b = draw_double(r1, -53, 348);
+            a = 1.0;
+            got = div_one(b);
+            want = 1.0 / b;
         } else {
             // Roe denominators sqrt(rhoL) + sqrt(rhoR) in [2^-50, 2^51],
             // numerators zero or +-[2^-800, 2^600]
@@ -1155,7 +1170,7 @@ avh_status avh_stats_read(avh_stats* t, int save, int primitive, double* mean, d
 avh_status avh_arith_selftest(avh_ctx* ctx, int kind, uint64_t seed, int64_t n, int64_t* mismatches,
                               double* first_bad) {
     if (!ctx || !mismatches) return fail(AVH_EINVAL, "null argument");
-    if (kind < ARITH_SQRT || kind > ARITH_FREXP) return fail(AVH_EINVAL, "unknown self-test kind");
+    if (kind < ARITH_SQRT || kind > ARITH_DIV_ONE) return fail(AVH_EINVAL, "unknown self-test kind");
     if (n < 0) return fail(AVH_EINVAL, "negative operand count");
     AVH_HIP(hipSetDevice(ctx->device));
     void* mem = nullptr;

@@ -53,6 +53,11 @@ __device__ __forceinline__ double div_shared(double n, double d, double r) {
     const double q0 = n * r;
     return fma(-fma(d, q0, -n), r, q0);
 }
+// 1/d: div_shared with numerator 1, whose first product is r itself.
+__device__ __forceinline__ double div_one(double d) {
+    const double r = div_recip(d);
+    return fma(-fma(d, r, -1.0), r, r);
+}
 // lo <= n <= hi (false for zero, negative values, inf and NaN)
 __device__ __forceinline__ bool positive_within(double n, double lo, double hi) {
     return (n >= lo) & (n <= hi);
@@ -65,29 +70,41 @@ __device__ __forceinline__ int frexp_exp(double x) { return __builtin_amdgcn_fre
 
 // Arithmetic of an interface's reconstruction and flux.
 //   PlainOps   the compiler's sqrt and divide everywhere.
-//   SharedOps  sqrt_core, and shared reciprocals for the divisions by rho,
-//              by sqrt(rhoL) + sqrt(rhoR) and by the WENO weight sum; every
-//              operand is checked against the range where this gives the
-//              bits of PlainOps, and a failed check clears `ok`, after which
-//              the caller recomputes the interface with PlainOps.  The
-//              checks feed a flag instead of branching so that the interface
-//              stays one straight-line block for the scheduler.
-// The checks combine with non-short-circuit '&' so that they stay lane
-// masks and never turn into branches.
+//   SharedOps  sqrt_core and div_recip / div_shared wherever operands provably
+//              lie where these give PlainOps' bits; otherwise `ok` is cleared
+//              and the caller recomputes the interface with PlainOps.
+// What has to be checked for that is spread so that most of it is paid once
+// per cell and not once per interface (the stage is bound by the FP64 pipe,
+// and a check costs the same issue slot as an addition):
+//   per launch     gamma in [1 + 2^-20, 2^10]             (EQ::gamma_admitted)
+//   per cell       sum of |q_v| <= 2^85, momenta zero or at least 2^-600
+//                  (EQ::admitted, of every cell of the tile and its halo)
+//   per interface  each side: rho >= 2^-90, gamma p >= 2^-300, momenta zero or
+//                  at least 2^-390; HLL3: the two star denominators and two
+//                  star numerators; HLL: the denominator and the numerators.
+// Measured against per-interface checks of every operand and the compiler's
+// divisions for the WENO terms and star quotients (one MI355X, same box): 16
+// RK3 steps at 1024^2 2381 -> 2114 us, 4 at 256^3 13.93 -> 12.80 ms; about 55
+// fewer VALU instructions and 3 fewer quarter-rate reciprocals an interface.
+// The bounds the cell check leaves on the face values and everything formed
+// from them (faces are combinations of three cells with weights of magnitude
+// at most 11/6, so at most 2^87):
+//   u = m/rho: zero or in [2^-477, 2^177]; 0.5 m.m: zero or in [2^-781, 2^176]
+//   p <= 2^97, p >= 2^-310; sound speeds in [2^-194, 2^99] (squares likewise
+//   far inside sqrt_core's range); the two sides' sqrt(rho) in [2^-45, 2^44].
+// "Zero or at least" carries through sums because doubles of magnitude at
+// least 2^-k are multiples of 2^(-k-52), and so is any rounded sum of them:
+// a difference of such values is zero or at least 2^(-k-52).
+// The checks feed a flag instead of branching, and combine with
+// non-short-circuit '&', so that they stay lane masks and an interface stays
+// one straight-line block for the scheduler.
 struct PlainOps {
     static constexpr bool SHARED = false;
-    __device__ __forceinline__ static double sqrt_(double x, bool&) { return sqrt(x); }
-    // sqrt of an argument already known to lie in [2^-767, DBL_MAX] under
-    // SharedOps (a density that passed make_all_ops' check, or a quotient
-    // of checked operands)
     __device__ __forceinline__ static double sqrt_in_range(double x) { return sqrt(x); }
 };
 struct SharedOps {
     static constexpr bool SHARED = true;
-    __device__ __forceinline__ static double sqrt_(double x, bool& ok) {
-        ok = ok & (x >= 0x1p-767) & (x <= 0x1.fffffffffffffp+1023);
-        return sqrt_core(x);
-    }
+    // sqrt of an argument known to lie in [2^-767, DBL_MAX]
     __device__ __forceinline__ static double sqrt_in_range(double x) { return sqrt_core(x); }
 };
 template <bool SHARED>
@@ -122,6 +139,9 @@ struct BurgersEq {
         return !__builtin_isnan(u) && !__builtin_isinf(u);
     }
     __device__ __forceinline__ static bool obeys_fast(const double* q, double g) { return obeys(q, g); }
+    // no shared-reciprocal path: nothing to admit
+    __device__ __forceinline__ static bool gamma_admitted(double) { return true; }
+    __device__ __forceinline__ static bool admitted(const double*) { return true; }
 };
 
 template <int NSD_>
@@ -154,14 +174,30 @@ struct EulerEq {
         a.rinv = 0.0;
         return a;
     }
+    // The two checks SharedOps rests on beside its own per-interface ones
+    // (see SharedOps): the equation's gamma, once per launch, and a cell's
+    // conserved state, once per cell of a tile.  The sum of magnitudes bounds
+    // every variable, and is NaN or infinite when one of them is.  Momenta
+    // below 2^-600 (products with a WENO weight, at least 2^-404, could then
+    // be subnormal) are left to PlainOps, so that halving the weights instead
+    // of the sums (weno2_face) loses no bit.
+    __device__ __forceinline__ static bool gamma_admitted(double gamma) {
+        return positive_within(gamma, 0x1.00001p0, 0x1p10);
+    }
+    __device__ __forceinline__ static bool admitted(const double* q) {
+        double s = fabs(q[0]);
+        int emin = frexp_exp(q[1]);
+#pragma unroll
+        for (int v = 1; v < NV; ++v) s = s + fabs(q[v]);
+#pragma unroll
+        for (int c = 1; c < NSD_; ++c) emin = min(emin, frexp_exp(q[1 + c]));
+        return (s <= 0x1p85) & (emin >= -599);
+    }
     // make_all under OPS.  SharedOps forms one reciprocal of rho for the
-    // divisions by rho.  It checks that rho is in [2^-100, 2^100], that
-    // m.m <= 2^580 (so every |m[c]| <= 2^290 (1 + 2^-54); false for inf and
-    // NaN) and, by binary exponent, that every momentum is zero or
-    // |m[c]| >= 2^-433.  Then the numerators m[c] are zero or within
-    // [2^-433, 2^291] and 0.5*m.m is zero or within [2^-867, 2^579] (the
-    // computed sum of squares is at least its largest term, 2^-866 or more,
-    // and nothing underflows), so every quotient lies within [2^-967, 2^679].
+    // divisions by rho; rho in [2^-90, 2^87] and the momenta's bounds put
+    // every quotient in [2^-868, 2^266] or at zero.  0.5 m.m / rho is formed
+    // as 0.5 (m.m / rho), and subtracted in one fused step: halving is exact
+    // here, so neither changes a bit.
     template <class OPS>
     __device__ __forceinline__ static All make_all_ops(const double* q, double gamma, bool& ok) {
         if constexpr (!OPS::SHARED) {
@@ -176,9 +212,9 @@ struct EulerEq {
             int emin = frexp_exp(a.m[0]);
 #pragma unroll
             for (int c = 1; c < NSD_; ++c) emin = min(emin, frexp_exp(a.m[c]));
-            ok = ok & positive_within(a.rho, 0x1p-100, 0x1p100) & (mm <= 0x1p580) & (emin >= -432);
+            ok = ok & (a.rho >= 0x1p-90) & (emin >= -389);
             const double r = div_recip(a.rho);
-            const double ie = a.E - div_shared(0.5 * mm, a.rho, r);
+            const double ie = fma(-0.5, div_shared(mm, a.rho, r), a.E);
 #pragma unroll
             for (int c = 0; c < NSD_; ++c) a.u[c] = div_shared(a.m[c], a.rho, r);
             a.rinv = r;
@@ -187,39 +223,43 @@ struct EulerEq {
         }
     }
     // sqrt(g*p / rho) for a state a from make_all_ops<OPS> (the sound speed;
-    // n = g*p).  SharedOps checks that n lies in [2^-600, 2^600], so that the
-    // quotient lies in [2^-700, 2^700], inside sqrt_core's range, and that
-    // gamma lies in [2^-20, 2^20] (div_roe's bounds on p rest on it).
+    // n = g*p).  SharedOps checks n >= 2^-300 (p is then positive, and so
+    // bounded above by (gamma - 1) E): the quotient lies in [2^-387, 2^197].
     template <class OPS>
-    __device__ __forceinline__ static double sqrt_div_rho(double n, double g, const All& a, bool& ok) {
+    __device__ __forceinline__ static double sqrt_div_rho(double n, const All& a, bool& ok) {
         if constexpr (!OPS::SHARED) {
             return sqrt(n / a.rho);
         } else {
-            ok = ok & positive_within(n, 0x1p-600, 0x1p600) & positive_within(g, 0x1p-20, 0x1p20);
+            ok = ok & (n >= 0x1p-300);
             return sqrt_core(div_shared(n, a.rho, a.rinv));
         }
     }
     // (n1, n2) / (wl + wr) with wl, wr the square roots of the two sides'
-    // densities: n1 = uL wl + uR wr, n2 = wl pL + wr pR.  Under SharedOps the
-    // densities passed make_all_ops' check, so wl + wr is in [2^-50, 2^51],
-    // and the interface's other checks bound the numerators: |u| <= 2^391
-    // (make_all_ops) and, with gamma in [2^-20, 2^20], p in [2^-620, 2^620]
-    // on both sides (sqrt_div_rho), so |n1| <= 2^442 and n2, a sum of two
-    // positive terms, lies in [2^-671, 2^671].  Only n1 can be small: it is checked, by
-    // binary exponent, to be zero or at least 2^-800 in magnitude (it is
-    // finite when the other checks pass).
+    // densities: n1 = uL wl + uR wr, n2 = wl pL + wr pR.  Under SharedOps
+    // wl + wr is in [2^-44, 2^45], n1 zero or in [2^-574, 2^222] and n2, a sum
+    // of two positive terms, in [2^-355, 2^142].
     template <class OPS>
     __device__ __forceinline__ static void div_roe(double n1, double n2, double wl, double wr, double& q1,
-                                                   double& q2, bool& ok) {
+                                                   double& q2) {
         if constexpr (!OPS::SHARED) {
             q1 = n1 / (wl + wr);
             q2 = n2 / (wl + wr);
         } else {
-            ok = ok & (frexp_exp(n1) >= -799);
             const double den = wl + wr;
             const double r = div_recip(den);
             q1 = div_shared(n1, den, r);
             q2 = div_shared(n2, den, r);
+        }
+    }
+    // sqrt(g*p / rho) at the Roe pressure, which lies between the two sides'
+    // (up to rounding), and the mean density: under SharedOps the quotient is
+    // in [2^-389, 2^198] and needs no check of its own.
+    template <class OPS>
+    __device__ __forceinline__ static double sqrt_roe(double n, double rho) {
+        if constexpr (!OPS::SHARED) {
+            return sqrt(n / rho);
+        } else {
+            return sqrt_core(div_shared(n, rho, div_recip(rho)));
         }
     }
     // computePointFlux along DIR (Euler.hpp:172-181)
@@ -243,22 +283,22 @@ struct EulerEq {
         for (int c = 0; c < NSD_; ++c) ok = ok && !__builtin_isnan(a.u[c]) && !__builtin_isinf(a.u[c]);
         return ok && (a.rho > 0) && (a.p > 0);
     }
-    // obeys() with computeExtra's quotients through one reciprocal of rho
-    // (make_all_ops<SharedOps>) where the state lies in that range, which
-    // gives the same extra variables and so the same answer; any other
+    // obeys() decided without a division where the answer is plain: a state
+    // whose magnitudes sum to at most 2^85 has no NaN or infinity, rho >=
+    // 2^-90 makes every velocity and the kinetic energy finite, and the
+    // pressure is positive if E exceeds the kinetic energy by more than the
+    // rounding of either form: 2 rho E - m.m > 2^-40 (2 rho E), with 2 rho E >=
+    // 2^-900 so that nothing underflows, and gamma - 1 >= 2^-20.  Any other
     // state takes obeys() itself.
     __device__ __forceinline__ static bool obeys_fast(const double* q, double gamma) {
-        bool in_range = true;
-        const All a = make_all_ops<SharedOps>(q, gamma, in_range);
-        bool ok = true;
+        double s = fabs(q[0]);
 #pragma unroll
-        for (int i = 0; i < NV; ++i) ok = ok & !__builtin_isnan(q[i]) & !__builtin_isinf(q[i]);
-        ok = ok & !__builtin_isnan(a.p) & !__builtin_isinf(a.p);
-#pragma unroll
-        for (int c = 0; c < NSD_; ++c) ok = ok & !__builtin_isnan(a.u[c]) & !__builtin_isinf(a.u[c]);
-        ok = ok & (a.rho > 0) & (a.p > 0);
-        if (!in_range) ok = obeys(q, gamma);
-        return ok;
+        for (int v = 1; v < NV; ++v) s = s + fabs(q[v]);
+        const double e2 = 2 * q[0] * q[NSD_ + 1];
+        const double gap = e2 - dot(q + 1);
+        bool plain = (s <= 0x1p85) & (q[0] >= 0x1p-90) & (e2 >= 0x1p-900) & (gap > 0x1p-40 * e2);
+        plain = plain & gamma_admitted(gamma);
+        return plain ? true : obeys(q, gamma);
     }
 };
 
@@ -308,10 +348,10 @@ struct HLLFluxT {
         const double wr = OPS::sqrt_in_range(R.rho);
         const double rho = (L.rho + R.rho) / 2;
         double ud, p;
-        EQ::template div_roe<OPS>(L.u[DIR] * wl + R.u[DIR] * wr, L.p * wl + R.p * wr, wl, wr, ud, p, ok);
-        const double cs = OPS::sqrt_(g * p / rho, ok);
-        const double cfl = EQ::template sqrt_div_rho<OPS>(g * L.p, g, L, ok);
-        const double cfr = EQ::template sqrt_div_rho<OPS>(g * R.p, g, R, ok);
+        EQ::template div_roe<OPS>(L.u[DIR] * wl + R.u[DIR] * wr, L.p * wl + R.p * wr, wl, wr, ud, p);
+        const double cs = EQ::template sqrt_roe<OPS>(g * p, rho);
+        const double cfl = EQ::template sqrt_div_rho<OPS>(g * L.p, L, ok);
+        const double cfr = EQ::template sqrt_div_rho<OPS>(g * R.p, R, ok);
         const double sl = fmin(L.u[DIR] - cfl, ud - cs);
         const double sr = fmax(R.u[DIR] + cfr, ud + cs);
         double fl[NV], fr[NV], ul[NV], ur[NV];
@@ -328,10 +368,27 @@ struct HLLFluxT {
         ur[NSD + 1] = R.E;
         const double srsl = sr * sl;
         const double den = sr - sl;
+        double num[NV], mid[NV];
+#pragma unroll
+        for (int i = 0; i < NV; ++i) num[i] = sr * fl[i] - sl * fr[i] + srsl * (ur[i] - ul[i]);
+        if constexpr (OPS::SHARED) {
+            // one reciprocal for the NV quotients: den in [2^-100, 2^180] (the
+            // speeds are at most 2^179) and every numerator zero or in
+            // [2^-701, 2^456] put them in [2^-881, 2^556] or at zero
+            int emin = frexp_exp(num[0]);
+#pragma unroll
+            for (int i = 1; i < NV; ++i) emin = min(emin, frexp_exp(num[i]));
+            ok = ok & (den >= 0x1p-100) & (emin >= -700);
+            const double r = div_recip(den);
+#pragma unroll
+            for (int i = 0; i < NV; ++i) mid[i] = div_shared(num[i], den, r);
+        } else {
+#pragma unroll
+            for (int i = 0; i < NV; ++i) mid[i] = num[i] / den;
+        }
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
-            const double mid = (sr * fl[i] - sl * fr[i] + srsl * (ur[i] - ul[i])) / den;
-            double v = mid;
+            double v = mid[i];
             v = (sr < 0) ? fr[i] : v;
             v = (sl > 0) ? fl[i] : v;
             v = (sl == 0) ? 0.0 : v;
@@ -353,15 +410,33 @@ struct HLL3FluxT {
     // its point flux `fk`, formed from side k's values by point_flux's
     // operations (the same bits as selecting between both point fluxes).
     // The transverse momentum fluxes in the star velocities are m[c] * u[DIR].
-    template <int DIR, class EQ>
+    // SharedOps forms one reciprocal for the quotients over aa and one for
+    // those over s_m - s_k.  With |speeds| <= 2^179 and |u - speed| zero or at
+    // least 2^-477 (a speed is a multiple of 2^-248, and u - 0 is u):
+    //   -aa in [2^-150, 2^80] (aa < 0 in any flow; checked), numerators zero or
+    //   in [2^-919, 2^268]: quotients in [2^-999, 2^418] or zero.  Both are
+    //   negated, because div_shared keeps the sign of a zero for a positive
+    //   denominator.
+    //   |s_m - s_k| in [2^-100, 2^150], numerators checked at least 2^-700 and
+    //   2^-800 in magnitude and at most 2^630: quotients in [2^-950, 2^730].
+    template <class OPS, int DIR, class EQ>
     __device__ __forceinline__ static void star_side(const typename EQ::All& L, const typename EQ::All& R, double sl,
-                                                     double sr, double& sk, double* mid, double* uc, double* fk) {
+                                                     double sr, double& sk, double* mid, double* uc, double* fk,
+                                                     bool& ok) {
         constexpr int NSD = EQ::NSD;
         const double pl = L.p, pr = R.p;
         const double udl = L.u[DIR] - sl;
         const double udr = R.u[DIR] - sr;
         const double aa = udr * R.rho - udl * L.rho;
-        const double sm = (R.m[DIR] * udr - L.m[DIR] * udl + pr - pl) / aa;
+        const double nm = R.m[DIR] * udr - L.m[DIR] * udl + pr - pl;
+        double ra = 0.0, sm;
+        if constexpr (OPS::SHARED) {
+            ok = ok & positive_within(-aa, 0x1p-150, 0x1p80);
+            ra = div_recip(-aa);
+            sm = div_shared(-nm, -aa, ra);
+        } else {
+            sm = nm / aa;
+        }
 
         const bool left = sm >= 0;
         const double rk = left ? L.rho : R.rho;
@@ -371,17 +446,32 @@ struct HLL3FluxT {
         const double uk = left ? L.u[DIR] : R.u[DIR];
         const double ek = left ? L.E : R.E;
 
-        mid[0] = rk * udk / (sm - sk);
+        const double ds = sm - sk;
+        const double n0 = rk * udk;
+        const double pm = pk + rk * (uk - sm) * udk;
+        const double ne = udk * ek + pk * uk - pm * sm;
+        if constexpr (OPS::SHARED) {
+            ok = ok & (fabs(ds) >= 0x1p-100) & (fabs(ds) <= 0x1p150) & (fabs(n0) >= 0x1p-700) &
+                 (fabs(ne) >= 0x1p-800);
+            const double rs = div_recip(ds);
+            mid[0] = div_shared(n0, ds, rs);
+            mid[NSD + 1] = div_shared(ne, ds, rs);
+        } else {
+            mid[0] = n0 / ds;
+            mid[NSD + 1] = ne / ds;
+        }
 #pragma unroll
         for (int c = 0; c < NSD; ++c) {
             // us = (fR.m - fL.m - sR*mR + sL*mL)/aa with us[DIR] = sm
-            const double us = (c == DIR) ? sm
-                                         : (R.m[c] * R.u[DIR] - L.m[c] * L.u[DIR] - R.m[c] * sr + L.m[c] * sl) / aa;
+            double us = sm;
+            if (c != DIR) {
+                const double nt = R.m[c] * R.u[DIR] - L.m[c] * L.u[DIR] - R.m[c] * sr + L.m[c] * sl;
+                if constexpr (OPS::SHARED) us = div_shared(-nt, -aa, ra);
+                else us = nt / aa;
+            }
             mid[1 + c] = us * mid[0];
             uc[1 + c] = left ? L.m[c] : R.m[c];
         }
-        const double pm = pk + rk * (uk - sm) * udk;
-        mid[NSD + 1] = (udk * ek + pk * uk - pm * sm) / (sm - sk);
         uc[0] = rk;
         uc[NSD + 1] = ek;
         fk[0] = uc[1 + DIR];
@@ -406,13 +496,25 @@ struct HLL3FluxT {
         const double wr = OPS::sqrt_in_range(R.rho);
         const double rho = (L.rho + R.rho) / 2;
         double ud, p;
-        EQ::template div_roe<OPS>(L.u[DIR] * wl + R.u[DIR] * wr, wl * L.p + wr * R.p, wl, wr, ud, p, ok);
-        const double cfl = EQ::template sqrt_div_rho<OPS>(g * L.p, g, L, ok);
-        const double cfr = EQ::template sqrt_div_rho<OPS>(g * R.p, g, R, ok);
-        const double correct = 0.5 * fmax(0.0, L.u[DIR] - R.u[DIR]);
-        const double cs = OPS::sqrt_(g * p / rho, ok);
-        const double sl = fmin(L.u[DIR] + correct - cfl, ud - cs);
-        const double sr = fmax(R.u[DIR] - correct + cfr, ud + cs);
+        EQ::template div_roe<OPS>(L.u[DIR] * wl + R.u[DIR] * wr, wl * L.p + wr * R.p, wl, wr, ud, p);
+        const double cfl = EQ::template sqrt_div_rho<OPS>(g * L.p, L, ok);
+        const double cfr = EQ::template sqrt_div_rho<OPS>(g * R.p, R, ok);
+        // correct = jump/2; halving is exact but for subnormal jumps, which a
+        // velocity sum of SharedOps' range does not notice, so there it is
+        // fused into the sums
+        const double jump = fmax(0.0, L.u[DIR] - R.u[DIR]);
+        double ul, ur;
+        if constexpr (OPS::SHARED) {
+            ul = fma(0.5, jump, L.u[DIR]);
+            ur = fma(-0.5, jump, R.u[DIR]);
+        } else {
+            const double correct = 0.5 * jump;
+            ul = L.u[DIR] + correct;
+            ur = R.u[DIR] - correct;
+        }
+        const double cs = EQ::template sqrt_roe<OPS>(g * p, rho);
+        const double sl = fmin(ul - cfl, ud - cs);
+        const double sr = fmax(ur + cfr, ud + cs);
 
         // subsonic interfaces (sL < 0 < sR) take the star branch.  Under
         // SharedOps a wavefront that is subsonic throughout skips the other
@@ -421,7 +523,7 @@ struct HLL3FluxT {
         // formed first, as the general branch selects between them.
         const bool star = !(sl == 0) && !(sl > 0) && !(sr < 0);
         double sk, mid[NV], uc[NV], fk[NV];
-        star_side<DIR, EQ>(L, R, sl, sr, sk, mid, uc, fk);
+        star_side<OPS, DIR, EQ>(L, R, sl, sr, sk, mid, uc, fk, ok);
         if (__all(star)) {
 #pragma unroll
             for (int i = 0; i < NV; ++i) F[i] = fk[i] + sk * (mid[i] - uc[i]);
@@ -474,31 +576,54 @@ struct ReconTraits<RECON_ENO3> {
 // WENO2 (alsfvm/include/alsfvm/reconstruction/WENO2.hpp:31-95; epsilon 1e-8,
 // WENOCoefficients.hpp:21).  RIGHT selects the value at the cell's right face
 // (the reference's `right` volume), otherwise the left face.
-// Under SharedOps the two weights share the reciprocal of a0 + a1, checked
-// to need a0, a1 >= 2^-400: both are at most 2/(3*eps^2) < 2^53, so the
-// numerators, the denominator and the quotients (within [2^-454, 1]) are in
-// the range where div_shared equals the division.
-template <class OPS>
-__device__ __forceinline__ void weno2_weights(double a0, double a1, double& w0, double& w1, bool& ok) {
-    if constexpr (OPS::SHARED) {
-        ok = ok & (a0 >= 0x1p-400) & (a1 >= 0x1p-400);
-        const double den = a0 + a1;
-        const double r = div_recip(den);
-        w0 = div_shared(a0, den, r);
-        w1 = div_shared(a1, den, r);
-    } else {
-        w0 = a0 / (a0 + a1);
-        w1 = a1 / (a0 + a1);
-    }
+__device__ __forceinline__ void weno2_weights(double a0, double a1, double& w0, double& w1) {
+    w0 = a0 / (a0 + a1);
+    w1 = a1 / (a0 + a1);
+}
+
+// Under SharedOps a face's weights come from the reciprocals r = 1/d of the
+// smoothness terms d = 3 (eps + b)^2 of the differences ahead (r0) and behind
+// (r1), so 2/d is 2r (doubling is exact) and one reciprocal serves both
+// quotients of a face.  The weights are formed halved: the 0.5 of the face
+// value is a power of two, so it commutes with the rounding of every product
+// and sum (no product is subnormal unless the face is below 2^-390, which
+// the interface check excludes; EQ::admitted).  For the right face
+// 0.5 * 2 r0 / (2 r0 + r1) is r0 / (2 r0 + r1): no multiplication at all.
+// Admitted cells give d in [2^-53, 2^348]: r, the sum, and the quotients
+// (at least 2^-404) need no check.
+__device__ __forceinline__ double weno2_recip(double diff) {
+    const double e = 1e-8 + diff * diff;
+    return div_one(3 * e * e);
+}
+template <bool RIGHT>
+__device__ __forceinline__ void weno2_half_weights(double r0, double r1, double& h0, double& h1) {
+    const double den = RIGHT ? fma(2.0, r0, r1) : fma(2.0, r1, r0);
+    const double r = div_recip(den);
+    h0 = div_shared(r0, den, r);
+    h1 = div_shared(r1, den, r);
+    if (RIGHT) h1 = 0.5 * h1;
+    else h0 = 0.5 * h0;
 }
 
 template <int NV, bool RIGHT, class OPS>
-__device__ __forceinline__ void weno2_face(const double* s, int vs, int i, int sd, double* out, bool& ok) {
+__device__ __forceinline__ void weno2_face(const double* s, int vs, int i, int sd, double* out) {
     const double eps = 1e-8;
     const double w0 = s[i];
     const double dp = s[i + sd] - w0;
-    const double b0 = dp * dp;
     const double dm = w0 - s[i - sd];
+    if constexpr (OPS::SHARED) {
+        double h0, h1;
+        weno2_half_weights<RIGHT>(weno2_recip(dp), weno2_recip(dm), h0, h1);
+        const double hc = RIGHT ? 3 * h1 + h0 : 3 * h0 + h1;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const double* u = s + v * vs;
+            out[v] = RIGHT ? h0 * u[i + sd] + hc * u[i] - h1 * u[i - sd]
+                           : h1 * u[i - sd] + hc * u[i] - h0 * u[i + sd];
+        }
+        return;
+    }
+    const double b0 = dp * dp;
     const double b1 = dm * dm;
     const double d0 = 3 * (eps + b0) * (eps + b0);
     const double d1 = 3 * (eps + b1) * (eps + b1);
@@ -506,7 +631,7 @@ __device__ __forceinline__ void weno2_face(const double* s, int vs, int i, int s
         const double a0 = 2 / d0;
         const double a1 = 1 / d1;
         double w0r, w1r;
-        weno2_weights<OPS>(a0, a1, w0r, w1r, ok);
+        weno2_weights(a0, a1, w0r, w1r);
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
             const double* u = s + v * vs;
@@ -516,7 +641,7 @@ __device__ __forceinline__ void weno2_face(const double* s, int vs, int i, int s
         const double a0 = 1 / d0;
         const double a1 = 2 / d1;
         double w0l, w1l;
-        weno2_weights<OPS>(a0, a1, w0l, w1l, ok);
+        weno2_weights(a0, a1, w0l, w1l);
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
             const double* u = s + v * vs;
@@ -582,23 +707,17 @@ __device__ __forceinline__ void eno_face(const double* s, int vs, int i, int sd,
 }
 
 template <int RECON, int NV, bool RIGHT, class OPS>
-__device__ __forceinline__ void recon_face_ops(const double* s, int vs, int i, int sd, double* out, bool& ok) {
+__device__ __forceinline__ void recon_face_ops(const double* s, int vs, int i, int sd, double* out) {
     if (RECON == RECON_NONE) {
 #pragma unroll
         for (int v = 0; v < NV; ++v) out[v] = s[v * vs + i];
     } else if (RECON == RECON_WENO2) {
-        weno2_face<NV, RIGHT, OPS>(s, vs, i, sd, out, ok);
+        weno2_face<NV, RIGHT, OPS>(s, vs, i, sd, out);
     } else if (RECON == RECON_ENO2) {
         eno_face<2, NV, RIGHT>(s, vs, i, sd, out);
     } else {
         eno_face<3, NV, RIGHT>(s, vs, i, sd, out);
     }
-}
-
-template <int RECON, int NV, bool RIGHT>
-__device__ __forceinline__ void recon_face(const double* s, int vs, int i, int sd, double* out) {
-    bool ok = true;
-    recon_face_ops<RECON, NV, RIGHT, PlainOps>(s, vs, i, sd, out, ok);
 }
 
 }  // namespace avh

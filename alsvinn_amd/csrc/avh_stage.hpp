@@ -276,13 +276,14 @@ struct StageKernel {
     }
 
     // reconstruct both sides of the interface between cell ia and ia + SD
-    // (LDS indices) and evaluate the numerical flux under OPS
+    // (LDS indices) and evaluate the numerical flux under OPS; `ok` comes in
+    // as whether the cells are admitted to SharedOps
     template <class OPS, int DIR>
     __device__ __forceinline__ static double interface(const double* su, int ia, int SD, double gamma,
                                                        double* F, bool& ok) {
         double qa[NV], qb[NV];
-        recon_face_ops<RECON, NV, true, OPS>(su, LT, ia, SD, qa, ok);        // right face of a
-        recon_face_ops<RECON, NV, false, OPS>(su, LT, ia + SD, SD, qb, ok);  // left face of b
+        recon_face_ops<RECON, NV, true, OPS>(su, LT, ia, SD, qa);        // right face of a
+        recon_face_ops<RECON, NV, false, OPS>(su, LT, ia + SD, SD, qb);  // left face of b
         const typename EQ::All aL = EQ::template make_all_ops<OPS>(qa, gamma, ok);
         const typename EQ::All aR = EQ::template make_all_ops<OPS>(qb, gamma, ok);
         return FLUX::template flux_ops<OPS, DIR, EQ>(aL, aR, gamma, F, ok);
@@ -321,9 +322,10 @@ struct StageKernel {
     // interface with shared reciprocals (SharedOps); the interfaces whose
     // operands fall outside the range where that is exact are redone with
     // PlainOps in a second loop, after the first one's registers are free.
+    // `adm`: every cell of the tile and its halo is admitted to SharedOps.
     template <int DIR>
     __device__ __forceinline__ static void flux_pass(const double* su, double* sf, int ox, int oy, int oz,
-                                                     const int* n, double gamma, double& ws) {
+                                                     const int* n, double gamma, bool adm, double& ws) {
         constexpr int NI = DIR == 0 ? NI_X : (DIR == 1 ? NI_Y : NI_Z);
         constexpr int SD = DIR == 0 ? 1 : (DIR == 1 ? LX : LX * LY);
         static_assert((NI + NT - 1) / NT <= 32, "one redo bit per iteration");
@@ -334,7 +336,7 @@ struct StageKernel {
             int ia;
             if (!interface_cell<DIR>(it, ox, oy, oz, n, ia)) continue;
             double F[NV];
-            bool ok = true;
+            bool ok = adm;
             const double w = interface<Ops, DIR>(su, ia, SD, gamma, F, ok);
             if (ok) {
                 ws = ws_max(ws, w);
@@ -399,6 +401,7 @@ struct StageKernel {
     __device__ static void run_tile(const StageParams& P, const unsigned int tile, const VolumeParams* V = nullptr) {
         __shared__ double lds[NV * LT + NV * NI_MAX];
         __shared__ double s_ws[3][NT / 64];
+        __shared__ int s_adm[NT / 64];
         double* su = lds;
         double* sf = lds + NV * LT;
 
@@ -463,7 +466,22 @@ struct StageKernel {
 #pragma unroll
             for (int v = 0; v < NV; ++v) su[v * LT + p] = sv[k][v];
         }
+        // whether SharedOps may run on this tile: one vote per wavefront
+        // through LDS, read by all after the barrier that publishes the tile
+        bool adm = EQ::gamma_admitted(P.gamma);
+        if constexpr (FLUX::FAST) {
+#pragma unroll
+            for (int k = 0; k < SPT; ++k) adm = adm & EQ::admitted(sv[k]);
+            const bool all = __all(adm);
+            if ((threadIdx.x & 63) == 0) s_adm[threadIdx.x >> 6] = all;
+        }
         __syncthreads();
+        if constexpr (FLUX::FAST) {
+            int all = s_adm[0];
+#pragma unroll
+            for (int i = 1; i < NT / 64; ++i) all = all & s_adm[i];
+            adm = all != 0;
+        }
 
         double acc[CPT][NV];
 #pragma unroll
@@ -473,18 +491,18 @@ struct StageKernel {
         double ws[3] = {0.0, 0.0, 0.0};
 
         // 2./3. per direction: interface fluxes into LDS, then accumulate
-        flux_pass<0>(su, sf, ox, oy, oz, P.n, P.gamma, ws[0]);
+        flux_pass<0>(su, sf, ox, oy, oz, P.n, P.gamma, adm, ws[0]);
         __syncthreads();
         accumulate<0>(sf, acc);
         if (DIM >= 2) {
             __syncthreads();
-            flux_pass<DIM >= 2 ? 1 : 0>(su, sf, ox, oy, oz, P.n, P.gamma, ws[1]);
+            flux_pass<DIM >= 2 ? 1 : 0>(su, sf, ox, oy, oz, P.n, P.gamma, adm, ws[1]);
             __syncthreads();
             accumulate<DIM >= 2 ? 1 : 0>(sf, acc);
         }
         if (DIM >= 3) {
             __syncthreads();
-            flux_pass<DIM >= 3 ? 2 : 0>(su, sf, ox, oy, oz, P.n, P.gamma, ws[2]);
+            flux_pass<DIM >= 3 ? 2 : 0>(su, sf, ox, oy, oz, P.n, P.gamma, adm, ws[2]);
             __syncthreads();
             accumulate<DIM >= 3 ? 2 : 0>(sf, acc);
         }

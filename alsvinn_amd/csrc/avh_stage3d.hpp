@@ -23,10 +23,9 @@ namespace avh {
 
 // ENO / WENO2 / none on a register window: u[i][v], stencil centre `c`
 // (compile-time), unit stride.  Selects replace ENO's data-dependent index.
-// OPS as in recon_face_ops (the WENO2 weights may share a reciprocal).
-template <int RECON, int NV, bool RIGHT, int WZ, class OPS = PlainOps>
-__device__ __forceinline__ void recon_face_reg(const double (&u)[WZ][NV], const int c, double* out,
-                                               bool& ok) {
+// The plain arithmetic; recon_faces_reg has the SharedOps form of WENO2.
+template <int RECON, int NV, bool RIGHT, int WZ>
+__device__ __forceinline__ void recon_face_reg(const double (&u)[WZ][NV], const int c, double* out) {
     if (RECON == RECON_NONE) {
 #pragma unroll
         for (int v = 0; v < NV; ++v) out[v] = u[c][v];
@@ -43,7 +42,7 @@ __device__ __forceinline__ void recon_face_reg(const double (&u)[WZ][NV], const 
             const double a0 = 2 / d0;
             const double a1 = 1 / d1;
             double w0r, w1r;
-            weno2_weights<OPS>(a0, a1, w0r, w1r, ok);
+            weno2_weights(a0, a1, w0r, w1r);
 #pragma unroll
             for (int v = 0; v < NV; ++v)
                 out[v] = 0.5 * (w0r * u[c + 1][v] + (3 * w1r + w0r) * u[c][v] - w1r * u[c - 1][v]);
@@ -51,7 +50,7 @@ __device__ __forceinline__ void recon_face_reg(const double (&u)[WZ][NV], const 
             const double a0 = 1 / d0;
             const double a1 = 2 / d1;
             double w0l, w1l;
-            weno2_weights<OPS>(a0, a1, w0l, w1l, ok);
+            weno2_weights(a0, a1, w0l, w1l);
 #pragma unroll
             for (int v = 0; v < NV; ++v)
                 out[v] = 0.5 * (w1l * u[c - 1][v] + (3 * w0l + w1l) * u[c][v] - w0l * u[c + 1][v]);
@@ -92,43 +91,30 @@ __device__ __forceinline__ void recon_face_reg(const double (&u)[WZ][NV], const 
     }
 }
 
-template <int RECON, int NV, bool RIGHT, int WZ>
-__device__ __forceinline__ void recon_face_reg(const double (&u)[WZ][NV], const int c, double* out) {
-    bool ok = true;
-    recon_face_reg<RECON, NV, RIGHT, WZ, PlainOps>(u, c, out, ok);
-}
-
-// Both faces of the window's cell c.  WENO2 under SharedOps divides once per
-// denominator: the left face takes a0 = 1/d0, a1 = 2/d1 and the right face
-// a0 = 2/d0, a1 = 1/d1, and 2/d is formed as 2 * (1/d).  Doubling is exact
-// and commutes with rounding while 2/d stays normal; the weight checks
-// (every a0, a1 >= 2^-400, so 1/d0, 1/d1 >= 2^-400 and d0, d1 <= 2^400) hold
-// only there, so a pair that passes them has the bits of the two divisions.
+// Both faces of the window's cell c.  WENO2 under SharedOps: rb comes in as
+// 1/d of the difference behind the cell and goes out as 1/d of the one ahead
+// (weno2_recip), which is the one behind the next cell of the march, so each
+// difference is inverted once.
 template <int RECON, int NV, int WZ, class OPS>
-__device__ __forceinline__ void recon_faces_reg(const double (&u)[WZ][NV], const int c, double* outl,
-                                                double* outr, bool& ok) {
+__device__ __forceinline__ void recon_faces_reg(const double (&u)[WZ][NV], const int c, double& rb, double* outl,
+                                                double* outr) {
     if constexpr (RECON == RECON_WENO2 && OPS::SHARED) {
-        const double eps = 1e-8;
-        const double w0 = u[c][0];
-        const double dp = u[c + 1][0] - w0;
-        const double b0 = dp * dp;
-        const double dm = w0 - u[c - 1][0];
-        const double b1 = dm * dm;
-        const double d0 = 3 * (eps + b0) * (eps + b0);
-        const double d1 = 3 * (eps + b1) * (eps + b1);
-        const double r0 = 1 / d0;
-        const double r1 = 1 / d1;
-        double w0l, w1l, w0r, w1r;
-        weno2_weights<OPS>(r0, 2 * r1, w0l, w1l, ok);
-        weno2_weights<OPS>(2 * r0, r1, w0r, w1r, ok);
+        const double r1 = rb;
+        const double r0 = weno2_recip(u[c + 1][0] - u[c][0]);
+        double h0l, h1l, h0r, h1r;
+        weno2_half_weights<false>(r0, r1, h0l, h1l);
+        weno2_half_weights<true>(r0, r1, h0r, h1r);
+        const double hl = 3 * h0l + h1l;
+        const double hr = 3 * h1r + h0r;
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
-            outl[v] = 0.5 * (w1l * u[c - 1][v] + (3 * w0l + w1l) * u[c][v] - w0l * u[c + 1][v]);
-            outr[v] = 0.5 * (w0r * u[c + 1][v] + (3 * w1r + w0r) * u[c][v] - w1r * u[c - 1][v]);
+            outl[v] = h1l * u[c - 1][v] + hl * u[c][v] - h0l * u[c + 1][v];
+            outr[v] = h0r * u[c + 1][v] + hr * u[c][v] - h1r * u[c - 1][v];
         }
+        rb = r0;
     } else {
-        recon_face_reg<RECON, NV, false, WZ, OPS>(u, c, outl, ok);
-        recon_face_reg<RECON, NV, true, WZ, OPS>(u, c, outr, ok);
+        recon_face_reg<RECON, NV, false, WZ>(u, c, outl);
+        recon_face_reg<RECON, NV, true, WZ>(u, c, outr);
     }
 }
 
@@ -209,8 +195,8 @@ struct MarchKernel3 {
     __device__ __forceinline__ static double plane_interface(const double* sp, int ia, int SD, double gamma,
                                                              double* F, bool& ok) {
         double qa[NV], qb[NV];
-        recon_face_ops<RECON, NV, true, OPS>(sp, LP, ia, SD, qa, ok);
-        recon_face_ops<RECON, NV, false, OPS>(sp, LP, ia + SD, SD, qb, ok);
+        recon_face_ops<RECON, NV, true, OPS>(sp, LP, ia, SD, qa);
+        recon_face_ops<RECON, NV, false, OPS>(sp, LP, ia + SD, SD, qb);
         const typename EQ::All aL = EQ::template make_all_ops<OPS>(qa, gamma, ok);
         const typename EQ::All aR = EQ::template make_all_ops<OPS>(qb, gamma, ok);
         return FLUX::template flux_ops<OPS, DIR, EQ>(aL, aR, gamma, F, ok);
@@ -233,9 +219,10 @@ struct MarchKernel3 {
     // A FAST flux evaluates each interface with SharedOps and redoes those
     // whose operands leave the guarded range with PlainOps (as the 2D stage
     // kernel's flux_pass); otherwise PlainOps throughout.
+    // `adm`: every cell of the plane tile is admitted to SharedOps.
     template <int DIR>
     __device__ __forceinline__ static void plane_pass(const double* sp, double* sf, int ox, int oy, const int* n,
-                                                      double gamma, double& ws) {
+                                                      double gamma, bool adm, double& ws) {
         constexpr int NI = DIR == 0 ? NIX : NIY;
         constexpr int SD = DIR == 0 ? 1 : LXP;
         static_assert((NI + NT - 1) / NT <= 32, "one redo bit per turn");
@@ -246,7 +233,7 @@ struct MarchKernel3 {
             int ia;
             if (!plane_item<DIR>(it, ox, oy, n, ia)) continue;
             double F[NV];
-            bool ok = true;
+            bool ok = adm;
             const double w = plane_interface<Ops, DIR>(sp, ia, SD, gamma, F, ok);
             if (ok) ws = ws_max(ws, w);
             else redo |= 1u << m;
@@ -274,6 +261,7 @@ struct MarchKernel3 {
         __shared__ double sf_y[TWO_BARRIERS ? NV * NIMAX : 1];
         __shared__ double s_ws[3][NT / 64];
         __shared__ double su0[U0RING ? RING * NV * NC : 1];
+        __shared__ int s_adm[NBUF][NT / 64];
         double* const sfx = sf;
         double* const sfy = TWO_BARRIERS ? sf_y : sf;
 
@@ -304,6 +292,11 @@ struct MarchKernel3 {
         double ws[3] = {0.0, 0.0, 0.0};
         double w[WZ][NV];
         double rprev[NV], fprev[NV];
+        double rb = 0.0;  // 1/d of the difference behind the next z-reconstructed cell (WENO2)
+        // whether SharedOps may run on this column: every cell its window has
+        // held is admitted (a column that meets one that is not stays with
+        // PlainOps to the end of the chunk)
+        bool col_adm = EQ::gamma_admitted(P.gamma);
 #pragma unroll
         for (int i = 0; i < WZ; ++i)
 #pragma unroll
@@ -331,6 +324,10 @@ struct MarchKernel3 {
                 for (int v = 0; v < NV; ++v) w[i][v] = w[i + 1][v];
             fetch(P, otf, s, gidx(gxc, gyc, bc_map(z0 + HW, n2, P.bc), n0, n1), w[WZ - 1],
                   ring ? slot(z0 + HW) : nullptr);
+            if constexpr (FLUX::FAST) {
+#pragma unroll
+                for (int i = 0; i < WZ; ++i) col_adm = col_adm & EQ::admitted(w[i]);
+            }
             if (col_ok) {
                 double l0[NV];
                 recon_face_reg<RECON, NV, false, WZ>(w, HW, l0);
@@ -346,6 +343,10 @@ struct MarchKernel3 {
                 for (int v = 0; v < NV; ++v) w[i][v] = w[i + 1][v];
             fetch(P, otf, s, gidx(gxc, gyc, bc_map(z0 + 1 + HW, n2, P.bc), n0, n1), w[WZ - 1],
                   ring ? slot(z0 + 1 + HW) : nullptr);
+            if constexpr (FLUX::FAST) {
+                col_adm = col_adm & EQ::admitted(w[WZ - 1]);
+                if (RECON == RECON_WENO2) rb = weno2_recip(w[HW][0] - w[HW - 1][0]);
+            }
         }
 
         bool bad = false;
@@ -430,18 +431,33 @@ struct MarchKernel3 {
 #pragma unroll
                 for (int v = 0; v < NV; ++v) sp[v * LP + (cy + G) * LXP + (cx + G)] = w[HW - 1][v];
             }
+            bool adm = col_adm;
 #pragma unroll
             for (int j = 0; j < HPT; ++j) {
                 if (has_halo[j]) {
+                    double q[NV];
 #pragma unroll
                     for (int v = 0; v < NV; ++v) {
-                        double val = pin[j][v];
-                        if (otf) val = val * s + pu0[j][v];
-                        sp[v * LP + halo_lds[j]] = val;
+                        q[v] = pin[j][v];
+                        if (otf) q[v] = q[v] * s + pu0[j][v];
+                        sp[v * LP + halo_lds[j]] = q[v];
                     }
+                    if constexpr (FLUX::FAST) adm = adm & EQ::admitted(q);
                 }
             }
+            // one vote per wavefront through LDS, read by all after the barrier
+            int* const va = s_adm[TWO_BARRIERS ? ((k - z0) & 1) : 0];
+            if constexpr (FLUX::FAST) {
+                const bool all = __all(adm);
+                if ((threadIdx.x & 63) == 0) va[threadIdx.x >> 6] = all;
+            }
             __syncthreads();
+            if constexpr (FLUX::FAST) {
+                int all = va[0];
+#pragma unroll
+                for (int i = 1; i < NT / 64; ++i) all = all & va[i];
+                adm = all != 0;
+            }
             if (k + 1 < z1) {
                 AVH_PREFETCH_RING(k + 1)
             }
@@ -459,8 +475,8 @@ struct MarchKernel3 {
                 if (col_ok) {
                     typedef typename OpsFor<FLUX::FAST>::type Ops;
                     double lz[NV];
-                    bool ok = true;
-                    recon_faces_reg<RECON, NV, WZ, Ops>(w, HW, lz, rnext, ok);
+                    bool ok = col_adm;
+                    recon_faces_reg<RECON, NV, WZ, Ops>(w, HW, rb, lz, rnext);
                     typename EQ::All aL = EQ::template make_all_ops<Ops>(rprev, P.gamma, ok);
                     typename EQ::All aR = EQ::template make_all_ops<Ops>(lz, P.gamma, ok);
                     double wz = FLUX::template flux_ops<Ops, 2, EQ>(aL, aR, P.gamma, fz, ok);
@@ -495,18 +511,18 @@ struct MarchKernel3 {
             if constexpr (TWO_BARRIERS) {
                 // every flux of the plane, then one barrier, then the sums in
                 // the reference's x, y, z order
-                plane_pass<0>(sp, sfx, ox, oy, P.n, P.gamma, ws[0]);
-                plane_pass<1>(sp, sfy, ox, oy, P.n, P.gamma, ws[1]);
+                plane_pass<0>(sp, sfx, ox, oy, P.n, P.gamma, adm, ws[0]);
+                plane_pass<1>(sp, sfy, ox, oy, P.n, P.gamma, adm, ws[1]);
                 z_flux();
                 __syncthreads();
                 add_x();
                 add_y();
             } else {
-                plane_pass<0>(sp, sfx, ox, oy, P.n, P.gamma, ws[0]);
+                plane_pass<0>(sp, sfx, ox, oy, P.n, P.gamma, adm, ws[0]);
                 __syncthreads();
                 add_x();
                 __syncthreads();
-                plane_pass<1>(sp, sfy, ox, oy, P.n, P.gamma, ws[1]);
+                plane_pass<1>(sp, sfy, ox, oy, P.n, P.gamma, adm, ws[1]);
                 __syncthreads();
                 add_y();
                 z_flux();
@@ -576,6 +592,7 @@ struct MarchKernel3 {
                 }
 #pragma unroll
                 for (int v = 0; v < NV; ++v) w[WZ - 1][v] = otf ? cin[v] * s + cu0[v] : cin[v];
+                if constexpr (FLUX::FAST) col_adm = col_adm & EQ::admitted(w[WZ - 1]);
             }
             // one plane buffer: every thread must be done reading it (and the
             // flux buffer) before the next plane is written

@@ -236,42 +236,35 @@ struct Launchers {
     VolumeLauncher volume = nullptr;
 };
 
-template <class EQ, class FLUX, int DIM>
-Launchers pick_recon(int recon) {
+template <class EQ, int RECON, class FLUX, int DIM>
+Launchers launchers_of() {
     Launchers L;
-    switch (recon) {
-    case RECON_NONE:
-        L.stage = &launch_stage<EQ, RECON_NONE, FLUX, DIM>;
-        L.batch = &launch_batch_stage<EQ, RECON_NONE, FLUX, DIM>;
-        L.volume = &launch_volume_stage<EQ, RECON_NONE, FLUX, DIM>;
-        break;
-    case RECON_WENO2:
-        L.stage = &launch_stage<EQ, RECON_WENO2, FLUX, DIM>;
-        L.batch = &launch_batch_stage<EQ, RECON_WENO2, FLUX, DIM>;
-        L.volume = &launch_volume_stage<EQ, RECON_WENO2, FLUX, DIM>;
-        break;
-    case RECON_ENO2:
-        L.stage = &launch_stage<EQ, RECON_ENO2, FLUX, DIM>;
-        L.batch = &launch_batch_stage<EQ, RECON_ENO2, FLUX, DIM>;
-        L.volume = &launch_volume_stage<EQ, RECON_ENO2, FLUX, DIM>;
-        break;
-    case RECON_ENO3:
-        L.stage = &launch_stage<EQ, RECON_ENO3, FLUX, DIM>;
-        L.batch = &launch_batch_stage<EQ, RECON_ENO3, FLUX, DIM>;
-        L.volume = &launch_volume_stage<EQ, RECON_ENO3, FLUX, DIM>;
-        break;
-    }
-    if (DIM == 3) L.batch = nullptr;
+    L.stage = &launch_stage<EQ, RECON, FLUX, DIM>;
+    if (DIM < 3) L.batch = &launch_batch_stage<EQ, RECON, FLUX, DIM>;
+    L.volume = &launch_volume_stage<EQ, RECON, FLUX, DIM>;
     return L;
 }
 
-template <class EQ, class FLUX>
+template <class EQ, class FLUX, int DIM>
+Launchers pick_recon(int recon) {
+    switch (recon) {
+    case RECON_NONE: return launchers_of<EQ, RECON_NONE, FLUX, DIM>();
+    case RECON_WENO2: return launchers_of<EQ, RECON_WENO2, FLUX, DIM>();
+    case RECON_ENO2: return launchers_of<EQ, RECON_ENO2, FLUX, DIM>();
+    case RECON_ENO3: return launchers_of<EQ, RECON_ENO3, FLUX, DIM>();
+    }
+    return Launchers();
+}
+
+// grids of one or two active axes, and of three where the caller's
+// translation unit holds those kernels too
+template <class EQ, class FLUX, int MAX_DIM = 3>
 Launchers pick_dim(int recon, int dim) {
     if (dim == 1) return pick_recon<EQ, FLUX, 1>(recon);
     if constexpr (EQ::NSD >= 2) {
         if (dim == 2) return pick_recon<EQ, FLUX, 2>(recon);
     }
-    if constexpr (EQ::NSD >= 3) {
+    if constexpr (EQ::NSD >= 3 && MAX_DIM >= 3) {
         if (dim == 3) return pick_recon<EQ, FLUX, 3>(recon);
     }
     return Launchers();
@@ -282,5 +275,11 @@ Launchers get_launchers_burgers(int recon, int flux, int dim);
 Launchers get_launchers_euler1(int recon, int flux, int dim);
 Launchers get_launchers_euler2(int recon, int flux, int dim);
 Launchers get_launchers_euler3(int recon, int flux, int dim);
+// euler3 on three active axes, one translation unit per reconstruction (they
+// take most of the build's time)
+Launchers get_launchers_euler3_3d_none(int flux);
+Launchers get_launchers_euler3_3d_weno2(int flux);
+Launchers get_launchers_euler3_3d_eno2(int flux);
+Launchers get_launchers_euler3_3d_eno3(int flux);
 
 }  // namespace avh

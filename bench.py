@@ -46,7 +46,9 @@ WORKLOADS = {
 # digest of the sources it was measured on, and its traffic / instruction
 # figures are reported only while the sources still match.
 KERNEL_SOURCES = ["avh_physics.hpp", "avh_stage.hpp", "avh_stage3d.hpp", "avh_stage_inst.hpp", "avh_batch.hpp",
-                  "avh_stage_burgers.hip", "avh_stage_euler1.hip", "avh_stage_euler2.hip", "avh_stage_euler3.hip"]
+                  "avh_stage_burgers.hip", "avh_stage_euler1.hip", "avh_stage_euler2.hip", "avh_stage_euler3.hip",
+                  "avh_stage_euler3_none.hip", "avh_stage_euler3_weno2.hip", "avh_stage_euler3_eno2.hip",
+                  "avh_stage_euler3_eno3.hip"]
 
 
 def kernel_source_digest():
