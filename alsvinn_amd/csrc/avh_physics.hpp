@@ -489,7 +489,6 @@ struct HLL3FluxT {
     template <class OPS, int DIR, class EQ>
     __device__ __forceinline__ static double flux_ops(const typename EQ::All& L, const typename EQ::All& R,
                                                       double g, double* F, bool& ok) {
-        constexpr int NSD = EQ::NSD;
         constexpr int NV = EQ::NV;
         // computeHLLSpeeds
         const double wl = OPS::sqrt_in_range(L.rho);

@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <cstring>
 #include <limits>
+#include <mutex>
 #include <new>
 #include <random>
 #include <vector>
@@ -121,29 +122,50 @@ __global__ __launch_bounds__(256) void kh2d_fill_kernel(double* state, long long
 }
 
 
+// Sum over the 256 threads of a workgroup, the same tree every time: lanes of
+// a wavefront, then the four wavefronts.  The total is thread 0's.
+__device__ __forceinline__ double block_sum(double v) {
+    __shared__ double s_part[4];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v = v + __shfl_xor(v, off, 64);
+    if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = v;
+    __syncthreads();
+    return (s_part[0] + s_part[1]) + (s_part[2] + s_part[3]);
+}
+
 // Kinetic energy of one velocity component per sample,
 //   E_c = (sum over cells of 0.5 * rho * u_c * u_c) * dV,  u_c = m_c / rho,
 // a functional of the conserved state modelled on the Moment functional
-// (alsfvm/src/functional/Moment.cpp:31-45).  One block per sample; each
-// thread sums a strided subset in cell order, then a fixed tree, so the
-// result does not depend on timing.
+// (alsfvm/src/functional/Moment.cpp:31-45).  Block (x, y) sums cells
+// x * 256, ... of every gridDim.x-th 256 of sample y; sums_finish_kernel adds
+// the blocks' sums in block order, so the result does not depend on timing.
+// Bound by reading two of the state's variables; one block a sample left all
+// but a few CUs idle (16 samples of 256^2: 85 us, now 7 us in 32 blocks each).
 __global__ __launch_bounds__(256) void kinetic_energy_kernel(const double* state, long long stride, long long ncells,
-                                                             int comp, double dv, double* out) {
-    __shared__ double red[256];
-    const double* q = state + (long long)blockIdx.x * stride;
+                                                             int comp, double* partial) {
+    const double* q = state + (long long)blockIdx.y * stride;
     double acc = 0.0;
-    for (long long i = threadIdx.x; i < ncells; i += 256) {
+    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < ncells; i += (long long)gridDim.x * 256) {
         const double rho = q[i];
         const double u = q[(long long)(1 + comp) * ncells + i] / rho;
         acc = acc + 0.5 * rho * (u * u);
     }
-    red[threadIdx.x] = acc;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] = red[threadIdx.x] + red[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[blockIdx.x] = red[0] * dv;
+    const double sum = block_sum(acc);
+    if (threadIdx.x == 0) partial[(long long)blockIdx.y * gridDim.x + blockIdx.x] = sum;
+}
+
+// out[t] = scale * (sum of the n partials of t), one wavefront each
+__global__ __launch_bounds__(256) void sums_finish_kernel(const double* partial, int n, int count, double scale,
+                                                          double* out) {
+    const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    if (t >= count) return;
+    const double* q = partial + (long long)t * n;
+    double acc = 0.0;
+    for (int k = lane; k < n; k += 64) acc = acc + q[k];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) acc = acc + __shfl_xor(acc, off, 64);
+    if (lane == 0) out[t] = scale * acc;
 }
 
 template <int P>
@@ -155,12 +177,24 @@ __device__ __forceinline__ double fast_power(double x) {
     }
 }
 
+// acc + |d|^P (P = 0: any power p)
+template <int P>
+__device__ __forceinline__ double add_power(double acc, double d, double p) {
+    if constexpr (P == 2) {
+        return fma(d, d, acc);
+    } else if constexpr (P > 0) {
+        return acc + fast_power<P>(fabs(d));
+    } else {
+        return acc + pow(fabs(d), p);
+    }
+}
+
 __device__ __forceinline__ int bc_value_index(int x, int n, int bc) {
     // ValueAtBoundary: periodic wraps, neumann clamps to the interior
     // (alsfvm/include/alsfvm/boundary/ValueAtBoundary.hpp)
     if (bc == AVH_BC_PERIODIC) {
-        while (x < 0) x += n;
-        return x % n;
+        x %= n;
+        return x < 0 ? x + n : x;
     }
     return x < 0 ? 0 : (x > n - 1 ? n - 1 : x);
 }
@@ -169,68 +203,171 @@ __device__ __forceinline__ int bc_value_index(int x, int n, int bc) {
 // statistic, alsfvm/include/alsfvm/functional/structure_common.hpp:36-154):
 // for every cell and lag h, |u - u'|^p summed over the cells u' on the
 // boundary of the square of half-width h around it (2 points in 1D, 8h in
-// 2D), divided by the number of cells.  Block = 256 consecutive cells of one
-// sample at one lag; partial sums in fixed order.
+// 2D), divided by the number of cells.
+//
+// 1D: block (x, y, z) sums 256 cells of sample z at lag y + 1.
 template <int P>
-__global__ __launch_bounds__(256) void structure_partial_kernel(const double* state, long long stride, int var, int nx,
-                                                                int ny, int dims, int bc, double p, double* partial) {
-    __shared__ double red[256];
-    const long long ncells = (long long)nx * ny;
+__global__ __launch_bounds__(256) void structure_line_kernel(const double* state, long long stride, int var, int nx,
+                                                             int bc, double p, double* partial) {
     const int h = blockIdx.y + 1;
-    const double* u = state + (long long)blockIdx.z * stride + (long long)var * ncells;
-    const long long c = (long long)blockIdx.x * 256 + threadIdx.x;
+    const double* u = state + (long long)blockIdx.z * stride + (long long)var * nx;
+    const int c = blockIdx.x * 256 + threadIdx.x;
     double acc = 0.0;
-    if (c < ncells) {
-        const int i = (int)(c % nx), j = (int)(c / nx);
+    if (c < nx) {
         const double uc = u[c];
-        auto term = [&](int x, int y) {
-            const double d = fabs(uc - u[(long long)bc_value_index(y, ny, bc) * nx + bc_value_index(x, nx, bc)]);
-            if constexpr (P > 0) {
-                acc = acc + fast_power<P>(d);
+        acc = add_power<P>(acc, uc - u[bc_value_index(c - h, nx, bc)], p);
+        acc = add_power<P>(acc, uc - u[bc_value_index(c + h, nx, bc)], p);
+    }
+    const double sum = block_sum(acc);
+    if (threadIdx.x == 0)
+        partial[((long long)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] = sum;
+}
+
+// Transposed copy of one variable of each sample: out[s][x][y] = u[s][y][x],
+// 32 x 32 cells a workgroup through LDS.
+__global__ __launch_bounds__(256) void transpose_kernel(const double* state, long long stride, int var, int nx, int ny,
+                                                        double* out) {
+    __shared__ double tile[32][33];
+    const long long ncells = (long long)nx * ny;
+    const double* u = state + (long long)blockIdx.z * stride + (long long)var * ncells;
+    double* o = out + (long long)blockIdx.z * ncells;
+    const int ntx = (nx + 31) / 32;
+    const int x0 = ((int)blockIdx.x % ntx) * 32, y0 = ((int)blockIdx.x / ntx) * 32;
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    for (int r = ty; r < 32; r += 8)
+        if (x0 + tx < nx && y0 + r < ny) tile[r][tx] = u[(long long)(y0 + r) * nx + x0 + tx];
+    __syncthreads();
+    for (int r = ty; r < 32; r += 8)
+        if (x0 + r < nx && y0 + tx < ny) o[(long long)(x0 + r) * ny + y0 + tx] = tile[tx][r];
+}
+
+// 2D.  The ring of lag h is two columns x -/+ h (y - h + 1 .. y + h - 1) and
+// two rows y -/+ h (x - h .. x + h); a row of the field is a column of its
+// transpose, so both are sweeps down a column: a lane owns a cell column and
+// SWEEP_ROWS cells of it in registers, and every value loaded from column
+// x + h serves all of them.  With periodic boundaries the pair at -h is the
+// pair at +h seen from its other cell, so one side is swept and the finish
+// doubles it; with neumann boundaries both are.
+// Bound by the FP64 pipe (a subtraction and an FMA a pair for p = 2); the
+// loads, one per SWEEP_ROWS pairs, come from L1 and L2.  One thread per cell
+// gathering its ring with wrapped indices took 17.2 ms for 16 samples of
+// 256^2 and 62 lags; this takes 0.70 ms (60 % of the pipe).
+// Block = 64 columns x 4 * SWEEP_ROWS rows of one sample at one lag, of the
+// field (blockIdx.x < cu) or of its transpose; the longest lags start first.
+constexpr int SWEEP_ROWS = 8;
+
+struct SweepParams {
+    const double* state;  // sample 0's state; stride doubles from one sample to the next
+    const double* trans;  // transposed copies
+    long long stride;
+    int var, nx, ny, bc;
+    int cu;               // blocks covering the field, the others cover the transpose
+    int nlags;            // lags 1 .. nlags
+    double p;
+    double* partial;      // [sample][lag][block]
+};
+
+template <int P>
+__global__ __launch_bounds__(256) void structure_sweep_kernel(SweepParams S) {
+    constexpr int R = SWEEP_ROWS;
+    const int h = S.nlags - (int)blockIdx.y;
+    const long long ncells = (long long)S.nx * S.ny;
+    const bool flip = (int)blockIdx.x >= S.cu;
+    const double* v = flip ? S.trans + (long long)blockIdx.z * ncells
+                           : S.state + (long long)blockIdx.z * S.stride + (long long)S.var * ncells;
+    const int nc = flip ? S.ny : S.nx, nr = flip ? S.nx : S.ny;  // columns, rows
+    const int L = flip ? h : h - 1;
+    const int tile = flip ? (int)blockIdx.x - S.cu : (int)blockIdx.x;
+    const int ntx = (nc + 63) / 64;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int x = (tile % ntx) * 64 + lane;
+    const int xc = x < nc ? x : nc - 1;
+    const int y0 = ((tile / ntx) * 4 + wave) * R;
+    double acc[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = 0.0;
+    if (y0 < nr) {
+        double c[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) c[r] = v[(long long)(y0 + r < nr ? y0 + r : nr - 1) * nc + xc];
+        const bool wrap = S.bc == AVH_BC_PERIODIC;
+        for (int side = 0; side < (wrap ? 1 : 2); ++side) {
+            const int xo = bc_value_index(side ? xc - h : xc + h, nc, S.bc);
+            // rows y0 - L + t for t = 0 .. 2L + R - 1; row t meets the cells
+            // r with t - 2L <= r <= t
+            int k = y0 - L;
+            int row = bc_value_index(k, nr, S.bc);
+            auto next = [&]() {
+                const double val = v[(long long)row * nc + xo];
+                ++k;
+                if (wrap) row = row + 1 == nr ? 0 : row + 1;
+                else row = k < 0 ? 0 : (k > nr - 1 ? nr - 1 : k);
+                return val;
+            };
+            if (2 * L >= R - 1) {
+#pragma unroll
+                for (int t = 0; t < R - 1; ++t) {
+                    const double val = next();
+#pragma unroll
+                    for (int r = 0; r <= t; ++r) acc[r] = add_power<P>(acc[r], c[r] - val, S.p);
+                }
+                int left = 2 * L + 2 - R;
+                for (; left >= 8; left -= 8) {
+                    double val[8];
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) val[i] = next();
+#pragma unroll
+                    for (int i = 0; i < 8; ++i)
+#pragma unroll
+                        for (int r = 0; r < R; ++r) acc[r] = add_power<P>(acc[r], c[r] - val[i], S.p);
+                }
+                for (; left > 0; --left) {
+                    const double val = next();
+#pragma unroll
+                    for (int r = 0; r < R; ++r) acc[r] = add_power<P>(acc[r], c[r] - val, S.p);
+                }
+#pragma unroll
+                for (int t = 1; t < R; ++t) {
+                    const double val = next();
+#pragma unroll
+                    for (int r = t; r < R; ++r) acc[r] = add_power<P>(acc[r], c[r] - val, S.p);
+                }
             } else {
-                acc = acc + pow(d, p);
-            }
-        };
-        if (dims == 1) {
-            term(i - h, 0);
-            term(i + h, 0);
-        } else {
-            // d = 0: columns x = i -/+ h, y in [j-h+1, j+h-1]
-            for (int side = 0; side < 2; ++side) {
-                const int x = side == 0 ? i - h : i + h;
-                for (int y = j - h + 1; y < j + h; ++y) term(x, y);
-            }
-            // d = 1: rows y = j -/+ h, x in [i-h, i+h]
-            for (int side = 0; side < 2; ++side) {
-                const int y = side == 0 ? j - h : j + h;
-                for (int x = i - h; x < i + h + 1; ++x) term(x, y);
+                for (int t = 0; t < 2 * L + R; ++t) {
+                    const double val = next();
+#pragma unroll
+                    for (int r = 0; r < R; ++r)
+                        if (r >= t - 2 * L && r <= t) acc[r] = add_power<P>(acc[r], c[r] - val, S.p);
+                }
             }
         }
     }
-    red[threadIdx.x] = acc;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] = red[threadIdx.x] + red[threadIdx.x + w];
-        __syncthreads();
-    }
+    double sum = 0.0;
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+        if (y0 + r < nr) sum = sum + acc[r];
+    sum = block_sum(x < nc ? sum : 0.0);
     if (threadIdx.x == 0)
-        partial[((long long)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] = red[0];
+        S.partial[((long long)blockIdx.z * S.nlags + (h - 1)) * gridDim.x + blockIdx.x] = sum;
 }
 
-// out[s][0] = 0, out[s][h] = (sum of the partials of (s, h) in block order) / cells
-__global__ __launch_bounds__(256) void structure_finish_kernel(const double* partial, int nchunks, int nh, int nsamples,
-                                                               double ncells, double* out) {
-    const int t = blockIdx.x * 256 + threadIdx.x;
+// out[s][0] = 0, out[s][h] = scale * (sum of the n partials of (s, h)), one
+// wavefront each
+__global__ __launch_bounds__(256) void structure_finish_kernel(const double* partial, int n, int nh, int nsamples,
+                                                               double ncells, double factor, double* out) {
+    const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
     if (t >= nsamples * nh) return;
     const int s = t / nh, h = t % nh;
-    if (h == 0) {
-        out[t] = 0.0;
-        return;
-    }
-    const double* q = partial + ((long long)s * (nh - 1) + (h - 1)) * nchunks;
     double acc = 0.0;
-    for (int k = 0; k < nchunks; ++k) acc = acc + q[k];
-    out[t] = acc / ncells;
+    if (h > 0) {
+        const double* q = partial + ((long long)s * (nh - 1) + (h - 1)) * n;
+        for (int k = lane; k < n; k += 64) acc = acc + q[k];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) acc = acc + __shfl_xor(acc, off, 64);
+    }
+    if (lane == 0) out[t] = h > 0 ? factor * acc / ncells : 0.0;
 }
 
 // End time of every sample: samples with t < t_end (and no constraint
@@ -319,6 +456,11 @@ struct avh_batch {
     // groups the stage and element-wise launches cover: a group whose
     // samples have all stopped is dropped until the next avh_batch_advance
     bool live[MAX_GROUPS] = {true, true, true, true};
+    // workspace of the observables (at most OBS_SLAB_BYTES and one sample's
+    // share), kept until the batch goes; `obs_lock` serialises its users
+    std::mutex obs_lock;
+    double* work = nullptr;
+    size_t work_cap = 0;
 };
 
 namespace {
@@ -343,8 +485,34 @@ void free_batch(avh_batch* b) {
         (void)hipFree(G.counts);
         (void)hipFree(G.active_count);
     }
+    (void)hipFree(b->work);
     if (b->stream) (void)hipStreamDestroy(b->stream);
     delete b;
+}
+
+// Samples of an observable are taken in slabs whose workspace stays below this
+// (or one sample at a time where a sample needs more).
+constexpr size_t OBS_SLAB_BYTES = (size_t)64 << 20;
+
+int slab_samples(size_t doubles_per_sample, int nsamples) {
+    const size_t per = doubles_per_sample * sizeof(double);
+    const size_t fit = per ? OBS_SLAB_BYTES / per : (size_t)nsamples;
+    return (int)std::max<size_t>(1, std::min<size_t>(fit, (size_t)nsamples));
+}
+
+// b->work with room for n doubles (b->obs_lock is held)
+avh_status ensure_work(avh_batch* b, size_t n) {
+    if (n <= b->work_cap) return AVH_OK;
+    (void)hipFree(b->work);
+    b->work = nullptr;
+    b->work_cap = 0;
+    if (hipMalloc(&b->work, sizeof(double) * n) != hipSuccess) {
+        b->work = nullptr;
+        (void)hipGetLastError();
+        return fail(AVH_ENOMEM, "device allocation failed");
+    }
+    b->work_cap = n;
+    return AVH_OK;
 }
 
 // Launch parameters over the live groups (slot j of P is group index[j]);
@@ -859,15 +1027,50 @@ avh_status avh_batch_kinetic_energy(avh_batch* b, int group, int component, doub
     double dv = 1.0;
     for (int d = 0; d < 3; ++d)
         if (G.n[d] > 1) dv *= (b->cfg.upper[d] - b->cfg.lower[d]) / double(G.n[d]);
-    double* d = nullptr;
-    AVH_HIP(hipMalloc(&d, sizeof(double) * G.nsamples));
-    hipLaunchKernelGGL(kinetic_energy_kernel, dim3(G.nsamples), dim3(256), 0, b->stream, G.A,
-                       (long long)b->nv * G.ncells, G.ncells, component, dv, d);
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipMemcpyAsync(out, d, sizeof(double) * G.nsamples, hipMemcpyDeviceToHost, b->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
-    (void)hipFree(d);
-    if (e != hipSuccess) return fail(AVH_EHIP, std::string("kinetic energy: ") + hipGetErrorString(e));
+    std::lock_guard<std::mutex> lock(b->obs_lock);
+    // 2048 cells a block: 8 a thread
+    const int nblk = (int)std::max<long long>(1, std::min<long long>((G.ncells + 2047) / 2048, 1024));
+    const int slab = std::min(slab_samples((size_t)nblk + 1, G.nsamples), 65535);
+    if ((r = ensure_work(b, (size_t)slab * (nblk + 1)))) return r;
+    double* d = b->work + (size_t)slab * nblk;
+    const long long stride = (long long)b->nv * G.ncells;
+    for (int s0 = 0; s0 < G.nsamples; s0 += slab) {
+        const int m = std::min(slab, G.nsamples - s0);
+        hipLaunchKernelGGL(kinetic_energy_kernel, dim3(nblk, m), dim3(256), 0, b->stream, G.A + s0 * stride, stride,
+                           G.ncells, component, b->work);
+        AVH_HIP(hipGetLastError());
+        hipLaunchKernelGGL(sums_finish_kernel, dim3((m + 3) / 4), dim3(256), 0, b->stream, b->work, nblk, m, dv, d);
+        AVH_HIP(hipGetLastError());
+        AVH_HIP(hipMemcpyAsync(out + s0, d, sizeof(double) * m, hipMemcpyDeviceToHost, b->stream));
+        AVH_HIP(hipStreamSynchronize(b->stream));
+    }
+    return AVH_OK;
+}
+
+static avh_status launch_structure_line(int pi, dim3 grid, hipStream_t st, const double* state, long long stride,
+                                        int var, int nx, int bc, double p, double* partial) {
+    switch (pi) {
+    case 1: hipLaunchKernelGGL(structure_line_kernel<1>, grid, dim3(256), 0, st, state, stride, var, nx, bc, p, partial); break;
+    case 2: hipLaunchKernelGGL(structure_line_kernel<2>, grid, dim3(256), 0, st, state, stride, var, nx, bc, p, partial); break;
+    case 3: hipLaunchKernelGGL(structure_line_kernel<3>, grid, dim3(256), 0, st, state, stride, var, nx, bc, p, partial); break;
+    case 4: hipLaunchKernelGGL(structure_line_kernel<4>, grid, dim3(256), 0, st, state, stride, var, nx, bc, p, partial); break;
+    case 5: hipLaunchKernelGGL(structure_line_kernel<5>, grid, dim3(256), 0, st, state, stride, var, nx, bc, p, partial); break;
+    default: hipLaunchKernelGGL(structure_line_kernel<0>, grid, dim3(256), 0, st, state, stride, var, nx, bc, p, partial); break;
+    }
+    AVH_HIP(hipGetLastError());
+    return AVH_OK;
+}
+
+static avh_status launch_structure_sweep(int pi, dim3 grid, hipStream_t st, const SweepParams& S) {
+    switch (pi) {
+    case 1: hipLaunchKernelGGL(structure_sweep_kernel<1>, grid, dim3(256), 0, st, S); break;
+    case 2: hipLaunchKernelGGL(structure_sweep_kernel<2>, grid, dim3(256), 0, st, S); break;
+    case 3: hipLaunchKernelGGL(structure_sweep_kernel<3>, grid, dim3(256), 0, st, S); break;
+    case 4: hipLaunchKernelGGL(structure_sweep_kernel<4>, grid, dim3(256), 0, st, S); break;
+    case 5: hipLaunchKernelGGL(structure_sweep_kernel<5>, grid, dim3(256), 0, st, S); break;
+    default: hipLaunchKernelGGL(structure_sweep_kernel<0>, grid, dim3(256), 0, st, S); break;
+    }
+    AVH_HIP(hipGetLastError());
     return AVH_OK;
 }
 
@@ -882,38 +1085,53 @@ avh_status avh_batch_structure_cube(avh_batch* b, int group, int var, int number
     if (!(p > 0)) return fail(AVH_EINVAL, "p must be positive");
     if (G.nsamples > 65535) return fail(AVH_EINVAL, "structure functions: at most 65535 samples per group");
     AVH_HIP(hipSetDevice(b->ctx->device));
-    const unsigned int nchunks = (unsigned int)((G.ncells + 255) / 256);
-    const size_t npart = (size_t)nchunks * (number_of_h - 1) * G.nsamples;
-    double *part = nullptr, *d = nullptr;
-    AVH_HIP(hipMalloc(&part, sizeof(double) * npart));
-    if (hipMalloc(&d, sizeof(double) * G.nsamples * number_of_h) != hipSuccess) {
-        (void)hipFree(part);
-        return fail(AVH_ENOMEM, "device allocation failed");
-    }
-    const dim3 grid(nchunks, number_of_h - 1, G.nsamples);
+    const int nx = G.n[0], ny = G.n[1], nlags = number_of_h - 1;
+    const bool two = b->dim == 2;
+    const int cu = two ? ((nx + 63) / 64) * ((ny + 4 * SWEEP_ROWS - 1) / (4 * SWEEP_ROWS)) : (nx + 255) / 256;
+    const int ct = two ? ((ny + 63) / 64) * ((nx + 4 * SWEEP_ROWS - 1) / (4 * SWEEP_ROWS)) : 0;
+    const size_t npart = (size_t)(cu + ct) * nlags;
+    const size_t per = npart + (two ? (size_t)G.ncells : 0) + number_of_h;
+    const int slab = slab_samples(per, G.nsamples);
+    std::lock_guard<std::mutex> lock(b->obs_lock);
+    if ((r = ensure_work(b, per * slab))) return r;
+    double* const part = b->work;
+    double* const trans = part + npart * slab;
+    double* const d = trans + (two ? (size_t)G.ncells * slab : 0);
     const long long stride = (long long)b->nv * G.ncells;
     const int pi = p == 1.0 ? 1 : p == 2.0 ? 2 : p == 3.0 ? 3 : p == 4.0 ? 4 : p == 5.0 ? 5 : 0;
-    switch (pi) {
-    case 1: hipLaunchKernelGGL(structure_partial_kernel<1>, grid, dim3(256), 0, b->stream, G.A, stride, var, G.n[0], G.n[1], b->dim, b->cfg.boundary, p, part); break;
-    case 2: hipLaunchKernelGGL(structure_partial_kernel<2>, grid, dim3(256), 0, b->stream, G.A, stride, var, G.n[0], G.n[1], b->dim, b->cfg.boundary, p, part); break;
-    case 3: hipLaunchKernelGGL(structure_partial_kernel<3>, grid, dim3(256), 0, b->stream, G.A, stride, var, G.n[0], G.n[1], b->dim, b->cfg.boundary, p, part); break;
-    case 4: hipLaunchKernelGGL(structure_partial_kernel<4>, grid, dim3(256), 0, b->stream, G.A, stride, var, G.n[0], G.n[1], b->dim, b->cfg.boundary, p, part); break;
-    case 5: hipLaunchKernelGGL(structure_partial_kernel<5>, grid, dim3(256), 0, b->stream, G.A, stride, var, G.n[0], G.n[1], b->dim, b->cfg.boundary, p, part); break;
-    default: hipLaunchKernelGGL(structure_partial_kernel<0>, grid, dim3(256), 0, b->stream, G.A, stride, var, G.n[0], G.n[1], b->dim, b->cfg.boundary, p, part); break;
+    for (int s0 = 0; s0 < G.nsamples; s0 += slab) {
+        const int m = std::min(slab, G.nsamples - s0);
+        const double* state = G.A + s0 * stride;
+        if (two) {
+            hipLaunchKernelGGL(transpose_kernel, dim3(((nx + 31) / 32) * ((ny + 31) / 32), 1, m), dim3(256), 0, b->stream,
+                               state, stride, var, nx, ny, trans);
+            AVH_HIP(hipGetLastError());
+            SweepParams S;
+            S.state = state;
+            S.trans = trans;
+            S.stride = stride;
+            S.var = var;
+            S.nx = nx;
+            S.ny = ny;
+            S.bc = b->cfg.boundary;
+            S.cu = cu;
+            S.nlags = nlags;
+            S.p = p;
+            S.partial = part;
+            r = launch_structure_sweep(pi, dim3(cu + ct, nlags, m), b->stream, S);
+        } else {
+            r = launch_structure_line(pi, dim3(cu, nlags, m), b->stream, state, stride, var, nx, b->cfg.boundary, p,
+                                      part);
+        }
+        if (r) return r;
+        const double factor = two && b->cfg.boundary == AVH_BC_PERIODIC ? 2.0 : 1.0;
+        hipLaunchKernelGGL(structure_finish_kernel, dim3((m * number_of_h + 3) / 4), dim3(256), 0, b->stream, part,
+                           cu + ct, number_of_h, m, (double)G.ncells, factor, d);
+        AVH_HIP(hipGetLastError());
+        AVH_HIP(hipMemcpyAsync(out + (size_t)s0 * number_of_h, d, sizeof(double) * m * number_of_h,
+                               hipMemcpyDeviceToHost, b->stream));
+        AVH_HIP(hipStreamSynchronize(b->stream));
     }
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess) {
-        const int nt = G.nsamples * number_of_h;
-        hipLaunchKernelGGL(structure_finish_kernel, dim3((nt + 255) / 256), dim3(256), 0, b->stream, part, (int)nchunks,
-                           number_of_h, G.nsamples, (double)G.ncells, d);
-        e = hipGetLastError();
-    }
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(out, d, sizeof(double) * G.nsamples * number_of_h, hipMemcpyDeviceToHost, b->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
-    (void)hipFree(part);
-    (void)hipFree(d);
-    if (e != hipSuccess) return fail(AVH_EHIP, std::string("structure function: ") + hipGetErrorString(e));
     return AVH_OK;
 }
 
