@@ -14,6 +14,11 @@
 //   backward  dW_l = dZ_l^T . X_l           (operands dZ_l^T, X_l^T)
 //             dX_l = dZ_l . W_l             (operands dZ_l, W_l^T)
 //             dZ_{l-1} = dX_l * gelu'(Z_{l-1})
+// Networks whose layers fit a workgroup's LDS (FUSED_MAX_DIM) run a training
+// step in two launches -- mlp_rows_kernel takes 16 rows through every layer
+// and back, mlp_update_kernel forms all gradients and applies Adam -- and a
+// prediction in one; wider ones run layer by layer (mlp_gemm_kernel).  Both
+// form every product with the same matrix instructions in the same order.
 // No reference counterpart: the reference has no learned model; this is the
 // surrogate of its Monte Carlo runs (alsuq/src/run/Runner.cpp:39-90).
 #include <hip/hip_runtime.h>
@@ -54,6 +59,13 @@ __device__ __forceinline__ float gelu_grad(float x) {
     const float cdf = 0.5f * (1.0f + erff(x * 0.70710678118654752f));
     const float pdf = 0.39894228040143268f * expf(-0.5f * x * x);
     return cdf + x * pdf;
+}
+// both from one erff: the same bits as gelu and gelu_grad
+__device__ __forceinline__ float gelu_both(float x, float& grad) {
+    const float e = 1.0f + erff(x * 0.70710678118654752f);
+    const float pdf = 0.39894228040143268f * expf(-0.5f * x * x);
+    grad = 0.5f * e + x * pdf;
+    return 0.5f * x * e;
 }
 
 enum GemmEpilogue { EPI_HIDDEN = 0, EPI_OUT = 1, EPI_DX = 2, EPI_DW = 3 };
@@ -192,6 +204,19 @@ __global__ __launch_bounds__(256) void mlp_bias_grad_kernel(const uint16_t* dZT,
     grad[mem * p_ms + b_off + o] = acc;
 }
 
+// Tile layout of a 16-bit operand [rows][K] of the fused path (rows and K
+// multiples of 16): 16 rows x 32 of K are 1 KiB in the order in which the
+// lanes of a matrix instruction take them (lane = row % 16 + 16 * (k % 32 / 8),
+// 8 values each), a last 16 of K likewise with 4 values a lane.  A wave's
+// operand load is then one contiguous block; row-major rows of 512 bytes put
+// its 64 lanes on 16 cache lines of the same banks (a 256-wide layer's weights
+// took 9000 cycles to arrive, 2048 at L1's rate).
+__host__ __device__ __forceinline__ int tiled(int row, int k, int K) {
+    const int full = K & ~31, tile = (row >> 4) * 16 * K;
+    if (k < full) return tile + (k >> 5) * 512 + ((k & 31) >> 3) * 128 + (row & 15) * 8 + (k & 7);
+    return tile + full * 16 + ((k & 15) >> 2) * 64 + (row & 15) * 4 + (k & 3);
+}
+
 struct LayerDesc {
     int nin, nout;
     long long w_off, b_off;  // in the fp32 parameter block of a member
@@ -206,7 +231,29 @@ struct AdamArgs {
     LayerDesc L[MAX_LAYERS];
     float lr, b1, b2, eps, c1, c2;  // c1 = 1 - b1^t, c2 = 1 - b2^t
     float wd;                       // decoupled weight decay of the weights (not the biases)
+    int tiles;                      // bf16 weights in the fused path's tile layout
 };
+
+// where weight (o, k) of a layer goes in the bf16 blocks
+__device__ __forceinline__ int weight_at(const AdamArgs& a, const LayerDesc& L, int o, int k) {
+    return a.tiles ? tiled(o, k, L.nin) : o * L.nin + k;
+}
+__device__ __forceinline__ int weight_t_at(const AdamArgs& a, const LayerDesc& L, int o, int k) {
+    return a.tiles ? tiled(k, o, L.nout) : k * L.nout + o;
+}
+
+// Adam's update of one parameter; writes p, m, v and returns the new value.
+__device__ __forceinline__ float adam_update(const AdamArgs& a, long long i, float g, float p0, float m0, float v0,
+                                             bool weight) {
+    const float m = a.b1 * m0 + (1.f - a.b1) * g;
+    const float v = a.b2 * v0 + (1.f - a.b2) * (g * g);
+    a.m[i] = m;
+    a.v[i] = v;
+    float p = p0 - a.lr * (m / a.c1) / (sqrtf(v / a.c2) + a.eps);
+    if (weight && a.wd != 0.f) p = p - a.lr * a.wd * p0;
+    a.p[i] = p;
+    return p;
+}
 
 // Adam (bias-corrected) on the fp32 master parameters of layer blockIdx.y,
 // with decoupled weight decay on the weights (AdamW, Loshchilov and Hutter,
@@ -219,20 +266,12 @@ __global__ __launch_bounds__(256) void mlp_adam_kernel(AdamArgs a) {
     const long long e = (long long)blockIdx.x * 256 + threadIdx.x;
     if (e >= nw + L.nout) return;
     const long long i = mem * a.p_ms + (e < nw ? L.w_off + e : L.b_off + (e - nw));
-    const float g = a.g[i];
-    const float m = a.b1 * a.m[i] + (1.f - a.b1) * g;
-    const float v = a.b2 * a.v[i] + (1.f - a.b2) * (g * g);
-    a.m[i] = m;
-    a.v[i] = v;
-    const float p0 = a.p[i];
-    float p = p0 - a.lr * (m / a.c1) / (sqrtf(v / a.c2) + a.eps);
-    if (e < nw && a.wd != 0.f) p = p - a.lr * a.wd * p0;
-    a.p[i] = p;
+    const float p = adam_update(a, i, a.g[i], a.p[i], a.m[i], a.v[i], e < nw);
     if (e < nw) {
         const int o = (int)(e / L.nin), k = (int)(e % L.nin);
         const uint16_t b = f2bf(p);
-        a.wb[mem * a.wb_ms + L.wb_off + e] = b;
-        a.wtb[mem * a.wb_ms + L.wb_off + (long long)k * L.nout + o] = b;
+        a.wb[mem * a.wb_ms + L.wb_off + weight_at(a, L, o, k)] = b;
+        a.wtb[mem * a.wb_ms + L.wb_off + weight_t_at(a, L, o, k)] = b;
     }
 }
 
@@ -245,8 +284,465 @@ __global__ __launch_bounds__(256) void mlp_cast_kernel(AdamArgs a) {
     if (e >= nw) return;
     const int o = (int)(e / L.nin), k = (int)(e % L.nin);
     const uint16_t b = f2bf(a.p[mem * a.p_ms + L.w_off + e]);
-    a.wb[mem * a.wb_ms + L.wb_off + e] = b;
-    a.wtb[mem * a.wb_ms + L.wb_off + (long long)k * L.nout + o] = b;
+    a.wb[mem * a.wb_ms + L.wb_off + weight_at(a, L, o, k)] = b;
+    a.wtb[mem * a.wb_ms + L.wb_off + weight_t_at(a, L, o, k)] = b;
+}
+
+// ---------------------------------------------------------------------------
+// The fused step.  One Adam step of the study's ensemble (5 members, 256 rows,
+// 40 -> 256^4 -> 66) is 1.7 GFLOP and was 22 dependent launches of 3 to 40 us:
+// latency, not arithmetic, bounds it, so the layers' activations stay in one
+// workgroup's LDS and the launches go (347 -> 40 us a step, of which
+// mlp_rows_kernel 25 and mlp_update_kernel 14).
+
+// Widest layer of a network that takes the fused path: its two activation
+// buffers take 33 KB of LDS, and no measured shape up to it is faster layer
+// by layer (us a training step, fused / layered: 5 members of 512 x 4, 256
+// rows 122 / 387; of 256 x 4, 4096 rows 401 / 3660; 64 members of 512 x 4,
+// 1024 rows 2802 / 6605).  Wider layers would need a larger share of LDS, and
+// every workgroup reads all of a member's weights.
+constexpr int FUSED_MAX_DIM = 512;
+constexpr int ROWS = 16;  // minibatch rows of a workgroup: one MFMA tile
+
+struct RowsArgs {
+    const float *X, *Y;     // data rows
+    const int* idx;         // [member] rows of the minibatch, null: rows in order
+    long long idx_ms;
+    int rows;               // rows there are (later rows of a tile are zero)
+    int nin, pin, nout, pout, B, M, W, nl;
+    int pitch;              // LDS elements from one row to the next
+    const float *mu_in, *sd_in, *mu_out, *sd_out;
+    const uint16_t *wb, *wtb;
+    long long wb_ms;
+    const float* params;
+    long long p_ms;
+    LayerDesc L[MAX_LAYERS];
+    float* dg;              // [hidden][member][B][W] gelu' of the pre-activations
+    uint16_t *x0t, *at;     // transposed activations, for the gradients (tile layout)
+    uint16_t* dzt;          // [layer][member][dz_w][B] transposed dZ (tile layout)
+    int dz_w;
+    float* loss_part;       // [member][workgroup]
+    float* out;             // prediction: [member][rows][nout], data units
+};
+
+// bf16 by the hardware's conversion (round to nearest even, as f2bf)
+__device__ __forceinline__ uint16_t cvt_bf(float f) {
+    const __bf16 b = (__bf16)f;
+    uint16_t u;
+    __builtin_memcpy(&u, &b, 2);
+    return u;
+}
+
+// One 16 x 16 tile of C = A . B^T: A's rows from LDS, B's tile (in tile
+// layout) from global memory.  Of a K of 256 or more the first 256 of B are
+// loaded ahead (load_ahead) and run without a branch; the steps' order is
+// mlp_gemm_kernel's.
+constexpr int AHEAD = 8;
+__device__ __forceinline__ bf16x8 load8(const uint16_t* tile, int k0, int lane) {
+    return *reinterpret_cast<const bf16x8*>(tile + k0 * 16 + lane * 8);
+}
+__device__ __forceinline__ bf16x4 load4(const uint16_t* tile, int k0, int lane) {
+    return *reinterpret_cast<const bf16x4*>(tile + k0 * 16 + lane * 4);
+}
+__device__ __forceinline__ void load_ahead(const uint16_t* tile, int K, int lane, bf16x8 (&wreg)[AHEAD]) {
+    if (K >= AHEAD * 32) {
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) wreg[i] = load8(tile, i * 32, lane);
+    }
+}
+__device__ __forceinline__ f32x4 tile_product(const uint16_t* A, const uint16_t* tile, int K, int lane,
+                                              const bf16x8 (&wreg)[AHEAD]) {
+    const int kq = lane >> 4;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    int k0 = 0;
+    if (K >= AHEAD * 32) {
+        bf16x8 a[AHEAD];
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) a[i] = *reinterpret_cast<const bf16x8*>(A + i * 32 + 8 * kq);
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], wreg[i], acc, 0, 0, 0);
+        k0 = AHEAD * 32;
+    }
+#pragma unroll 2
+    for (; k0 + 32 <= K; k0 += 32) {
+        const bf16x8 a = *reinterpret_cast<const bf16x8*>(A + k0 + 8 * kq);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, load8(tile, k0, lane), acc, 0, 0, 0);
+    }
+    if (k0 < K) {
+        const bf16x4 a = *reinterpret_cast<const bf16x4*>(A + k0 + 4 * kq);
+        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, load4(tile, k0, lane), acc, 0, 0, 0);
+    }
+    return acc;
+}
+
+__device__ __forceinline__ void store4(uint16_t* to, const uint16_t (&v)[4]) {
+    uint2 w;
+    w.x = (uint32_t)v[0] | ((uint32_t)v[1] << 16);
+    w.y = (uint32_t)v[2] | ((uint32_t)v[3] << 16);
+    *reinterpret_cast<uint2*>(to) = w;
+}
+
+// Workgroup (x, member) takes ROWS rows through every layer, its waves sharing
+// the layer's 16-column tiles; with TRAIN on to the loss and back to dZ of
+// every layer.  Activations and backward signals alternate between two LDS
+// buffers, one barrier a layer; a row's pitch is 16 bytes past a multiple of
+// 32, so that the rows of a tile start in different banks.  TRAIN leaves what
+// the gradients need (transposed activations and dZ) in global memory: a lane
+// holds four consecutive rows of a column, one 8-byte store.  A wave loads its
+// tile's weights, bias and gelu' of the next layer before it issues those
+// stores: vector memory completes in order, and loads behind the stores would
+// wait for them in every layer.  GELU and its derivative, an erff and an expf,
+// are the longest part of a layer's chain and are formed together, forward.
+// (5 members x 256 rows: 25 us in 80 workgroups; with the weights in rows
+// 38 us; 160 workgroups of 8 rows, each wave with two tiles, 26 us.)
+template <bool TRAIN>
+__global__ __launch_bounds__(1024) void mlp_rows_kernel(RowsArgs g) {
+    extern __shared__ __align__(16) uint16_t lds[];
+    __shared__ int s_src[ROWS];
+    __shared__ float s_loss[16];
+    uint16_t* cur = lds;
+    uint16_t* nxt = lds + ROWS * g.pitch;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    const int kq = lane >> 4, lo = lane & 15;
+    const int mr = 4 * kq;  // the lane's first row of a result tile
+    const int mem = blockIdx.y;
+    const int row0 = blockIdx.x * ROWS;
+    const uint16_t* wb = g.wb + mem * g.wb_ms;
+    const uint16_t* wtb = g.wtb + mem * g.wb_ms;
+    const float* params = g.params + mem * g.p_ms;
+    // Every wave takes a 16-column tile of each product (waves past the last
+    // repeat it and write the same values), so the code below has no branch
+    // around its loads and stores; further tiles follow in a loop.
+    auto first_tile = [&](int N) { return wave < N / 16 ? wave : N / 16 - 1; };
+    bf16x8 wreg[AHEAD];
+    auto product = [&](const uint16_t* W, int t, int K) {
+        return tile_product(cur + lo * g.pitch, W + t * 16 * K, K, lane, wreg);
+    };
+    float bn = 0.f;  // the lane's bias in the next layer
+    auto next_layer = [&](int l) {
+        const LayerDesc L = g.L[l];
+        const int t = first_tile(L.nout);
+        load_ahead(wb + L.wb_off + t * 16 * L.nin, L.nin, lane, wreg);
+        bn = params[L.b_off + t * 16 + lo];
+    };
+    float dg[4] = {0.f, 0.f, 0.f, 0.f};  // and gelu' in the next layer back
+    auto dg_rows = [&](int l) { return g.dg + (((long long)l * g.M + mem) * g.B + row0 + mr) * g.W; };
+    auto next_back = [&](int l) {
+        const LayerDesc L = g.L[l];
+        const int t = first_tile(L.nin);
+        load_ahead(wtb + L.wb_off + t * 16 * L.nout, L.nout, lane, wreg);
+        const float* d = dg_rows(l - 1) + t * 16 + lo;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) dg[r] = d[r * g.W];
+    };
+    auto swap = [&]() {
+        lds_barrier();
+        uint16_t* const sw = cur;
+        cur = nxt;
+        nxt = sw;
+    };
+    next_layer(0);
+
+    if (threadIdx.x < ROWS) {
+        const int r = row0 + threadIdx.x;
+        s_src[threadIdx.x] = r < g.rows ? (g.idx ? g.idx[mem * g.idx_ms + r] : r) : -1;
+    }
+    lds_barrier();
+    for (int e = threadIdx.x; e < ROWS * g.pin; e += blockDim.x) {
+        const int r = e / g.pin, k = e % g.pin;
+        const int src = s_src[r];
+        float v = 0.f;
+        if (src >= 0 && k < g.nin) v = (g.X[(long long)src * g.nin + k] - g.mu_in[k]) / g.sd_in[k];
+        cur[r * g.pitch + k] = cvt_bf(v);
+    }
+    // normalised targets; those of the wave's output turn are loaded now
+    auto target = [&](int m, int n) {
+        const int src = s_src[m];
+        return src >= 0 && n < g.nout ? (g.Y[(long long)src * g.nout + n] - g.mu_out[n]) / g.sd_out[n] : 0.f;
+    };
+    float y[4] = {0.f, 0.f, 0.f, 0.f};
+    if (TRAIN) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) y[r] = target(mr + r, first_tile(g.pout) * 16 + lo);
+    }
+    lds_barrier();
+    if (TRAIN) {
+        for (int e = threadIdx.x; e < 4 * g.pin; e += blockDim.x) {
+            const int k = e >> 2, r = (e & 3) * 4;
+            uint16_t q[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) q[i] = cur[(r + i) * g.pitch + k];
+            store4(g.x0t + (long long)mem * g.pin * g.B + tiled(k, row0 + r, g.B), q);
+        }
+    }
+
+    // hidden layers
+    for (int l = 0; l + 1 < g.nl; ++l) {
+        const LayerDesc L = g.L[l];
+        const int N = L.nout;
+        uint16_t* at = g.at + ((long long)l * g.M + mem) * g.W * g.B;
+        float* dgl = dg_rows(l);
+        uint16_t q[4];
+        float grad[4];
+        auto activate = [&](const f32x4& acc, int n, float b) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) q[r] = cvt_bf(TRAIN ? gelu_both(acc[r] + b, grad[r]) : gelu(acc[r] + b));
+#pragma unroll
+            for (int r = 0; r < 4; ++r) nxt[(mr + r) * g.pitch + n] = q[r];
+        };
+        auto keep = [&](int n) {
+            if (!TRAIN) return;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) dgl[r * g.W + n] = grad[r];
+            store4(at + tiled(n, row0 + mr, g.B), q);
+        };
+        const uint16_t* W = wb + L.wb_off;
+        const f32x4 acc = product(W, first_tile(N), L.nin);
+        const float b = bn;
+        for (int t = wave + nw; t < N / 16; t += nw) {
+            load_ahead(W + t * 16 * L.nin, L.nin, lane, wreg);
+            const int n = t * 16 + lo;
+            activate(product(W, t, L.nin), n, params[L.b_off + n]);
+            keep(n);
+        }
+        const int n = first_tile(N) * 16 + lo;
+        activate(acc, n, b);
+        next_layer(l + 1);
+        keep(n);
+        swap();
+    }
+
+    // output layer
+    float loss = 0.f;
+    {
+        const int l = g.nl - 1;
+        const LayerDesc L = g.L[l];
+        const int N = L.nout;
+        const uint16_t* W = wb + L.wb_off;
+        const float scale = 2.0f / (float)(g.B * g.nout);
+        uint16_t* dzt = g.dzt + ((long long)l * g.M + mem) * g.dz_w * g.B;
+        uint16_t q[4];
+        auto finish = [&](const f32x4& acc, int t, float b) {
+            const int n = t * 16 + lo;
+            if (TRAIN) {
+                const bool own = t == wave || t >= nw;  // not a repeat
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float v = acc[r] + b;
+                    const float d = n < g.nout ? v - (t < nw ? y[r] : target(mr + r, n)) : 0.f;
+                    loss += own ? d * d : 0.f;
+                    q[r] = cvt_bf(d * scale);
+                    nxt[(mr + r) * g.pitch + n] = q[r];
+                }
+            } else if (n < g.nout) {
+                const float sd = g.sd_out[n], mu = g.mu_out[n];
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (row0 + mr + r < g.rows)
+                        g.out[((long long)mem * g.rows + row0 + mr + r) * g.nout + n] = (acc[r] + b) * sd + mu;
+            }
+        };
+        const f32x4 acc = product(W, first_tile(N), L.nin);
+        for (int t = wave + nw; t < N / 16; t += nw) {
+            load_ahead(W + t * 16 * L.nin, L.nin, lane, wreg);
+            finish(product(W, t, L.nin), t, params[L.b_off + t * 16 + lo]);
+            if (TRAIN) store4(dzt + tiled(t * 16 + lo, row0 + mr, g.B), q);
+        }
+        finish(acc, first_tile(N), bn);
+        if (!TRAIN) return;
+        next_back(l);
+        store4(dzt + tiled(first_tile(N) * 16 + lo, row0 + mr, g.B), q);
+        swap();
+    }
+
+    // dZ_{l-1} = (dZ_l . W_l) * gelu'(Z_{l-1})
+    for (int l = g.nl - 1; l > 0; --l) {
+        const LayerDesc L = g.L[l];
+        const int K = L.nout, N = L.nin;
+        const uint16_t* W = wtb + L.wb_off;
+        uint16_t* dzt = g.dzt + ((long long)(l - 1) * g.M + mem) * g.dz_w * g.B;
+        uint16_t q[4];
+        auto finish = [&](const f32x4& acc, int n, const float (&d)[4]) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                q[r] = cvt_bf(acc[r] * d[r]);
+                nxt[(mr + r) * g.pitch + n] = q[r];
+            }
+        };
+        const f32x4 acc = product(W, first_tile(N), K);
+        for (int t = wave + nw; t < N / 16; t += nw) {
+            load_ahead(W + t * 16 * K, K, lane, wreg);
+            const int n = t * 16 + lo;
+            float d[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) d[r] = dg_rows(l - 1)[r * g.W + n];
+            finish(product(W, t, K), n, d);
+            store4(dzt + tiled(n, row0 + mr, g.B), q);
+        }
+        const int n = first_tile(N) * 16 + lo;
+        finish(acc, n, dg);
+        if (l > 1) next_back(l - 1);
+        store4(dzt + tiled(n, row0 + mr, g.B), q);
+        swap();
+    }
+
+    // the workgroup's share of the loss, the same tree every time
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off, 64);
+    if (lane == 0) s_loss[wave] = loss;
+    lds_barrier();
+    if (threadIdx.x == 0) {
+        float sum = 0.f;
+        for (int w = 0; w < nw; ++w) sum += s_loss[w];
+        g.loss_part[(long long)mem * gridDim.x + blockIdx.x] = sum;
+    }
+}
+
+struct UpdateArgs {
+    AdamArgs a;
+    float* grad;
+    const uint16_t *x0t, *at, *dzt;
+    int pin, W, B, M, nl, dz_w, nout;
+    int bias_blocks;            // workgroups of the biases, the first ones
+    int first[MAX_LAYERS + 1];  // first workgroup of each layer's weights among the others, and their number
+    const float* loss_part;
+    int nparts;
+    float* loss;
+};
+
+// Gradients of every layer, dW = dZ^T . X over the minibatch rows and db in
+// row order, with Adam on the spot (ADAM) and the bf16 copies of the weights.
+// Bound by the latency of its operands in L2 and of the master weights and
+// moments in HBM; a wave takes a 16 x 32 tile of dW, whose moments and weights
+// it loads before the products.  The first workgroups sum the biases (one lane
+// an output: a chain of B additions, the longest work here) and the loss.
+template <bool ADAM>
+__global__ __launch_bounds__(256) void mlp_update_kernel(UpdateArgs u) {
+    const AdamArgs& a = u.a;
+    const int mem = blockIdx.y, part = blockIdx.x;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (part >= u.bias_blocks) {
+        const int b = part - u.bias_blocks;
+        // the layer, selected from all of the table: a search step by step
+        // would wait for a scalar load at every step
+        int l = 0, first = 0;
+        LayerDesc L = a.L[0];
+#pragma unroll
+        for (int i = 1; i < MAX_LAYERS; ++i)
+            if (i < u.nl && b >= u.first[i]) {
+                l = i;
+                first = u.first[i];
+                L = a.L[i];
+            }
+        const int ntn = (L.nin + 31) / 32;
+        const int tile = (b - first) * 4 + wave;
+        const int tm = tile / ntn, tn = tile % ntn;
+        if (tm * 16 >= L.nout) return;
+        const int kq = lane >> 4, lo = lane & 15;
+        const uint16_t* A = u.dzt + (((long long)l * u.M + mem) * u.dz_w + tm * 16) * u.B;
+        const uint16_t* X = l == 0 ? u.x0t + (long long)mem * u.pin * u.B
+                                   : u.at + ((long long)(l - 1) * u.M + mem) * u.W * u.B;
+        const bool two = tn * 32 + 16 < L.nin;  // the second half of the tile exists
+        const int n[2] = {tn * 32 + lo, two ? tn * 32 + 16 + lo : tn * 32 + lo};
+        long long at[2][4];
+        float p0[2][4], m0[2][4], v0[2][4];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                at[h][r] = mem * a.p_ms + L.w_off + (long long)(tm * 16 + 4 * kq + r) * L.nin + n[h];
+                if (ADAM) {
+                    p0[h][r] = a.p[at[h][r]];
+                    m0[h][r] = a.m[at[h][r]];
+                    v0[h][r] = a.v[at[h][r]];
+                }
+            }
+        const uint16_t* X0 = X + tn * 32 * u.B;
+        const uint16_t* X1 = two ? X0 + 16 * u.B : X0;
+        f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+        int k0 = 0;
+#pragma unroll 4
+        for (; k0 + 32 <= u.B; k0 += 32) {
+            const bf16x8 x = load8(A, k0, lane), y0 = load8(X0, k0, lane), y1 = load8(X1, k0, lane);
+            acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y0, acc[0], 0, 0, 0);
+            acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y1, acc[1], 0, 0, 0);
+        }
+        if (k0 < u.B) {
+            const bf16x4 x = load4(A, k0, lane), y0 = load4(X0, k0, lane), y1 = load4(X1, k0, lane);
+            acc[0] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(x, y0, acc[0], 0, 0, 0);
+            acc[1] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(x, y1, acc[1], 0, 0, 0);
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            if (h == 1 && !two) break;
+            uint16_t q[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float g = acc[h][r];
+                u.grad[at[h][r]] = g;
+                if (ADAM) {
+                    q[r] = cvt_bf(adam_update(a, at[h][r], g, p0[h][r], m0[h][r], v0[h][r], true));
+                    a.wb[mem * a.wb_ms + L.wb_off + tiled(tm * 16 + 4 * kq + r, n[h], L.nin)] = q[r];
+                }
+            }
+            if (ADAM) store4(a.wtb + mem * a.wb_ms + L.wb_off + tiled(n[h], tm * 16 + 4 * kq, L.nout), q);
+        }
+        return;
+    }
+    // biases: output t of all layers in turn, a lane each
+    int t = part * 256 + threadIdx.x;
+    if (t == 0) {
+        float sum = 0.f;
+        for (int i = 0; i < u.nparts; ++i) sum += u.loss_part[(long long)mem * u.nparts + i];
+        u.loss[mem] += sum / (float)(u.B * u.nout);
+    }
+    int l = -1, at = 0;
+    long long b_off = 0;
+#pragma unroll
+    for (int i = 0, base = 0; i < MAX_LAYERS; ++i)
+        if (i < u.nl) {
+            if (t >= base && t < base + a.L[i].nout) {
+                l = i;
+                at = base;
+                b_off = a.L[i].b_off;
+            }
+            base += a.L[i].nout;
+        }
+    if (l < 0) return;
+    t -= at;
+    const uint16_t* dz = u.dzt + ((long long)l * u.M + mem) * u.dz_w * u.B;
+    const long long i = mem * a.p_ms + b_off + t;
+    float acc = 0.f;
+#pragma unroll 8
+    for (int r = 0; r < u.B; r += 4) {
+        const uint2 w = *reinterpret_cast<const uint2*>(dz + tiled(t, r, u.B));
+        acc += __uint_as_float(w.x << 16);
+        acc += __uint_as_float(w.x & 0xffff0000u);
+        acc += __uint_as_float(w.y << 16);
+        acc += __uint_as_float(w.y & 0xffff0000u);
+    }
+    u.grad[i] = acc;
+    if (ADAM) adam_update(a, i, acc, a.p[i], a.m[i], a.v[i], false);
+}
+
+// The fp32 block of a member (parameters or gradients) in the caller's order:
+// W[out][in] without padding, then b[out], layer by layer.
+struct PackArgs {
+    const float* src;
+    float* dst;
+    long long src_ms, dst_ms;
+    LayerDesc L[MAX_LAYERS];
+    int fin[MAX_LAYERS], fout[MAX_LAYERS];  // unpadded widths
+    long long off[MAX_LAYERS];              // layer's first value in the caller's order
+};
+__global__ __launch_bounds__(256) void mlp_pack_kernel(PackArgs a) {
+    const int l = blockIdx.y, mem = blockIdx.z;
+    const long long nw = (long long)a.fin[l] * a.fout[l];
+    const long long e = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (e >= nw + a.fout[l]) return;
+    const LayerDesc& L = a.L[l];
+    const long long i = e < nw ? L.w_off + e / a.fin[l] * L.nin + e % a.fin[l] : L.b_off + (e - nw);
+    a.dst[mem * a.dst_ms + a.off[l] + e] = a.src[mem * a.src_ms + i];
 }
 
 inline int pad16(int x) { return (x + 15) / 16 * 16; }
@@ -273,6 +769,11 @@ struct avh_mlp {
     int* idx = nullptr;
     long long icap = 0;
     long long t = 0;  // Adam steps taken
+    bool fused = false;         // the fused path serves this network
+    uint16_t* dztl = nullptr;   // [layer][M][dz_w][B] transposed dZ (fused)
+    float* loss_part = nullptr; // [M][row tiles] (fused)
+    float* outbuf = nullptr;    // what a call hands to the host: predictions, packed parameters
+    long long ocap = 0;
     long long epochs_done = 0;  // epochs of avh_mlp_train so far (seeds the shuffles)
     float wd = 0.f;   // decoupled weight decay
     hipStream_t stream = nullptr;
@@ -286,7 +787,7 @@ void free_mlp(avh_mlp* n) {
     if (n->stream) (void)hipStreamSynchronize(n->stream);
     void* ptrs[] = {n->params, n->m, n->v, n->grad, n->wb, n->wtb, n->x0, n->x0t, n->z, n->a, n->at, n->yhat,
                     n->yn, n->dz[0], n->dz[1], n->dzt[0], n->dzt[1], n->mu_in, n->sd_in, n->mu_out, n->sd_out,
-                    n->loss, n->dx, n->dy, n->idx};
+                    n->loss, n->dx, n->dy, n->idx, n->dztl, n->loss_part, n->outbuf};
     for (void* p : ptrs) (void)hipFree(p);
     if (n->stream) (void)hipStreamDestroy(n->stream);
     delete n;
@@ -303,6 +804,7 @@ AdamArgs adam_args(const avh_mlp* n) {
     a.wtb = n->wtb;
     a.p_ms = n->P;
     a.wb_ms = n->WB;
+    a.tiles = n->fused ? 1 : 0;
     for (int l = 0; l < n->nl; ++l) a.L[l] = n->L[l];
     return a;
 }
@@ -459,7 +961,8 @@ avh_status backward(avh_mlp* n) {
     return AVH_OK;
 }
 
-avh_status adam_step(avh_mlp* n, float lr) {
+// Adam's arguments for the next step (counts it)
+AdamArgs next_adam(avh_mlp* n, float lr) {
     n->t += 1;
     AdamArgs a = adam_args(n);
     a.lr = lr;
@@ -469,8 +972,169 @@ avh_status adam_step(avh_mlp* n, float lr) {
     a.eps = n->cfg.eps;
     a.c1 = (float)(1.0 - std::pow((double)n->cfg.beta1, (double)n->t));
     a.c2 = (float)(1.0 - std::pow((double)n->cfg.beta2, (double)n->t));
+    return a;
+}
+
+avh_status adam_step(avh_mlp* n, float lr) {
+    const AdamArgs a = next_adam(n, lr);
     hipLaunchKernelGGL(mlp_adam_kernel, dim3(max_layer_blocks(n), n->nl, n->M), dim3(256), 0, n->stream, a);
     AVH_HIP(hipGetLastError());
+    return AVH_OK;
+}
+
+int dz_width(const avh_mlp* n) { return std::max(n->maxw, n->pout); }
+
+RowsArgs rows_args(const avh_mlp* n) {
+    RowsArgs g;
+    std::memset(&g, 0, sizeof g);
+    g.X = n->dx;
+    g.nin = n->cfg.n_in;
+    g.pin = n->pin;
+    g.nout = n->cfg.n_out;
+    g.pout = n->pout;
+    g.B = n->B;
+    g.M = n->M;
+    g.W = n->maxw;
+    g.nl = n->nl;
+    g.pitch = std::max(std::max(n->pin, n->pout), n->maxw) + 8;
+    g.mu_in = n->mu_in;
+    g.sd_in = n->sd_in;
+    g.mu_out = n->mu_out;
+    g.sd_out = n->sd_out;
+    g.wb = n->wb;
+    g.wtb = n->wtb;
+    g.wb_ms = n->WB;
+    g.params = n->params;
+    g.p_ms = n->P;
+    for (int l = 0; l < n->nl; ++l) g.L[l] = n->L[l];
+    g.dg = n->z;
+    g.x0t = n->x0t;
+    g.at = n->at;
+    g.dzt = n->dztl;
+    g.dz_w = dz_width(n);
+    g.loss_part = n->loss_part;
+    return g;
+}
+
+// a wave for each column tile of the widest layer, at least 4 and at most 16
+template <bool TRAIN>
+avh_status launch_rows(const avh_mlp* n, const RowsArgs& g) {
+    const int tiles = std::max(n->maxw, n->pout) / 16;
+    hipLaunchKernelGGL(mlp_rows_kernel<TRAIN>, dim3((g.rows + ROWS - 1) / ROWS, n->M),
+                       dim3(64 * std::max(4, std::min(16, tiles))), 2 * sizeof(uint16_t) * ROWS * (size_t)g.pitch,
+                       n->stream, g);
+    AVH_HIP(hipGetLastError());
+    return AVH_OK;
+}
+
+// Loss and gradients of the minibatch rows idx[member][row0 ...] of the device
+// data, and with `adam` the update of every parameter, in two launches.
+avh_status fused_step(avh_mlp* n, long long row0, long long idx_ms, const AdamArgs* adam) {
+    RowsArgs g = rows_args(n);
+    g.Y = n->dy;
+    g.idx = n->idx + row0;
+    g.idx_ms = idx_ms;
+    g.rows = n->B;
+    avh_status r = launch_rows<true>(n, g);
+    if (r) return r;
+    UpdateArgs u;
+    std::memset(&u, 0, sizeof u);
+    u.a = adam ? *adam : adam_args(n);
+    u.grad = n->grad;
+    u.x0t = n->x0t;
+    u.at = n->at;
+    u.dzt = n->dztl;
+    u.pin = n->pin;
+    u.W = n->maxw;
+    u.B = n->B;
+    u.M = n->M;
+    u.nl = n->nl;
+    u.dz_w = dz_width(n);
+    u.nout = n->cfg.n_out;
+    int first = 0, outs = 0;
+    for (int l = 0; l < n->nl; ++l) {
+        u.first[l] = first;
+        first += ((n->L[l].nout / 16) * ((n->L[l].nin + 31) / 32) + 3) / 4;
+        outs += n->L[l].nout;
+    }
+    u.first[n->nl] = first;
+    u.loss_part = n->loss_part;
+    u.nparts = n->B / ROWS;
+    u.loss = n->loss;
+    u.bias_blocks = (outs + 255) / 256;
+    const dim3 grid(u.bias_blocks + first, n->M);
+    if (adam) hipLaunchKernelGGL(mlp_update_kernel<true>, grid, dim3(256), 0, n->stream, u);
+    else hipLaunchKernelGGL(mlp_update_kernel<false>, grid, dim3(256), 0, n->stream, u);
+    AVH_HIP(hipGetLastError());
+    return AVH_OK;
+}
+
+avh_status ensure_outbuf(avh_mlp* n, long long count) {
+    if (count <= n->ocap) return AVH_OK;
+    (void)hipFree(n->outbuf);
+    n->outbuf = nullptr;
+    n->ocap = 0;
+    AVH_HIP(hipMalloc(&n->outbuf, sizeof(float) * count));
+    n->ocap = count;
+    return AVH_OK;
+}
+
+// `count` members' blocks from `src` (the first's) to the host in the
+// caller's order: packed on the device, so that the copy needs no pass of the
+// host over its values
+avh_status read_packed(avh_mlp* n, const float* src, int count, float* host) {
+    PackArgs a;
+    std::memset(&a, 0, sizeof a);
+    long long np = 0, most = 0;
+    for (int l = 0; l < n->nl; ++l) {
+        a.L[l] = n->L[l];
+        a.fin[l] = l == 0 ? n->cfg.n_in : n->cfg.width;
+        a.fout[l] = l == n->nl - 1 ? n->cfg.n_out : n->cfg.width;
+        a.off[l] = np;
+        const long long vals = (long long)a.fin[l] * a.fout[l] + a.fout[l];
+        np += vals;
+        most = std::max(most, vals);
+    }
+    avh_status r = ensure_outbuf(n, np * count);
+    if (r) return r;
+    a.src = src;
+    a.dst = n->outbuf;
+    a.src_ms = n->P;
+    a.dst_ms = np;
+    hipLaunchKernelGGL(mlp_pack_kernel, dim3((unsigned int)((most + 255) / 256), n->nl, count), dim3(256), 0,
+                       n->stream, a);
+    AVH_HIP(hipGetLastError());
+    AVH_HIP(hipMemcpyAsync(host, n->outbuf, sizeof(float) * np * count, hipMemcpyDeviceToHost, n->stream));
+    AVH_HIP(hipStreamSynchronize(n->stream));
+    return AVH_OK;
+}
+
+// Outputs of every member for the first `rows` device rows, in data units,
+// slab by slab of at most PREDICT_SLAB rows (the outputs of a call then take
+// at most 16 MiB a member at 64 outputs).
+constexpr long long PREDICT_SLAB = 65536;
+avh_status fused_predict(avh_mlp* n, long long rows, float* out) {
+    const long long slab = std::min(rows, PREDICT_SLAB);
+    const long long need = slab * n->M * n->cfg.n_out;
+    avh_status r = ensure_outbuf(n, need);
+    if (r) return r;
+    for (long long c0 = 0; c0 < rows; c0 += slab) {
+        RowsArgs g = rows_args(n);
+        g.rows = (int)std::min(slab, rows - c0);
+        g.X = n->dx + c0 * n->cfg.n_in;
+        g.out = n->outbuf;
+        if ((r = launch_rows<false>(n, g))) return r;
+        const size_t part = sizeof(float) * (size_t)g.rows * n->cfg.n_out;
+        if (g.rows == rows) {
+            AVH_HIP(hipMemcpyAsync(out, n->outbuf, part * n->M, hipMemcpyDeviceToHost, n->stream));
+        } else {
+            for (int mem = 0; mem < n->M; ++mem)
+                AVH_HIP(hipMemcpyAsync(out + ((size_t)mem * rows + c0) * n->cfg.n_out,
+                                       n->outbuf + (size_t)mem * g.rows * n->cfg.n_out, part, hipMemcpyDeviceToHost,
+                                       n->stream));
+        }
+        AVH_HIP(hipStreamSynchronize(n->stream));
+    }
     return AVH_OK;
 }
 
@@ -519,6 +1183,7 @@ avh_status avh_mlp_create(avh_ctx* ctx, const avh_mlp_config* cfg, avh_mlp** out
     }
     n->P = P;
     n->WB = WB;
+    n->fused = std::max(std::max(n->pin, n->pout), n->maxw) <= FUSED_MAX_DIM;
     const long long M = n->M, B = n->B, W = cfg->width, H = cfg->hidden;
     const long long dzw = B * std::max<long long>(W, n->pout);
     bool ok = hipStreamCreateWithFlags(&n->stream, hipStreamNonBlocking) == hipSuccess;
@@ -546,6 +1211,10 @@ avh_status avh_mlp_create(avh_ctx* ctx, const avh_mlp_config* cfg, avh_mlp** out
     alloc((void**)&n->mu_out, sizeof(float) * cfg->n_out);
     alloc((void**)&n->sd_out, sizeof(float) * cfg->n_out);
     alloc((void**)&n->loss, sizeof(float) * M);
+    if (n->fused) {
+        alloc((void**)&n->dztl, 2 * M * n->nl * dzw);
+        alloc((void**)&n->loss_part, sizeof(float) * M * (B / ROWS));
+    }
     if (!ok) {
         free_mlp(n);
         return fail(AVH_ENOMEM, "device allocation failed");
@@ -630,19 +1299,7 @@ avh_status avh_mlp_set_normalization(avh_mlp* n, const float* in_mean, const flo
 avh_status avh_mlp_get_params(avh_mlp* n, int member, float* out) {
     if (!n || !out || member < 0 || member >= n->M) return fail(AVH_EINVAL, "bad argument");
     AVH_HIP(hipSetDevice(n->ctx->device));
-    AVH_HIP(hipStreamSynchronize(n->stream));
-    std::vector<float> h(n->P);
-    AVH_HIP(hipMemcpy(h.data(), n->params + member * n->P, sizeof(float) * n->P, hipMemcpyDeviceToHost));
-    size_t o = 0;
-    for (int l = 0; l < n->nl; ++l) {
-        const LayerDesc& L = n->L[l];
-        const int fin = l == 0 ? n->cfg.n_in : n->cfg.width;
-        const int fout = l == n->nl - 1 ? n->cfg.n_out : n->cfg.width;
-        for (int r = 0; r < fout; ++r)
-            for (int k = 0; k < fin; ++k) out[o++] = h[L.w_off + (long long)r * L.nin + k];
-        for (int r = 0; r < fout; ++r) out[o++] = h[L.b_off + r];
-    }
-    return AVH_OK;
+    return read_packed(n, n->params + member * n->P, 1, out);
 }
 
 avh_status avh_mlp_set_params(avh_mlp* n, int member, const float* in) {
@@ -679,29 +1336,15 @@ avh_status avh_mlp_gradients(avh_mlp* n, const float* X, const float* Y, int64_t
     for (int i = 0; i < rows; ++i) id[i] = i;
     AVH_HIP(hipMemcpyAsync(n->idx, id.data(), sizeof(int) * rows, hipMemcpyHostToDevice, n->stream));
     AVH_HIP(hipMemsetAsync(n->loss, 0, sizeof(float) * n->M, n->stream));
-    if ((r = gather(n, 0, 0, (int)rows, true))) return r;
-    if ((r = forward(n))) return r;
-    if ((r = backward(n))) return r;
-    std::vector<float> h((size_t)(n->M * n->P));
-    AVH_HIP(hipMemcpyAsync(h.data(), n->grad, sizeof(float) * n->M * n->P, hipMemcpyDeviceToHost, n->stream));
-    AVH_HIP(hipMemcpyAsync(loss, n->loss, sizeof(float) * n->M, hipMemcpyDeviceToHost, n->stream));
-    AVH_HIP(hipStreamSynchronize(n->stream));
-    int64_t np = 0;
-    avh_mlp_num_params(n, &np);
-    for (int mem = 0; mem < n->M; ++mem) {
-        size_t o = 0;
-        const float* src = h.data() + (size_t)mem * n->P;
-        float* dst = grads + (size_t)mem * np;
-        for (int l = 0; l < n->nl; ++l) {
-            const LayerDesc& L = n->L[l];
-            const int fin = l == 0 ? n->cfg.n_in : n->cfg.width;
-            const int fout = l == n->nl - 1 ? n->cfg.n_out : n->cfg.width;
-            for (int rr = 0; rr < fout; ++rr)
-                for (int k = 0; k < fin; ++k) dst[o++] = src[L.w_off + (long long)rr * L.nin + k];
-            for (int rr = 0; rr < fout; ++rr) dst[o++] = src[L.b_off + rr];
-        }
+    if (n->fused) {
+        if ((r = fused_step(n, 0, 0, nullptr))) return r;
+    } else {
+        if ((r = gather(n, 0, 0, (int)rows, true))) return r;
+        if ((r = forward(n))) return r;
+        if ((r = backward(n))) return r;
     }
-    return AVH_OK;
+    AVH_HIP(hipMemcpyAsync(loss, n->loss, sizeof(float) * n->M, hipMemcpyDeviceToHost, n->stream));
+    return read_packed(n, n->grad, n->M, grads);
 }
 
 // One Adam step of every member from the gradients of the last
@@ -750,6 +1393,11 @@ avh_status avh_mlp_train(avh_mlp* n, const float* X, const float* Y, int64_t row
         for (long long s = 0; s < steps_per_epoch; ++s, ++k) {
             const double c = 0.5 * (1.0 + std::cos(3.14159265358979323846 * (double)k / (double)total));
             const float lr_k = lr * (final_lr_fraction + (1.f - final_lr_fraction) * (float)c);
+            if (n->fused) {
+                const AdamArgs a = next_adam(n, lr_k);
+                if ((r = fused_step(n, s * n->B, rows, &a))) return r;
+                continue;
+            }
             if ((r = gather(n, s * n->B, rows, n->B, true))) return r;
             if ((r = forward(n))) return r;
             if ((r = backward(n))) return r;
@@ -779,6 +1427,7 @@ avh_status avh_mlp_predict(avh_mlp* n, const float* X, int64_t rows, float* out)
     AVH_HIP(hipSetDevice(n->ctx->device));
     avh_status r = upload_data(n, X, nullptr, rows);
     if (r) return r;
+    if (n->fused) return fused_predict(n, rows, out);
     const long long padded = (rows + n->B - 1) / n->B * n->B;
     if ((r = ensure_idx(n, padded))) return r;
     std::vector<int> id(padded);

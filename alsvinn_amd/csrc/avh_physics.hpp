@@ -10,6 +10,16 @@
 
 namespace avh {
 
+// Workgroup barrier for data exchanged through LDS alone.  __syncthreads also
+// waits for the wavefront's global loads and stores in flight, which here
+// would put prefetched tiles and the write-back of results on the critical
+// path of every plane or layer.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Correctly rounded FP64 square root for x in [2^-767, DBL_MAX]: the
 // operation sequence the compiler emits for sqrt() on gfx950 -- v_rsq_f64,
 // then g = x*r, h = r/2 and two Goldschmidt / Newton corrections by fused
