@@ -86,6 +86,7 @@ struct StageParams {
     // 1: the launch is the step's last stage and its last workgroup runs the
     // end of the step (end_step); 0: the caller runs finish_step_kernel
     int finish = 0;
+    int lz = 0;  // 3D: planes a workgroup marches through (set by the launcher)
 };
 
 // The reference's Volume (alsfvm/src/volume/Volume.cpp:44-60): one array per

@@ -118,13 +118,13 @@ __device__ __forceinline__ void recon_faces_reg(const double (&u)[WZ][NV], const
     }
 }
 
-// TWO_BARRIERS: the plane tile is double-buffered and the x- and y-interface
-// fluxes have LDS buffers of their own, so a plane takes two barriers (plane
-// published; fluxes published) instead of five, and the x, y and z flux
-// evaluations of a plane run in one barrier-free stretch.
+// The plane tile is double-buffered and the x- and y-interface fluxes have LDS
+// buffers of their own, so a plane takes two barriers (plane published; fluxes
+// published) and its x, y and z flux evaluations run in one barrier-free
+// stretch.  A workgroup marches through P.lz planes.
 // MODE_CT >= 0 compiles the kernel for that StageMode alone (P.mode must
 // equal it): the other modes' branches and registers drop out.
-template <class EQ, int RECON, class FLUX, int TX, int TY, int LZ, int NTH, bool TWO_BARRIERS = false, int MODE_CT = -1>
+template <class EQ, int RECON, class FLUX, int TX, int TY, int NTH, int MODE_CT = -1>
 struct MarchKernel3 {
     static constexpr int NV = EQ::NV;
     static constexpr int NC = TX * TY;  // columns: one per thread, threads past them work on the planes only
@@ -141,8 +141,8 @@ struct MarchKernel3 {
     static constexpr int NIMAX = NIX > NIY ? NIX : NIY;
     static constexpr int NHALO = LP - TX * TY;
 
-    __host__ __device__ static unsigned int tiles(const int* n) {
-        return (unsigned int)(((n[0] + TX - 1) / TX) * ((n[1] + TY - 1) / TY) * ((n[2] + LZ - 1) / LZ));
+    __host__ __device__ static unsigned int tiles(const int* n, int lz) {
+        return (unsigned int)(((n[0] + TX - 1) / TX) * ((n[1] + TY - 1) / TY) * ((n[2] + lz - 1) / lz));
     }
 
     // Cell indices.  The kernels compiled for the first two RK3 stages index
@@ -187,7 +187,7 @@ struct MarchKernel3 {
     // allows no more).
     static constexpr int RING = 2 + HW;
     static constexpr int LDS_BASE =
-        8 * ((TWO_BARRIERS ? 2 : 1) * NV * LP + (TWO_BARRIERS ? 2 : 1) * NV * NIMAX + 3 * (NT / 64));
+        8 * (2 * NV * LP + 2 * NV * NIMAX + 3 * (NT / 64)) + 8 * (NT / 64);
     static constexpr bool U0RING = MODE_CT == MODE_RK3_2 && LDS_BASE + 8 * RING * NV * NC <= 80 * 1024;
 
     // interface between plane cells ia and ia + SD under OPS
@@ -255,15 +255,12 @@ struct MarchKernel3 {
     }
 
     __device__ static void run(const StageParams& P) {
-        constexpr int NBUF = TWO_BARRIERS ? 2 : 1;
-        __shared__ double sp_buf[NBUF][NV * LP];
-        __shared__ double sf[NV * NIMAX];
-        __shared__ double sf_y[TWO_BARRIERS ? NV * NIMAX : 1];
+        __shared__ double sp_buf[2][NV * LP];
+        __shared__ double sfx[NV * NIMAX];
+        __shared__ double sfy[NV * NIMAX];
         __shared__ double s_ws[3][NT / 64];
         __shared__ double su0[U0RING ? RING * NV * NC : 1];
-        __shared__ int s_adm[NBUF][NT / 64];
-        double* const sfx = sf;
-        double* const sfy = TWO_BARRIERS ? sf_y : sf;
+        __shared__ int s_adm[2][NT / 64];
 
         Control* ctrl = P.ctrl;
         const int mode = MODE_CT >= 0 ? MODE_CT : P.mode;
@@ -275,8 +272,8 @@ struct MarchKernel3 {
         const int tx = tile % ntx;
         const int ty = (tile / ntx) % nty;
         const int tz = tile / (ntx * nty);
-        const int ox = tx * TX, oy = ty * TY, z0 = tz * LZ;
-        const int z1 = (z0 + LZ < n2) ? z0 + LZ : n2;
+        const int ox = tx * TX, oy = ty * TY, z0 = tz * P.lz;
+        const int z1 = (z0 + P.lz < n2) ? z0 + P.lz : n2;
         const bool otf = (mode == MODE_RK3_2);
         const double s = (mode == MODE_FLUX_ONLY || mode == MODE_L) ? 0.0 : step_dt(ctrl) / ctrl->cell[0];
 
@@ -343,10 +340,7 @@ struct MarchKernel3 {
                 for (int v = 0; v < NV; ++v) w[i][v] = w[i + 1][v];
             fetch(P, otf, s, gidx(gxc, gyc, bc_map(z0 + 1 + HW, n2, P.bc), n0, n1), w[WZ - 1],
                   ring ? slot(z0 + 1 + HW) : nullptr);
-            if constexpr (FLUX::FAST) {
-                col_adm = col_adm & EQ::admitted(w[WZ - 1]);
-                if (RECON == RECON_WENO2) rb = weno2_recip(w[HW][0] - w[HW - 1][0]);
-            }
+            if (FLUX::FAST && RECON == RECON_WENO2) rb = weno2_recip(w[HW][0] - w[HW - 1][0]);
         }
 
         bool bad = false;
@@ -424,7 +418,7 @@ struct MarchKernel3 {
         }
 
         for (int k = z0; k < z1; ++k) {
-            double* const sp = sp_buf[TWO_BARRIERS ? ((k - z0) & 1) : 0];
+            double* const sp = sp_buf[(k - z0) & 1];
             // plane k into LDS: own column from the window (w[HW-1] is plane k),
             // the halo ring from the prefetched registers
             if (has_col) {
@@ -446,12 +440,12 @@ struct MarchKernel3 {
                 }
             }
             // one vote per wavefront through LDS, read by all after the barrier
-            int* const va = s_adm[TWO_BARRIERS ? ((k - z0) & 1) : 0];
+            int* const va = s_adm[(k - z0) & 1];
             if constexpr (FLUX::FAST) {
                 const bool all = __all(adm);
                 if ((threadIdx.x & 63) == 0) va[threadIdx.x >> 6] = all;
             }
-            __syncthreads();
+            lds_barrier();
             if constexpr (FLUX::FAST) {
                 int all = va[0];
 #pragma unroll
@@ -472,6 +466,10 @@ struct MarchKernel3 {
             // (only for the tile's columns inside the grid: a column past the
             // grid edge supplies the plane's halo but has no cells to update)
             auto z_flux = [&]() {
+                // the window's newest plane, here where it is first needed
+                if constexpr (FLUX::FAST) {
+                    if (has_col) col_adm = col_adm & EQ::admitted(w[WZ - 1]);
+                }
                 if (col_ok) {
                     typedef typename OpsFor<FLUX::FAST>::type Ops;
                     double lz[NV];
@@ -508,25 +506,14 @@ struct MarchKernel3 {
                         acc[v] = acc[v] + ((-sfy[v * NIMAX + ip]) + sfy[v * NIMAX + ip - TX]);
                 }
             };
-            if constexpr (TWO_BARRIERS) {
-                // every flux of the plane, then one barrier, then the sums in
-                // the reference's x, y, z order
-                plane_pass<0>(sp, sfx, ox, oy, P.n, P.gamma, adm, ws[0]);
-                plane_pass<1>(sp, sfy, ox, oy, P.n, P.gamma, adm, ws[1]);
-                z_flux();
-                __syncthreads();
-                add_x();
-                add_y();
-            } else {
-                plane_pass<0>(sp, sfx, ox, oy, P.n, P.gamma, adm, ws[0]);
-                __syncthreads();
-                add_x();
-                __syncthreads();
-                plane_pass<1>(sp, sfy, ox, oy, P.n, P.gamma, adm, ws[1]);
-                __syncthreads();
-                add_y();
-                z_flux();
-            }
+            // every flux of the plane, then one barrier, then the sums in the
+            // reference's x, y, z order
+            plane_pass<0>(sp, sfx, ox, oy, P.n, P.gamma, adm, ws[0]);
+            plane_pass<1>(sp, sfy, ox, oy, P.n, P.gamma, adm, ws[1]);
+            z_flux();
+            lds_barrier();
+            add_x();
+            add_y();
 #pragma unroll
             for (int v = 0; v < NV; ++v) acc[v] = acc[v] + ((-fz[v]) + fprev[v]);
 
@@ -592,11 +579,7 @@ struct MarchKernel3 {
                 }
 #pragma unroll
                 for (int v = 0; v < NV; ++v) w[WZ - 1][v] = otf ? cin[v] * s + cu0[v] : cin[v];
-                if constexpr (FLUX::FAST) col_adm = col_adm & EQ::admitted(w[WZ - 1]);
             }
-            // one plane buffer: every thread must be done reading it (and the
-            // flux buffer) before the next plane is written
-            if constexpr (!TWO_BARRIERS) __syncthreads();
         }
 
 #undef AVH_PREFETCH_RING

@@ -27,21 +27,20 @@ typedef hipError_t (*VolumeLauncher)(const StageParams& P, const VolumeParams& V
 //       lanes have an item, so shapes whose interface counts sit just under
 //       a multiple of 256 waste the least: 32x15 (495 x- / 512 y-interfaces),
 //       24x20 (500 / 504) and 16x15 (255 / 256), against 32x16 (528 / 544).
-//   3D: columns marching over 32 planes, 256 threads: 32x8 (264 / 288
-//       plane interfaces), 16x15 or 32x7 (at most 256 each: one turn; the
-//       threads past the columns only work on the planes); then 16x15 over
-//       32 and over 16 planes and 32x7 over 32 planes with two barriers
-//       per plane (double-buffered plane tile); then 16x15 over 32 planes,
-//       two barriers, fluxes under SharedOps with the PlainOps redo.
+//   3D: 16x15 or 32x7 columns marching over 2 to 32 planes, 256 threads (at
+//       most 256 interfaces a plane in each direction: one turn; the threads
+//       past the columns only work on the planes).  A chunk pays a z flux
+//       and the loads of its window before its first plane, so long chunks
+//       win where a grid still gives every CU its two workgroups (us of an RK3
+//       stage pair, 4 / 8 / 16 / 32 planes: 256^3 2520 / 2262 / 2133 / 2100,
+//       200x150x120 575 / 539 / 598 / 722, 97x83x61 120 / 140 / 173 / 326).
 constexpr int NSHAPES1 = 2, NSHAPES2 = 5, NSHAPES3 = 7;
 constexpr int SHAPE1_TX[NSHAPES1] = {256, 64};
 constexpr int SHAPE2_TX[NSHAPES2] = {32, 16, 64, 32, 24};
 constexpr int SHAPE2_TY[NSHAPES2] = {16, 15, 4, 15, 20};
-constexpr int SHAPE3_TX[NSHAPES3] = {32, 16, 32, 16, 16, 32, 16};
-constexpr int SHAPE3_TY[NSHAPES3] = {8, 15, 7, 15, 15, 7, 15};
-constexpr int SHAPE3_LZ[NSHAPES3] = {32, 32, 32, 32, 16, 32, 32};
-constexpr bool SHAPE3_TWO_BARRIERS[NSHAPES3] = {false, false, false, true, true, true, true};
-constexpr bool SHAPE3_SHARED[NSHAPES3] = {false, false, false, false, false, false, true};
+constexpr int SHAPE3_TX[NSHAPES3] = {16, 16, 32, 32, 16, 16, 16};
+constexpr int SHAPE3_TY[NSHAPES3] = {15, 15, 7, 7, 15, 15, 15};
+constexpr int SHAPE3_LZ[NSHAPES3] = {4, 8, 8, 32, 16, 2, 32};
 
 inline int num_shapes(int dim) { return dim == 1 ? NSHAPES1 : (dim == 2 ? NSHAPES2 : NSHAPES3); }
 
@@ -127,50 +126,34 @@ hipError_t launch_stage_k(const StageParams& P, hipStream_t stream) {
 
 template <class K>
 hipError_t launch_march_k(const StageParams& P, hipStream_t stream) {
-    hipLaunchKernelGGL(march_kernel3<K>, dim3(K::tiles(P.n)), dim3(K::NT), 0, stream, P);
+    hipLaunchKernelGGL(march_kernel3<K>, dim3(K::tiles(P.n, P.lz)), dim3(K::NT), 0, stream, P);
     return hipGetLastError();
+}
+
+// one column tile: each stage mode has a kernel compiled for it; flux-only
+// launches, and grids whose cells need 64-bit indices, take the kernel that
+// reads the mode
+template <class EQ, int RECON, class FLUX, int TX, int TY>
+hipError_t launch_march(const StageParams& P, hipStream_t stream) {
+    if (P.ncells < MODE_KERNEL_MAX_CELLS) {
+        switch (P.mode) {
+        case MODE_L: return launch_march_k<MarchKernel3<EQ, RECON, FLUX, TX, TY, 256, MODE_L>>(P, stream);
+        case MODE_RK2_2: return launch_march_k<MarchKernel3<EQ, RECON, FLUX, TX, TY, 256, MODE_RK2_2>>(P, stream);
+        case MODE_RK3_2: return launch_march_k<MarchKernel3<EQ, RECON, FLUX, TX, TY, 256, MODE_RK3_2>>(P, stream);
+        case MODE_RK3_3: return launch_march_k<MarchKernel3<EQ, RECON, FLUX, TX, TY, 256, MODE_RK3_3>>(P, stream);
+        }
+    }
+    return launch_march_k<MarchKernel3<EQ, RECON, FLUX, TX, TY, 256>>(P, stream);
 }
 
 template <class EQ, int RECON, class FLUX, int DIM>
 hipError_t launch_stage(const StageParams& P, int shape, hipStream_t stream) {
     if constexpr (DIM == 3) {
-        // shapes without SharedOps use the compiler's sqrt and divide throughout
-#define AVH_MARCH_CASE(S)                                                                                   \
-    case S:                                                                                                 \
-        return launch_march_k<MarchKernel3<EQ, RECON,                                                       \
-                                           typename std::conditional<SHAPE3_SHARED[S], FLUX,                \
-                                                                     typename FLUX::Plain>::type,           \
-                                           SHAPE3_TX[S], SHAPE3_TY[S], SHAPE3_LZ[S], 256,                   \
-                                           SHAPE3_TWO_BARRIERS[S]>>(P, stream);
-        switch (shape) {
-            AVH_MARCH_CASE(0)
-            AVH_MARCH_CASE(1)
-            AVH_MARCH_CASE(2)
-            AVH_MARCH_CASE(3)
-            AVH_MARCH_CASE(4)
-            AVH_MARCH_CASE(5)
-        case 6: {
-            // the RK3 stages of the shape a 3D run normally takes, each compiled
-            // for its mode; other modes take the kernel that reads P.mode
-            typedef typename std::conditional<SHAPE3_SHARED[6], FLUX, typename FLUX::Plain>::type F6;
-            if (P.ncells >= MODE_KERNEL_MAX_CELLS)  // the per-mode kernels index with 32-bit values
-                return launch_march_k<MarchKernel3<EQ, RECON, F6, SHAPE3_TX[6], SHAPE3_TY[6], SHAPE3_LZ[6], 256,
-                                                   SHAPE3_TWO_BARRIERS[6]>>(P, stream);
-            if (P.mode == MODE_L)
-                return launch_march_k<MarchKernel3<EQ, RECON, F6, SHAPE3_TX[6], SHAPE3_TY[6], SHAPE3_LZ[6], 256,
-                                                   SHAPE3_TWO_BARRIERS[6], MODE_L>>(P, stream);
-            if (P.mode == MODE_RK3_2)
-                return launch_march_k<MarchKernel3<EQ, RECON, F6, SHAPE3_TX[6], SHAPE3_TY[6], SHAPE3_LZ[6], 256,
-                                                   SHAPE3_TWO_BARRIERS[6], MODE_RK3_2>>(P, stream);
-            if (P.mode == MODE_RK3_3)
-                return launch_march_k<MarchKernel3<EQ, RECON, F6, SHAPE3_TX[6], SHAPE3_TY[6], SHAPE3_LZ[6], 256,
-                                                   SHAPE3_TWO_BARRIERS[6], MODE_RK3_3>>(P, stream);
-            return launch_march_k<MarchKernel3<EQ, RECON, F6, SHAPE3_TX[6], SHAPE3_TY[6], SHAPE3_LZ[6], 256,
-                                               SHAPE3_TWO_BARRIERS[6]>>(P, stream);
-        }
-        }
-#undef AVH_MARCH_CASE
-        return hipErrorInvalidValue;
+        if (shape < 0 || shape >= NSHAPES3) return hipErrorInvalidValue;
+        StageParams Q = P;
+        Q.lz = SHAPE3_LZ[shape];
+        return SHAPE3_TX[shape] == 16 ? launch_march<EQ, RECON, FLUX, 16, 15>(Q, stream)
+                                      : launch_march<EQ, RECON, FLUX, 32, 7>(Q, stream);
     } else if constexpr (DIM == 1) {
         switch (shape) {
         case 0: return launch_stage_k<typename KernelFor<EQ, RECON, FLUX, 1, 0>::type>(P, stream);

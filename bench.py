@@ -27,9 +27,9 @@ import time
 
 HBM_PEAK_GBS = 8000.0
 SHAPE_NAMES = {1: ["256", "64"], 2: ["32x16", "16x15", "64x4", "32x15", "24x20"],
-               3: ["32x8 columns x 32 planes", "16x15 columns x 32 planes", "32x7 columns x 32 planes",
-                   "16x15 columns x 32 planes, 2 barriers", "16x15 columns x 16 planes, 2 barriers",
-                   "32x7 columns x 32 planes, 2 barriers", "16x15 columns x 32 planes, 2 barriers, shared reciprocals"]}
+               3: ["16x15 columns x 4 planes", "16x15 columns x 8 planes", "32x7 columns x 8 planes",
+                   "32x7 columns x 32 planes", "16x15 columns x 16 planes", "16x15 columns x 2 planes",
+                   "16x15 columns x 32 planes"]}
 
 WORKLOADS = {
     # the bench line
