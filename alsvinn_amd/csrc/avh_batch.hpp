@@ -119,18 +119,26 @@ __global__ __launch_bounds__(256) void batch_ew_kernel(BatchParams B, int fe_fin
     Control* ctrl = G.ctrl + sample;
     if (!ctrl->active) return;
     constexpr int NV = EQ::NV;
+    const long long o = (long long)sample * G.stride;
+    double l[NV], u[NV];
+    if (i < G.ncells) {
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            l[v] = G.in[o + v * G.ncells + i];
+            u[v] = G.u0[o + v * G.ncells + i];
+        }
+    }
     const double s = step_dt(ctrl) / ctrl->cell[0];
     bool bad = false;
     if (i < G.ncells) {
-        const long long o = (long long)sample * G.stride;
         double r[NV];
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
-            double x = G.in[o + v * G.ncells + i] * s;
-            x = x + G.u0[o + v * G.ncells + i];
+            double x = l[v] * s;
+            x = x + u[v];
             r[v] = x;
         }
-        if (fe_finish) bad = !EQ::obeys(r, B.gamma);
+        if (fe_finish) bad = !EQ::obeys_fast(r, B.gamma);
 #pragma unroll
         for (int v = 0; v < NV; ++v) G.out[o + v * G.ncells + i] = r[v];
     }
@@ -142,28 +150,36 @@ __global__ __launch_bounds__(256) void batch_ew_kernel(BatchParams B, int fe_fin
 // One sample's end of step (same bookkeeping as finish_step_kernel).
 // Returns the statistics save index this step reached, or -1.
 __device__ __forceinline__ int finish_sample(Control* c, int stats_adj) {
+    const StepInputs k = step_inputs(c);
+    const double t_end = c->t_end;
+    const long long steps = c->steps;
+    const int violated = c->violated, failed = c->block_violation;
+    int pending = c->saves_pending;
     if (!c->active) return -1;
-    const double dt = step_dt(c);
+    const double dt = step_dt(k);
+    const double t = k.t + dt;
     c->dt = dt;
-    c->scale = dt / c->cell[0];
-    c->t = c->t + dt;
-    c->steps = c->steps + 1;
+    c->scale = dt / k.cell[0];
+    c->t = t;
+    c->steps = steps + 1;
     c->last_dt = dt;
     int hit = -1;
-    if (c->block_violation) {
+    if (failed) {
         c->violated = 1;
     } else {
-        for (int i = 0; i < c->n_adj; ++i) {
-            if (c->t >= (double)c->adj_saved[i] * c->adj_interval[i] + c->adj_start[i]) {
-                if (i == stats_adj) hit = (int)c->adj_saved[i];
-                c->adj_saved[i] = c->adj_saved[i] + 1;
-                c->saves_pending = c->saves_pending + 1;
+#pragma unroll
+        for (int i = 0; i < MAX_ADJ; ++i) {
+            if (i < k.n_adj && t >= (double)k.saved[i] * k.interval[i] + k.start[i]) {
+                if (i == stats_adj) hit = (int)k.saved[i];
+                c->adj_saved[i] = k.saved[i] + 1;
+                ++pending;
             }
         }
+        c->saves_pending = pending;
     }
     c->block_violation = 0;
     clear_wave_speeds(c);
-    c->active = (!(c->t >= c->t_end) && !c->violated) ? 1 : 0;
+    c->active = (!(t >= t_end) && !violated && !failed) ? 1 : 0;
     return hit;
 }
 

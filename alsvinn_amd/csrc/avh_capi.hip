@@ -49,22 +49,41 @@ enum EwMode { EW_FE_FINISH = 0, EW_RK2_U1 = 1 };
 template <class EQ>
 __global__ __launch_bounds__(256) void ew_kernel(const double* L, const double* u0, double* out,
                                                  Control* ctrl, long long nc, int mode, double gamma) {
-    if (!ctrl->active) return;
     constexpr int NV = EQ::NV;
+    const long long step = (long long)gridDim.x * blockDim.x;
+    long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    // the first cell's values are in flight while dt is formed
+    double l[NV], u[NV];
+    if (i < nc) {
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            l[v] = L[v * nc + i];
+            u[v] = u0[v * nc + i];
+        }
+    }
+    if (!ctrl->active) return;
     const double s = step_dt(ctrl) / ctrl->cell[0];
     bool bad = false;
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < nc;
-         i += (long long)gridDim.x * blockDim.x) {
+    while (i < nc) {
         double r[NV];
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
-            double o = L[v * nc + i] * s;
-            o = o + u0[v * nc + i];
+            double o = l[v] * s;
+            o = o + u[v];
             r[v] = o;
         }
-        if (mode == EW_FE_FINISH) bad = bad || !EQ::obeys(r, gamma);
+        const long long at = i;
+        i += step;
+        if (i < nc) {
 #pragma unroll
-        for (int v = 0; v < NV; ++v) out[v * nc + i] = r[v];
+            for (int v = 0; v < NV; ++v) {
+                l[v] = L[v * nc + i];
+                u[v] = u0[v * nc + i];
+            }
+        }
+        if (mode == EW_FE_FINISH) bad = bad || !EQ::obeys_fast(r, gamma);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) out[v * nc + at] = r[v];
     }
     if (mode == EW_FE_FINISH) {
         if (__syncthreads_or(bad) && threadIdx.x == 0) atomicOr(&ctrl->block_violation, 1);
@@ -509,11 +528,11 @@ static TuneKey tune_key(const avh_solver* s) {
                    s->cfg.n[2]);
 }
 
-// Times every tile shape on the current state and keeps the fastest: a
-// flux-only launch (writing the L0 buffer, which stage 1 overwrites), and
-// for RK3 also the second stage on its output (input formed on the fly from
-// L0 and U0, writing the U2 buffer), whose extra reads weigh differently on
-// different shapes.  The state is not written; the wave-speed maxima the
+// Times every tile shape on the current state and keeps the fastest: the
+// first stage (writing the L0 buffer, which every step overwrites; flux-only
+// if the solver has stopped), and for RK3 also the second stage on its output
+// (input formed on the fly from L0 and U0, writing the U2 buffer), whose extra
+// reads weigh differently on different shapes.  The state is not written; the wave-speed maxima the
 // launches add to are restored.
 static avh_status autotune(avh_solver* s, int* best, double* ms, int* nshapes) {
     const int ns = num_shapes(s->dim);
@@ -529,7 +548,7 @@ static avh_status autotune(avh_solver* s, int* best, double* ms, int* nshapes) {
     P.in = s->A;
     P.u0 = s->A;
     P.out = s->B;
-    P.mode = MODE_FLUX_ONLY;
+    P.mode = s->h.active ? MODE_L : MODE_FLUX_ONLY;
     StageParams P2 = P;
     P2.in = s->B;
     P2.out = s->C;

@@ -614,6 +614,20 @@ __device__ __forceinline__ void weno2_half_weights(double r0, double r1, double&
     else h0 = 0.5 * h0;
 }
 
+// A face of cell i from the reciprocals ahead (r0) and behind (r1) of it.
+template <int NV, bool RIGHT>
+__device__ __forceinline__ void weno2_face_recips(const double* s, int vs, int i, int sd, double r0, double r1,
+                                                  double* out) {
+    double h0, h1;
+    weno2_half_weights<RIGHT>(r0, r1, h0, h1);
+    const double hc = RIGHT ? 3 * h1 + h0 : 3 * h0 + h1;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+        const double* u = s + v * vs;
+        out[v] = RIGHT ? h0 * u[i + sd] + hc * u[i] - h1 * u[i - sd] : h1 * u[i - sd] + hc * u[i] - h0 * u[i + sd];
+    }
+}
+
 template <int NV, bool RIGHT, class OPS>
 __device__ __forceinline__ void weno2_face(const double* s, int vs, int i, int sd, double* out) {
     const double eps = 1e-8;
@@ -621,15 +635,7 @@ __device__ __forceinline__ void weno2_face(const double* s, int vs, int i, int s
     const double dp = s[i + sd] - w0;
     const double dm = w0 - s[i - sd];
     if constexpr (OPS::SHARED) {
-        double h0, h1;
-        weno2_half_weights<RIGHT>(weno2_recip(dp), weno2_recip(dm), h0, h1);
-        const double hc = RIGHT ? 3 * h1 + h0 : 3 * h0 + h1;
-#pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            const double* u = s + v * vs;
-            out[v] = RIGHT ? h0 * u[i + sd] + hc * u[i] - h1 * u[i - sd]
-                           : h1 * u[i - sd] + hc * u[i] - h0 * u[i + sd];
-        }
+        weno2_face_recips<NV, RIGHT>(s, vs, i, sd, weno2_recip(dp), weno2_recip(dm), out);
         return;
     }
     const double b0 = dp * dp;

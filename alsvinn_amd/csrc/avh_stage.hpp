@@ -184,23 +184,51 @@ __host__ __device__ __forceinline__ void clear_wave_speeds(Control* c) {
 // first stage accumulated; every launch after it evaluates this same
 // expression, so all of them use the identical dt without a grid-wide
 // barrier or fence.
-__device__ __forceinline__ double step_dt(const Control* c) {
+// Everything it reads is loaded before anything is used: the loads then cost
+// one latency, which on small grids is a good part of a launch.
+struct StepInputs {
+    double ws[3], cell[3], cfl, t;
+    double interval[MAX_ADJ], start[MAX_ADJ];
+    long long saved[MAX_ADJ];
+    int n_adj;
+};
+__device__ __forceinline__ StepInputs step_inputs(const Control* c) {
+    StepInputs k;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        k.ws[d] = wave_speed(c, d);
+        k.cell[d] = c->cell[d];
+    }
+    k.cfl = c->cfl;
+    k.t = c->t;
+    k.n_adj = c->n_adj;
+#pragma unroll
+    for (int i = 0; i < MAX_ADJ; ++i) {
+        k.interval[i] = c->adj_interval[i];
+        k.start[i] = c->adj_start[i];
+        k.saved[i] = c->adj_saved[i];
+    }
+    return k;
+}
+__device__ __forceinline__ double step_dt(const StepInputs& k) {
     double total = 0;
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-        if (c->cell[d] == 0) continue;
-        total += wave_speed(c, d) / c->cell[d];
+        if (k.cell[d] == 0) continue;
+        total += k.ws[d] / k.cell[d];
     }
-    double dt = c->cfl / total;
-    for (int i = 0; i < c->n_adj; ++i) {
-        if (c->adj_saved[i] > 0) {
-            const double next = (double)c->adj_saved[i] * c->adj_interval[i] + c->adj_start[i];
-            const double cand = next - c->t;
+    double dt = k.cfl / total;
+#pragma unroll
+    for (int i = 0; i < MAX_ADJ; ++i) {
+        if (i < k.n_adj && k.saved[i] > 0) {
+            const double next = (double)k.saved[i] * k.interval[i] + k.start[i];
+            const double cand = next - k.t;
             dt = (cand < dt) ? cand : dt;
         }
     }
     return dt;
 }
+__device__ __forceinline__ double step_dt(const Control* c) { return step_dt(step_inputs(c)); }
 
 // End of a step, one thread: t += dt, constraint flag, then the writers'
 // save counters (alsfvm/src/simulator/Simulator.cpp:81-85, 180-214;
@@ -208,25 +236,33 @@ __device__ __forceinline__ double step_dt(const Control* c) {
 // `t >= endTime` (Simulator.cpp:77-79); clears the wave-speed maxima for the
 // next step.
 __device__ __forceinline__ void end_step(Control* c, bool violation) {
-    const double dt = step_dt(c);
+    const StepInputs k = step_inputs(c);
+    const double t_end = c->t_end;
+    const long long steps = c->steps;
+    const int violated = c->violated, pause = c->pause_on_save;
+    int pending = c->saves_pending;
+    const double dt = step_dt(k);
+    const double t = k.t + dt;
     c->dt = dt;
-    c->scale = dt / c->cell[0];
-    c->t = c->t + dt;
-    c->steps = c->steps + 1;
+    c->scale = dt / k.cell[0];
+    c->t = t;
+    c->steps = steps + 1;
     c->last_dt = dt;
     if (violation) {
         c->violated = 1;
     } else {
-        for (int i = 0; i < c->n_adj; ++i) {
-            if (c->t >= (double)c->adj_saved[i] * c->adj_interval[i] + c->adj_start[i]) {
-                c->adj_saved[i] = c->adj_saved[i] + 1;
-                c->saves_pending = c->saves_pending + 1;
+#pragma unroll
+        for (int i = 0; i < MAX_ADJ; ++i) {
+            if (i < k.n_adj && t >= (double)k.saved[i] * k.interval[i] + k.start[i]) {
+                c->adj_saved[i] = k.saved[i] + 1;
+                ++pending;
             }
         }
+        c->saves_pending = pending;
     }
     c->block_violation = 0;
     clear_wave_speeds(c);
-    const bool more = !(c->t >= c->t_end) && !c->violated && !(c->pause_on_save && c->saves_pending > 0);
+    const bool more = !(t >= t_end) && !violated && !violation && !(pause && pending > 0);
     c->active = more ? 1 : 0;
 }
 
@@ -242,6 +278,37 @@ __device__ __forceinline__ void arrive_final(Control* c, bool bad) {
     if ((unsigned int)prev == gridDim.x - 1) {
         c->arrive = 0ull;
         end_step(c, ((prev + add) >> 32) != 0ull);
+    }
+}
+
+// What a workgroup leaves behind after its cells.  First stage and flux-only:
+// the wave speeds, a wavefront reduction, then one atomicMax per direction
+// (non-negative doubles order like their bit patterns).  Final stage: whether
+// a cell broke the constraints, and the end of the step.
+template <int NT>
+__device__ __forceinline__ void end_of_tile(const StageParams& P, Control* ctrl, int mode, double w0, double w1,
+                                            double w2, double (*s_ws)[NT / 64], bool bad) {
+    if (mode == MODE_FLUX_ONLY || mode == MODE_L) {
+        const double ws[3] = {w0, w1, w2};
+        const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            const double w = wave_max(ws[d]);
+            if (lane == 0) s_ws[d][wid] = w;
+        }
+        lds_barrier();
+        if (threadIdx.x < 3) {
+            double w = 0.0;
+#pragma unroll
+            for (int i = 0; i < NT / 64; ++i) w = ws_max(w, s_ws[threadIdx.x][i]);
+            if (w > 0.0) atomicMax(&ctrl->ws_bits[threadIdx.x], (unsigned long long)__double_as_longlong(w));
+        }
+    } else if (mode == MODE_RK2_2 || mode == MODE_RK3_3) {
+        const int any_bad = __syncthreads_or(bad);
+        if (threadIdx.x == 0) {
+            if (P.finish) arrive_final(ctrl, any_bad != 0);
+            else if (any_bad) atomicOr(&ctrl->block_violation, 1);
+        }
     }
 }
 
@@ -571,30 +638,7 @@ struct StageKernel {
             }
         }
 
-        if (mode == MODE_FLUX_ONLY || mode == MODE_L) {
-            // wave speed: wavefront reduction, then one atomicMax per direction
-            // per workgroup (non-negative doubles order like their bit patterns)
-            const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                const double w = wave_max(ws[d]);
-                if (lane == 0) s_ws[d][wid] = w;
-            }
-            __syncthreads();
-            if (threadIdx.x < 3) {
-                double w = 0.0;
-#pragma unroll
-                for (int i = 0; i < NT / 64; ++i) w = ws_max(w, s_ws[threadIdx.x][i]);
-                if (w > 0.0)
-                    atomicMax(&ctrl->ws_bits[threadIdx.x], (unsigned long long)__double_as_longlong(w));
-            }
-        } else if (final_stage) {
-            const int any_bad = __syncthreads_or(bad);
-            if (threadIdx.x == 0) {
-                if (P.finish) arrive_final(ctrl, any_bad != 0);
-                else if (any_bad) atomicOr(&ctrl->block_violation, 1);
-            }
-        }
+        end_of_tile<NT>(P, ctrl, mode, ws[0], ws[1], ws[2], s_ws, bad);
     }
 };
 

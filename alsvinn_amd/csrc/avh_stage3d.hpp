@@ -583,28 +583,7 @@ struct MarchKernel3 {
         }
 
 #undef AVH_PREFETCH_RING
-        if (mode == MODE_FLUX_ONLY || mode == MODE_L) {
-            const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                const double wv = wave_max(ws[d]);
-                if (lane == 0) s_ws[d][wid] = wv;
-            }
-            __syncthreads();
-            if (threadIdx.x < 3) {
-                double wv = 0.0;
-#pragma unroll
-                for (int i = 0; i < NT / 64; ++i) wv = ws_max(wv, s_ws[threadIdx.x][i]);
-                if (wv > 0.0)
-                    atomicMax(&ctrl->ws_bits[threadIdx.x], (unsigned long long)__double_as_longlong(wv));
-            }
-        } else if (final_stage) {
-            const int any_bad = __syncthreads_or(bad);
-            if (threadIdx.x == 0) {
-                if (P.finish) arrive_final(ctrl, any_bad != 0);
-                else if (any_bad) atomicOr(&ctrl->block_violation, 1);
-            }
-        }
+        end_of_tile<NT>(P, ctrl, mode, ws[0], ws[1], ws[2], s_ws, bad);
     }
 };
 

@@ -3,6 +3,7 @@
 #pragma once
 #include "avh_batch.hpp"
 #include "avh_stage.hpp"
+#include "avh_stage2d.hpp"
 #include "avh_stage3d.hpp"
 
 namespace avh {
@@ -20,13 +21,13 @@ typedef hipError_t (*VolumeLauncher)(const StageParams& P, const VolumeParams& V
 // order, so the choice never changes a result bit.
 //   1D: (cells, threads) = (256, 256) or (64, 64): small grids get more
 //       workgroups from the smaller tile.
-//   2D: 32x16, 16x15, 64x4, 32x15 or 24x20 cells, 256 threads (LDS 40.8,
-//       20.7, 28.0, 38.6 and 38.0 KB for euler2 with WENO2).  A
-//       flux pass hands interface items to threads in turns of 256, and a
-//       turn costs a wave its full instruction stream however few of its
-//       lanes have an item, so shapes whose interface counts sit just under
-//       a multiple of 256 waste the least: 32x15 (495 x- / 512 y-interfaces),
-//       24x20 (500 / 504) and 16x15 (255 / 256), against 32x16 (528 / 544).
+//   2D: 64x7, 16x15, 16x7, 32x15 or 16x28 cells, 256 threads.  A flux pass
+//       costs a wave its full instruction stream however few of its lanes
+//       have an item, so the shapes' items sit just under the 256 threads:
+//       two interfaces a thread for 64x7 (231 x / 256 y turns), 32x15 (255 /
+//       256) and 16x28 (252 / 240), one for 16x15 (255 / 256), and one for
+//       both directions together for 16x7 (119 + 128), the shape of small
+//       grids: more workgroups and half the chain.
 //   3D: 16x15 or 32x7 columns marching over 2 to 32 planes, 256 threads (at
 //       most 256 interfaces a plane in each direction: one turn; the threads
 //       past the columns only work on the planes).  A chunk pays a z flux
@@ -36,8 +37,8 @@ typedef hipError_t (*VolumeLauncher)(const StageParams& P, const VolumeParams& V
 //       200x150x120 575 / 539 / 598 / 722, 97x83x61 120 / 140 / 173 / 326).
 constexpr int NSHAPES1 = 2, NSHAPES2 = 5, NSHAPES3 = 7;
 constexpr int SHAPE1_TX[NSHAPES1] = {256, 64};
-constexpr int SHAPE2_TX[NSHAPES2] = {32, 16, 64, 32, 24};
-constexpr int SHAPE2_TY[NSHAPES2] = {16, 15, 4, 15, 20};
+constexpr int SHAPE2_TX[NSHAPES2] = {64, 16, 16, 32, 16};
+constexpr int SHAPE2_TY[NSHAPES2] = {7, 15, 7, 15, 28};
 constexpr int SHAPE3_TX[NSHAPES3] = {16, 16, 32, 32, 16, 16, 16};
 constexpr int SHAPE3_TY[NSHAPES3] = {15, 15, 7, 7, 15, 15, 15};
 constexpr int SHAPE3_LZ[NSHAPES3] = {4, 8, 8, 32, 16, 2, 32};
@@ -52,17 +53,16 @@ struct KernelFor<EQ, RECON, FLUX, 1, S> {
 };
 template <class EQ, int RECON, class FLUX, int S>
 struct KernelFor<EQ, RECON, FLUX, 2, S> {
-    typedef StageKernel<EQ, RECON, FLUX, 2, SHAPE2_TX[S], SHAPE2_TY[S], 1, 256> type;
+    typedef TileKernel2<EQ, RECON, FLUX, SHAPE2_TX[S], SHAPE2_TY[S], 256> type;
 };
 // 2D shapes whose RK3 stages are each compiled for their mode (the shapes
-// the autotuner takes for the benchmark grids and the batched set); those
-// kernels index cells with 32-bit values, so they serve grids of fewer than
-// 2^29 cells (per sample in a batch)
-constexpr bool SHAPE2_BY_MODE[NSHAPES2] = {false, false, false, true, true};
+// the autotuner takes most); those kernels index cells with 32-bit values, so
+// they serve grids of fewer than 2^29 cells (per sample in a batch)
+constexpr bool SHAPE2_BY_MODE[NSHAPES2] = {false, false, true, true, false};
 constexpr long long MODE_KERNEL_MAX_CELLS = 1ll << 29;
 template <class EQ, int RECON, class FLUX, int S, int MODE>
 struct KernelForMode {
-    typedef StageKernel<EQ, RECON, FLUX, 2, SHAPE2_TX[S], SHAPE2_TY[S], 1, 256, MODE> type;
+    typedef TileKernel2<EQ, RECON, FLUX, SHAPE2_TX[S], SHAPE2_TY[S], 256, MODE> type;
 };
 
 // stage tiles (workgroups) covering one grid of the 1D / 2D kernels
@@ -199,7 +199,7 @@ struct VolumeKernelFor<EQ, RECON, FLUX, 1> {
 };
 template <class EQ, int RECON, class FLUX>
 struct VolumeKernelFor<EQ, RECON, FLUX, 2> {
-    typedef StageKernel<EQ, RECON, FLUX, 2, 32, 15, 1, 256> type;
+    typedef TileKernel2<EQ, RECON, FLUX, 32, 15, 256> type;
 };
 template <class EQ, int RECON, class FLUX>
 struct VolumeKernelFor<EQ, RECON, FLUX, 3> {

@@ -591,9 +591,10 @@ TuneKey batch_tune_key(const avh_batch* b) {
                    b->g[0].n[1], total);
 }
 
-// Times every tile shape with flux-only launches over all samples (they write
-// the L0 buffers and add to the per-sample wave-speed maxima; the control
-// blocks are restored afterwards) and keeps the fastest.
+// Times every tile shape over all samples with the first stage (flux-only if
+// every sample has stopped) and, for RK3, the second stage, and keeps the
+// fastest.  They write the L0 and U2 buffers and add to the per-sample
+// wave-speed maxima; the control blocks are restored afterwards.
 void set_all_live(avh_batch* b);
 
 avh_status batch_autotune(avh_batch* b, int* best, double* ms, int* nshapes) {
@@ -606,6 +607,10 @@ avh_status batch_autotune(avh_batch* b, int* best, double* ms, int* nshapes) {
         AVH_HIP(hipMemcpy(saved[i].data(), b->g[i].ctrl, sizeof(Control) * b->g[i].nsamples,
                           hipMemcpyDeviceToHost));
     }
+    bool active = false;
+    for (const auto& cs : saved)
+        for (const Control& c : cs) active = active || c.active;
+    const bool rk3 = active && b->cfg.integrator == AVH_INT_RUNGEKUTTA3;
     const int keep = b->shape;
     int bst = 0;
     double tmin = 0;
@@ -615,13 +620,21 @@ avh_status batch_autotune(avh_batch* b, int* best, double* ms, int* nshapes) {
         if (ns > 1) {
             b->shape = k;
             unsigned int nb = 0;
-            BatchParams P = batch_params(b, MODE_FLUX_ONLY, false, &nb);
+            BatchParams P = batch_params(b, active ? MODE_L : MODE_FLUX_ONLY, false, &nb);
+            BatchParams P2 = batch_params(b, MODE_RK3_2, false, &nb);
             for (int i = 0; i < b->ngroups; ++i) {
-                P.g[i].in = b->g[i].A;
-                P.g[i].u0 = b->g[i].A;
+                P.g[i].in = P.g[i].u0 = P2.g[i].u0 = b->g[i].A;
                 P.g[i].out = b->g[i].B;
+                P2.g[i].in = b->g[i].B;
+                P2.g[i].out = b->g[i].C;
             }
-            r = time_launches(b->stream, 3, [&]() { return b->stage(P, nb, k, b->stream); }, &t);
+            r = time_launches(b->stream, 3,
+                              [&]() {
+                                  hipError_t e = b->stage(P, nb, k, b->stream);
+                                  if (e == hipSuccess && rk3) e = b->stage(P2, nb, k, b->stream);
+                                  return e;
+                              },
+                              &t);
         }
         if (ms) ms[k] = t;
         if (k == 0 || t < tmin) {

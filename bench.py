@@ -26,7 +26,7 @@ import sys
 import time
 
 HBM_PEAK_GBS = 8000.0
-SHAPE_NAMES = {1: ["256", "64"], 2: ["32x16", "16x15", "64x4", "32x15", "24x20"],
+SHAPE_NAMES = {1: ["256", "64"], 2: ["64x7", "16x15", "16x7", "32x15", "16x28"],
                3: ["16x15 columns x 4 planes", "16x15 columns x 8 planes", "32x7 columns x 8 planes",
                    "32x7 columns x 32 planes", "16x15 columns x 16 planes", "16x15 columns x 2 planes",
                    "16x15 columns x 32 planes"]}
@@ -45,7 +45,7 @@ WORKLOADS = {
 # Sources of the stage kernels: a profile summary under profiles/ records the
 # digest of the sources it was measured on, and its traffic / instruction
 # figures are reported only while the sources still match.
-KERNEL_SOURCES = ["avh_physics.hpp", "avh_stage.hpp", "avh_stage3d.hpp", "avh_stage_inst.hpp", "avh_batch.hpp",
+KERNEL_SOURCES = ["avh_physics.hpp", "avh_stage.hpp", "avh_stage2d.hpp", "avh_stage3d.hpp", "avh_stage_inst.hpp", "avh_batch.hpp",
                   "avh_stage_burgers.hip", "avh_stage_euler1.hip", "avh_stage_euler2.hip", "avh_stage_euler3.hip",
                   "avh_stage_euler3_none.hip", "avh_stage_euler3_weno2.hip", "avh_stage_euler3_eno2.hip",
                   "avh_stage_euler3_eno3.hip"]
