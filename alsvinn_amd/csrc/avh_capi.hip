@@ -443,10 +443,12 @@ struct avh_solver {
     Control h{};  // host mirror of ctrl, valid after pull()
     hipStream_t stream = nullptr;
     StageLauncher stage = nullptr;
+    LineLauncher line = nullptr;  // small 1D grids: steps in one workgroup
     EwLauncher ew = nullptr;
     int graph_steps = 16;  // steps per captured hipGraph (0: ordinary launches)
     StepGraph graph;
     int shape = -1;        // tile shape of the stage kernel; -1: autotune on first use
+    bool shape_fixed = false;  // by avh_set_tile_shape
 };
 
 static avh_status use_device(const avh_solver* s) {
@@ -595,7 +597,26 @@ static avh_status ensure_shape(avh_solver* s) {
     return autotune(s, nullptr, nullptr, nullptr);
 }
 
+// the solver's steps run in one workgroup (a fixed tile shape asks for the
+// stage kernels)
+static bool line_steps(const avh_solver* s) { return s->line && !s->shape_fixed; }
+
 static avh_status enqueue_steps(avh_solver* s, int64_t n) {
+    if (line_steps(s)) {
+        LineParams P;
+        P.state = s->A;
+        P.ctrl = s->ctrl;
+        P.n = s->cfg.n[0];
+        P.bc = s->cfg.boundary;
+        P.integrator = s->cfg.integrator == AVH_INT_FORWARDEULER ? 0 : (s->cfg.integrator == AVH_INT_RUNGEKUTTA2 ? 1 : 2);
+        P.gamma = s->cfg.gamma;
+        // a launch of at most 4096 steps keeps it to some ten milliseconds
+        for (; n > 0; n -= P.steps) {
+            P.steps = (int)std::min<int64_t>(n, 4096);
+            AVH_HIP(s->line(P, s->stream));
+        }
+        return AVH_OK;
+    }
     avh_status r = ensure_shape(s);
     if (r) return r;
     return enqueue_steps_graphed(s->graph, s->graph_steps, s->stream, n, [s]() { return enqueue_step(s); });
@@ -663,8 +684,8 @@ avh_status avh_solver_create(avh_ctx* ctx, const avh_config* cfg, avh_solver** o
     for (int d = 0; d < dim; ++d)
         if (cfg->n[d] < ng)
             return fail(AVH_EINVAL, "too few cells: every active axis needs at least as many cells as ghost cells");
-    const StageLauncher st = launchers_for(cfg->equation, cfg->reconstruction, cfg->flux, dim).stage;
-    if (!st)
+    const Launchers launchers = launchers_for(cfg->equation, cfg->reconstruction, cfg->flux, dim);
+    if (!launchers.stage)
         return fail(AVH_EINVAL,
                     "unsupported combination of equation, flux and grid dimension (burgers: godunov; "
                     "euler<n>: hll, hll3 with at most n active axes)");
@@ -682,7 +703,9 @@ avh_status avh_solver_create(avh_ctx* ctx, const avh_config* cfg, avh_solver** o
     s->g[2] = dim > 2 ? ng : 0;
     s->ncells = (long long)cfg->n[0] * cfg->n[1] * cfg->n[2];
     s->nghosted = (long long)(cfg->n[0] + 2 * s->g[0]) * (cfg->n[1] + 2 * s->g[1]) * (cfg->n[2] + 2 * s->g[2]);
-    s->stage = st;
+    s->stage = launchers.stage;
+    if (dim == 1 && cfg->n[0] + (cfg->boundary == AVH_BC_PERIODIC ? 0 : 1) <= line_interfaces(s->nv))
+        s->line = launchers.line;
     s->ew = ew_for(cfg->equation);
     const size_t bytes = (size_t)nv * s->ncells * sizeof(double);
     if (hipMalloc(&s->A, bytes) != hipSuccess || hipMalloc(&s->B, bytes) != hipSuccess ||
@@ -934,6 +957,7 @@ avh_status avh_prepare_graph(avh_solver* s) {
     if (!s) return fail(AVH_EINVAL, "null argument");
     avh_status r = use_device(s);
     if (r) return r;
+    if (line_steps(s)) return AVH_OK;  // nothing to capture
     if ((r = ensure_shape(s))) return r;
     return ensure_step_graph(s->graph, s->graph_steps, s->stream, [s]() { return enqueue_step(s); });
 }
@@ -956,6 +980,7 @@ avh_status avh_set_tile_shape(avh_solver* s, int shape) {
     AVH_HIP(hipStreamSynchronize(s->stream));
     s->graph.reset();
     s->shape = shape;
+    s->shape_fixed = shape >= 0;
     return AVH_OK;
 }
 
@@ -1043,8 +1068,7 @@ avh_status avh_step(avh_solver* s, double* dt_out) {
     s->h.pause_on_save = 0;
     s->h.active = 1;
     if ((r = push(s))) return r;
-    if ((r = ensure_shape(s))) return r;
-    if ((r = enqueue_step(s))) return r;
+    if ((r = enqueue_steps(s, 1))) return r;
     if ((r = pull(s))) return r;
     s->h.t_end = t_end;
     s->h.pause_on_save = pause;

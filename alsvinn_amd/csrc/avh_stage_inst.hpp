@@ -2,6 +2,7 @@
 // reconstruction, flux and grid dimension the equation supports.
 #pragma once
 #include "avh_batch.hpp"
+#include "avh_line.hpp"
 #include "avh_stage.hpp"
 #include "avh_stage2d.hpp"
 #include "avh_stage3d.hpp"
@@ -213,8 +214,31 @@ hipError_t launch_volume_stage(const StageParams& P, const VolumeParams& V, hipS
     return hipGetLastError();
 }
 
+// Steps of a small 1D grid in one workgroup (avh_line.hpp), for burgers and
+// euler1.
+typedef hipError_t (*LineLauncher)(const LineParams& P, hipStream_t stream);
+
+template <class K>
+hipError_t launch_line_k(const LineParams& P, int threads, hipStream_t stream) {
+    hipLaunchKernelGGL(line_kernel<K>, dim3(1), dim3(threads), K::lds_bytes(P.n), stream, P);
+    return hipGetLastError();
+}
+
+template <class EQ, int RECON, class FLUX>
+hipError_t launch_line(const LineParams& P, hipStream_t stream) {
+    const int ni = P.bc == BC_PERIODIC ? P.n : P.n + 1;
+    const int cpt = ni <= 512 ? 1 : (ni <= 1024 ? 2 : 4);
+    const int threads = ((ni + cpt - 1) / cpt + 63) / 64 * 64;
+    if (ni > line_interfaces(EQ::NV)) return hipErrorInvalidValue;
+    if (cpt == 1) return launch_line_k<LineKernel<EQ, RECON, FLUX, 1>>(P, threads, stream);
+    if (cpt == 2) return launch_line_k<LineKernel<EQ, RECON, FLUX, 2>>(P, threads, stream);
+    if constexpr (EQ::NV == 1) return launch_line_k<LineKernel<EQ, RECON, FLUX, 4>>(P, threads, stream);
+    return hipErrorInvalidValue;
+}
+
 struct Launchers {
     StageLauncher stage = nullptr;
+    LineLauncher line = nullptr;
     BatchLauncher batch = nullptr;
     VolumeLauncher volume = nullptr;
 };
@@ -224,6 +248,7 @@ Launchers launchers_of() {
     Launchers L;
     L.stage = &launch_stage<EQ, RECON, FLUX, DIM>;
     if (DIM < 3) L.batch = &launch_batch_stage<EQ, RECON, FLUX, DIM>;
+    if constexpr (DIM == 1 && EQ::NV <= 3) L.line = &launch_line<EQ, RECON, FLUX>;
     L.volume = &launch_volume_stage<EQ, RECON, FLUX, DIM>;
     return L;
 }
