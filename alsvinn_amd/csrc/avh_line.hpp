@@ -13,14 +13,14 @@
 // A workgroup takes at most 512 threads and up to four interfaces a thread:
 // each wavefront evaluates dt and the bookkeeping for itself, about 200
 // instructions a step, and with 1024 threads these were a good part of a step
-// (burgers, weno2, 1024 cells: 7.6 us a step with 1024 threads, 5.5 with 512).
+// (burgers, eno3, 1024 cells: 6.5 us a step with 1024 threads, 4.5 with 512).
 // What is left at 200 cells is the chain of one interface's operations, three
 // times a step; from 1024 cells on it is the issue rate of the one compute
 // unit.  Time of a step, rk3, in microseconds, against three stage launches:
 //   cells              64    200    512   1024   1500   2048   3000
-//   burgers none      1.3    1.7    2.1    2.8    4.3    4.4    7.2
+//   burgers none      1.3    1.7    2.1    2.8    4.3    4.5    7.2
 //     stages          9.5   10.2   11.2   11.3   11.9   11.1   11.7
-//   burgers weno2     2.0    2.4    3.4    5.5    9.6    9.9   18.0
+//   burgers weno2     2.1    2.5    3.4    5.1    8.8    8.9
 //     stages         11.3   11.3   12.8   12.9   12.5   12.7   12.9
 //   euler1 none       3.6    4.0    5.6    9.8   18.0   18.1   38.1
 //     stages         13.5   13.8   16.2   16.3   16.2   16.0   16.3

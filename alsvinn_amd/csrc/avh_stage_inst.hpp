@@ -256,10 +256,10 @@ Launchers launchers_of() {
 template <class EQ, class FLUX, int DIM>
 Launchers pick_recon(int recon) {
     switch (recon) {
-    case RECON_NONE: return launchers_of<EQ, RECON_NONE, FLUX, DIM>();
-    case RECON_WENO2: return launchers_of<EQ, RECON_WENO2, FLUX, DIM>();
-    case RECON_ENO2: return launchers_of<EQ, RECON_ENO2, FLUX, DIM>();
-    case RECON_ENO3: return launchers_of<EQ, RECON_ENO3, FLUX, DIM>();
+    case RECON_NONE: return launchers_of<EQ, RECON_NONE, typename FLUX::template For<RECON_NONE>, DIM>();
+    case RECON_WENO2: return launchers_of<EQ, RECON_WENO2, typename FLUX::template For<RECON_WENO2>, DIM>();
+    case RECON_ENO2: return launchers_of<EQ, RECON_ENO2, typename FLUX::template For<RECON_ENO2>, DIM>();
+    case RECON_ENO3: return launchers_of<EQ, RECON_ENO3, typename FLUX::template For<RECON_ENO3>, DIM>();
     }
     return Launchers();
 }

@@ -107,3 +107,38 @@ def test_guard_bounds_bitwise(equation, n, bound):
                 assert np.array_equal(np.isnan(out_h), nan)
                 assert np.array_equal(np.asarray(ws_h).view(np.uint64), np.asarray(ws_o).view(np.uint64))
                 assert np.array_equal(got[~nan], want[~nan]), "shape %d" % shape
+
+
+BURGERS = {"zeros": None, "tiny": (-1070, -590), "about 2^-600": (-606, -594), "about 2^85": (80, 90),
+           "all": (-1070, 200)}
+
+
+@pytest.mark.parametrize("bound", sorted(BURGERS))
+@pytest.mark.parametrize("n", [(97,), (45, 34), (19, 17, 9)])
+def test_burgers_guard_bounds_bitwise(n, bound):
+    """Burgers' WENO2 weights on both sides of the cell check: the net flux on
+    every tile shape, and in 1D a step (the one-workgroup path)."""
+    from oracle import pyoracle
+    r = np.random.default_rng(len(bound) * 10 + len(n))
+    q = np.ascontiguousarray(smooth_state("burgers", n, seed=len(bound), jump=True))
+    at = _pick(r, q)
+    q[0][at] = (r.choice([-0.0, 0.0], size=q[0].shape) if BURGERS[bound] is None else
+                _pow2(r, q[0].shape, BURGERS[bound]) * r.choice([-1.0, 1.0], size=q[0].shape))[at]
+    print("case burgers guard", bound, n, flush=True)
+    o, h = make_pair(pyoracle, "burgers", "weno2", "godunov", "rungekutta3", "periodic", n, 0.4)
+    o.set_interior(q)
+    U = o.get_state()
+    out_o, ws_o = pyoracle.compute_flux(o.cfg, U, np.zeros_like(U))
+    want = np.ascontiguousarray(o.interior(out_o)).view(np.uint64)
+    for shape in range((2, 5, 7)[len(n) - 1]):
+        h.set_tile_shape(shape)
+        h.set_interior(q)
+        out_h, ws_h = h.compute_flux()
+        assert np.array_equal(np.asarray(ws_h).view(np.uint64), np.asarray(ws_o).view(np.uint64))
+        assert np.array_equal(np.ascontiguousarray(out_h).view(np.uint64), want), "shape %d" % shape
+    h.set_tile_shape(-1)
+    h.set_interior(q)
+    h.perform_step()
+    o.step()
+    assert np.array_equal(h.get_interior().view(np.uint64),
+                          np.ascontiguousarray(o.interior(o.get_state())).view(np.uint64))
