@@ -328,7 +328,6 @@ struct EulerEq {
 // of 1024 cells, rk3: 5.5 -> 5.1 us).
 template <bool FAST_>
 struct GodunovFluxT {
-    typedef GodunovFluxT<false> Plain;
     template <int RECON>
     using For = GodunovFluxT<RECON == RECON_WENO2>;
     static constexpr bool FAST = FAST_;
@@ -351,12 +350,10 @@ typedef GodunovFluxT<false> GodunovFlux;
 // euler::HLL (alsfvm/include/alsfvm/numflux/euler/HLL.hpp).  The reference's
 // if/else chain is evaluated branch-free: every candidate is computed and the
 // chain's answer is selected, which gives the same value as the branch taken.
-template <bool FAST_>
-struct HLLFluxT {
-    typedef HLLFluxT<false> Plain;
+struct HLLFlux {
     template <int RECON>
-    using For = HLLFluxT;
-    static constexpr bool FAST = FAST_;  // the stage kernel runs flux_ops<SharedOps> first
+    using For = HLLFlux;
+    static constexpr bool FAST = true;  // the stage kernel runs flux_ops<SharedOps> first
     template <int DIR, class EQ>
     __device__ __forceinline__ static double flux(const typename EQ::All& L, const typename EQ::All& R,
                                                   double g, double* F) {
@@ -425,12 +422,10 @@ struct HLLFluxT {
 // euler::HLL3 (alsfvm/include/alsfvm/numflux/euler/HLL3.hpp:52-148).  The two
 // star-state branches (sm >= 0 / sm < 0) share one formula on the side's
 // variables, so the side is selected first and the formula evaluated once.
-template <bool FAST_>
-struct HLL3FluxT {
-    typedef HLL3FluxT<false> Plain;
+struct HLL3Flux {
     template <int RECON>
-    using For = HLL3FluxT;
-    static constexpr bool FAST = FAST_;  // the stage kernel runs flux_ops<SharedOps> first
+    using For = HLL3Flux;
+    static constexpr bool FAST = true;  // the stage kernel runs flux_ops<SharedOps> first
     // The star state of side k (k = L when s_m >= 0, else R): its speed sk,
     // the star conserved state `mid`, the side's conserved state `uc` and
     // its point flux `fk`, formed from side k's values by point_flux's
@@ -568,9 +563,6 @@ struct HLL3FluxT {
         return fmax(fabs(sl), fabs(sr));
     }
 };
-
-typedef HLLFluxT<true> HLLFlux;
-typedef HLL3FluxT<true> HLL3Flux;
 
 // ---------------------------------------------------------------------------
 // Reconstructions on an LDS tile.  `s` points at variable 0 of the tile,

@@ -1,16 +1,17 @@
-// Fused FP64 finite-volume stage kernel.
+// Fused FP64 finite-volume stage kernels: what all of them share, and the 1D
+// one (2D: avh_stage2d.hpp, 3D: avh_stage3d.hpp).
 //
-// One launch = one RK stage over the whole grid.  Each workgroup owns a
-// TX x TY x TZ tile of interior cells:
+// One launch = one RK stage over the whole grid.  Each workgroup owns a tile
+// of interior cells:
 //   1. stage the tile plus a GHOST-wide halo of the stage input into LDS;
 //      halo cells outside the domain are read through the boundary map
 //      (periodic wrap / neumann mirror), which is the ghost fill of the
 //      reference done at load time; in the on-the-fly modes the stage input
 //      is formed while loading as U1 = L0*s + U0;
-//   2. per direction: one work item per interface, reconstructing the right
-//      face of the left cell and the left face of the right cell and
-//      evaluating the numerical flux; fluxes go to LDS, the interface wave
-//      speeds to a per-thread max;
+//   2. per direction: every interface, reconstructing the right face of the
+//      left cell and the left face of the right cell and evaluating the
+//      numerical flux; fluxes go to LDS, the interface wave speeds to a
+//      per-thread max;
 //   3. each thread accumulates the net flux of its cells in registers,
 //      out = 0 + ((-F[i+1/2]) + F[i-1/2]) per direction, exactly as
 //      NumericalFluxCPU::computeNetFlux does on a zeroed output;
@@ -101,6 +102,9 @@ struct VolumeParams {
     int tot[3];    // cells per axis including ghosts
     int ghost[3];  // ghost cells per axis of the volume
     int org[3];    // first cell of the box, interior coordinates
+    // a combination in place of the net flux L: out = ((L*s + in) * ca + u0) * cb
+    const double* u0[5];
+    double s, ca, cb;
 };
 
 __device__ __forceinline__ long long volume_index(const VolumeParams& V, int x, int y, int z) {
@@ -312,144 +316,28 @@ __device__ __forceinline__ void end_of_tile(const StageParams& P, Control* ctrl,
     }
 }
 
-// MODE_CT >= 0 compiles the kernel for that StageMode alone (P.mode must
-// equal it): the other modes' branches and registers drop out.
-template <class EQ, int RECON, class FLUX, int DIM, int TX, int TY, int TZ, int NT, int MODE_CT = -1>
-struct StageKernel {
-    // the kernels compiled per stage mode index cells with 32-bit values
-    // (their launchers take them only for grids of fewer than 2^29 cells)
-    static constexpr bool OFF32 = MODE_CT >= 0;
-    typedef typename std::conditional<OFF32, unsigned int, long long>::type Idx;
+// 1D grids too large for one workgroup (avh_line.hpp): a tile of TX cells.
+template <class EQ, int RECON, class FLUX, int TX, int NT>
+struct StageKernel1 {
+    typedef typename OpsFor<FLUX::FAST>::type Ops;
     static constexpr int NV = EQ::NV;
     static constexpr int G = ReconTraits<RECON>::GHOST;
-    static constexpr int HX = G;
-    static constexpr int HY = DIM >= 2 ? G : 0;
-    static constexpr int HZ = DIM >= 3 ? G : 0;
-    static constexpr int LX = TX + 2 * HX;
-    static constexpr int LY = TY + 2 * HY;
-    static constexpr int LZ = TZ + 2 * HZ;
-    static constexpr int LT = LX * LY * LZ;  // tile cells incl. halo
-    static constexpr int NI_X = (TX + 1) * TY * TZ;
-    static constexpr int NI_Y = DIM >= 2 ? TX * (TY + 1) * TZ : 0;
-    static constexpr int NI_Z = DIM >= 3 ? TX * TY * (TZ + 1) : 0;
-    static constexpr int NI_MAX = NI_X > NI_Y ? (NI_X > NI_Z ? NI_X : NI_Z) : (NI_Y > NI_Z ? NI_Y : NI_Z);
-    static constexpr int TC = TX * TY * TZ;
-    static constexpr int TXC = TX, TYC = TY, TZC = TZ;
+    static constexpr int LT = TX + 2 * G;  // tile cells incl. halo
+    static constexpr int NI = TX + 1;
     static constexpr int NTHREADS = NT;
-    static constexpr int CPT = (TC + NT - 1) / NT;  // cells per thread in phase 3
-    static constexpr int LDS_BYTES = (NV * LT + NV * NI_MAX) * 8;
+    static constexpr int CPT = (TX + NT - 1) / NT;  // cells per thread
 
-    __device__ __forceinline__ static int lidx(int cx, int cy, int cz) {
-        return ((cz + HZ) * LY + (cy + HY)) * LX + (cx + HX);
-    }
-
-    // reconstruct both sides of the interface between cell ia and ia + SD
-    // (LDS indices) and evaluate the numerical flux under OPS; `ok` comes in
-    // as whether the cells are admitted to SharedOps
-    template <class OPS, int DIR>
-    __device__ __forceinline__ static double interface(const double* su, int ia, int SD, double gamma,
-                                                       double* F, bool& ok) {
+    // reconstruct both sides of the interface between cells ia and ia + 1 (LDS
+    // indices) and evaluate the numerical flux under OPS; `ok` comes in as
+    // whether the cells are admitted to SharedOps
+    template <class OPS>
+    __device__ __forceinline__ static double interface(const double* su, int ia, double gamma, double* F, bool& ok) {
         double qa[NV], qb[NV];
-        recon_face_ops<RECON, NV, true, OPS>(su, LT, ia, SD, qa);        // right face of a
-        recon_face_ops<RECON, NV, false, OPS>(su, LT, ia + SD, SD, qb);  // left face of b
+        recon_face_ops<RECON, NV, true, OPS>(su, LT, ia, 1, qa);       // right face of a
+        recon_face_ops<RECON, NV, false, OPS>(su, LT, ia + 1, 1, qb);  // left face of b
         const typename EQ::All aL = EQ::template make_all_ops<OPS>(qa, gamma, ok);
         const typename EQ::All aR = EQ::template make_all_ops<OPS>(qb, gamma, ok);
-        return FLUX::template flux_ops<OPS, DIR, EQ>(aL, aR, gamma, F, ok);
-    }
-
-    // cell a = (cx, cy, cz) left of interface `it` along DIR, and whether the
-    // interface lies inside the grid
-    template <int DIR>
-    __device__ __forceinline__ static bool interface_cell(int it, int ox, int oy, int oz, const int* n, int& ia) {
-        int cx, cy, cz, k;
-        if (DIR == 0) {
-            k = it % (TX + 1);
-            const int r = it / (TX + 1);
-            cy = r % TY;
-            cz = r / TY;
-            cx = k - 1;
-        } else if (DIR == 1) {
-            cx = it % TX;
-            const int r = it / TX;
-            k = r % (TY + 1);
-            cz = r / (TY + 1);
-            cy = k - 1;
-        } else {
-            cx = it % TX;
-            cy = (it / TX) % TY;
-            k = it / (TX * TY);
-            cz = k - 1;
-        }
-        ia = lidx(cx, cy, cz);
-        const int ga = (DIR == 0 ? ox + cx : (DIR == 1 ? oy + cy : oz + cz));
-        return (ga < n[DIR]) && (oy + (DIR == 1 ? 0 : cy) < n[1]) && (ox + (DIR == 0 ? 0 : cx) < n[0]) &&
-               (oz + (DIR == 2 ? 0 : cz) < n[2]);
-    }
-
-    // Fluxes of every interface along DIR into sf.  A FAST flux evaluates each
-    // interface with shared reciprocals (SharedOps); the interfaces whose
-    // operands fall outside the range where that is exact are redone with
-    // PlainOps in a second loop, after the first one's registers are free.
-    // `adm`: every cell of the tile and its halo is admitted to SharedOps.
-    template <int DIR>
-    __device__ __forceinline__ static void flux_pass(const double* su, double* sf, int ox, int oy, int oz,
-                                                     const int* n, double gamma, bool adm, double& ws) {
-        constexpr int NI = DIR == 0 ? NI_X : (DIR == 1 ? NI_Y : NI_Z);
-        constexpr int SD = DIR == 0 ? 1 : (DIR == 1 ? LX : LX * LY);
-        static_assert((NI + NT - 1) / NT <= 32, "one redo bit per iteration");
-        typedef typename OpsFor<FLUX::FAST>::type Ops;
-        unsigned int redo = 0;
-        int m = 0;
-        for (int it = threadIdx.x; it < NI; it += NT, ++m) {
-            int ia;
-            if (!interface_cell<DIR>(it, ox, oy, oz, n, ia)) continue;
-            double F[NV];
-            bool ok = adm;
-            const double w = interface<Ops, DIR>(su, ia, SD, gamma, F, ok);
-            if (ok) {
-                ws = ws_max(ws, w);
-            } else {
-                redo |= 1u << m;
-            }
-#pragma unroll
-            for (int v = 0; v < NV; ++v) sf[v * NI_MAX + it] = F[v];
-        }
-        if (FLUX::FAST && redo != 0) {
-            m = 0;
-            for (int it = threadIdx.x; it < NI; it += NT, ++m) {
-                int ia;
-                if (!((redo >> m) & 1u) || !interface_cell<DIR>(it, ox, oy, oz, n, ia)) continue;
-                double F[NV];
-                bool ok = true;
-                ws = ws_max(ws, interface<PlainOps, DIR>(su, ia, SD, gamma, F, ok));
-#pragma unroll
-                for (int v = 0; v < NV; ++v) sf[v * NI_MAX + it] = F[v];
-            }
-        }
-    }
-
-    template <int DIR>
-    __device__ __forceinline__ static void accumulate(const double* sf, double (&acc)[CPT][NV]) {
-#pragma unroll
-        for (int m = 0; m < CPT; ++m) {
-            const int c = threadIdx.x + m * NT;
-            if (TC % NT != 0 && c >= TC) continue;
-            const int cx = c % TX;
-            const int cy = (c / TX) % TY;
-            const int cz = c / (TX * TY);
-            int ip;
-            if (DIR == 0) ip = (cz * TY + cy) * (TX + 1) + cx + 1;
-            else if (DIR == 1) ip = (cz * (TY + 1) + cy + 1) * TX + cx;
-            else ip = ((cz + 1) * TY + cy) * TX + cx;
-            constexpr int STEP = DIR == 0 ? 1 : (DIR == 1 ? TX : TX * TY);
-#pragma unroll
-            for (int v = 0; v < NV; ++v) {
-                const double fp = sf[v * NI_MAX + ip];
-                const double fm = sf[v * NI_MAX + ip - STEP];
-                // temp = -F; out[i] += temp[i] + (-1)*temp[i-1]
-                acc[m][v] = acc[m][v] + ((-fp) + fm);
-            }
-        }
+        return FLUX::template flux_ops<OPS, 0, EQ>(aL, aR, gamma, F, ok);
     }
 
     __device__ static void run(const StageParams& P) { run_tile(P, tile_id_xcd(blockIdx.x, gridDim.x)); }
@@ -458,60 +346,45 @@ struct StageKernel {
     }
 
     // number of tiles covering a grid of n cells
-    __host__ __device__ static unsigned int tiles(const int* n) {
-        return (unsigned int)(((n[0] + TX - 1) / TX) * ((n[1] + TY - 1) / TY) * ((n[2] + TZ - 1) / TZ));
-    }
+    __host__ __device__ static unsigned int tiles(const int* n) { return (unsigned int)((n[0] + TX - 1) / TX); }
 
-    // VOL: the cells live in a reference Volume (V) and P.n is the extent of
-    // the box the launch covers; otherwise in the interior-only buffers of P
-    // with the boundary map for the halo.
+    // VOL: the cells live in a reference Volume (V; MODE_FLUX_ONLY, or
+    // MODE_RK3_3 for the combination V describes) and P.n is the extent of the
+    // box the launch covers; otherwise in the interior-only buffers of P with
+    // the boundary map for the halo.
     template <bool VOL = false>
     __device__ static void run_tile(const StageParams& P, const unsigned int tile, const VolumeParams* V = nullptr) {
-        __shared__ double lds[NV * LT + NV * NI_MAX];
+        __shared__ double su[NV * LT];
+        __shared__ double sf[NV * NI];
         __shared__ double s_ws[3][NT / 64];
         __shared__ int s_adm[NT / 64];
-        double* su = lds;
-        double* sf = lds + NV * LT;
 
         Control* ctrl = P.ctrl;
-        const int mode = MODE_CT >= 0 ? MODE_CT : P.mode;
-        if (!ctrl->active && mode != MODE_FLUX_ONLY) return;  // step past the end: no-op
+        const int mode = P.mode;
+        if (!VOL && !ctrl->active && mode != MODE_FLUX_ONLY) return;  // step past the end: no-op
 
-        const int n0 = P.n[0], n1 = P.n[1], n2 = P.n[2];
-        const int ntx = (n0 + TX - 1) / TX, nty = (n1 + TY - 1) / TY;
-        const int tx = tile % ntx;
-        const int ty = (tile / ntx) % nty;
-        const int tz = tile / (ntx * nty);
-        const int ox = tx * TX, oy = ty * TY, oz = tz * TZ;
+        const int n0 = P.n[0];
+        const int ox = (int)tile * TX;
         const long long nc = P.ncells;
         const bool otf = (mode == MODE_RK3_2);
-        const double s = (mode == MODE_FLUX_ONLY || mode == MODE_L) ? 0.0 : step_dt(ctrl) / ctrl->cell[0];
+        const double s = (mode == MODE_FLUX_ONLY || mode == MODE_L) ? 0.0
+                         : VOL                                       ? V->s
+                                                                     : step_dt(ctrl) / ctrl->cell[0];
 
         // 1. stage input tile + halo into LDS through the boundary map.  Each
         // thread issues the loads of all its points before writing any of
         // them, so that their global-memory latencies overlap; points past
         // the tile repeat the last one and are not written.
         constexpr int SPT = (LT + NT - 1) / NT;  // staged points per thread
-        Idx sg[SPT];
+        long long sg[SPT];
 #pragma unroll
         for (int k = 0; k < SPT; ++k) {
             int p = threadIdx.x + k * NT;
             p = p < LT ? p : LT - 1;
-            const int lx = p % LX;
-            const int ly = (p / LX) % LY;
-            const int lz = p / (LX * LY);
-            int gx = ox + lx - HX, gy = oy + ly - HY, gz = oz + lz - HZ;
-            gx = gx < n0 + HX ? gx : n0 + HX - 1;
-            gy = gy < n1 + HY ? gy : n1 + HY - 1;
-            gz = gz < n2 + HZ ? gz : n2 + HZ - 1;
-            if constexpr (VOL) {
-                sg[k] = volume_index(*V, gx, DIM >= 2 ? gy : 0, DIM >= 3 ? gz : 0);
-            } else {
-                gx = bc_map(gx, n0, P.bc);
-                gy = DIM >= 2 ? bc_map(gy, n1, P.bc) : 0;
-                gz = DIM >= 3 ? bc_map(gz, n2, P.bc) : 0;
-                sg[k] = ((Idx)gz * n1 + gy) * n0 + gx;
-            }
+            int gx = ox + p - G;
+            gx = gx < n0 + G ? gx : n0 + G - 1;
+            if constexpr (VOL) sg[k] = volume_index(*V, gx, 0, 0);
+            else sg[k] = bc_map(gx, n0, P.bc);
         }
         double sv[SPT][NV];
 #pragma unroll
@@ -519,13 +392,13 @@ struct StageKernel {
 #pragma unroll
             for (int v = 0; v < NV; ++v) {
                 if constexpr (VOL) sv[k][v] = V->in[v][sg[k]];
-                else sv[k][v] = soa_ld<OFF32>(P.in, nc, v, sg[k]);
+                else sv[k][v] = P.in[v * nc + sg[k]];
             }
         if (otf) {
 #pragma unroll
             for (int k = 0; k < SPT; ++k)
 #pragma unroll
-                for (int v = 0; v < NV; ++v) sv[k][v] = sv[k][v] * s + soa_ld<OFF32>(P.u0, nc, v, sg[k]);
+                for (int v = 0; v < NV; ++v) sv[k][v] = sv[k][v] * s + P.u0[v * nc + sg[k]];
         }
 #pragma unroll
         for (int k = 0; k < SPT; ++k) {
@@ -543,7 +416,7 @@ struct StageKernel {
             const bool all = __all(adm);
             if ((threadIdx.x & 63) == 0) s_adm[threadIdx.x >> 6] = all;
         }
-        __syncthreads();
+        lds_barrier();
         if constexpr (FLUX::FAST) {
             int all = s_adm[0];
 #pragma unroll
@@ -551,79 +424,68 @@ struct StageKernel {
             adm = all != 0;
         }
 
-        double acc[CPT][NV];
+        // 2. interface fluxes into LDS; interface i lies right of cell i - 1.
+        // A FAST flux evaluates each with SharedOps, and with PlainOps where
+        // the operands leave the range in which SharedOps is exact.
+        double ws = 0.0;
+        for (int it = threadIdx.x; it < NI; it += NT) {
+            if (ox + it - 1 >= n0) continue;
+            double F[NV];
+            bool ok = adm;
+            double w = interface<Ops>(su, it - 1 + G, P.gamma, F, ok);
+            if (FLUX::FAST && !ok) {
+                ok = true;
+                w = interface<PlainOps>(su, it - 1 + G, P.gamma, F, ok);
+            }
+            ws = ws_max(ws, w);
 #pragma unroll
-        for (int m = 0; m < CPT; ++m)
-#pragma unroll
-            for (int v = 0; v < NV; ++v) acc[m][v] = 0.0;
-        double ws[3] = {0.0, 0.0, 0.0};
-
-        // 2./3. per direction: interface fluxes into LDS, then accumulate
-        flux_pass<0>(su, sf, ox, oy, oz, P.n, P.gamma, adm, ws[0]);
-        __syncthreads();
-        accumulate<0>(sf, acc);
-        if (DIM >= 2) {
-            __syncthreads();
-            flux_pass<DIM >= 2 ? 1 : 0>(su, sf, ox, oy, oz, P.n, P.gamma, adm, ws[1]);
-            __syncthreads();
-            accumulate<DIM >= 2 ? 1 : 0>(sf, acc);
+            for (int v = 0; v < NV; ++v) sf[v * NI + it] = F[v];
         }
-        if (DIM >= 3) {
-            __syncthreads();
-            flux_pass<DIM >= 3 ? 2 : 0>(su, sf, ox, oy, oz, P.n, P.gamma, adm, ws[2]);
-            __syncthreads();
-            accumulate<DIM >= 3 ? 2 : 0>(sf, acc);
-        }
+        lds_barrier();
 
-        // 4. RK combination and write-back; the U0 loads of all the thread's
-        // cells are issued first (cells outside the grid load element 0 and
-        // write nothing)
+        // 3. net flux, RK combination and write-back; the U0 loads of all the
+        // thread's cells are issued first (cells outside the grid load element
+        // 0 and write nothing)
         bool bad = false;
-        const bool final_stage = (mode == MODE_RK2_2 || mode == MODE_RK3_3);
+        const bool final_stage = !VOL && (mode == MODE_RK2_2 || mode == MODE_RK3_3);
         const bool combine = !(mode == MODE_FLUX_ONLY || mode == MODE_L);
-        Idx gc[CPT];
+        long long gc[CPT];
         bool inside[CPT];
 #pragma unroll
         for (int m = 0; m < CPT; ++m) {
             const int c = threadIdx.x + m * NT;
-            const int cx = c % TX;
-            const int cy = (c / TX) % TY;
-            const int cz = c / (TX * TY);
-            const int gx = ox + cx, gy = oy + cy, gz = oz + cz;
-            inside[m] = (TC % NT == 0 || c < TC) && gx < n0 && gy < n1 && gz < n2;
-            if constexpr (VOL) gc[m] = inside[m] ? volume_index(*V, gx, gy, gz) : 0;
-            else gc[m] = inside[m] ? ((Idx)gz * n1 + gy) * n0 + gx : 0;
+            inside[m] = (TX % NT == 0 || c < TX) && ox + c < n0;
+            if constexpr (VOL) gc[m] = inside[m] ? volume_index(*V, ox + c, 0, 0) : 0;
+            else gc[m] = inside[m] ? ox + c : 0;
         }
-        const double ca = mode == MODE_RK3_2 ? 1. / 3. : (mode == MODE_RK3_3 ? 2.0 : 1.0);
-        const double cb = mode == MODE_RK2_2 ? 0.5 : (mode == MODE_RK3_2 ? 3. / 4. : 1. / 3.);
+        const double ca = VOL ? V->ca : (mode == MODE_RK3_2 ? 1. / 3. : (mode == MODE_RK3_3 ? 2.0 : 1.0));
+        const double cb = VOL ? V->cb : (mode == MODE_RK2_2 ? 0.5 : (mode == MODE_RK3_2 ? 3. / 4. : 1. / 3.));
         double u0c[CPT][NV];
         if (combine) {
 #pragma unroll
             for (int m = 0; m < CPT; ++m)
 #pragma unroll
-                for (int v = 0; v < NV; ++v) u0c[m][v] = soa_ld<OFF32>(P.u0, nc, v, gc[m]);
+                for (int v = 0; v < NV; ++v) {
+                    if constexpr (VOL) u0c[m][v] = V->u0[v][gc[m]];
+                    else u0c[m][v] = P.u0[v * nc + gc[m]];
+                }
         }
 #pragma unroll
         for (int m = 0; m < CPT; ++m) {
             if (!inside[m]) continue;
             const int c = threadIdx.x + m * NT;
-            const int cx = c % TX;
-            const int cy = (c / TX) % TY;
-            const int cz = c / (TX * TY);
-            const Idx gi = gc[m];
-            const int li = lidx(cx, cy, cz);
             double r[NV];
 #pragma unroll
             for (int v = 0; v < NV; ++v) {
-                const double l = acc[m][v];
+                // temp = -F; out[i] = 0 + (temp[i] + (-1)*temp[i-1])
+                const double l = 0.0 + ((-sf[v * NI + c + 1]) + sf[v * NI + c]);
                 if (!combine) {
                     r[v] = l;
                 } else {
                     // ((L*s + U) * ca + U0) * cb; the factor 1 of the RK2
                     // stage is exact, so every mode keeps its own rounding
-                    const double us = su[v * LT + li];
                     double o = l * s;
-                    o = o + us;
+                    o = o + su[v * LT + c + G];
                     o = o * ca;
                     o = o + u0c[m][v];
                     o = o * cb;
@@ -633,12 +495,11 @@ struct StageKernel {
             if (final_stage) bad = bad || !EQ::obeys_fast(r, P.gamma);
 #pragma unroll
             for (int v = 0; v < NV; ++v) {
-                if constexpr (VOL) V->out[v][gi] = r[v];
-                else soa_st<OFF32>(P.out, nc, v, gi, r[v]);
+                if constexpr (VOL) V->out[v][gc[m]] = r[v];
+                else P.out[v * nc + gc[m]] = r[v];
             }
         }
-
-        end_of_tile<NT>(P, ctrl, mode, ws[0], ws[1], ws[2], s_ws, bad);
+        if (!VOL || mode == MODE_FLUX_ONLY) end_of_tile<NT>(P, ctrl, mode, ws, 0.0, 0.0, s_ws, bad);
     }
 };
 
@@ -647,7 +508,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void s
     K::run(P);
 }
 
-// A stage over a box of a reference Volume (flux-only mode)
+// A stage over a box of a reference Volume
 template <class K>
 __global__ __launch_bounds__(256) void volume_stage_kernel(StageParams P, VolumeParams V) {
     K::run_volume(P, V);

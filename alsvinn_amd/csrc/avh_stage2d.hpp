@@ -161,8 +161,9 @@ struct TileKernel2 {
         run_tile<true>(P, tile_id_xcd(blockIdx.x, gridDim.x), &V);
     }
 
-    // VOL: the cells live in a reference Volume (V) and P.n is the extent of
-    // the box the launch covers; otherwise in the interior-only buffers of P
+    // VOL: the cells live in a reference Volume (V; MODE_FLUX_ONLY, or
+    // MODE_RK3_3 for the combination V describes) and P.n is the extent of the
+    // box the launch covers; otherwise in the interior-only buffers of P
     // with the boundary map for the halo.  LOAD_FIRST: the tile's loads are
     // issued before the test whether the step runs at all (a single grid's
     // steps nearly always do; of a batch's samples many may have ended).
@@ -175,7 +176,7 @@ struct TileKernel2 {
 
         Control* ctrl = P.ctrl;
         const int mode = MODE_CT >= 0 ? MODE_CT : P.mode;
-        if (!LOAD_FIRST && !ctrl->active && mode != MODE_FLUX_ONLY) return;  // step past the end: no-op
+        if (!VOL && !LOAD_FIRST && !ctrl->active && mode != MODE_FLUX_ONLY) return;  // step past the end: no-op
 
         const int n0 = P.n[0], n1 = P.n[1];
         const int ntx = (n0 + TX - 1) / TX;
@@ -214,9 +215,11 @@ struct TileKernel2 {
 #pragma unroll
                 for (int v = 0; v < NV; ++v) s0[k][v] = soa_ld<OFF32>(P.u0, nc, v, sg[k]);
         }
-        if (LOAD_FIRST && !ctrl->active && mode != MODE_FLUX_ONLY) return;
+        if (!VOL && LOAD_FIRST && !ctrl->active && mode != MODE_FLUX_ONLY) return;
         // dt / dx, formed while the loads are in flight
-        const double s = (mode == MODE_FLUX_ONLY || mode == MODE_L) ? 0.0 : step_dt(ctrl) / ctrl->cell[0];
+        const double s = (mode == MODE_FLUX_ONLY || mode == MODE_L) ? 0.0
+                         : VOL                                       ? V->s
+                                                                     : step_dt(ctrl) / ctrl->cell[0];
         if (otf) {
 #pragma unroll
             for (int k = 0; k < SW; ++k)
@@ -275,7 +278,7 @@ struct TileKernel2 {
         // cells are issued first (cells outside the grid load element 0 and
         // write nothing)
         bool bad = false;
-        const bool final_stage = (mode == MODE_RK2_2 || mode == MODE_RK3_3);
+        const bool final_stage = !VOL && (mode == MODE_RK2_2 || mode == MODE_RK3_3);
         const bool combine = !(mode == MODE_FLUX_ONLY || mode == MODE_L);
         Idx gc[CPT];
         bool inside[CPT];
@@ -287,14 +290,17 @@ struct TileKernel2 {
             if constexpr (VOL) gc[m] = inside[m] ? volume_index(*V, x, y, 0) : 0;
             else gc[m] = inside[m] ? (Idx)y * n0 + x : 0;
         }
-        const double ca = mode == MODE_RK3_2 ? 1. / 3. : (mode == MODE_RK3_3 ? 2.0 : 1.0);
-        const double cb = mode == MODE_RK2_2 ? 0.5 : (mode == MODE_RK3_2 ? 3. / 4. : 1. / 3.);
+        const double ca = VOL ? V->ca : (mode == MODE_RK3_2 ? 1. / 3. : (mode == MODE_RK3_3 ? 2.0 : 1.0));
+        const double cb = VOL ? V->cb : (mode == MODE_RK2_2 ? 0.5 : (mode == MODE_RK3_2 ? 3. / 4. : 1. / 3.));
         double u0c[CPT][NV];
         if (combine) {
 #pragma unroll
             for (int m = 0; m < CPT; ++m)
 #pragma unroll
-                for (int v = 0; v < NV; ++v) u0c[m][v] = soa_ld<OFF32>(P.u0, nc, v, gc[m]);
+                for (int v = 0; v < NV; ++v) {
+                    if constexpr (VOL) u0c[m][v] = V->u0[v][gc[m]];
+                    else u0c[m][v] = soa_ld<OFF32>(P.u0, nc, v, gc[m]);
+                }
         }
 #pragma unroll
         for (int m = 0; m < CPT; ++m) {
@@ -325,7 +331,7 @@ struct TileKernel2 {
                 else soa_st<OFF32>(P.out, nc, v, gc[m], r[v]);
             }
         }
-        end_of_tile<NT>(P, ctrl, mode, ws[0], ws[1], 0.0, s_ws, bad);
+        if (!VOL || mode == MODE_FLUX_ONLY) end_of_tile<NT>(P, ctrl, mode, ws[0], ws[1], 0.0, s_ws, bad);
     }
 };
 

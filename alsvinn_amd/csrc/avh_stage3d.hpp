@@ -124,7 +124,11 @@ __device__ __forceinline__ void recon_faces_reg(const double (&u)[WZ][NV], const
 // stretch.  A workgroup marches through P.lz planes.
 // MODE_CT >= 0 compiles the kernel for that StageMode alone (P.mode must
 // equal it): the other modes' branches and registers drop out.
-template <class EQ, int RECON, class FLUX, int TX, int TY, int NTH, int MODE_CT = -1>
+// VOL: the cells live in a reference Volume (V; MODE_FLUX_ONLY, or
+// MODE_RK3_3 for the combination V describes) and P.n is the extent of the box
+// the launch covers; otherwise in the interior-only buffers of P with the
+// boundary map for the halo.
+template <class EQ, int RECON, class FLUX, int TX, int TY, int NTH, int MODE_CT = -1, bool VOL = false>
 struct MarchKernel3 {
     static constexpr int NV = EQ::NV;
     static constexpr int NC = TX * TY;  // columns: one per thread, threads past them work on the planes only
@@ -151,27 +155,50 @@ struct MarchKernel3 {
     // 32-bit offset from a variable's base held in scalar registers, with no
     // 64-bit address arithmetic per lane.  (The final stage, which also
     // stores, runs out of scalar registers that way and is slower.)
-    static constexpr bool OFF32 = MODE_CT == MODE_L || MODE_CT == MODE_RK3_2;
+    static constexpr bool OFF32 = !VOL && (MODE_CT == MODE_L || MODE_CT == MODE_RK3_2);
     typedef typename std::conditional<OFF32, unsigned int, long long>::type Idx;
-    __device__ __forceinline__ static Idx gidx(int x, int y, int z, int n0, int n1) {
-        return ((Idx)z * n1 + y) * n0 + x;
+    // rows and planes of the buffers, and where cell (0, 0, 0) of the box lies
+    struct Layout {
+        Idx origin, row, plane;
+        __device__ __forceinline__ Idx at(int x, int y, int z) const { return origin + z * plane + y * row + x; }
+    };
+    __device__ __forceinline__ static Layout layout(const StageParams& P, const VolumeParams* V) {
+        if constexpr (VOL) return Layout{volume_index(*V, 0, 0, 0), V->tot[0], (Idx)V->tot[0] * V->tot[1]};
+        else return Layout{0, (Idx)P.n[0], (Idx)P.n[0] * P.n[1]};
     }
-    __device__ __forceinline__ static double ld(const double* base, long long ncells, int v, Idx gi) {
-        return soa_ld<OFF32>(base, ncells, v, gi);
+    __device__ __forceinline__ static double ld_in(const StageParams& P, const VolumeParams* V, int v, Idx gi) {
+        if constexpr (VOL) return V->in[v][gi];
+        else return soa_ld<OFF32>(P.in, P.ncells, v, gi);
     }
-    __device__ __forceinline__ static void st(double* base, long long ncells, int v, Idx gi, double x) {
-        soa_st<OFF32>(base, ncells, v, gi, x);
+    __device__ __forceinline__ static double ld_u0(const StageParams& P, const VolumeParams* V, int v, Idx gi) {
+        if constexpr (VOL) return V->u0[v][gi];
+        else return soa_ld<OFF32>(P.u0, P.ncells, v, gi);
+    }
+    // coordinate g of the buffers for a cell at most G outside the box
+    __device__ __forceinline__ static int map_in(int g, int n, int bc) {
+        g = g < n + G ? g : n + G - 1;
+        return VOL ? g : bc_map(g, n, bc);
+    }
+    // as map_in along z, where a window wider than the stencil (HW > G - 1)
+    // may reach further out; those planes are not used
+    __device__ __forceinline__ static int map_z(int g, int n, int bc) {
+        if constexpr (VOL) {
+            g = g > -G ? g : -G;
+            return g < n + G ? g : n + G - 1;
+        } else {
+            return bc_map(g, n, bc);
+        }
     }
 
-    // one input value at a (boundary-mapped) global cell; in the on-the-fly
-    // stage U0's values are also written to `keep` (stride NC) when given
-    __device__ __forceinline__ static void fetch(const StageParams& P, bool otf, double s, Idx gi, double* q,
-                                                 double* keep = nullptr) {
+    // one input value at a cell; in the on-the-fly stage U0's values are also
+    // written to `keep` (stride NC) when given
+    __device__ __forceinline__ static void fetch(const StageParams& P, const VolumeParams* V, bool otf, double s,
+                                                 Idx gi, double* q, double* keep = nullptr) {
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
-            double val = ld(P.in, P.ncells, v, gi);
+            double val = ld_in(P, V, v, gi);
             if (otf) {
-                const double u = ld(P.u0, P.ncells, v, gi);
+                const double u = ld_u0(P, V, v, gi);
                 if (keep) keep[v * NC] = u;
                 val = val * s + u;
             }
@@ -254,7 +281,7 @@ struct MarchKernel3 {
         }
     }
 
-    __device__ static void run(const StageParams& P) {
+    __device__ static void run(const StageParams& P, const VolumeParams* V = nullptr) {
         __shared__ double sp_buf[2][NV * LP];
         __shared__ double sfx[NV * NIMAX];
         __shared__ double sfy[NV * NIMAX];
@@ -264,7 +291,7 @@ struct MarchKernel3 {
 
         Control* ctrl = P.ctrl;
         const int mode = MODE_CT >= 0 ? MODE_CT : P.mode;
-        if (!ctrl->active && mode != MODE_FLUX_ONLY) return;
+        if (!VOL && !ctrl->active && mode != MODE_FLUX_ONLY) return;
 
         const int n0 = P.n[0], n1 = P.n[1], n2 = P.n[2];
         const int ntx = (n0 + TX - 1) / TX, nty = (n1 + TY - 1) / TY;
@@ -275,7 +302,10 @@ struct MarchKernel3 {
         const int ox = tx * TX, oy = ty * TY, z0 = tz * P.lz;
         const int z1 = (z0 + P.lz < n2) ? z0 + P.lz : n2;
         const bool otf = (mode == MODE_RK3_2);
-        const double s = (mode == MODE_FLUX_ONLY || mode == MODE_L) ? 0.0 : step_dt(ctrl) / ctrl->cell[0];
+        const double s = (mode == MODE_FLUX_ONLY || mode == MODE_L) ? 0.0
+                         : VOL                                       ? V->s
+                                                                     : step_dt(ctrl) / ctrl->cell[0];
+        const Layout lay = layout(P, V);
 
         // this thread's column.  A column past the grid edge (partial tile)
         // sits where the tile's x/y halo lies, so it loads the boundary image
@@ -283,8 +313,8 @@ struct MarchKernel3 {
         const bool has_col = (int)threadIdx.x < NC;
         const int cx = threadIdx.x % TX, cy = has_col ? (int)threadIdx.x / TX : 0;
         const bool col_ok = has_col && (ox + cx < n0) && (oy + cy < n1);
-        const int gxc = bc_map(ox + cx < n0 + G ? ox + cx : n0 + G - 1, n0, P.bc);
-        const int gyc = bc_map(oy + cy < n1 + G ? oy + cy : n1 + G - 1, n1, P.bc);
+        const int gxc = map_in(ox + cx, n0, P.bc);
+        const int gyc = map_in(oy + cy, n1, P.bc);
 
         double ws[3] = {0.0, 0.0, 0.0};
         double w[WZ][NV];
@@ -310,8 +340,8 @@ struct MarchKernel3 {
         if (has_col) {
 #pragma unroll
             for (int i = 0; i < WZ; ++i) {
-                const int gz = bc_map(z0 - 1 - HW + i, n2, P.bc);
-                fetch(P, otf, s, gidx(gxc, gyc, gz, n0, n1), w[i], (ring && i > HW) ? slot(z0 - 1 - HW + i) : nullptr);
+                const int gz = map_z(z0 - 1 - HW + i, n2, P.bc);
+                fetch(P, V, otf, s, lay.at(gxc, gyc, gz), w[i], (ring && i > HW) ? slot(z0 - 1 - HW + i) : nullptr);
             }
             double rm1[NV];
             recon_face_reg<RECON, NV, true, WZ>(w, HW, rm1);
@@ -319,7 +349,7 @@ struct MarchKernel3 {
             for (int i = 0; i < WZ - 1; ++i)
 #pragma unroll
                 for (int v = 0; v < NV; ++v) w[i][v] = w[i + 1][v];
-            fetch(P, otf, s, gidx(gxc, gyc, bc_map(z0 + HW, n2, P.bc), n0, n1), w[WZ - 1],
+            fetch(P, V, otf, s, lay.at(gxc, gyc, map_z(z0 + HW, n2, P.bc)), w[WZ - 1],
                   ring ? slot(z0 + HW) : nullptr);
             if constexpr (FLUX::FAST) {
 #pragma unroll
@@ -338,13 +368,13 @@ struct MarchKernel3 {
             for (int i = 0; i < WZ - 1; ++i)
 #pragma unroll
                 for (int v = 0; v < NV; ++v) w[i][v] = w[i + 1][v];
-            fetch(P, otf, s, gidx(gxc, gyc, bc_map(z0 + 1 + HW, n2, P.bc), n0, n1), w[WZ - 1],
+            fetch(P, V, otf, s, lay.at(gxc, gyc, map_z(z0 + 1 + HW, n2, P.bc)), w[WZ - 1],
                   ring ? slot(z0 + 1 + HW) : nullptr);
             if (FLUX::FAST && RECON == RECON_WENO2) rb = weno2_recip(w[HW][0] - w[HW - 1][0]);
         }
 
         bool bad = false;
-        const bool final_stage = (mode == MODE_RK2_2 || mode == MODE_RK3_3);
+        const bool final_stage = !VOL && (mode == MODE_RK2_2 || mode == MODE_RK3_3);
         // This thread's cells of the x/y halo ring (HPT per thread at most):
         // their LDS slots and boundary-mapped positions in a plane do not
         // change with k.  The ring rows above and below the tile come first,
@@ -373,16 +403,10 @@ struct MarchKernel3 {
                     const int c2 = r % (2 * G);
                     lx = c2 < G ? c2 : TX + c2;
                 }
-                int gx = ox + lx - G, gy = oy + ly - G;
-                gx = gx < n0 + G ? gx : n0 + G - 1;
-                gy = gy < n1 + G ? gy : n1 + G - 1;
-                gx = bc_map(gx, n0, P.bc);
-                gy = bc_map(gy, n1, P.bc);
                 halo_lds[j] = ly * LXP + lx;
-                halo_xy[j] = (Idx)gy * n0 + gx;
+                halo_xy[j] = lay.at(map_in(ox + lx - G, n0, P.bc), map_in(oy + ly - G, n1, P.bc), 0);
             }
         }
-        const Idx plane = (Idx)n0 * n1;
         // the ring of the next plane is loaded while the current plane is
         // computed: raw input (and U0 for the on-the-fly stage) in registers
         double pin[HPT][NV], pu0[HPT][NV];
@@ -393,10 +417,10 @@ struct MarchKernel3 {
 #define AVH_PREFETCH_RING(KP)                                                   \
     _Pragma("unroll") for (int j = 0; j < HPT; ++j) {                           \
         if (has_halo[j]) {                                                      \
-            const Idx gi = (Idx)(KP) * plane + halo_xy[j];                      \
+            const Idx gi = (Idx)(KP) * lay.plane + halo_xy[j];                  \
             _Pragma("unroll") for (int v = 0; v < NV; ++v) {                    \
-                pin[j][v] = ld(P.in, P.ncells, v, gi);                            \
-                if (otf) pu0[j][v] = ld(P.u0, P.ncells, v, gi);                   \
+                pin[j][v] = ld_in(P, V, v, gi);                                 \
+                if (otf) pu0[j][v] = ld_u0(P, V, v, gi);                        \
             }                                                                   \
         }                                                                       \
     }
@@ -406,15 +430,15 @@ struct MarchKernel3 {
         // stage is exact); U0 of the column's next plane is loaded one plane
         // ahead, with the window's next plane
         const bool combine = !(mode == MODE_FLUX_ONLY || mode == MODE_L);
-        const double ca = mode == MODE_RK3_2 ? 1. / 3. : (mode == MODE_RK3_3 ? 2.0 : 1.0);
-        const double cb = mode == MODE_RK2_2 ? 0.5 : (mode == MODE_RK3_2 ? 3. / 4. : 1. / 3.);
+        const double ca = VOL ? V->ca : (mode == MODE_RK3_2 ? 1. / 3. : (mode == MODE_RK3_3 ? 2.0 : 1.0));
+        const double cb = VOL ? V->cb : (mode == MODE_RK2_2 ? 0.5 : (mode == MODE_RK3_2 ? 3. / 4. : 1. / 3.));
         double u0n[NV];
 #pragma unroll
         for (int v = 0; v < NV; ++v) u0n[v] = 0.0;
         if (combine && col_ok && !ring) {
-            const Idx gi = gidx(ox + cx, oy + cy, z0, n0, n1);
+            const Idx gi = lay.at(ox + cx, oy + cy, z0);
 #pragma unroll
-            for (int v = 0; v < NV; ++v) u0n[v] = ld(P.u0, P.ncells, v, gi);
+            for (int v = 0; v < NV; ++v) u0n[v] = ld_u0(P, V, v, gi);
         }
 
         for (int k = z0; k < z1; ++k) {
@@ -518,7 +542,7 @@ struct MarchKernel3 {
             for (int v = 0; v < NV; ++v) acc[v] = acc[v] + ((-fz[v]) + fprev[v]);
 
             if (col_ok) {
-                const Idx gi = gidx(ox + cx, oy + cy, k, n0, n1);
+                const Idx gi = lay.at(ox + cx, oy + cy, k);
                 if (ring) {
                     const double* const u0k = slot(k);
 #pragma unroll
@@ -541,7 +565,10 @@ struct MarchKernel3 {
                 }
                 if (final_stage) bad = bad || !EQ::obeys_fast(r, P.gamma);
 #pragma unroll
-                for (int v = 0; v < NV; ++v) st(P.out, P.ncells, v, gi, r[v]);
+                for (int v = 0; v < NV; ++v) {
+                    if constexpr (VOL) V->out[v][gi] = r[v];
+                    else soa_st<OFF32>(P.out, P.ncells, v, gi, r[v]);
+                }
             }
 #pragma unroll
             for (int v = 0; v < NV; ++v) {
@@ -556,21 +583,21 @@ struct MarchKernel3 {
             // the window's next plane and the next write-back's U0, issued
             // together so that their latencies overlap
             if (has_col && k + 1 < z1) {
-                const Idx gn = gidx(gxc, gyc, bc_map(k + 2 + HW, n2, P.bc), n0, n1);
-                const Idx gw = gidx(ox + cx, oy + cy, k + 1, n0, n1);
+                const Idx gn = lay.at(gxc, gyc, map_z(k + 2 + HW, n2, P.bc));
+                const Idx gw = lay.at(ox + cx, oy + cy, k + 1);
                 double cin[NV], cu0[NV];
 #pragma unroll
                 for (int v = 0; v < NV; ++v) {
-                    cin[v] = ld(P.in, P.ncells, v, gn);
+                    cin[v] = ld_in(P, V, v, gn);
                     cu0[v] = 0.0;
                 }
                 if (otf) {
 #pragma unroll
-                    for (int v = 0; v < NV; ++v) cu0[v] = ld(P.u0, P.ncells, v, gn);
+                    for (int v = 0; v < NV; ++v) cu0[v] = ld_u0(P, V, v, gn);
                 }
                 if (combine && col_ok && !ring) {
 #pragma unroll
-                    for (int v = 0; v < NV; ++v) u0n[v] = ld(P.u0, P.ncells, v, gw);
+                    for (int v = 0; v < NV; ++v) u0n[v] = ld_u0(P, V, v, gw);
                 }
                 if (ring && k + 2 + HW < z1) {
                     double* const kp = slot(k + 2 + HW);
@@ -583,13 +610,19 @@ struct MarchKernel3 {
         }
 
 #undef AVH_PREFETCH_RING
-        end_of_tile<NT>(P, ctrl, mode, ws[0], ws[1], ws[2], s_ws, bad);
+        if (!VOL || mode == MODE_FLUX_ONLY) end_of_tile<NT>(P, ctrl, mode, ws[0], ws[1], ws[2], s_ws, bad);
     }
 };
 
 template <class K>
 __global__ __launch_bounds__(256) void march_kernel3(StageParams P) {
     K::run(P);
+}
+
+// A stage over a box of a reference Volume
+template <class K>
+__global__ __launch_bounds__(256) void volume_march_kernel3(StageParams P, VolumeParams V) {
+    K::run(P, &V);
 }
 
 }  // namespace avh

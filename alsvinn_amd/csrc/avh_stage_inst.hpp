@@ -32,17 +32,19 @@ typedef hipError_t (*VolumeLauncher)(const StageParams& P, const VolumeParams& V
 //   3D: 16x15 or 32x7 columns marching over 2 to 32 planes, 256 threads (at
 //       most 256 interfaces a plane in each direction: one turn; the threads
 //       past the columns only work on the planes).  A chunk pays a z flux
-//       and the loads of its window before its first plane, so long chunks
-//       win where a grid still gives every CU its two workgroups (us of an RK3
-//       stage pair, 4 / 8 / 16 / 32 planes: 256^3 2520 / 2262 / 2133 / 2100,
-//       200x150x120 575 / 539 / 598 / 722, 97x83x61 120 / 140 / 173 / 326).
+//       and the loads of its window before its first plane, so the best length
+//       is the one that fills the CUs evenly (march_chunk; the fixed lengths
+//       stand beside it for grids where its model is off).  us of an RK3 stage
+//       pair, 4 / 8 / 16 / 32 planes and march_chunk's: 200x150x120
+//       566 / 539 / 582 / 700 / 528, 128^3 317 / 313 / 352 / 449 / 302, 64^3
+//       76 / 87 / 159 / 299 / 64, 160^3 616 / 559 / 585 / 710 / 555.
 constexpr int NSHAPES1 = 2, NSHAPES2 = 5, NSHAPES3 = 7;
 constexpr int SHAPE1_TX[NSHAPES1] = {256, 64};
 constexpr int SHAPE2_TX[NSHAPES2] = {64, 16, 16, 32, 16};
 constexpr int SHAPE2_TY[NSHAPES2] = {7, 15, 7, 15, 28};
 constexpr int SHAPE3_TX[NSHAPES3] = {16, 16, 32, 32, 16, 16, 16};
 constexpr int SHAPE3_TY[NSHAPES3] = {15, 15, 7, 7, 15, 15, 15};
-constexpr int SHAPE3_LZ[NSHAPES3] = {4, 8, 8, 32, 16, 2, 32};
+constexpr int SHAPE3_LZ[NSHAPES3] = {4, 0, 8, 32, 16, 2, 32};  // 0: march_chunk
 
 inline int num_shapes(int dim) { return dim == 1 ? NSHAPES1 : (dim == 2 ? NSHAPES2 : NSHAPES3); }
 
@@ -50,7 +52,7 @@ template <class EQ, int RECON, class FLUX, int DIM, int S>
 struct KernelFor;
 template <class EQ, int RECON, class FLUX, int S>
 struct KernelFor<EQ, RECON, FLUX, 1, S> {
-    typedef StageKernel<EQ, RECON, FLUX, 1, SHAPE1_TX[S], 1, 1, SHAPE1_TX[S]> type;
+    typedef StageKernel1<EQ, RECON, FLUX, SHAPE1_TX[S], SHAPE1_TX[S]> type;
 };
 template <class EQ, int RECON, class FLUX, int S>
 struct KernelFor<EQ, RECON, FLUX, 2, S> {
@@ -125,6 +127,28 @@ hipError_t launch_stage_k(const StageParams& P, hipStream_t stream) {
     return hipGetLastError();
 }
 
+// Planes per chunk for a box of n cells, by a model of the launch.  The
+// workgroups of a CU share its FP64 pipe, so a launch takes as long as the CU
+// with the most of them, each worth its planes and about one more for its
+// prologue; one alone leaves about a quarter of the pipe idle.
+// 128^3, 16x15 columns, us of a volume substep's launch at 8 / 13 / 16 / 32
+// planes and at the 19 this picks: 165 / 163 / 192 / 240 and 158.
+template <class K>
+int march_chunk(const int* n) {
+    const int CUS = 256;
+    int best = 1;
+    long long cost = 0;
+    for (int lz = 2; lz <= 64; ++lz) {
+        const long long per_cu = (K::tiles(n, lz) + CUS - 1) / CUS;
+        const long long c = (2 * per_cu < 3 ? 3 : 2 * per_cu) * (lz + 1);
+        if (lz == 2 || c < cost) {
+            best = lz;
+            cost = c;
+        }
+    }
+    return best;
+}
+
 template <class K>
 hipError_t launch_march_k(const StageParams& P, hipStream_t stream) {
     hipLaunchKernelGGL(march_kernel3<K>, dim3(K::tiles(P.n, P.lz)), dim3(K::NT), 0, stream, P);
@@ -153,6 +177,7 @@ hipError_t launch_stage(const StageParams& P, int shape, hipStream_t stream) {
         if (shape < 0 || shape >= NSHAPES3) return hipErrorInvalidValue;
         StageParams Q = P;
         Q.lz = SHAPE3_LZ[shape];
+        if (Q.lz == 0) Q.lz = march_chunk<MarchKernel3<EQ, RECON, FLUX, 16, 15, 256>>(P.n);
         return SHAPE3_TX[shape] == 16 ? launch_march<EQ, RECON, FLUX, 16, 15>(Q, stream)
                                       : launch_march<EQ, RECON, FLUX, 32, 7>(Q, stream);
     } else if constexpr (DIM == 1) {
@@ -189,29 +214,37 @@ hipError_t launch_stage(const StageParams& P, int shape, hipStream_t stream) {
 }
 
 // The reference-Volume kernels: one tile per dimension -- 1D 256 cells, 2D
-// 32x15, 3D 8x4x4 bricks on 128 threads (the ghost-width-3 halo of a brick
-// still fits one workgroup's LDS for euler3) -- since this path serves the
-// reference's unfused per-call interfaces.
-template <class EQ, int RECON, class FLUX, int DIM>
-struct VolumeKernelFor;
+// 32x15, 3D 16x15 columns.  P.mode is MODE_FLUX_ONLY, or MODE_RK3_3 for the
+// combination V describes.
 template <class EQ, int RECON, class FLUX>
-struct VolumeKernelFor<EQ, RECON, FLUX, 1> {
-    typedef StageKernel<EQ, RECON, FLUX, 1, 256, 1, 1, 256> type;
+struct VolumeKernel1 {
+    typedef StageKernel1<EQ, RECON, FLUX, 256, 256> type;
 };
 template <class EQ, int RECON, class FLUX>
-struct VolumeKernelFor<EQ, RECON, FLUX, 2> {
+struct VolumeKernel2 {
     typedef TileKernel2<EQ, RECON, FLUX, 32, 15, 256> type;
 };
-template <class EQ, int RECON, class FLUX>
-struct VolumeKernelFor<EQ, RECON, FLUX, 3> {
-    typedef StageKernel<EQ, RECON, typename FLUX::Plain, 3, 8, 4, 4, 128> type;
-};
+
+template <class K>
+hipError_t launch_volume_march(const StageParams& P, const VolumeParams& V, hipStream_t stream) {
+    StageParams Q = P;
+    Q.lz = march_chunk<K>(P.n);
+    hipLaunchKernelGGL(volume_march_kernel3<K>, dim3(K::tiles(P.n, Q.lz)), dim3(K::NT), 0, stream, Q, V);
+    return hipGetLastError();
+}
 
 template <class EQ, int RECON, class FLUX, int DIM>
 hipError_t launch_volume_stage(const StageParams& P, const VolumeParams& V, hipStream_t stream) {
-    typedef typename VolumeKernelFor<EQ, RECON, FLUX, DIM>::type K;
-    hipLaunchKernelGGL(volume_stage_kernel<K>, dim3(K::tiles(P.n)), dim3(K::NTHREADS), 0, stream, P, V);
-    return hipGetLastError();
+    if constexpr (DIM == 3) {
+        if (P.mode == MODE_FLUX_ONLY)
+            return launch_volume_march<MarchKernel3<EQ, RECON, FLUX, 16, 15, 256, MODE_FLUX_ONLY, true>>(P, V, stream);
+        return launch_volume_march<MarchKernel3<EQ, RECON, FLUX, 16, 15, 256, MODE_RK3_3, true>>(P, V, stream);
+    } else {
+        typedef typename std::conditional<DIM == 1, VolumeKernel1<EQ, RECON, FLUX>,
+                                          VolumeKernel2<EQ, RECON, FLUX>>::type::type K;
+        hipLaunchKernelGGL(volume_stage_kernel<K>, dim3(K::tiles(P.n)), dim3(K::NTHREADS), 0, stream, P, V);
+        return hipGetLastError();
+    }
 }
 
 // Steps of a small 1D grid in one workgroup (avh_line.hpp), for burgers and

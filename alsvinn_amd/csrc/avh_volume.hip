@@ -7,18 +7,21 @@
 // map; these entry points instead read and write the reference's layout, so
 // that the reference's own Simulator, ConservedSystem and Integrator can
 // drive the hip platform call by call:
-//   numerical flux  the stage kernel in flux-only mode over a box of the
-//                   interior, halo from the caller's ghost cells;
+//   numerical flux  the stage kernels over a box of the interior, halo from
+//                   the caller's ghost cells;
 //   reconstruction  one thread per cell, a register window along the
 //                   direction;
 //   boundary        ghost cells from the interior by the boundary map;
 //   constraints     every cell, ghosts included;
 //   substep         numerical flux over the interior, dt from the wave
 //                   speeds, then the integrator's Volume operations on
-//                   every cell.
+//                   every cell; from the second substep on, where dt is
+//                   given, the stage kernel applies them to the interior
+//                   itself.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <cstdint>
 #include <cstring>
 #include <limits>
 #include <mutex>
@@ -84,6 +87,17 @@ bool same_shape(const avh_volume* a, const avh_volume* b) {
     for (int d = 0; d < 3; ++d)
         if (a->n[d] != b->n[d] || a->ghosts[d] != b->ghosts[d]) return false;
     return true;
+}
+
+// whether two volumes of the same shape share memory
+bool overlap(const avh_volume* a, const avh_volume* b) {
+    const uintptr_t bytes = (uintptr_t)shape_of(a).cells * sizeof(double);
+    for (int i = 0; i < a->nvars; ++i)
+        for (int j = 0; j < b->nvars; ++j) {
+            const uintptr_t p = (uintptr_t)a->var[i], q = (uintptr_t)b->var[j];
+            if (p < q + bytes && q < p + bytes) return true;
+        }
+    return false;
 }
 
 avh_status ctx_scratch(avh_ctx* ctx, Scratch** out) {
@@ -200,7 +214,6 @@ bool launch_volume_reconstruct(int recon, const ReconVolParams& R, unsigned nb, 
 
 struct VolPtrs {
     double* v[5];
-    int nv;
     int n[3];
     int g[3];
     int tot[3];
@@ -209,7 +222,6 @@ struct VolPtrs {
 VolPtrs ptrs_of(const avh_volume* a) {
     VolPtrs p;
     for (int i = 0; i < 5; ++i) p.v[i] = i < a->nvars ? a->var[i] : nullptr;
-    p.nv = a->nvars;
     for (int d = 0; d < 3; ++d) {
         p.n[d] = a->n[d];
         p.g[d] = a->ghosts[d];
@@ -218,21 +230,67 @@ VolPtrs ptrs_of(const avh_volume* a) {
     return p;
 }
 
+// The ghost cells of a volume, counted: the planes below and above the
+// interior, then in the planes between them the rows before and behind it,
+// then the cells left and right of it.  Ghost passes enumerate these alone
+// (128^3 with two ghost cells: 0.2 of 2.3 M cells).
+struct GhostCells {
+    int n[3], g[3], tot[3];
+    long long planes, rows, all;  // running ends of the three kinds
+};
+
+GhostCells ghost_cells(const int* n, const int* g) {
+    GhostCells c;
+    for (int d = 0; d < 3; ++d) {
+        c.n[d] = n[d];
+        c.g[d] = g[d];
+        c.tot[d] = n[d] + 2 * g[d];
+    }
+    c.planes = 2ll * g[2] * c.tot[1] * c.tot[0];
+    c.rows = c.planes + (long long)n[2] * 2 * g[1] * c.tot[0];
+    c.all = c.rows + (long long)n[2] * n[1] * 2 * g[0];
+    return c;
+}
+
+// 0 .. 2g-1 to the positions outside the interior: -g .. -1, n .. n+g-1
+__device__ __forceinline__ int outside(int k, int n, int g) { return k < g ? k - g : n + k - g; }
+
+// interior coordinates of ghost cell i; returns its index in the volume
+__device__ __forceinline__ long long ghost_cell(const GhostCells& C, long long i, int& x, int& y, int& z) {
+    if (i < C.planes) {
+        x = (int)(i % C.tot[0]) - C.g[0];
+        i /= C.tot[0];
+        y = (int)(i % C.tot[1]) - C.g[1];
+        z = outside((int)(i / C.tot[1]), C.n[2], C.g[2]);
+    } else if (i < C.rows) {
+        i -= C.planes;
+        x = (int)(i % C.tot[0]) - C.g[0];
+        i /= C.tot[0];
+        y = outside((int)(i % (2 * C.g[1])), C.n[1], C.g[1]);
+        z = (int)(i / (2 * C.g[1]));
+    } else {
+        i -= C.rows;
+        x = outside((int)(i % (2 * C.g[0])), C.n[0], C.g[0]);
+        i /= 2 * C.g[0];
+        y = (int)(i % C.n[1]);
+        z = (int)(i / C.n[1]);
+    }
+    return ((long long)(z + C.g[2]) * C.tot[1] + (y + C.g[1])) * C.tot[0] + (x + C.g[0]);
+}
+
 // Every ghost cell takes the value of the interior cell the boundary map
 // assigns to it; interior cells are only read, so the order does not matter.
-__global__ __launch_bounds__(256) void volume_boundary_kernel(VolPtrs V, int bc) {
-    const long long total = (long long)V.tot[0] * V.tot[1] * V.tot[2];
-    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < total; i += (long long)gridDim.x * 256) {
-        const int x = (int)(i % V.tot[0]) - V.g[0];
-        const int y = (int)((i / V.tot[0]) % V.tot[1]) - V.g[1];
-        const int z = (int)(i / ((long long)V.tot[0] * V.tot[1])) - V.g[2];
-        const bool ghost = x < 0 || x >= V.n[0] || y < 0 || y >= V.n[1] || z < 0 || z >= V.n[2];
-        if (!ghost) continue;
+// One variable a block (blockIdx.y), so that a thread pays one load's latency.
+__global__ __launch_bounds__(256) void volume_boundary_kernel(VolPtrs V, GhostCells C, int bc) {
+    for (long long j = (long long)blockIdx.x * 256 + threadIdx.x; j < C.all; j += (long long)gridDim.x * 256) {
+        int x, y, z;
+        const long long i = ghost_cell(C, j, x, y, z);
         const int sx = bc_map(x, V.n[0], bc);
         const int sy = V.g[1] ? bc_map(y, V.n[1], bc) : y;
         const int sz = V.g[2] ? bc_map(z, V.n[2], bc) : z;
         const long long si = ((long long)(sz + V.g[2]) * V.tot[1] + (sy + V.g[1])) * V.tot[0] + (sx + V.g[0]);
-        for (int v = 0; v < V.nv; ++v) V.v[v][i] = V.v[v][si];
+        double* const a = V.v[blockIdx.y];
+        a[i] = a[si];
     }
 }
 
@@ -245,7 +303,7 @@ __global__ __launch_bounds__(256) void volume_constraints_kernel(VolPtrs V, doub
         double q[NV];
 #pragma unroll
         for (int v = 0; v < NV; ++v) q[v] = V.v[v][i];
-        bad = bad || !EQ::obeys(q, gamma);
+        bad = bad || !EQ::obeys_fast(q, gamma);
     }
     if (__syncthreads_or(bad) && threadIdx.x == 0) atomicOr(flag, 1);
 }
@@ -262,31 +320,56 @@ struct CombineParams {
     double* out[5];
     const double* us[5];
     const double* u0[5];
-    int nv;
     long long cells;
     int mode;
-    double s;
+    double s;  // dt / dx, unless ctrl is given: its wave speeds then set dt
+    const Control* ctrl;
+    double cell[3], cfl, cap;
+    GhostCells ghosts;
 };
 
+// dt of the step: cfl / sum_d(ws_d / dx_d), at most `cap`
+__host__ __device__ double step_of(const double* ws, const double* cell, double cfl, double cap) {
+    double total = 0;
+    for (int d = 0; d < 3; ++d) {
+        if (cell[d] == 0) continue;
+        total += ws[d] / cell[d];
+    }
+    const double dt = cfl / total;
+    return (cap < dt) ? cap : dt;
+}
+
+// On every cell, or (GHOSTS) on the ghost cells alone; one variable a block.
+template <bool GHOSTS>
 __global__ __launch_bounds__(256) void volume_combine_kernel(CombineParams C) {
-    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < C.cells; i += (long long)gridDim.x * 256) {
-        for (int v = 0; v < C.nv; ++v) {
-            double o = C.out[v][i] * C.s;
-            o = o + C.us[v][i];
-            if (C.mode == COMBINE_RK2_1) {
-                o = o + C.u0[v][i];
-                o = o * 0.5;
-            } else if (C.mode == COMBINE_RK3_1) {
-                o = o * (1. / 3.);
-                o = o + C.u0[v][i];
-                o = o * (3. / 4.);
-            } else if (C.mode == COMBINE_RK3_2) {
-                o = o * 2;
-                o = o + C.u0[v][i];
-                o = o * (1. / 3.);
-            }
-            C.out[v][i] = o;
+    double s = C.s;
+    if (C.ctrl) {
+        double ws[3];
+        for (int d = 0; d < 3; ++d) ws[d] = wave_speed(C.ctrl, d);
+        s = step_of(ws, C.cell, C.cfl, C.cap) / C.cell[0];
+    }
+    double* const out = C.out[blockIdx.y];
+    const double* const us = C.us[blockIdx.y];
+    const double* const u0 = C.u0[blockIdx.y];
+    const long long total = GHOSTS ? C.ghosts.all : C.cells;
+    for (long long j = (long long)blockIdx.x * 256 + threadIdx.x; j < total; j += (long long)gridDim.x * 256) {
+        int x, y, z;
+        const long long i = GHOSTS ? ghost_cell(C.ghosts, j, x, y, z) : j;
+        double o = out[i] * s;
+        o = o + us[i];
+        if (C.mode == COMBINE_RK2_1) {
+            o = o + u0[i];
+            o = o * 0.5;
+        } else if (C.mode == COMBINE_RK3_1) {
+            o = o * (1. / 3.);
+            o = o + u0[i];
+            o = o * (3. / 4.);
+        } else if (C.mode == COMBINE_RK3_2) {
+            o = o * 2;
+            o = o + u0[i];
+            o = o * (1. / 3.);
         }
+        out[i] = o;
     }
 }
 
@@ -297,9 +380,17 @@ unsigned grid_blocks(long long cells) {
     return (unsigned)nb;
 }
 
-// flux over the box [start, n + end) into out; ws_host[3] the maxima
+// What the stage kernel writes in place of the net flux L:
+// ((L * s + in) * ca + u0) * cb.
+struct FusedCombine {
+    const avh_volume* u0;
+    double s, ca, cb;
+};
+
+// flux over the box [start, n + end) into out, enqueued; the wave speeds are
+// left in the context's scratch (none with `fuse`)
 avh_status volume_flux(avh_ctx* ctx, const avh_config* cfg, const avh_volume* in, avh_volume* out, const int* start,
-                       const int* end, double* ws_host, hipStream_t st) {
+                       const int* end, hipStream_t st, const FusedCombine* fuse = nullptr) {
     const int nv = nvars_of(cfg->equation);
     if (!nv) return fail(AVH_EINVAL, "unknown equation");
     const int G = ghosts_of(cfg->reconstruction);
@@ -336,21 +427,31 @@ avh_status volume_flux(avh_ctx* ctx, const avh_config* cfg, const avh_volume* in
     }
     Scratch* sc = nullptr;
     if ((r = ctx_scratch(ctx, &sc))) return r;
-    if (empty) {
-        for (int d = 0; d < 3; ++d) ws_host[d] = 0.0;
-        return AVH_OK;
-    }
     P.ctrl = &sc->ctrl;
     P.mode = MODE_FLUX_ONLY;
     P.gamma = cfg->gamma;
     P.ncells = 0;
+    if (fuse) {
+        P.mode = MODE_RK3_3;
+        for (int v = 0; v < nv; ++v) V.u0[v] = fuse->u0->var[v];
+        V.s = fuse->s;
+        V.ca = fuse->ca;
+        V.cb = fuse->cb;
+        AVH_HIP(L.volume(P, V, st));
+        return AVH_OK;
+    }
     hipLaunchKernelGGL(clear_scratch_kernel, dim3(1), dim3(64), 0, st, sc);
     AVH_HIP(hipGetLastError());
-    AVH_HIP(L.volume(P, V, st));
+    if (!empty) AVH_HIP(L.volume(P, V, st));
+    return AVH_OK;
+}
+
+// the wave speeds of the launches before, once they are done
+avh_status read_wave_speeds(avh_ctx* ctx, double* ws, hipStream_t st) {
     unsigned long long bits[3];
-    AVH_HIP(hipMemcpyAsync(bits, sc->ctrl.ws_bits, sizeof bits, hipMemcpyDeviceToHost, st));
+    AVH_HIP(hipMemcpyAsync(bits, ((Scratch*)ctx->scratch)->ctrl.ws_bits, sizeof bits, hipMemcpyDeviceToHost, st));
     AVH_HIP(hipStreamSynchronize(st));
-    for (int d = 0; d < 3; ++d) std::memcpy(&ws_host[d], &bits[d], sizeof(double));
+    for (int d = 0; d < 3; ++d) std::memcpy(&ws[d], &bits[d], sizeof(double));
     return AVH_OK;
 }
 
@@ -363,7 +464,9 @@ avh_status avh_numerical_flux(avh_ctx* ctx, const avh_config* cfg, const avh_vol
     if (!ctx || !cfg || !start || !end || !ws) return fail(AVH_EINVAL, "null argument");
     std::lock_guard<std::mutex> g(ctx->lock);
     AVH_HIP(hipSetDevice(ctx->device));
-    return volume_flux(ctx, cfg, in, out, start, end, ws, (hipStream_t)stream);
+    const hipStream_t st = (hipStream_t)stream;
+    const avh_status r = volume_flux(ctx, cfg, in, out, start, end, st);
+    return r ? r : read_wave_speeds(ctx, ws, st);
 }
 
 avh_status avh_reconstruction(avh_ctx* ctx, const avh_config* cfg, const avh_volume* in, int direction,
@@ -436,10 +539,12 @@ avh_status avh_apply_boundary(avh_ctx* ctx, int boundary, avh_volume* volume, vo
     std::lock_guard<std::mutex> g(ctx->lock);
     AVH_HIP(hipSetDevice(ctx->device));
     const hipStream_t st = (hipStream_t)stream;
-    const VolShape s = shape_of(volume);
-    hipLaunchKernelGGL(volume_boundary_kernel, dim3(grid_blocks(s.cells)), dim3(256), 0, st, ptrs_of(volume),
-                       boundary);
-    AVH_HIP(hipGetLastError());
+    const GhostCells c = ghost_cells(volume->n, volume->ghosts);
+    if (c.all > 0) {
+        hipLaunchKernelGGL(volume_boundary_kernel, dim3(grid_blocks(c.all), volume->nvars), dim3(256), 0, st,
+                           ptrs_of(volume), c, boundary);
+        AVH_HIP(hipGetLastError());
+    }
     AVH_HIP(hipStreamSynchronize(st));
     return AVH_OK;
 }
@@ -491,26 +596,12 @@ avh_status avh_substep(avh_ctx* ctx, const avh_config* cfg, const avh_volume* co
     std::lock_guard<std::mutex> g(ctx->lock);
     AVH_HIP(hipSetDevice(ctx->device));
     const hipStream_t st = (hipStream_t)stream;
-    // ConservedSystem: the interior plus the side strips equal one call over
-    // the whole interior (start = end = 0)
-    const int zero[3] = {0, 0, 0};
-    double ws[3];
-    if ((r = volume_flux(ctx, cfg, inputs[substep], out, zero, zero, ws, st))) return r;
     // Grid::computeCellLengths (alsfvm/src/grid/Grid.cpp:24-41): 1 on
     // single-cell axes
     double cell[3];
     for (int d = 0; d < 3; ++d) cell[d] = (cfg->upper[d] - cfg->lower[d]) / double(out->n[d]);
     if (out->n[1] == 1) cell[1] = 1;
     if (out->n[2] == 1) cell[2] = 1;
-    if (substep == 0) {
-        double total = 0;
-        for (int d = 0; d < 3; ++d) {
-            if (cell[d] == 0) continue;
-            total += ws[d] / cell[d];
-        }
-        dt = cfg->cfl / total;
-        dt = (dt_cap < dt) ? dt_cap : dt;
-    }
     CombineParams C;
     std::memset(&C, 0, sizeof C);
     for (int v = 0; v < nv; ++v) {
@@ -518,16 +609,50 @@ avh_status avh_substep(avh_ctx* ctx, const avh_config* cfg, const avh_volume* co
         C.us[v] = inputs[substep]->var[v];
         C.u0[v] = inputs[0]->var[v];
     }
-    C.nv = nv;
     C.cells = shape_of(out).cells;
-    C.s = dt / cell[0];
+    C.ghosts = ghost_cells(out->n, out->ghosts);
     C.mode = COMBINE_PLAIN;
     if (cfg->integrator == AVH_INT_RUNGEKUTTA2 && substep == 1) C.mode = COMBINE_RK2_1;
     if (cfg->integrator == AVH_INT_RUNGEKUTTA3 && substep == 1) C.mode = COMBINE_RK3_1;
     if (cfg->integrator == AVH_INT_RUNGEKUTTA3 && substep == 2) C.mode = COMBINE_RK3_2;
-    hipLaunchKernelGGL(volume_combine_kernel, dim3(grid_blocks(C.cells)), dim3(256), 0, st, C);
+    // ConservedSystem: the interior plus the side strips equal one call over
+    // the whole interior (start = end = 0)
+    const int zero[3] = {0, 0, 0};
+    // With dt given, the stage kernel combines as it writes (128^3, euler3: flux
+    // and combination 158 + 49 us apart, 159 + 14 for the ghost cells so).  The
+    // combination reads the inputs' cells after their stencils were read, so
+    // this needs an output apart from them; the ghost cells, which have no
+    // flux, take the Volume operations as before.
+    if (substep > 0 && !overlap(out, inputs[0]) && !overlap(out, inputs[substep])) {
+        FusedCombine f;
+        f.u0 = inputs[0];
+        f.s = C.s = dt / cell[0];
+        f.ca = C.mode == COMBINE_RK3_1 ? 1. / 3. : (C.mode == COMBINE_RK3_2 ? 2.0 : 1.0);
+        f.cb = C.mode == COMBINE_RK2_1 ? 0.5 : (C.mode == COMBINE_RK3_1 ? 3. / 4. : 1. / 3.);
+        if ((r = volume_flux(ctx, cfg, inputs[substep], out, zero, zero, st, &f))) return r;
+        if (C.ghosts.all > 0) {
+            hipLaunchKernelGGL(volume_combine_kernel<true>, dim3(grid_blocks(C.ghosts.all), nv), dim3(256), 0, st,
+                               C);
+            AVH_HIP(hipGetLastError());
+        }
+        AVH_HIP(hipStreamSynchronize(st));
+        *dt_out = dt;
+        return AVH_OK;
+    }
+    if ((r = volume_flux(ctx, cfg, inputs[substep], out, zero, zero, st))) return r;
+    if (substep == 0) {
+        C.ctrl = &((Scratch*)ctx->scratch)->ctrl;
+        for (int d = 0; d < 3; ++d) C.cell[d] = cell[d];
+        C.cfl = cfg->cfl;
+        C.cap = dt_cap;
+    } else {
+        C.s = dt / cell[0];
+    }
+    hipLaunchKernelGGL(volume_combine_kernel<false>, dim3(grid_blocks(C.cells), nv), dim3(256), 0, st, C);
     AVH_HIP(hipGetLastError());
-    AVH_HIP(hipStreamSynchronize(st));
+    double ws[3];
+    if ((r = read_wave_speeds(ctx, ws, st))) return r;
+    if (substep == 0) dt = step_of(ws, cell, cfg->cfl, dt_cap);
     *dt_out = dt;
     return AVH_OK;
 }
