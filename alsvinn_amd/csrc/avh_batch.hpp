@@ -193,6 +193,7 @@ struct StatsGroup {
     int* list_len;
     long long* counts;    // per save index: samples folded in so far
     int* active_count;
+    int* host_active;     // the same number in pinned host memory
     double* mean_c;       // [nsaves][nv][ncells]
     double* m2_c;
     double* mean_p;       // rho, u..., p

@@ -69,6 +69,7 @@ __global__ __launch_bounds__(1024) void batch_finish_kernel(StatsParams S) {
         }
         *G.list_len = s_base;
         *G.active_count = s_active;
+        __hip_atomic_store(G.host_active, s_active, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -456,6 +457,10 @@ struct avh_batch {
     // groups the stage and element-wise launches cover: a group whose
     // samples have all stopped is dropped until the next avh_batch_advance
     bool live[MAX_GROUPS] = {true, true, true, true};
+    // running samples per group, written by the end of a step into pinned
+    // memory, and the marks after which avh_batch_advance reads them
+    int* running = nullptr;
+    hipEvent_t passed[2] = {nullptr, nullptr};
     // workspace of the observables (at most OBS_SLAB_BYTES and one sample's
     // share), kept until the batch goes; `obs_lock` serialises its users
     std::mutex obs_lock;
@@ -486,6 +491,9 @@ void free_batch(avh_batch* b) {
         (void)hipFree(G.active_count);
     }
     (void)hipFree(b->work);
+    (void)hipHostFree(b->running);
+    for (hipEvent_t e : b->passed)
+        if (e) (void)hipEventDestroy(e);
     if (b->stream) (void)hipStreamDestroy(b->stream);
     delete b;
 }
@@ -572,6 +580,7 @@ StatsParams stats_params(const avh_batch* b, unsigned int* nblocks) {
         T.list_len = G.list_len;
         T.counts = G.counts;
         T.active_count = G.active_count;
+        T.host_active = b->running + i;
         T.mean_c = G.mean_c;
         T.m2_c = G.m2_c;
         T.mean_p = G.mean_p;
@@ -814,6 +823,12 @@ avh_status avh_batch_create(avh_ctx* ctx, const avh_config* cfg, int ngroups, co
         free_batch(b);
         return fail(AVH_EHIP, "hipStreamCreate failed");
     }
+    bool marks = hipHostMalloc(&b->running, sizeof(int) * MAX_GROUPS, hipHostMallocDefault) == hipSuccess;
+    for (hipEvent_t& e : b->passed) marks = marks && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+    if (!marks) {
+        free_batch(b);
+        return fail(AVH_ENOMEM, "host allocation failed");
+    }
     for (int i = 0; i < ngroups; ++i) {
         GroupHost& G = b->g[i];
         for (int d = 0; d < 3; ++d) G.n[d] = groups[i].n[d];
@@ -944,6 +959,28 @@ avh_status avh_batch_set_kh2d(avh_batch* b, int group, const double* host_interf
     return AVH_OK;
 }
 
+// Enqueues n steps.  They go out a graph's worth at a time, two ahead of the
+// device, so that what would follow the last sample's end is not launched at
+// all: a launch in which every sample has stopped still deals all its
+// workgroups (84 samples of 128^2 to 512^2: 9 us, and three of them a step).
+static avh_status enqueue_until_stopped(avh_batch* b, int64_t n) {
+    const int64_t unit = b->graph_steps >= 2 ? b->graph_steps : 8;
+    for (int64_t k = 0; n > 0; ++k, n -= unit) {
+        const hipEvent_t mark = b->passed[k % 2];
+        if (k >= 2) {
+            AVH_HIP(hipEventSynchronize(mark));
+            int running = 0;
+            for (int i = 0; i < b->ngroups; ++i) running += __atomic_load_n(b->running + i, __ATOMIC_RELAXED);
+            if (running == 0) return AVH_OK;
+        }
+        const avh_status r = enqueue_steps_graphed(b->graph, b->graph_steps, b->stream, std::min<int64_t>(n, unit),
+                                                   [b]() { return enqueue_batch_step(b); });
+        if (r) return r;
+        AVH_HIP(hipEventRecord(mark, b->stream));
+    }
+    return AVH_OK;
+}
+
 avh_status avh_batch_advance(avh_batch* b, int64_t max_steps, int chunk, int64_t* steps_done, int64_t* active_left) {
     if (!b) return fail(AVH_EINVAL, "null argument");
     if (chunk < 1) chunk = 1;
@@ -966,8 +1003,7 @@ avh_status avh_batch_advance(avh_batch* b, int64_t max_steps, int chunk, int64_t
     int64_t done = 0, left = 0;
     while (done < max_steps) {
         const int64_t k = std::min<int64_t>(chunk, max_steps - done);
-        avh_status r = enqueue_steps_graphed(b->graph, b->graph_steps, b->stream, k,
-                                             [b]() { return enqueue_batch_step(b); });
+        const avh_status r = enqueue_until_stopped(b, k);
         if (r) return r;
         done += k;
         AVH_HIP(hipStreamSynchronize(b->stream));
