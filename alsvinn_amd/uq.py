@@ -17,7 +17,7 @@ import ctypes
 import numpy as np
 
 from . import _abi
-from .initial_data import kh_interfaces
+from .initial_data import kh_interfaces_many
 from .simulator import (BOUNDARIES, EQUATIONS, FLUXES, INTEGRATORS, NVARS, RECONSTRUCTIONS, _lookup,
                         default_context, resolve_cfl, resolve_integrator)
 
@@ -143,12 +143,7 @@ class BatchRunner:
         """params: (nsamples, 40) perturbation parameters per sample."""
         n = self.groups[group][0]
         params = np.asarray(params, dtype=np.float64)
-        iface = np.empty((params.shape[0], 2, n[0]))
-        for s in range(params.shape[0]):
-            lo, hi = kh_interfaces(n[0], params[s])
-            iface[s, 0] = lo
-            iface[s, 1] = hi
-        iface = np.ascontiguousarray(iface)
+        iface = kh_interfaces_many(n[0], params)
         _abi.check(_abi.load().avh_batch_set_kh2d(self._h, int(group), iface.ctypes.data))
 
     def run(self, max_steps=1 << 62, chunk=64):
