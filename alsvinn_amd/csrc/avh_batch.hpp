@@ -85,7 +85,7 @@ __device__ __forceinline__ int batch_group(const BatchParams& B, unsigned int b)
 }
 
 template <class K>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void batch_stage_kernel(BatchParams B) {
+__global__ __launch_bounds__(K::NTHREADS) __attribute__((amdgpu_waves_per_eu(4))) void batch_stage_kernel(BatchParams B) {
     int gi = 0;
     unsigned int sample = 0, tile = 0;
     if (!batch_stage_decode(B, blockIdx.x, gi, sample, tile)) return;

@@ -504,7 +504,7 @@ struct StageKernel1 {
 };
 
 template <class K>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void stage_kernel(StageParams P) {
+__global__ __launch_bounds__(K::NTHREADS) __attribute__((amdgpu_waves_per_eu(4))) void stage_kernel(StageParams P) {
     K::run(P);
 }
 

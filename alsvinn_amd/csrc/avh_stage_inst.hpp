@@ -22,13 +22,18 @@ typedef hipError_t (*VolumeLauncher)(const StageParams& P, const VolumeParams& V
 // order, so the choice never changes a result bit.
 //   1D: (cells, threads) = (256, 256) or (64, 64): small grids get more
 //       workgroups from the smaller tile.
-//   2D: 64x7, 16x15, 16x7, 32x15 or 16x28 cells, 256 threads.  A flux pass
-//       costs a wave its full instruction stream however few of its lanes
-//       have an item, so the shapes' items sit just under the 256 threads:
-//       two interfaces a thread for 64x7 (231 x / 256 y turns), 32x15 (255 /
-//       256) and 16x28 (252 / 240), one for 16x15 (255 / 256), and one for
-//       both directions together for 16x7 (119 + 128), the shape of small
-//       grids: more workgroups and half the chain.
+//   2D: a flux pass costs a wavefront its full instruction stream however few
+//       of its lanes have an item, so the shapes' items sit just under their
+//       threads.  32x15 on 256 threads (255 x / 256 y turns of two
+//       interfaces) and 32x11 on 192 do the least work a cell and take the
+//       large grids.  On smaller ones a workgroup's chain is what counts:
+//       16x15 on 512 threads, 32x15 on 1024 and 16x7 on 256 evaluate both
+//       directions side by side, one interface a thread (a lone tile takes
+//       5.6, 7.7 and 4.8 us, 32x15 on 256 threads 8.9).  us of an RK3 stage
+//       pair, 32x15 on 256 / 16x15 on 512 / 16x7: 64^2 17.9 / 11.2 / 9.6,
+//       256^2 19.8 / 17.3 / 18.8, 501x333 27.4 / 25.9 / 33.8, 1024^2
+//       91 / 112 / 165; 700x300, eno3, hll, first stage: 16.4, 32x15 on 1024
+//       threads 15.5.
 //   3D: 16x15 or 32x7 columns marching over 2 to 32 planes, 256 threads (at
 //       most 256 interfaces a plane in each direction: one turn; the threads
 //       past the columns only work on the planes).  A chunk pays a z flux
@@ -40,8 +45,9 @@ typedef hipError_t (*VolumeLauncher)(const StageParams& P, const VolumeParams& V
 //       76 / 87 / 159 / 299 / 64, 160^3 616 / 559 / 585 / 710 / 555.
 constexpr int NSHAPES1 = 2, NSHAPES2 = 5, NSHAPES3 = 7;
 constexpr int SHAPE1_TX[NSHAPES1] = {256, 64};
-constexpr int SHAPE2_TX[NSHAPES2] = {64, 16, 16, 32, 16};
-constexpr int SHAPE2_TY[NSHAPES2] = {7, 15, 7, 15, 28};
+constexpr int SHAPE2_TX[NSHAPES2] = {32, 16, 16, 32, 32};
+constexpr int SHAPE2_TY[NSHAPES2] = {11, 15, 7, 15, 15};
+constexpr int SHAPE2_NT[NSHAPES2] = {192, 512, 256, 256, 1024};
 constexpr int SHAPE3_TX[NSHAPES3] = {16, 16, 32, 32, 16, 16, 16};
 constexpr int SHAPE3_TY[NSHAPES3] = {15, 15, 7, 7, 15, 15, 15};
 constexpr int SHAPE3_LZ[NSHAPES3] = {4, 0, 8, 32, 16, 2, 32};  // 0: march_chunk
@@ -56,16 +62,16 @@ struct KernelFor<EQ, RECON, FLUX, 1, S> {
 };
 template <class EQ, int RECON, class FLUX, int S>
 struct KernelFor<EQ, RECON, FLUX, 2, S> {
-    typedef TileKernel2<EQ, RECON, FLUX, SHAPE2_TX[S], SHAPE2_TY[S], 256> type;
+    typedef TileKernel2<EQ, RECON, FLUX, SHAPE2_TX[S], SHAPE2_TY[S], SHAPE2_NT[S]> type;
 };
 // 2D shapes whose RK3 stages are each compiled for their mode (the shapes
 // the autotuner takes most); those kernels index cells with 32-bit values, so
 // they serve grids of fewer than 2^29 cells (per sample in a batch)
-constexpr bool SHAPE2_BY_MODE[NSHAPES2] = {false, false, true, true, false};
+constexpr bool SHAPE2_BY_MODE[NSHAPES2] = {false, true, true, true, true};
 constexpr long long MODE_KERNEL_MAX_CELLS = 1ll << 29;
 template <class EQ, int RECON, class FLUX, int S, int MODE>
 struct KernelForMode {
-    typedef TileKernel2<EQ, RECON, FLUX, SHAPE2_TX[S], SHAPE2_TY[S], 256, MODE> type;
+    typedef TileKernel2<EQ, RECON, FLUX, SHAPE2_TX[S], SHAPE2_TY[S], SHAPE2_NT[S], MODE> type;
 };
 
 // stage tiles (workgroups) covering one grid of the 1D / 2D kernels
