@@ -32,6 +32,7 @@ struct GroupDesc {
     const double* in;
     const double* u0;
     double* out;
+    double* copy;              // StageParams::copy, or null
     Control* ctrl;             // nsamples consecutive Control blocks
     long long stride;          // doubles from one sample's state to the next
     long long ncells;
@@ -94,6 +95,7 @@ __global__ __launch_bounds__(K::NTHREADS) __attribute__((amdgpu_waves_per_eu(4))
     P.in = G.in + (long long)sample * G.stride;
     P.u0 = G.u0 + (long long)sample * G.stride;
     P.out = G.out + (long long)sample * G.stride;
+    P.copy = G.copy ? G.copy + (long long)sample * G.stride : nullptr;
     P.ctrl = G.ctrl + sample;
     P.ncells = G.ncells;
     P.n[0] = G.n[0];
@@ -105,11 +107,10 @@ __global__ __launch_bounds__(K::NTHREADS) __attribute__((amdgpu_waves_per_eu(4))
     K::run_tile(P, tile);
 }
 
-// Element-wise out = L*s + U0 for every sample (forward euler's finish with
-// the constraint check, or rk2's U1); blocks as in the stage launch but
-// 256 cells each.
+// Forward euler's finish for every sample: out = L*s + U0 element-wise and the
+// constraint check; blocks as in the stage launch but 256 cells each.
 template <class EQ>
-__global__ __launch_bounds__(256) void batch_ew_kernel(BatchParams B, int fe_finish) {
+__global__ __launch_bounds__(256) void batch_ew_kernel(BatchParams B) {
     const unsigned int b = blockIdx.x;
     const int gi = batch_group(B, b);
     const GroupDesc& G = B.g[gi];
@@ -138,13 +139,11 @@ __global__ __launch_bounds__(256) void batch_ew_kernel(BatchParams B, int fe_fin
             x = x + u[v];
             r[v] = x;
         }
-        if (fe_finish) bad = !EQ::obeys_fast(r, B.gamma);
+        bad = !EQ::obeys_fast(r, B.gamma);
 #pragma unroll
         for (int v = 0; v < NV; ++v) G.out[o + v * G.ncells + i] = r[v];
     }
-    if (fe_finish) {
-        if (__syncthreads_or(bad) && threadIdx.x == 0) atomicOr(&ctrl->block_violation, 1);
-    }
+    if (__syncthreads_or(bad) && threadIdx.x == 0) atomicOr(&ctrl->block_violation, 1);
 }
 
 // One sample's end of step (same bookkeeping as finish_step_kernel).

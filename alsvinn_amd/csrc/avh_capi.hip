@@ -9,7 +9,7 @@
 // Step sequences (reference: alsfvm/src/integrator/{ForwardEuler,RungeKutta2,
 // RungeKutta3}.cpp, Simulator::incrementSolution Simulator.cpp:191-214):
 //   forwardeuler: stage(L: A->B) ; ew(A = B*s + A, check, end step)
-//   rungekutta2 : stage(L: A->B) ; ew(C = B*s + A) ; stage(RK2_2: C, A -> A)
+//   rungekutta2 : stage(L: A->B, copy A->C) ; stage(RK2_2: B*s + C, C -> A)
 //   rungekutta3 : stage(L: A->B) ; stage(RK3_2: B*s+A on the fly -> C) ;
 //                 stage(RK3_3: C, A -> A)
 #include <hip/hip_runtime.h>
@@ -42,13 +42,11 @@ __global__ __launch_bounds__(64) void finish_step_kernel(Control* c) {
     end_step(c, c->block_violation != 0);
 }
 
-enum EwMode { EW_FE_FINISH = 0, EW_RK2_U1 = 1 };
-
-// out = L*s + U0 element-wise (Volume *= dt/dx; += U0).  EW_FE_FINISH writes
-// in place into U0, checks the constraints and closes the step.
+// Forward euler's finish: U = L*s + U element-wise (Volume *= dt/dx; += U) and
+// the constraint check.
 template <class EQ>
-__global__ __launch_bounds__(256) void ew_kernel(const double* L, const double* u0, double* out,
-                                                 Control* ctrl, long long nc, int mode, double gamma) {
+__global__ __launch_bounds__(256) void ew_kernel(const double* L, double* state, Control* ctrl, long long nc,
+                                                 double gamma) {
     constexpr int NV = EQ::NV;
     const long long step = (long long)gridDim.x * blockDim.x;
     long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -58,7 +56,7 @@ __global__ __launch_bounds__(256) void ew_kernel(const double* L, const double* 
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
             l[v] = L[v * nc + i];
-            u[v] = u0[v * nc + i];
+            u[v] = state[v * nc + i];
         }
     }
     if (!ctrl->active) return;
@@ -78,16 +76,14 @@ __global__ __launch_bounds__(256) void ew_kernel(const double* L, const double* 
 #pragma unroll
             for (int v = 0; v < NV; ++v) {
                 l[v] = L[v * nc + i];
-                u[v] = u0[v * nc + i];
+                u[v] = state[v * nc + i];
             }
         }
-        if (mode == EW_FE_FINISH) bad = bad || !EQ::obeys_fast(r, gamma);
+        bad = bad || !EQ::obeys_fast(r, gamma);
 #pragma unroll
-        for (int v = 0; v < NV; ++v) out[v * nc + at] = r[v];
+        for (int v = 0; v < NV; ++v) state[v * nc + at] = r[v];
     }
-    if (mode == EW_FE_FINISH) {
-        if (__syncthreads_or(bad) && threadIdx.x == 0) atomicOr(&ctrl->block_violation, 1);
-    }
+    if (__syncthreads_or(bad) && threadIdx.x == 0) atomicOr(&ctrl->block_violation, 1);
 }
 
 // Ghosted export: every cell of the (n+2g)-sized volume takes the value of
@@ -224,16 +220,13 @@ __global__ __launch_bounds__(256) void arith_selftest_kernel(int kind, unsigned 
     }
 }
 
-typedef void (*EwLauncher)(const double*, const double*, double*, Control*, long long, int, double,
-                           hipStream_t);
+typedef void (*EwLauncher)(const double*, double*, Control*, long long, double, hipStream_t);
 
 template <class EQ>
-void launch_ew(const double* L, const double* u0, double* out, Control* c, long long nc, int mode,
-               double gamma, hipStream_t st) {
+void launch_ew(const double* L, double* state, Control* c, long long nc, double gamma, hipStream_t st) {
     long long nb = (nc + 255) / 256;
     if (nb > 4096) nb = 4096;
-    hipLaunchKernelGGL(ew_kernel<EQ>, dim3((unsigned)nb), dim3(256), 0, st, L, u0, out, c, nc, mode,
-                       gamma);
+    hipLaunchKernelGGL(ew_kernel<EQ>, dim3((unsigned)nb), dim3(256), 0, st, L, state, c, nc, gamma);
 }
 
 // One sample folded into running mean / M2 arrays (Welford, n = samples
@@ -485,23 +478,21 @@ static avh_status enqueue_step(avh_solver* s, EventMarks* tm = nullptr) {
     P.u0 = s->A;
     P.out = s->B;
     P.mode = MODE_L;
+    P.copy = s->cfg.integrator == AVH_INT_RUNGEKUTTA2 ? s->C : nullptr;
     avh_status r;
     if ((r = mark(s, tm))) return r;
     AVH_HIP(s->stage(P, s->shape, s->stream));
     if ((r = mark(s, tm))) return r;
     if (s->cfg.integrator == AVH_INT_FORWARDEULER) {
-        s->ew(s->B, s->A, s->A, s->ctrl, s->ncells, EW_FE_FINISH, s->cfg.gamma, s->stream);
+        s->ew(s->B, s->A, s->ctrl, s->ncells, s->cfg.gamma, s->stream);
         AVH_HIP(hipGetLastError());
         if ((r = mark(s, tm))) return r;
         hipLaunchKernelGGL(finish_step_kernel, dim3(1), dim3(64), 0, s->stream, s->ctrl);
         AVH_HIP(hipGetLastError());
         if ((r = mark(s, tm))) return r;
     } else if (s->cfg.integrator == AVH_INT_RUNGEKUTTA2) {
-        s->ew(s->B, s->A, s->C, s->ctrl, s->ncells, EW_RK2_U1, s->cfg.gamma, s->stream);
-        AVH_HIP(hipGetLastError());
-        if ((r = mark(s, tm))) return r;
-        P.in = s->C;
-        P.u0 = s->A;
+        P.in = s->B;
+        P.u0 = s->C;
         P.out = s->A;
         P.mode = MODE_RK2_2;
         P.finish = 1;
@@ -532,10 +523,10 @@ static TuneKey tune_key(const avh_solver* s) {
 
 // Times every tile shape on the current state and keeps the fastest: the
 // first stage (writing the L0 buffer, which every step overwrites; flux-only
-// if the solver has stopped), and for RK3 also the second stage on its output
-// (input formed on the fly from L0 and U0, writing the U2 buffer), whose extra
-// reads weigh differently on different shapes.  The state is not written; the wave-speed maxima the
-// launches add to are restored.
+// if the solver has stopped), and for RK2 and RK3 also the second stage on its
+// output (input formed on the fly from L0 and U0, writing the U2 buffer), whose
+// extra reads weigh differently on different shapes.  The state is not written;
+// the control block, which the launches add to, is restored.
 static avh_status autotune(avh_solver* s, int* best, double* ms, int* nshapes) {
     const int ns = num_shapes(s->dim);
     avh_status r = pull(s);
@@ -551,11 +542,13 @@ static avh_status autotune(avh_solver* s, int* best, double* ms, int* nshapes) {
     P.u0 = s->A;
     P.out = s->B;
     P.mode = s->h.active ? MODE_L : MODE_FLUX_ONLY;
+    if (s->cfg.integrator == AVH_INT_RUNGEKUTTA2) P.copy = s->C;
     StageParams P2 = P;
+    P2.copy = nullptr;
     P2.in = s->B;
     P2.out = s->C;
-    P2.mode = MODE_RK3_2;
-    const bool rk3 = s->cfg.integrator == AVH_INT_RUNGEKUTTA3 && s->h.active;
+    P2.mode = s->cfg.integrator == AVH_INT_RUNGEKUTTA3 ? MODE_RK3_2 : MODE_RK2_2;
+    const bool second = s->cfg.integrator != AVH_INT_FORWARDEULER && s->h.active;
     int b = 0;
     double tmin = 0;
     for (int k = 0; k < ns; ++k) {
@@ -564,7 +557,7 @@ static avh_status autotune(avh_solver* s, int* best, double* ms, int* nshapes) {
             r = time_launches(s->stream, 5,
                               [&]() {
                                   hipError_t e = s->stage(P, k, s->stream);
-                                  if (e == hipSuccess && rk3) e = s->stage(P2, k, s->stream);
+                                  if (e == hipSuccess && second) e = s->stage(P2, k, s->stream);
                                   return e;
                               },
                               &t);
@@ -923,16 +916,16 @@ avh_status avh_step_noalloc(avh_ctx* ctx, const avh_config* cfg, double* state, 
     P.u0 = state;
     P.out = B;
     P.mode = MODE_L;
+    P.copy = cfg->integrator == AVH_INT_RUNGEKUTTA2 ? C : nullptr;
     AVH_HIP(stage(P, shape, st));
     if (cfg->integrator == AVH_INT_FORWARDEULER) {
-        ew(B, state, state, ctrl, ncells, EW_FE_FINISH, cfg->gamma, st);
+        ew(B, state, ctrl, ncells, cfg->gamma, st);
         AVH_HIP(hipGetLastError());
         hipLaunchKernelGGL(finish_step_kernel, dim3(1), dim3(64), 0, st, ctrl);
         AVH_HIP(hipGetLastError());
     } else if (cfg->integrator == AVH_INT_RUNGEKUTTA2) {
-        ew(B, state, C, ctrl, ncells, EW_RK2_U1, cfg->gamma, st);
-        AVH_HIP(hipGetLastError());
-        P.in = C;
+        P.in = B;
+        P.u0 = C;
         P.out = state;
         P.mode = MODE_RK2_2;
         P.finish = 1;
@@ -1005,10 +998,9 @@ avh_status avh_time_step_kernels(avh_solver* s, int64_t steps, double* ms, int* 
     if (!s || !ms || !kernels || steps < 1 || steps > 100000) return fail(AVH_EINVAL, "bad argument");
     avh_status r = use_device(s);
     if (r) return r;
-    // launches per step: the stages, the element-wise pass of forward euler
-    // / rk2, and forward euler's end-of-step kernel (the rk final stages end
-    // the step themselves)
-    const int nk = 3;
+    // launches per step: the stages, and forward euler's element-wise pass and
+    // end-of-step kernel (the rk final stages end the step themselves)
+    const int nk = s->cfg.integrator == AVH_INT_RUNGEKUTTA2 ? 2 : 3;
     if ((r = ensure_shape(s))) return r;
     EventMarks t;
     if ((r = t.create((size_t)steps * (nk + 1)))) return r;

@@ -66,17 +66,22 @@ struct Control {
 enum StageMode {
     MODE_FLUX_ONLY = 0,  // out = net flux, wave speeds accumulated, nothing else
     MODE_L = 1,          // first stage: out = L(U0), last block computes dt
-    MODE_RK2_2 = 2,      // in = U1;      out = ((L*s + U1) + U0) * 0.5, ends step
+    MODE_RK2_2 = 2,      // in = L0*s+U0; out = ((L*s + U1) + U0) * 0.5, ends step
     MODE_RK3_2 = 3,      // in = L0*s+U0; out = ((L*s + U1) * (1/3) + U0) * (3/4)
     MODE_RK3_3 = 4       // in = U2;      out = ((L*s + U2) * 2 + U0) * (1/3), ends step
 };
+
+// modes whose input is U1 = L0*s + U0, formed as the tile loads
+__host__ __device__ __forceinline__ constexpr bool on_the_fly(int mode) {
+    return mode == MODE_RK3_2 || mode == MODE_RK2_2;
+}
 
 enum { BC_PERIODIC = 0, BC_NEUMANN = 1 };
 
 struct StageParams {
     const double* in;  // stage input U_s, or L0 in the on-the-fly modes
     const double* u0;  // U0 (on-the-fly input and RK combination)
-    double* out;       // stage output (may equal u0 in MODE_RK2_2 / MODE_RK3_3:
+    double* out;       // stage output (may equal u0 in MODE_RK3_3:
                        // u0 is then read only at the cell being written)
     Control* ctrl;
     long long ncells;  // interior cells; variable stride of every buffer
@@ -87,6 +92,11 @@ struct StageParams {
     // 1: the launch is the step's last stage and its last workgroup runs the
     // end of the step (end_step); 0: the caller runs finish_step_kernel
     int finish = 0;
+    // MODE_L: where each cell's input is written as well, unless null.  RK2's
+    // second stage overwrites the state, and reads neighbours' U0 from here, to
+    // form U1 = L0*s + U0 as it loads: an element-wise pass for U1 took 6.6 of a
+    // 501x333 step's 46 us, the copy and the second operand together 2.
+    double* copy = nullptr;
     int lz = 0;  // 3D: planes a workgroup marches through (set by the launcher)
 };
 
@@ -366,7 +376,7 @@ struct StageKernel1 {
         const int n0 = P.n[0];
         const int ox = (int)tile * TX;
         const long long nc = P.ncells;
-        const bool otf = (mode == MODE_RK3_2);
+        const bool otf = on_the_fly(mode);
         const double s = (mode == MODE_FLUX_ONLY || mode == MODE_L) ? 0.0
                          : VOL                                       ? V->s
                                                                      : step_dt(ctrl) / ctrl->cell[0];
@@ -497,6 +507,10 @@ struct StageKernel1 {
             for (int v = 0; v < NV; ++v) {
                 if constexpr (VOL) V->out[v][gc[m]] = r[v];
                 else P.out[v * nc + gc[m]] = r[v];
+            }
+            if (mode == MODE_L && P.copy) {
+#pragma unroll
+                for (int v = 0; v < NV; ++v) P.copy[v * nc + gc[m]] = su[v * LT + c + G];
             }
         }
         if (!VOL || mode == MODE_FLUX_ONLY) end_of_tile<NT>(P, ctrl, mode, ws, 0.0, 0.0, s_ws, bad);

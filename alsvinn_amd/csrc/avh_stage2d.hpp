@@ -182,7 +182,7 @@ struct TileKernel2 {
         const int ntx = (n0 + TX - 1) / TX;
         const int ox = (int)(tile % ntx) * TX, oy = (int)(tile / ntx) * TY;
         const long long nc = P.ncells;
-        const bool otf = (mode == MODE_RK3_2);
+        const bool otf = on_the_fly(mode);
 
         // 1. stage input tile + halo into LDS through the boundary map.  All
         // loads are issued before the first is used; rows past the tile
@@ -329,6 +329,10 @@ struct TileKernel2 {
             for (int v = 0; v < NV; ++v) {
                 if constexpr (VOL) V->out[v][gc[m]] = r[v];
                 else soa_st<OFF32>(P.out, nc, v, gc[m], r[v]);
+            }
+            if (mode == MODE_L && P.copy) {
+#pragma unroll
+                for (int v = 0; v < NV; ++v) soa_st<OFF32>(P.copy, nc, v, gc[m], su[v * LT + li]);
             }
         }
         if (!VOL || mode == MODE_FLUX_ONLY) end_of_tile<NT>(P, ctrl, mode, ws[0], ws[1], 0.0, s_ws, bad);

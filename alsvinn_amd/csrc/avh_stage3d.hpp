@@ -206,7 +206,7 @@ struct MarchKernel3 {
         }
     }
 
-    // The kernel compiled for the on-the-fly stage (U1 = L0*s + U0 formed as
+    // A kernel compiled for an on-the-fly stage (U1 = L0*s + U0 formed as
     // the tile loads) reads the column's U0 with each window plane; its RK
     // combination needs the same U0 again RING planes later, by which time
     // the line has left L2.  A thread-private LDS ring of RING planes keeps
@@ -215,7 +215,7 @@ struct MarchKernel3 {
     static constexpr int RING = 2 + HW;
     static constexpr int LDS_BASE =
         8 * (2 * NV * LP + 2 * NV * NIMAX + 3 * (NT / 64)) + 8 * (NT / 64);
-    static constexpr bool U0RING = MODE_CT == MODE_RK3_2 && LDS_BASE + 8 * RING * NV * NC <= 80 * 1024;
+    static constexpr bool U0RING = on_the_fly(MODE_CT) && LDS_BASE + 8 * RING * NV * NC <= 80 * 1024;
 
     // interface between plane cells ia and ia + SD under OPS
     template <class OPS, int DIR>
@@ -301,7 +301,7 @@ struct MarchKernel3 {
         const int tz = tile / (ntx * nty);
         const int ox = tx * TX, oy = ty * TY, z0 = tz * P.lz;
         const int z1 = (z0 + P.lz < n2) ? z0 + P.lz : n2;
-        const bool otf = (mode == MODE_RK3_2);
+        const bool otf = on_the_fly(mode);
         const double s = (mode == MODE_FLUX_ONLY || mode == MODE_L) ? 0.0
                          : VOL                                       ? V->s
                                                                      : step_dt(ctrl) / ctrl->cell[0];
@@ -568,6 +568,10 @@ struct MarchKernel3 {
                 for (int v = 0; v < NV; ++v) {
                     if constexpr (VOL) V->out[v][gi] = r[v];
                     else soa_st<OFF32>(P.out, P.ncells, v, gi, r[v]);
+                }
+                if (mode == MODE_L && P.copy) {
+#pragma unroll
+                    for (int v = 0; v < NV; ++v) soa_st<OFF32>(P.copy, P.ncells, v, gi, w[HW - 1][v]);
                 }
             }
 #pragma unroll

@@ -64,7 +64,7 @@ template <class EQ, int RECON, class FLUX, int S>
 struct KernelFor<EQ, RECON, FLUX, 2, S> {
     typedef TileKernel2<EQ, RECON, FLUX, SHAPE2_TX[S], SHAPE2_TY[S], SHAPE2_NT[S]> type;
 };
-// 2D shapes whose RK3 stages are each compiled for their mode (the shapes
+// 2D shapes whose RK stages are each compiled for their mode (the shapes
 // the autotuner takes most); those kernels index cells with 32-bit values, so
 // they serve grids of fewer than 2^29 cells (per sample in a batch)
 constexpr bool SHAPE2_BY_MODE[NSHAPES2] = {false, true, true, true, true};
@@ -105,6 +105,9 @@ hipError_t launch_batch_stage(const BatchParams& B, unsigned int nblocks, int sh
             } else if (B.mode == MODE_L)                                                                    \
                 return launch_batch_k<typename KernelForMode<EQ, RECON, FLUX, S, MODE_L>::type>(B, nblocks, \
                                                                                                stream);     \
+            else if (B.mode == MODE_RK2_2)                                                                  \
+                return launch_batch_k<typename KernelForMode<EQ, RECON, FLUX, S, MODE_RK2_2>::type>(        \
+                    B, nblocks, stream);                                                                    \
             else if (B.mode == MODE_RK3_2)                                                                  \
                 return launch_batch_k<typename KernelForMode<EQ, RECON, FLUX, S, MODE_RK3_2>::type>(        \
                     B, nblocks, stream);                                                                    \
@@ -199,6 +202,9 @@ hipError_t launch_stage(const StageParams& P, int shape, hipStream_t stream) {
             if (P.ncells >= MODE_KERNEL_MAX_CELLS) {                                                        \
             } else if (P.mode == MODE_L)                                                                    \
                 return launch_stage_k<typename KernelForMode<EQ, RECON, FLUX, S, MODE_L>::type>(P, stream); \
+            else if (P.mode == MODE_RK2_2)                                                                  \
+                return launch_stage_k<typename KernelForMode<EQ, RECON, FLUX, S, MODE_RK2_2>::type>(P,      \
+                                                                                                 stream);   \
             else if (P.mode == MODE_RK3_2)                                                                  \
                 return launch_stage_k<typename KernelForMode<EQ, RECON, FLUX, S, MODE_RK3_2>::type>(P,      \
                                                                                                  stream);   \

@@ -405,14 +405,14 @@ struct GroupHost {
 };
 
 template <class EQ>
-void launch_batch_ew(const BatchParams& B, unsigned int nblocks, int fe_finish, hipStream_t st) {
-    hipLaunchKernelGGL(batch_ew_kernel<EQ>, dim3(nblocks), dim3(256), 0, st, B, fe_finish);
+void launch_batch_ew(const BatchParams& B, unsigned int nblocks, hipStream_t st) {
+    hipLaunchKernelGGL(batch_ew_kernel<EQ>, dim3(nblocks), dim3(256), 0, st, B);
 }
 template <class EQ>
 void launch_batch_stats(const StatsParams& S, unsigned int nblocks, hipStream_t st) {
     hipLaunchKernelGGL(batch_stats_kernel<EQ>, dim3(nblocks), dim3(256), 0, st, S);
 }
-typedef void (*BatchEw)(const BatchParams&, unsigned int, int, hipStream_t);
+typedef void (*BatchEw)(const BatchParams&, unsigned int, hipStream_t);
 typedef void (*BatchStats)(const StatsParams&, unsigned int, hipStream_t);
 
 BatchEw batch_ew_for(int eq) {
@@ -601,7 +601,7 @@ TuneKey batch_tune_key(const avh_batch* b) {
 }
 
 // Times every tile shape over all samples with the first stage (flux-only if
-// every sample has stopped) and, for RK3, the second stage, and keeps the
+// every sample has stopped) and, for RK2 and RK3, the second stage, and keeps the
 // fastest.  They write the L0 and U2 buffers and add to the per-sample
 // wave-speed maxima; the control blocks are restored afterwards.
 void set_all_live(avh_batch* b);
@@ -619,7 +619,7 @@ avh_status batch_autotune(avh_batch* b, int* best, double* ms, int* nshapes) {
     bool active = false;
     for (const auto& cs : saved)
         for (const Control& c : cs) active = active || c.active;
-    const bool rk3 = active && b->cfg.integrator == AVH_INT_RUNGEKUTTA3;
+    const bool second = active && b->cfg.integrator != AVH_INT_FORWARDEULER;
     const int keep = b->shape;
     int bst = 0;
     double tmin = 0;
@@ -630,17 +630,19 @@ avh_status batch_autotune(avh_batch* b, int* best, double* ms, int* nshapes) {
             b->shape = k;
             unsigned int nb = 0;
             BatchParams P = batch_params(b, active ? MODE_L : MODE_FLUX_ONLY, false, &nb);
-            BatchParams P2 = batch_params(b, MODE_RK3_2, false, &nb);
+            BatchParams P2 =
+                batch_params(b, b->cfg.integrator == AVH_INT_RUNGEKUTTA3 ? MODE_RK3_2 : MODE_RK2_2, false, &nb);
             for (int i = 0; i < b->ngroups; ++i) {
                 P.g[i].in = P.g[i].u0 = P2.g[i].u0 = b->g[i].A;
                 P.g[i].out = b->g[i].B;
+                if (b->cfg.integrator == AVH_INT_RUNGEKUTTA2) P.g[i].copy = b->g[i].C;
                 P2.g[i].in = b->g[i].B;
                 P2.g[i].out = b->g[i].C;
             }
             r = time_launches(b->stream, 3,
                               [&]() {
                                   hipError_t e = b->stage(P, nb, k, b->stream);
-                                  if (e == hipSuccess && rk3) e = b->stage(P2, nb, k, b->stream);
+                                  if (e == hipSuccess && second) e = b->stage(P2, nb, k, b->stream);
                                   return e;
                               },
                               &t);
@@ -675,11 +677,10 @@ avh_status batch_ensure_shape(avh_batch* b) {
     return batch_autotune(b, nullptr, nullptr, nullptr);
 }
 
-// Launches per batch step: the stages (plus forward euler's / rk2's
-// element-wise pass), the end-of-step kernel and, with statistics, the
-// statistics kernel.
+// Launches per batch step: the stages (plus forward euler's element-wise
+// pass), the end-of-step kernel and, with statistics, the statistics kernel.
 int batch_launches_per_step(const avh_batch* b) {
-    const int stages = b->cfg.integrator == AVH_INT_FORWARDEULER ? 2 : 3;
+    const int stages = b->cfg.integrator == AVH_INT_RUNGEKUTTA3 ? 3 : 2;
     return stages + 1 + (b->nsaves > 0 ? 1 : 0);
 }
 
@@ -712,27 +713,23 @@ avh_status enqueue_batch_step(avh_batch* b, EventMarks* tm = nullptr) {
         if (nb) AVH_HIP(b->stage(P, nb, b->shape, b->stream));
         return mark(tm, b->stream);
     };
-    auto ew = [&](BatchParams& E, int fe_finish) -> avh_status {
-        if (nbe) {
-            b->ew(E, nbe, fe_finish, b->stream);
-            AVH_HIP(hipGetLastError());
-        }
-        return mark(tm, b->stream);
-    };
     enum { A = 0, B = 1, C = 2 };
     BatchParams P = batch_params(b, MODE_L, false, &nb, index);
     set_ptrs(P, A, A, B);
+    if (b->cfg.integrator == AVH_INT_RUNGEKUTTA2)
+        for (int j = 0; j < P.ngroups; ++j) P.g[j].copy = b->g[index[j]].C;
     if ((r = stage(P))) return r;
     if (b->cfg.integrator == AVH_INT_FORWARDEULER) {
         BatchParams E = batch_params(b, MODE_L, true, &nbe, index);
         set_ptrs(E, B, A, A);
-        if ((r = ew(E, 1))) return r;
+        if (nbe) {
+            b->ew(E, nbe, b->stream);
+            AVH_HIP(hipGetLastError());
+        }
+        if ((r = mark(tm, b->stream))) return r;
     } else if (b->cfg.integrator == AVH_INT_RUNGEKUTTA2) {
-        BatchParams E = batch_params(b, MODE_L, true, &nbe, index);
-        set_ptrs(E, B, A, C);
-        if ((r = ew(E, 0))) return r;
         P = batch_params(b, MODE_RK2_2, false, &nb, index);
-        set_ptrs(P, C, A, A);
+        set_ptrs(P, B, C, A);
         if ((r = stage(P))) return r;
     } else {
         P = batch_params(b, MODE_RK3_2, false, &nb, index);
