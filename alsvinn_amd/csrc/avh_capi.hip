@@ -5,13 +5,14 @@
 // Buffers (interior-only SoA, nvars * ncells doubles each):
 //   A  the state U0 (always holds the current solution between steps)
 //   B  L0 = unscaled net flux of stage 1
-//   C  U1 (rungekutta2) or U2 (rungekutta3)
+//   C  U2 (rungekutta3), or a copy of U0
 // Step sequences (reference: alsfvm/src/integrator/{ForwardEuler,RungeKutta2,
 // RungeKutta3}.cpp, Simulator::incrementSolution Simulator.cpp:191-214):
 //   forwardeuler: stage(L: A->B) ; ew(A = B*s + A, check, end step)
 //   rungekutta2 : stage(L: A->B, copy A->C) ; stage(RK2_2: B*s + C, C -> A)
 //   rungekutta3 : stage(L: A->B) ; stage(RK3_2: B*s+A on the fly -> C) ;
-//                 stage(RK3_3: C, A -> A)
+//                 stage(RK3_3: C, A -> A); or, on small grids (avh_pair.hpp),
+//                 stage(L: A->B, copy A->C) ; pair(B, C -> A)
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -39,7 +40,10 @@ namespace {
 // (StageParams::finish).
 __global__ __launch_bounds__(64) void finish_step_kernel(Control* c) {
     if (threadIdx.x != 0 || !c->active) return;
-    end_step(c, c->block_violation != 0);
+    const StepInputs k = step_inputs(c);
+    StepEnd r;
+    prepare_end(k, end_inputs(c), step_dt(k), &r);
+    end_step(c, r, c->block_violation != 0);
 }
 
 // Forward euler's finish: U = L*s + U element-wise (Volume *= dt/dx; += U) and
@@ -436,6 +440,7 @@ struct avh_solver {
     Control h{};  // host mirror of ctrl, valid after pull()
     hipStream_t stream = nullptr;
     StageLauncher stage = nullptr;
+    PairLauncher pair = nullptr;
     LineLauncher line = nullptr;  // small 1D grids: steps in one workgroup
     EwLauncher ew = nullptr;
     int graph_steps = 16;  // steps per captured hipGraph (0: ordinary launches)
@@ -466,6 +471,51 @@ static void recompute_active(Control& h) {
 
 static avh_status mark(avh_solver* s, EventMarks* t) { return avh::mark(t, s->stream); }
 
+// The launches of an RK step, or forward euler's first: stage 1 writes L0 =
+// L(U0) to B and, where a later launch overwrites the state A but needs its
+// neighbours' U0, a copy of U0 to C.  P holds the grid; the result is in A.
+static avh_status enqueue_stages(const avh_config& cfg, StageLauncher stage, PairLauncher pair, int shape,
+                                 StageParams P, double* A, double* B, double* C, hipStream_t st, EventMarks* tm) {
+    const bool rk2 = cfg.integrator == AVH_INT_RUNGEKUTTA2;
+    avh_status r;
+    P.in = A;
+    P.u0 = A;
+    P.out = B;
+    P.mode = MODE_L;
+    P.copy = rk2 || pair ? C : nullptr;
+    if ((r = avh::mark(tm, st))) return r;
+    AVH_HIP(stage(P, shape, st));
+    if ((r = avh::mark(tm, st))) return r;
+    if (cfg.integrator == AVH_INT_FORWARDEULER) return AVH_OK;
+    P.copy = nullptr;
+    P.in = B;
+    P.u0 = C;
+    P.out = A;
+    if (rk2 || pair) {
+        P.mode = rk2 ? MODE_RK2_2 : MODE_RK3_3;
+        P.finish = 1;
+        AVH_HIP((rk2 ? stage : pair)(P, shape, st));
+        return avh::mark(tm, st);
+    }
+    P.u0 = A;
+    P.out = C;
+    P.mode = MODE_RK3_2;
+    AVH_HIP(stage(P, shape, st));
+    if ((r = avh::mark(tm, st))) return r;
+    P.in = C;
+    P.out = A;
+    P.mode = MODE_RK3_3;
+    P.finish = 1;
+    AVH_HIP(stage(P, shape, st));
+    return avh::mark(tm, st);
+}
+
+// the launcher of RK3's last two stages together, if this shape has it
+static PairLauncher pair_for(const avh_config& cfg, PairLauncher pair, int dim, int shape) {
+    if (cfg.integrator != AVH_INT_RUNGEKUTTA3) return nullptr;
+    return pair_shape(dim, shape, cfg.n, ghosts_of(cfg.reconstruction)) ? pair : nullptr;
+}
+
 static avh_status enqueue_step(avh_solver* s, EventMarks* tm = nullptr) {
     StageParams P;
     P.ctrl = s->ctrl;
@@ -473,47 +523,15 @@ static avh_status enqueue_step(avh_solver* s, EventMarks* tm = nullptr) {
     for (int d = 0; d < 3; ++d) P.n[d] = s->cfg.n[d];
     P.bc = s->cfg.boundary;
     P.gamma = s->cfg.gamma;
-    // stage 1: L0 = L(U0) into B, dt from the wave speeds
-    P.in = s->A;
-    P.u0 = s->A;
-    P.out = s->B;
-    P.mode = MODE_L;
-    P.copy = s->cfg.integrator == AVH_INT_RUNGEKUTTA2 ? s->C : nullptr;
-    avh_status r;
+    avh_status r = enqueue_stages(s->cfg, s->stage, pair_for(s->cfg, s->pair, s->dim, s->shape), s->shape, P, s->A,
+                                  s->B, s->C, s->stream, tm);
+    if (r || s->cfg.integrator != AVH_INT_FORWARDEULER) return r;
+    s->ew(s->B, s->A, s->ctrl, s->ncells, s->cfg.gamma, s->stream);
+    AVH_HIP(hipGetLastError());
     if ((r = mark(s, tm))) return r;
-    AVH_HIP(s->stage(P, s->shape, s->stream));
-    if ((r = mark(s, tm))) return r;
-    if (s->cfg.integrator == AVH_INT_FORWARDEULER) {
-        s->ew(s->B, s->A, s->ctrl, s->ncells, s->cfg.gamma, s->stream);
-        AVH_HIP(hipGetLastError());
-        if ((r = mark(s, tm))) return r;
-        hipLaunchKernelGGL(finish_step_kernel, dim3(1), dim3(64), 0, s->stream, s->ctrl);
-        AVH_HIP(hipGetLastError());
-        if ((r = mark(s, tm))) return r;
-    } else if (s->cfg.integrator == AVH_INT_RUNGEKUTTA2) {
-        P.in = s->B;
-        P.u0 = s->C;
-        P.out = s->A;
-        P.mode = MODE_RK2_2;
-        P.finish = 1;
-        AVH_HIP(s->stage(P, s->shape, s->stream));
-        if ((r = mark(s, tm))) return r;
-    } else {
-        P.in = s->B;
-        P.u0 = s->A;
-        P.out = s->C;
-        P.mode = MODE_RK3_2;
-        AVH_HIP(s->stage(P, s->shape, s->stream));
-        if ((r = mark(s, tm))) return r;
-        P.in = s->C;
-        P.u0 = s->A;
-        P.out = s->A;
-        P.mode = MODE_RK3_3;
-        P.finish = 1;
-        AVH_HIP(s->stage(P, s->shape, s->stream));
-        if ((r = mark(s, tm))) return r;
-    }
-    return AVH_OK;
+    hipLaunchKernelGGL(finish_step_kernel, dim3(1), dim3(64), 0, s->stream, s->ctrl);
+    AVH_HIP(hipGetLastError());
+    return mark(s, tm);
 }
 
 static TuneKey tune_key(const avh_solver* s) {
@@ -521,12 +539,12 @@ static TuneKey tune_key(const avh_solver* s) {
                    s->cfg.n[2]);
 }
 
-// Times every tile shape on the current state and keeps the fastest: the
-// first stage (writing the L0 buffer, which every step overwrites; flux-only
-// if the solver has stopped), and for RK2 and RK3 also the second stage on its
-// output (input formed on the fly from L0 and U0, writing the U2 buffer), whose
-// extra reads weigh differently on different shapes.  The state is not written;
-// the control block, which the launches add to, is restored.
+// Times every tile shape on the current state and keeps the fastest: the first
+// stage (writing the L0 buffer, which every step overwrites; flux-only if the
+// solver has stopped) and the launches after it, with outputs other than the
+// state: RK2's second stage and RK3's last two in one launch write the U2
+// buffer, RK3's third stage the L0 buffer.  The state is not written; the
+// control block, which the launches add to, is restored.
 static avh_status autotune(avh_solver* s, int* best, double* ms, int* nshapes) {
     const int ns = num_shapes(s->dim);
     avh_status r = pull(s);
@@ -542,22 +560,28 @@ static avh_status autotune(avh_solver* s, int* best, double* ms, int* nshapes) {
     P.u0 = s->A;
     P.out = s->B;
     P.mode = s->h.active ? MODE_L : MODE_FLUX_ONLY;
-    if (s->cfg.integrator == AVH_INT_RUNGEKUTTA2) P.copy = s->C;
     StageParams P2 = P;
-    P2.copy = nullptr;
     P2.in = s->B;
     P2.out = s->C;
-    P2.mode = s->cfg.integrator == AVH_INT_RUNGEKUTTA3 ? MODE_RK3_2 : MODE_RK2_2;
-    const bool second = s->cfg.integrator != AVH_INT_FORWARDEULER && s->h.active;
+    StageParams P3 = P2;
+    P3.in = s->C;
+    P3.out = s->B;
+    P3.mode = MODE_RK3_3;
+    const bool rk2 = s->cfg.integrator == AVH_INT_RUNGEKUTTA2;
+    const bool more = s->cfg.integrator != AVH_INT_FORWARDEULER && s->h.active;
     int b = 0;
     double tmin = 0;
     for (int k = 0; k < ns; ++k) {
         double t = 0;
         if (ns > 1) {
+            const PairLauncher pair = pair_for(s->cfg, s->pair, s->dim, k);
+            P.copy = rk2 || pair ? s->C : nullptr;
+            P2.mode = rk2 ? MODE_RK2_2 : (pair ? MODE_RK3_3 : MODE_RK3_2);
             r = time_launches(s->stream, 5,
                               [&]() {
                                   hipError_t e = s->stage(P, k, s->stream);
-                                  if (e == hipSuccess && second) e = s->stage(P2, k, s->stream);
+                                  if (e == hipSuccess && more) e = (pair ? pair : s->stage)(P2, k, s->stream);
+                                  if (e == hipSuccess && more && !rk2 && !pair) e = s->stage(P3, k, s->stream);
                                   return e;
                               },
                               &t);
@@ -697,6 +721,7 @@ avh_status avh_solver_create(avh_ctx* ctx, const avh_config* cfg, avh_solver** o
     s->ncells = (long long)cfg->n[0] * cfg->n[1] * cfg->n[2];
     s->nghosted = (long long)(cfg->n[0] + 2 * s->g[0]) * (cfg->n[1] + 2 * s->g[1]) * (cfg->n[2] + 2 * s->g[2]);
     s->stage = launchers.stage;
+    s->pair = launchers.pair;
     if (dim == 1 && cfg->n[0] + (cfg->boundary == AVH_BC_PERIODIC ? 0 : 1) <= line_interfaces(s->nv))
         s->line = launchers.line;
     s->ew = ew_for(cfg->equation);
@@ -879,8 +904,8 @@ avh_status avh_step_noalloc(avh_ctx* ctx, const avh_config* cfg, double* state, 
                       (long long)nv * ncells, NOALLOC_MAX_VALUES);
         return fail(AVH_EINVAL, buf);
     }
-    const StageLauncher stage = launchers_for(cfg->equation, cfg->reconstruction, cfg->flux, dim).stage;
-    if (!stage)
+    const Launchers launchers = launchers_for(cfg->equation, cfg->reconstruction, cfg->flux, dim);
+    if (!launchers.stage)
         return fail(AVH_EINVAL, "unsupported combination of equation, flux and grid dimension");
     AVH_HIP(hipSetDevice(ctx->device));
     double* sp = nullptr;
@@ -905,41 +930,20 @@ avh_status avh_step_noalloc(avh_ctx* ctx, const avh_config* cfg, double* state, 
     hipLaunchKernelGGL(noalloc_init_kernel, dim3(1), dim3(64), 0, st, ctrl, cell[0], cell[1], cell[2], cfg->cfl,
                        dt_cap);
     AVH_HIP(hipGetLastError());
-    const EwLauncher ew = ew_for(cfg->equation);
     StageParams P;
     P.ctrl = ctrl;
     P.ncells = ncells;
     for (int d = 0; d < 3; ++d) P.n[d] = cfg->n[d];
     P.bc = cfg->boundary;
     P.gamma = cfg->gamma;
-    P.in = state;
-    P.u0 = state;
-    P.out = B;
-    P.mode = MODE_L;
-    P.copy = cfg->integrator == AVH_INT_RUNGEKUTTA2 ? C : nullptr;
-    AVH_HIP(stage(P, shape, st));
+    if ((r = enqueue_stages(*cfg, launchers.stage, pair_for(*cfg, launchers.pair, dim, shape), shape, P, state, B, C,
+                            st, nullptr)))
+        return r;
     if (cfg->integrator == AVH_INT_FORWARDEULER) {
-        ew(B, state, ctrl, ncells, cfg->gamma, st);
+        ew_for(cfg->equation)(B, state, ctrl, ncells, cfg->gamma, st);
         AVH_HIP(hipGetLastError());
         hipLaunchKernelGGL(finish_step_kernel, dim3(1), dim3(64), 0, st, ctrl);
         AVH_HIP(hipGetLastError());
-    } else if (cfg->integrator == AVH_INT_RUNGEKUTTA2) {
-        P.in = B;
-        P.u0 = C;
-        P.out = state;
-        P.mode = MODE_RK2_2;
-        P.finish = 1;
-        AVH_HIP(stage(P, shape, st));
-    } else {
-        P.in = B;
-        P.out = C;
-        P.mode = MODE_RK3_2;
-        AVH_HIP(stage(P, shape, st));
-        P.in = C;
-        P.out = state;
-        P.mode = MODE_RK3_3;
-        P.finish = 1;
-        AVH_HIP(stage(P, shape, st));
     }
     hipLaunchKernelGGL(noalloc_result_kernel, dim3(1), dim3(64), 0, st, ctrl, dt_out, violated_out);
     AVH_HIP(hipGetLastError());
@@ -1000,8 +1004,9 @@ avh_status avh_time_step_kernels(avh_solver* s, int64_t steps, double* ms, int* 
     if (r) return r;
     // launches per step: the stages, and forward euler's element-wise pass and
     // end-of-step kernel (the rk final stages end the step themselves)
-    const int nk = s->cfg.integrator == AVH_INT_RUNGEKUTTA2 ? 2 : 3;
     if ((r = ensure_shape(s))) return r;
+    const bool two = s->cfg.integrator == AVH_INT_RUNGEKUTTA2 || pair_for(s->cfg, s->pair, s->dim, s->shape);
+    const int nk = two ? 2 : 3;
     EventMarks t;
     if ((r = t.create((size_t)steps * (nk + 1)))) return r;
     for (int64_t k = 0; k < steps; ++k)

@@ -172,6 +172,7 @@ struct TileKernel2 {
         __shared__ double su[NV * LT];
         __shared__ double sf[NV * NF];
         __shared__ double s_ws[3][NT / 64];
+        __shared__ StepEnd s_end;
         __shared__ int s_adm[NT / 64];
 
         Control* ctrl = P.ctrl;
@@ -219,7 +220,7 @@ struct TileKernel2 {
         // dt / dx, formed while the loads are in flight
         const double s = (mode == MODE_FLUX_ONLY || mode == MODE_L) ? 0.0
                          : VOL                                       ? V->s
-                                                                     : step_dt(ctrl) / ctrl->cell[0];
+                                                                     : stage_scale(P, ctrl, mode, &s_end);
         if (otf) {
 #pragma unroll
             for (int k = 0; k < SW; ++k)
@@ -335,7 +336,7 @@ struct TileKernel2 {
                 for (int v = 0; v < NV; ++v) soa_st<OFF32>(P.copy, nc, v, gc[m], su[v * LT + li]);
             }
         }
-        if (!VOL || mode == MODE_FLUX_ONLY) end_of_tile<NT>(P, ctrl, mode, ws[0], ws[1], 0.0, s_ws, bad);
+        if (!VOL || mode == MODE_FLUX_ONLY) end_of_tile<NT>(P, ctrl, mode, ws[0], ws[1], 0.0, s_ws, bad, s_end);
     }
 };
 

@@ -214,7 +214,7 @@ struct MarchKernel3 {
     // allows no more).
     static constexpr int RING = 2 + HW;
     static constexpr int LDS_BASE =
-        8 * (2 * NV * LP + 2 * NV * NIMAX + 3 * (NT / 64)) + 8 * (NT / 64);
+        8 * (2 * NV * LP + 2 * NV * NIMAX + 3 * (NT / 64)) + 8 * (NT / 64) + (int)sizeof(StepEnd);
     static constexpr bool U0RING = on_the_fly(MODE_CT) && LDS_BASE + 8 * RING * NV * NC <= 80 * 1024;
 
     // interface between plane cells ia and ia + SD under OPS
@@ -286,6 +286,7 @@ struct MarchKernel3 {
         __shared__ double sfx[NV * NIMAX];
         __shared__ double sfy[NV * NIMAX];
         __shared__ double s_ws[3][NT / 64];
+        __shared__ StepEnd s_end;
         __shared__ double su0[U0RING ? RING * NV * NC : 1];
         __shared__ int s_adm[2][NT / 64];
 
@@ -304,7 +305,7 @@ struct MarchKernel3 {
         const bool otf = on_the_fly(mode);
         const double s = (mode == MODE_FLUX_ONLY || mode == MODE_L) ? 0.0
                          : VOL                                       ? V->s
-                                                                     : step_dt(ctrl) / ctrl->cell[0];
+                                                                     : stage_scale(P, ctrl, mode, &s_end);
         const Layout lay = layout(P, V);
 
         // this thread's column.  A column past the grid edge (partial tile)
@@ -614,7 +615,7 @@ struct MarchKernel3 {
         }
 
 #undef AVH_PREFETCH_RING
-        if (!VOL || mode == MODE_FLUX_ONLY) end_of_tile<NT>(P, ctrl, mode, ws[0], ws[1], ws[2], s_ws, bad);
+        if (!VOL || mode == MODE_FLUX_ONLY) end_of_tile<NT>(P, ctrl, mode, ws[0], ws[1], ws[2], s_ws, bad, s_end);
     }
 };
 

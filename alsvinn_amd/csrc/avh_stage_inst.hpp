@@ -3,6 +3,7 @@
 #pragma once
 #include "avh_batch.hpp"
 #include "avh_line.hpp"
+#include "avh_pair.hpp"
 #include "avh_stage.hpp"
 #include "avh_stage2d.hpp"
 #include "avh_stage3d.hpp"
@@ -20,8 +21,8 @@ typedef hipError_t (*VolumeLauncher)(const StageParams& P, const VolumeParams& V
 // the solver's own grid and keeps the fastest.  Every shape computes each
 // interface flux and each cell update with the same operations in the same
 // order, so the choice never changes a result bit.
-//   1D: (cells, threads) = (256, 256) or (64, 64): small grids get more
-//       workgroups from the smaller tile.
+//   1D (grids above avh_line.hpp's): (cells, threads) = (256, 256), with
+//       RK3's last two stages in one launch, or (64, 64).
 //   2D: a flux pass costs a wavefront its full instruction stream however few
 //       of its lanes have an item, so the shapes' items sit just under their
 //       threads.  32x15 on 256 threads (255 x / 256 y turns of two
@@ -281,8 +282,33 @@ hipError_t launch_line(const LineParams& P, hipStream_t stream) {
     return hipErrorInvalidValue;
 }
 
+// RK3's last two stages in one launch (avh_pair.hpp): shape 2 of 2D grids
+// and shape 0 of 1D ones, where the grid is wide enough.
+typedef hipError_t (*PairLauncher)(const StageParams& P, int shape, hipStream_t stream);  // as StageLauncher
+
+template <class K>
+hipError_t launch_pair_k(const StageParams& P, hipStream_t stream) {
+    hipLaunchKernelGGL(pair_kernel<K>, dim3(K::tiles(P.n)), dim3(K::NTHREADS), 0, stream, P);
+    return hipGetLastError();
+}
+
+template <class EQ, int RECON, class FLUX, int DIM>
+hipError_t launch_pair(const StageParams& P, int, hipStream_t stream) {
+    if constexpr (DIM == 1) return launch_pair_k<PairKernel<EQ, RECON, FLUX, 1, 240, 1, 256>>(P, stream);
+    else return launch_pair_k<PairKernel<EQ, RECON, FLUX, 2, 16, 7, 512>>(P, stream);
+}
+
+// whether a shape's RK3 steps run their last two stages in one launch
+inline bool pair_shape(int dim, int shape, const int* n, int ghosts) {
+    if (dim > 2 || shape != (dim == 1 ? 0 : 2)) return false;
+    for (int d = 0; d < dim; ++d)
+        if (n[d] < 2 * ghosts) return false;
+    return true;
+}
+
 struct Launchers {
     StageLauncher stage = nullptr;
+    PairLauncher pair = nullptr;
     LineLauncher line = nullptr;
     BatchLauncher batch = nullptr;
     VolumeLauncher volume = nullptr;
@@ -293,6 +319,7 @@ Launchers launchers_of() {
     Launchers L;
     L.stage = &launch_stage<EQ, RECON, FLUX, DIM>;
     if (DIM < 3) L.batch = &launch_batch_stage<EQ, RECON, FLUX, DIM>;
+    if constexpr (DIM < 3) L.pair = &launch_pair<EQ, RECON, FLUX, DIM>;
     if constexpr (DIM == 1 && EQ::NV <= 3) L.line = &launch_line<EQ, RECON, FLUX>;
     L.volume = &launch_volume_stage<EQ, RECON, FLUX, DIM>;
     return L;
