@@ -233,7 +233,7 @@ struct PairKernel {
             bad = bad || !EQ::obeys_fast(r, P.gamma);
             const long long gi = (long long)(oy + cy) * n0 + ox + cx;
 #pragma unroll
-            for (int v = 0; v < NV; ++v) P.out[v * nc + gi] = r[v];
+            for (int v = 0; v < NV; ++v) store_through(P.out + v * nc + gi, r[v]);
         }
         end_of_tile<NT>(P, ctrl, MODE_RK3_3, 0.0, 0.0, 0.0, s_ws, bad, s_end);
     }

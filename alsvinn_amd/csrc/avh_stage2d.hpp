@@ -328,12 +328,12 @@ struct TileKernel2 {
             if (final_stage) bad = bad || !EQ::obeys_fast(r, P.gamma);
 #pragma unroll
             for (int v = 0; v < NV; ++v) {
-                if constexpr (VOL) V->out[v][gc[m]] = r[v];
-                else soa_st<OFF32>(P.out, nc, v, gc[m], r[v]);
+                if constexpr (VOL) store_through(V->out[v] + gc[m], r[v]);
+                else soa_st<OFF32, true>(P.out, nc, v, gc[m], r[v]);
             }
             if (mode == MODE_L && P.copy) {
 #pragma unroll
-                for (int v = 0; v < NV; ++v) soa_st<OFF32>(P.copy, nc, v, gc[m], su[v * LT + li]);
+                for (int v = 0; v < NV; ++v) soa_st<OFF32, true>(P.copy, nc, v, gc[m], su[v * LT + li]);
             }
         }
         if (!VOL || mode == MODE_FLUX_ONLY) end_of_tile<NT>(P, ctrl, mode, ws[0], ws[1], 0.0, s_ws, bad, s_end);

@@ -568,11 +568,11 @@ struct MarchKernel3 {
 #pragma unroll
                 for (int v = 0; v < NV; ++v) {
                     if constexpr (VOL) V->out[v][gi] = r[v];
-                    else soa_st<OFF32>(P.out, P.ncells, v, gi, r[v]);
+                    else soa_st<OFF32, false>(P.out, P.ncells, v, gi, r[v]);
                 }
                 if (mode == MODE_L && P.copy) {
 #pragma unroll
-                    for (int v = 0; v < NV; ++v) soa_st<OFF32>(P.copy, P.ncells, v, gi, w[HW - 1][v]);
+                    for (int v = 0; v < NV; ++v) soa_st<OFF32, false>(P.copy, P.ncells, v, gi, w[HW - 1][v]);
                 }
             }
 #pragma unroll
