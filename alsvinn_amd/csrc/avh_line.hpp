@@ -16,16 +16,17 @@
 // (burgers, eno3, 1024 cells: 6.5 us a step with 1024 threads, 4.5 with 512).
 // What is left at 200 cells is the chain of one interface's operations, three
 // times a step; from 1024 cells on it is the issue rate of the one compute
-// unit.  Time of a step, rk3, in microseconds, against three stage launches:
-//   cells              64    200    512   1024   1500   2048   3000
-//   burgers none      1.3    1.7    2.1    2.8    4.3    4.5    7.2
-//     stages          9.5   10.2   11.2   11.3   11.9   11.1   11.7
-//   burgers weno2     2.1    2.5    3.4    5.1    8.8    8.9
-//     stages         11.3   11.3   12.8   12.9   12.5   12.7   12.9
-//   euler1 none       3.6    4.0    5.6    9.8   18.0   18.1   38.1
-//     stages         13.5   13.8   16.2   16.3   16.2   16.0   16.3
-//   euler1 eno3       4.6    5.2    7.1   12.5   23.1   23.3   49.3
-//     stages         13.9   14.9   18.3   18.3   18.4   18.2   18.3
+// unit.  Time of a step, rk3, in microseconds, against stage launches (three,
+// or two with avh_pair.hpp):
+//   cells              64    200    512   1024   2048
+//   burgers none      1.1    1.5    1.9    2.7    4.2
+//     three           9.5   10.2   11.2   11.3   11.1
+//   burgers weno2     1.9    2.3    3.2    4.9    8.7
+//     three, two     11.3   11.3   12.8   12.9   12.7, 9.0
+//   euler1 none       3.5    3.9    5.6    9.5
+//     three          13.5   13.8   16.2   16.3
+//   euler1 eno3       4.5    5.1    7.0   12.4
+//     three, two     13.9   14.9   18.3   18.3, 12.8
 // so the line lies where the interfaces per thread stop paying: 2048 of them
 // for burgers, 1024 for euler1.
 #pragma once
@@ -187,8 +188,8 @@ struct LineKernel {
         int active = 1;
         for (int step = 0; step < P.steps && active; ++step) {
             // first stage: L(U0), the wave speed and dt
-            const double w = wave_max(fluxes(adm));
-            if ((tid & 63) == 0) s_ws[wave] = w;
+            const double w = wave_max63(fluxes(adm));
+            if ((tid & 63) == 63) s_ws[wave] = w;
             lds_barrier();
             k.ws[0] = 0.0;
 #pragma unroll

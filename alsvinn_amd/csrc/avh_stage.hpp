@@ -181,10 +181,23 @@ __device__ __forceinline__ double ws_max(double acc, double v) {
     return (acc < v) ? v : acc;
 }
 
-__device__ __forceinline__ double wave_max(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = ws_max(v, __shfl_xor(v, off, 64));
-    return v;
+// The largest of a wavefront's values, none negative or NaN, in lane 63: within
+// rows of 16 lanes, then rows of 32 and 64, by DPP moves (lanes without a
+// partner see 0).  Shuffles go through LDS and took 0.2 us of a 200-cell step.
+template <int CTRL>
+__device__ __forceinline__ double dpp_max(double v) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    const unsigned int lo = (unsigned int)__builtin_amdgcn_update_dpp(0, (int)(unsigned int)b, CTRL, 0xf, 0xf, false);
+    const unsigned int hi = (unsigned int)__builtin_amdgcn_update_dpp(0, (int)(unsigned int)(b >> 32), CTRL, 0xf, 0xf, false);
+    return fmax(v, __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo)));
+}
+__device__ __forceinline__ double wave_max63(double v) {
+    v = dpp_max<0x111>(v);  // row_shr:1, 2, 4, 8
+    v = dpp_max<0x112>(v);
+    v = dpp_max<0x114>(v);
+    v = dpp_max<0x118>(v);
+    v = dpp_max<0x142>(v);  // row_bcast:15, 31
+    return dpp_max<0x143>(v);
 }
 
 __device__ __forceinline__ unsigned int tile_id_xcd(unsigned int b, unsigned int nb) {
@@ -352,8 +365,8 @@ __device__ __forceinline__ void end_of_tile(const StageParams& P, Control* ctrl,
         const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
-            const double w = wave_max(ws[d]);
-            if (lane == 0) s_ws[d][wid] = w;
+            const double w = wave_max63(ws[d]);
+            if (lane == 63) s_ws[d][wid] = w;
         }
         lds_barrier();
         if (threadIdx.x < 3) {
