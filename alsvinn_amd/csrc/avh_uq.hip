@@ -491,7 +491,7 @@ void free_batch(avh_batch* b) {
         (void)hipFree(G.active_count);
     }
     (void)hipFree(b->work);
-    (void)hipHostFree(b->running);
+    pinned_give(b->ctx, b->running);
     for (hipEvent_t e : b->passed)
         if (e) (void)hipEventDestroy(e);
     if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -820,7 +820,7 @@ avh_status avh_batch_create(avh_ctx* ctx, const avh_config* cfg, int ngroups, co
         free_batch(b);
         return fail(AVH_EHIP, "hipStreamCreate failed");
     }
-    bool marks = hipHostMalloc(&b->running, sizeof(int) * MAX_GROUPS, hipHostMallocDefault) == hipSuccess;
+    bool marks = (b->running = (int*)pinned_take(b->ctx)) != nullptr;
     for (hipEvent_t& e : b->passed) marks = marks && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
     if (!marks) {
         free_batch(b);

@@ -181,13 +181,12 @@ avh_status avh_step_noalloc(avh_ctx* ctx, const avh_config* cfg, double* state, 
 avh_status avh_prepare_graph(avh_solver* solver);
 /* Tile shape of the fused stage kernel: -1 (default) lets the autotuner
  * pick on first use (cached per equation, reconstruction, flux and grid for
- * the process), 0..nshapes-1 fixes one (1D: 256 or 64 cells; 2D: 32x16,
- * 16x15, 64x4, 32x15 or 24x20; 3D columns marching over z-planes: 32x8,
- * 16x15 and 32x7 columns over 32 planes with one plane buffer, then 16x15
- * over 32 and over 16 planes and 32x7 over 32 planes with a double-buffered
- * plane and two barriers per plane, then 16x15 over 32 planes, two
- * barriers, fluxes with shared reciprocals).  Results are identical for
- * every shape.
+ * the process), 0..nshapes-1 fixes one (1D: 256 or 64 cells; 2D: 32x11 on 192
+ * threads, 16x15 on 512, 16x7 on 256, 32x15 on 256 or 32x15 on 1024; 3D columns
+ * marching over z-planes: 16x15 over 4 planes, 16x15 over as many as fill the
+ * compute units evenly, 32x7 over 8 and over 32, 16x15 over 16, 2 and 32).
+ * Results are identical for every shape.  Small 1D grids run whole steps in one
+ * workgroup unless a shape is fixed.
  * No reference counterpart: the reference's CUDA kernels use fixed block
  * sizes (alsfvm/src/numflux/NumericalFluxCUDA.cu:330-414). */
 avh_status avh_set_tile_shape(avh_solver* solver, int shape);
@@ -202,9 +201,9 @@ avh_status avh_autotune(avh_solver* solver, int* best_shape, double* ms_per_shap
  * ALSVINN_TIME_CUDA_BLOCK timers, alsutils/include/alsutils/timer/CudaTimer.hpp:11-48).
  * ms_per_launch[k] receives the average duration in milliseconds of the
  * k-th kernel of a step (k < *kernels_per_step <= 4), in launch order: the
- * stages and the element-wise pass of forward euler / RK2, and forward
- * euler's end-of-step kernel (the last RK2 / RK3 stage ends the step in its
- * last workgroup). */
+ * stages, or forward euler's element-wise pass and end-of-step kernel (the
+ * last RK2 / RK3 launch ends the step in its last workgroup; on small grids
+ * RK3's last two stages are one launch). */
 avh_status avh_time_step_kernels(avh_solver* solver, int64_t steps, double* ms_per_launch,
                                  int* kernels_per_step);
 
