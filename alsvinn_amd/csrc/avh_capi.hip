@@ -422,6 +422,18 @@ static __global__ void noalloc_init_kernel(Control* c, double c0, double c1, dou
     c->block_violation = 0;
 }
 
+// Opens a run to t_end: whether it has anything to do, and the steps done
+// before it (for the host, which has not looked).  A run that has broken its
+// constraints stays as it is.
+static __global__ void begin_run_kernel(Control* c, double t_end, int pause, long long* steps) {
+    if (threadIdx.x != 0) return;
+    __hip_atomic_store(steps, c->steps, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (c->violated) return;
+    c->t_end = t_end;
+    c->pause_on_save = pause;
+    c->active = (!(c->t >= t_end) && !(pause && c->saves_pending > 0)) ? 1 : 0;
+}
+
 static __global__ void noalloc_result_kernel(const Control* c, double* dt, int* violated) {
     if (threadIdx.x != 0) return;
     if (dt) dt[0] = c->last_dt;
@@ -438,7 +450,8 @@ struct avh_solver {
     double *A = nullptr, *B = nullptr, *C = nullptr, *staging = nullptr;
     Control* ctrl = nullptr;
     Control h{};  // host mirror of ctrl, valid after pull()
-    Control* pinned = nullptr;  // what travels between the two
+    Control* pinned = nullptr;  // what travels between the two, and behind it
+    long long* pinned_steps() { return (long long*)((char*)pinned + PINNED_SLOT) - 1; }  // a run's first step
     hipStream_t stream = nullptr;
     StageLauncher stage = nullptr;
     PairLauncher pair = nullptr;
@@ -458,7 +471,7 @@ static avh_status use_device(const avh_solver* s) {
 // The control block between the host mirror and the device, through pinned
 // memory on the solver's stream, one wait each: 20 us less a run than pageable
 // copies before and after a wait.
-static_assert(sizeof(Control) <= PINNED_SLOT, "a control block fits a slot");
+static_assert(sizeof(Control) + sizeof(long long) <= PINNED_SLOT, "a control block and a count fit a slot");
 static avh_status pull(avh_solver* s) {
     AVH_HIP(hipMemcpyAsync(s->pinned, s->ctrl, sizeof(Control), hipMemcpyDeviceToHost, s->stream));
     AVH_HIP(hipStreamSynchronize(s->stream));
@@ -466,17 +479,9 @@ static avh_status pull(avh_solver* s) {
     return AVH_OK;
 }
 
-// Behind whatever the stream holds, ahead of the launches that follow on it;
-// the caller waits for the stream (pull) before the next one.
-static avh_status push_ahead(avh_solver* s) {
+static avh_status push(avh_solver* s) {
     *s->pinned = s->h;
     AVH_HIP(hipMemcpyAsync(s->ctrl, s->pinned, sizeof(Control), hipMemcpyHostToDevice, s->stream));
-    return AVH_OK;
-}
-
-static avh_status push(avh_solver* s) {
-    const avh_status r = push_ahead(s);
-    if (r) return r;
     AVH_HIP(hipStreamSynchronize(s->stream));
     return AVH_OK;
 }
@@ -1100,24 +1105,41 @@ avh_status avh_advance(avh_solver* s, double t_end, int64_t max_steps, int chunk
     if (chunk < 1) chunk = 1;
     avh_status r = use_device(s);
     if (r) return r;
-    if ((r = pull(s))) return r;
-    if (s->h.violated) {
-        fill_progress(s, progress);
-        return constraint_error(s);
+    // The device opens the run itself (begin_run_kernel), ahead of its steps,
+    // unless the control block as last seen says that there is nothing to run:
+    // that may be out of date, so it decides only whether to look first.
+    Control seen = s->h;
+    seen.t_end = t_end;
+    seen.pause_on_save = pause_on_save ? 1 : 0;
+    recompute_active(seen);
+    if (max_steps <= 0 || !seen.active) {
+        if ((r = pull(s))) return r;
     }
-    s->h.t_end = t_end;
-    s->h.pause_on_save = pause_on_save ? 1 : 0;
-    recompute_active(s->h);
-    const bool runs = max_steps > 0 && s->h.active;
-    if ((r = runs ? push_ahead(s) : push(s))) return r;
     int64_t done = 0;
-    while (done < max_steps && s->h.active) {
+    bool open = false;
+    if (max_steps > 0) {
+        hipLaunchKernelGGL(begin_run_kernel, dim3(1), dim3(64), 0, s->stream, s->ctrl, t_end, seen.pause_on_save,
+                           s->pinned_steps());
+        AVH_HIP(hipGetLastError());
+        if (!seen.active) {
+            if ((r = pull(s))) return r;
+        }
+        open = seen.active || s->h.active;
+    } else if (!s->h.violated) {
+        s->h.t_end = t_end;
+        s->h.pause_on_save = seen.pause_on_save;
+        recompute_active(s->h);
+        if ((r = push(s))) return r;
+    }
+    for (bool first = true; open && done < max_steps; first = false) {
         const int64_t k = (max_steps - done) < chunk ? (max_steps - done) : chunk;
-        const int64_t before = s->h.steps;
+        const int64_t seen_steps = s->h.steps;
         if ((r = enqueue_steps(s, k))) return r;
         if ((r = pull(s))) return r;
-        done += s->h.steps - before;
-        if (s->h.steps - before < k) break;  // the device loop ended inside the chunk
+        const int64_t ran = s->h.steps - (first ? *s->pinned_steps() : seen_steps);
+        done += ran;
+        if (ran < k) break;  // the device loop ended inside the chunk
+        open = s->h.active;
     }
     fill_progress(s, progress);
     if (s->h.violated) return constraint_error(s);
