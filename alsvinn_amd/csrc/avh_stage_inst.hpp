@@ -35,9 +35,12 @@ typedef hipError_t (*VolumeLauncher)(const StageParams& P, const VolumeParams& V
 //       256^2 19.8 / 17.3 / 18.8, 501x333 27.4 / 25.9 / 33.8, 1024^2
 //       91 / 112 / 165; 700x300, eno3, hll, first stage: 16.4, 32x15 on 1024
 //       threads 15.5.
-//   3D: 16x15 or 32x7 columns marching over 2 to 32 planes, 256 threads (at
-//       most 256 interfaces a plane in each direction: one turn; the threads
-//       past the columns only work on the planes).  A chunk pays a z flux
+//   3D: 16x15, 17x14 or 14x17 columns marching through chunks of planes, 256
+//       threads (at most 255 interfaces a plane in each direction: one turn;
+//       the threads past the columns only work on the planes); the three
+//       waste different parts of a grid that they do not divide (97x83x61:
+//       42, 36 and 35 columns, 159 / 145 / 147 us of stages a step; 119x98x64
+//       203 / 189 / 211, 128^3 447 / 482 / 473).  A chunk pays a z flux
 //       and the loads of its window before its first plane, so the best length
 //       is the one that fills the CUs evenly (march_chunk; the fixed lengths
 //       stand beside it for grids where its model is off).  us of an RK3 stage
@@ -49,9 +52,9 @@ constexpr int SHAPE1_TX[NSHAPES1] = {256, 64};
 constexpr int SHAPE2_TX[NSHAPES2] = {32, 16, 16, 32, 32};
 constexpr int SHAPE2_TY[NSHAPES2] = {11, 15, 7, 15, 15};
 constexpr int SHAPE2_NT[NSHAPES2] = {192, 512, 256, 256, 1024};
-constexpr int SHAPE3_TX[NSHAPES3] = {16, 16, 32, 32, 16, 16, 16};
-constexpr int SHAPE3_TY[NSHAPES3] = {15, 15, 7, 7, 15, 15, 15};
-constexpr int SHAPE3_LZ[NSHAPES3] = {4, 0, 8, 32, 16, 2, 32};  // 0: march_chunk
+constexpr int SHAPE3_TX[NSHAPES3] = {16, 16, 17, 14, 16, 16, 16};
+constexpr int SHAPE3_TY[NSHAPES3] = {15, 15, 14, 17, 15, 15, 15};
+constexpr int SHAPE3_LZ[NSHAPES3] = {4, 0, 0, 0, 16, 2, 32};  // 0: march_chunk
 
 inline int num_shapes(int dim) { return dim == 1 ? NSHAPES1 : (dim == 2 ? NSHAPES2 : NSHAPES3); }
 
@@ -169,7 +172,8 @@ hipError_t launch_march_k(const StageParams& P, hipStream_t stream) {
 // launches, and grids whose cells need 64-bit indices, take the kernel that
 // reads the mode
 template <class EQ, int RECON, class FLUX, int TX, int TY>
-hipError_t launch_march(const StageParams& P, hipStream_t stream) {
+hipError_t launch_march(StageParams P, int lz, hipStream_t stream) {
+    P.lz = lz ? lz : march_chunk<MarchKernel3<EQ, RECON, FLUX, TX, TY, 256>>(P.n);
     if (P.ncells < MODE_KERNEL_MAX_CELLS) {
         switch (P.mode) {
         case MODE_L: return launch_march_k<MarchKernel3<EQ, RECON, FLUX, TX, TY, 256, MODE_L>>(P, stream);
@@ -185,11 +189,11 @@ template <class EQ, int RECON, class FLUX, int DIM>
 hipError_t launch_stage(const StageParams& P, int shape, hipStream_t stream) {
     if constexpr (DIM == 3) {
         if (shape < 0 || shape >= NSHAPES3) return hipErrorInvalidValue;
-        StageParams Q = P;
-        Q.lz = SHAPE3_LZ[shape];
-        if (Q.lz == 0) Q.lz = march_chunk<MarchKernel3<EQ, RECON, FLUX, 16, 15, 256>>(P.n);
-        return SHAPE3_TX[shape] == 16 ? launch_march<EQ, RECON, FLUX, 16, 15>(Q, stream)
-                                      : launch_march<EQ, RECON, FLUX, 32, 7>(Q, stream);
+        switch (SHAPE3_TX[shape]) {
+        case 14: return launch_march<EQ, RECON, FLUX, 14, 17>(P, SHAPE3_LZ[shape], stream);
+        case 17: return launch_march<EQ, RECON, FLUX, 17, 14>(P, SHAPE3_LZ[shape], stream);
+        }
+        return launch_march<EQ, RECON, FLUX, 16, 15>(P, SHAPE3_LZ[shape], stream);
     } else if constexpr (DIM == 1) {
         switch (shape) {
         case 0: return launch_stage_k<typename KernelFor<EQ, RECON, FLUX, 1, 0>::type>(P, stream);

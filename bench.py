@@ -27,8 +27,8 @@ import time
 
 HBM_PEAK_GBS = 8000.0
 SHAPE_NAMES = {1: ["256", "64"], 2: ["32x11", "16x15", "16x7", "32x15", "32x15 on 1024 threads"],
-               3: ["16x15 columns x 4 planes", "16x15 columns, balanced chunks", "32x7 columns x 8 planes",
-                   "32x7 columns x 32 planes", "16x15 columns x 16 planes", "16x15 columns x 2 planes",
+               3: ["16x15 columns x 4 planes", "16x15 columns, balanced chunks", "17x14 columns, balanced chunks",
+                   "14x17 columns, balanced chunks", "16x15 columns x 16 planes", "16x15 columns x 2 planes",
                    "16x15 columns x 32 planes"]}
 
 WORKLOADS = {

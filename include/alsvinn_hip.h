@@ -183,8 +183,8 @@ avh_status avh_prepare_graph(avh_solver* solver);
  * pick on first use (cached per equation, reconstruction, flux and grid for
  * the process), 0..nshapes-1 fixes one (1D: 256 or 64 cells; 2D: 32x11 on 192
  * threads, 16x15 on 512, 16x7 on 256, 32x15 on 256 or 32x15 on 1024; 3D columns
- * marching over z-planes: 16x15 over 4 planes, 16x15 over as many as fill the
- * compute units evenly, 32x7 over 8 and over 32, 16x15 over 16, 2 and 32).
+ * marching over z-planes: 16x15 over 4 planes, 16x15, 17x14 and 14x17 over as
+ * many as fill the compute units evenly, 16x15 over 16, 2 and 32).
  * Results are identical for every shape.  Small 1D grids run whole steps in one
  * workgroup unless a shape is fixed.
  * No reference counterpart: the reference's CUDA kernels use fixed block
