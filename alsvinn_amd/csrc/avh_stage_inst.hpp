@@ -147,7 +147,7 @@ hipError_t launch_stage_k(const StageParams& P, hipStream_t stream) {
 // 128^3, 16x15 columns, us of a volume substep's launch at 8 / 13 / 16 / 32
 // planes and at the 19 this picks: 165 / 163 / 192 / 240 and 158.
 template <class K>
-int march_chunk(const int* n) {
+int march_chunk(const int* n, long long* least = nullptr) {
     const int CUS = 256;
     int best = 1;
     long long cost = 0;
@@ -159,6 +159,7 @@ int march_chunk(const int* n) {
             cost = c;
         }
     }
+    if (least) *least = cost;
     return best;
 }
 
@@ -230,8 +231,7 @@ hipError_t launch_stage(const StageParams& P, int shape, hipStream_t stream) {
     }
 }
 
-// The reference-Volume kernels: one tile per dimension -- 1D 256 cells, 2D
-// 32x15, 3D 16x15 columns.  P.mode is MODE_FLUX_ONLY, or MODE_RK3_3 for the
+// The reference-Volume kernels: 1D 256 cells, 2D 32x15, 3D columns.  P.mode is MODE_FLUX_ONLY, or MODE_RK3_3 for the
 // combination V describes.
 template <class EQ, int RECON, class FLUX>
 struct VolumeKernel1 {
@@ -243,19 +243,36 @@ struct VolumeKernel2 {
 };
 
 template <class K>
-hipError_t launch_volume_march(const StageParams& P, const VolumeParams& V, hipStream_t stream) {
+hipError_t launch_volume_march_k(const StageParams& P, const VolumeParams& V, hipStream_t stream) {
     StageParams Q = P;
     Q.lz = march_chunk<K>(P.n);
     hipLaunchKernelGGL(volume_march_kernel3<K>, dim3(K::tiles(P.n, Q.lz)), dim3(K::NT), 0, stream, Q, V);
     return hipGetLastError();
 }
 
+// The columns whose launch the model finds shortest (a volume has no
+// autotuner): their workgroups do the same work a plane, so the costs compare.
+// us of an RK3 step through the volume interfaces, 16x15 alone and so: 97x83x61
+// 289 and 273, 119x98x64 340 and 327, 33x110x50 216 and 200, 128^3 the same.
+template <class EQ, int RECON, class FLUX, int MODE>
+hipError_t launch_volume_march(const StageParams& P, const VolumeParams& V, hipStream_t stream) {
+    typedef MarchKernel3<EQ, RECON, FLUX, 16, 15, 256, MODE, true> A;
+    typedef MarchKernel3<EQ, RECON, FLUX, 17, 14, 256, MODE, true> B;
+    typedef MarchKernel3<EQ, RECON, FLUX, 14, 17, 256, MODE, true> C;
+    long long a, b, c;
+    march_chunk<A>(P.n, &a);
+    march_chunk<B>(P.n, &b);
+    march_chunk<C>(P.n, &c);
+    if (a <= b && a <= c) return launch_volume_march_k<A>(P, V, stream);
+    return b <= c ? launch_volume_march_k<B>(P, V, stream) : launch_volume_march_k<C>(P, V, stream);
+}
+
 template <class EQ, int RECON, class FLUX, int DIM>
 hipError_t launch_volume_stage(const StageParams& P, const VolumeParams& V, hipStream_t stream) {
     if constexpr (DIM == 3) {
         if (P.mode == MODE_FLUX_ONLY)
-            return launch_volume_march<MarchKernel3<EQ, RECON, FLUX, 16, 15, 256, MODE_FLUX_ONLY, true>>(P, V, stream);
-        return launch_volume_march<MarchKernel3<EQ, RECON, FLUX, 16, 15, 256, MODE_RK3_3, true>>(P, V, stream);
+            return launch_volume_march<EQ, RECON, FLUX, MODE_FLUX_ONLY>(P, V, stream);
+        return launch_volume_march<EQ, RECON, FLUX, MODE_RK3_3>(P, V, stream);
     } else {
         typedef typename std::conditional<DIM == 1, VolumeKernel1<EQ, RECON, FLUX>,
                                           VolumeKernel2<EQ, RECON, FLUX>>::type::type K;

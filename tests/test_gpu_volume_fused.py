@@ -19,7 +19,8 @@ pytestmark = pytest.mark.gpu
 CASES = [("burgers", "weno2", "godunov", (300, 1, 1)), ("euler1", "eno3", "hll", (257, 1, 1)),
          ("burgers", "none", "godunov", (35, 17, 1)), ("euler2", "weno2", "hll3", (65, 47, 1)),
          ("burgers", "eno2", "godunov", (17, 16, 5)), ("euler3", "none", "hll", (16, 15, 3)),
-         ("euler3", "weno2", "hll3", (33, 31, 70)), ("euler3", "eno3", "hll3", (17, 46, 21))]
+         ("euler3", "weno2", "hll3", (33, 31, 70)), ("euler3", "eno3", "hll3", (17, 46, 21)),
+         ("euler3", "weno2", "hll3", (27, 33, 40)), ("euler3", "eno2", "hll", (32, 28, 19))]
 
 
 def _combine(integ, substep, L, us, u0, s):
