@@ -441,7 +441,8 @@ static __global__ void noalloc_result_kernel(const Control* c, double* dt, int* 
 }
 
 struct avh_solver {
-    avh_ctx* ctx = nullptr;
+    int device = 0;
+    PinnedSlot slot;
     avh_config cfg{};
     int dim = 1, nv = 0, ng = 0;
     int g[3] = {0, 0, 0};
@@ -464,7 +465,7 @@ struct avh_solver {
 };
 
 static avh_status use_device(const avh_solver* s) {
-    AVH_HIP(hipSetDevice(s->ctx->device));
+    AVH_HIP(hipSetDevice(s->device));
     return AVH_OK;
 }
 
@@ -660,6 +661,12 @@ static avh_status enqueue_steps(avh_solver* s, int64_t n) {
     return enqueue_steps_graphed(s->graph, s->graph_steps, s->stream, n, [s]() { return enqueue_step(s); });
 }
 
+static void* pinned_allocate(size_t bytes) {
+    void* p = nullptr;
+    return hipHostMalloc(&p, bytes, hipHostMallocDefault) == hipSuccess ? p : nullptr;
+}
+static void pinned_release(void* p) { (void)hipHostFree(p); }
+
 extern "C" {
 
 const char* avh_last_error(void) { return last_error_slot().c_str(); }
@@ -674,26 +681,29 @@ avh_status avh_ctx_create(int device, avh_ctx** ctx) {
     double* sp = nullptr;
     avh_status r = noalloc_scratch(device, &sp);
     if (r) return r;
-    auto c = new (std::nothrow) avh_ctx;
+    std::unique_ptr<avh_ctx> c(new (std::nothrow) avh_ctx);
     if (!c) return fail(AVH_ENOMEM, "host allocation failed");
     c->device = device;
-    *ctx = c;
+    try {
+        c->pinned = std::make_shared<PinnedPool>(pinned_allocate, pinned_release);
+    } catch (const std::bad_alloc&) {
+        return fail(AVH_ENOMEM, "host allocation failed");
+    }
+    *ctx = c.release();
     return AVH_OK;
 }
 
 avh_status avh_ctx_destroy(avh_ctx* ctx) {
-    if (ctx && (ctx->scratch || ctx->pinned)) {
-        (void)hipSetDevice(ctx->device);
-        (void)hipFree(ctx->scratch);
-        (void)hipHostFree(ctx->pinned);
-    }
+    if (!ctx) return AVH_OK;
+    (void)hipSetDevice(ctx->device);
+    (void)hipFree(ctx->scratch);
     delete ctx;
     return AVH_OK;
 }
 
 avh_status avh_solver_destroy(avh_solver* s) {
     if (!s) return AVH_OK;
-    (void)hipSetDevice(s->ctx->device);
+    (void)hipSetDevice(s->device);
     if (s->stream) (void)hipStreamSynchronize(s->stream);
     s->graph.reset();
     (void)hipFree(s->A);
@@ -701,7 +711,6 @@ avh_status avh_solver_destroy(avh_solver* s) {
     (void)hipFree(s->C);
     (void)hipFree(s->staging);
     (void)hipFree(s->ctrl);
-    pinned_give(s->ctx, s->pinned);
     if (s->stream) (void)hipStreamDestroy(s->stream);
     delete s;
     return AVH_OK;
@@ -733,7 +742,7 @@ avh_status avh_solver_create(avh_ctx* ctx, const avh_config* cfg, avh_solver** o
     AVH_HIP(hipSetDevice(ctx->device));
     auto s = new (std::nothrow) avh_solver;
     if (!s) return fail(AVH_ENOMEM, "host allocation failed");
-    s->ctx = ctx;
+    s->device = ctx->device;
     s->cfg = *cfg;
     s->dim = dim;
     s->nv = nv;
@@ -752,7 +761,7 @@ avh_status avh_solver_create(avh_ctx* ctx, const avh_config* cfg, avh_solver** o
     if (hipMalloc(&s->A, bytes) != hipSuccess || hipMalloc(&s->B, bytes) != hipSuccess ||
         hipMalloc(&s->C, bytes) != hipSuccess ||
         hipMalloc(&s->staging, (size_t)nv * s->nghosted * sizeof(double)) != hipSuccess ||
-        hipMalloc(&s->ctrl, sizeof(Control)) != hipSuccess || !(s->pinned = (Control*)pinned_take(ctx))) {
+        hipMalloc(&s->ctrl, sizeof(Control)) != hipSuccess || !(s->pinned = (Control*)s->slot.take(ctx->pinned))) {
         avh_solver_destroy(s);
         return fail(AVH_ENOMEM, "device allocation failed");
     }
@@ -1153,7 +1162,7 @@ avh_status avh_advance(avh_solver* s, double t_end, int64_t max_steps, int chunk
 // a sample count and mean / M2 arrays of the conserved and the primitive
 // variables.
 struct avh_stats {
-    avh_ctx* ctx = nullptr;
+    int device = 0;
     int equation = 0, nv = 0, nsaves = 0;
     long long ncells = 0;
     double gamma = 1.4;
@@ -1173,7 +1182,7 @@ avh_status avh_stats_create(avh_ctx* ctx, int equation, const int n[3], double g
     AVH_HIP(hipSetDevice(ctx->device));
     auto t = new (std::nothrow) avh_stats;
     if (!t) return fail(AVH_ENOMEM, "host allocation failed");
-    t->ctx = ctx;
+    t->device = ctx->device;
     t->equation = equation;
     t->nv = nv;
     t->nsaves = nsaves;
@@ -1198,7 +1207,7 @@ avh_status avh_stats_create(avh_ctx* ctx, int equation, const int n[3], double g
 
 avh_status avh_stats_destroy(avh_stats* t) {
     if (!t) return AVH_OK;
-    (void)hipSetDevice(t->ctx->device);
+    (void)hipSetDevice(t->device);
     (void)hipStreamSynchronize(t->stream);
     (void)hipFree(t->mem);
     (void)hipStreamDestroy(t->stream);
@@ -1208,7 +1217,7 @@ avh_status avh_stats_destroy(avh_stats* t) {
 
 avh_status avh_stats_reset(avh_stats* t) {
     if (!t) return fail(AVH_EINVAL, "null argument");
-    AVH_HIP(hipSetDevice(t->ctx->device));
+    AVH_HIP(hipSetDevice(t->device));
     AVH_HIP(hipStreamSynchronize(t->stream));
     AVH_HIP(hipMemset(t->mem, 0, sizeof(double) * 4 * (size_t)t->nsaves * t->nv * t->ncells));
     std::fill(t->count.begin(), t->count.end(), 0);
@@ -1219,7 +1228,7 @@ avh_status avh_stats_accumulate(avh_stats* t, avh_solver* s, int save) {
     if (!t || !s) return fail(AVH_EINVAL, "null argument");
     if (save < 0 || save >= t->nsaves) return fail(AVH_EINVAL, "no such statistics save");
     if (s->cfg.equation != t->equation || s->ncells != t->ncells) return fail(AVH_EINVAL, "solver does not match");
-    AVH_HIP(hipSetDevice(t->ctx->device));
+    AVH_HIP(hipSetDevice(t->device));
     // the solver's state is final once its stream is idle
     AVH_HIP(hipStreamSynchronize(s->stream));
     const long long n = ++t->count[save];
@@ -1235,7 +1244,7 @@ avh_status avh_stats_accumulate(avh_stats* t, avh_solver* s, int save) {
 avh_status avh_stats_read(avh_stats* t, int save, int primitive, double* mean, double* variance, int64_t* count) {
     if (!t || !mean || !variance || !count) return fail(AVH_EINVAL, "null argument");
     if (save < 0 || save >= t->nsaves) return fail(AVH_EINVAL, "no such statistics save");
-    AVH_HIP(hipSetDevice(t->ctx->device));
+    AVH_HIP(hipSetDevice(t->device));
     AVH_HIP(hipStreamSynchronize(t->stream));
     const size_t blk = (size_t)t->nsaves * t->nv * t->ncells;
     const size_t n = (size_t)t->nv * t->ncells;

@@ -4,12 +4,14 @@
 
 #include <cstdint>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <tuple>
 #include <vector>
 
 #include "../../include/alsvinn_hip.h"
+#include "avh_pinned.hpp"
 #include "avh_stage_inst.hpp"
 
 struct avh_ctx {
@@ -18,41 +20,10 @@ struct avh_ctx {
     // constraint flag), allocated on first use; `lock` serialises those calls
     std::mutex lock;
     void* scratch = nullptr;
-    // pinned host memory of the solvers and batches on this device, in slots:
-    // allocating a page of it takes 0.1 ms, as long as the rest of a solver
-    std::mutex pinned_lock;
-    char* pinned = nullptr;
-    unsigned long long pinned_used = 0;  // one bit a slot
+    std::shared_ptr<avh::PinnedPool> pinned;  // shared with its solvers and batches
 };
 
 namespace avh {
-
-constexpr size_t PINNED_SLOT = 512;
-constexpr int PINNED_SLOTS = 64;
-
-// A slot of pinned memory, or an allocation of its own once all are taken;
-// nullptr if there is none.  Whoever gives it back has waited for the device's
-// last access.
-inline void* pinned_take(avh_ctx* ctx) {
-    std::lock_guard<std::mutex> g(ctx->pinned_lock);
-    if (!ctx->pinned && hipHostMalloc((void**)&ctx->pinned, PINNED_SLOT * PINNED_SLOTS, hipHostMallocDefault) != hipSuccess)
-        ctx->pinned = nullptr;
-    for (int i = 0; ctx->pinned && i < PINNED_SLOTS; ++i)
-        if (!(ctx->pinned_used >> i & 1)) {
-            ctx->pinned_used |= 1ull << i;
-            return ctx->pinned + i * PINNED_SLOT;
-        }
-    void* p = nullptr;
-    return hipHostMalloc(&p, PINNED_SLOT, hipHostMallocDefault) == hipSuccess ? p : nullptr;
-}
-inline void pinned_give(avh_ctx* ctx, void* p) {
-    if (!p) return;
-    std::lock_guard<std::mutex> g(ctx->pinned_lock);
-    char* const c = (char*)p;
-    if (ctx->pinned && c >= ctx->pinned && c < ctx->pinned + PINNED_SLOT * PINNED_SLOTS)
-        ctx->pinned_used &= ~(1ull << ((c - ctx->pinned) / PINNED_SLOT));
-    else (void)hipHostFree(p);
-}
 
 inline std::string& last_error_slot() {
     static thread_local std::string s;

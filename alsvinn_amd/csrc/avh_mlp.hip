@@ -750,7 +750,7 @@ inline int pad16(int x) { return (x + 15) / 16 * 16; }
 }  // namespace
 
 struct avh_mlp {
-    avh_ctx* ctx = nullptr;
+    int device = 0;
     avh_mlp_config cfg{};
     int nl = 0, pin = 0, pout = 0, B = 0, M = 0, maxw = 0;
     LayerDesc L[MAX_LAYERS];
@@ -783,7 +783,7 @@ namespace {
 
 void free_mlp(avh_mlp* n) {
     if (!n) return;
-    (void)hipSetDevice(n->ctx->device);
+    (void)hipSetDevice(n->device);
     if (n->stream) (void)hipStreamSynchronize(n->stream);
     void* ptrs[] = {n->params, n->m, n->v, n->grad, n->wb, n->wtb, n->x0, n->x0t, n->z, n->a, n->at, n->yhat,
                     n->yn, n->dz[0], n->dz[1], n->dzt[0], n->dzt[1], n->mu_in, n->sd_in, n->mu_out, n->sd_out,
@@ -1161,7 +1161,7 @@ avh_status avh_mlp_create(avh_ctx* ctx, const avh_mlp_config* cfg, avh_mlp** out
     AVH_HIP(hipSetDevice(ctx->device));
     auto n = new (std::nothrow) avh_mlp;
     if (!n) return fail(AVH_ENOMEM, "host allocation failed");
-    n->ctx = ctx;
+    n->device = ctx->device;
     n->cfg = *cfg;
     n->nl = cfg->hidden + 1;
     n->pin = pad16(cfg->n_in);
@@ -1285,7 +1285,7 @@ avh_status avh_mlp_set_normalization(avh_mlp* n, const float* in_mean, const flo
         if (!(in_std[i] > 0)) return fail(AVH_EINVAL, "input scales must be positive");
     for (int i = 0; i < n->cfg.n_out; ++i)
         if (!(out_std[i] > 0)) return fail(AVH_EINVAL, "output scales must be positive");
-    AVH_HIP(hipSetDevice(n->ctx->device));
+    AVH_HIP(hipSetDevice(n->device));
     AVH_HIP(hipStreamSynchronize(n->stream));
     AVH_HIP(hipMemcpy(n->mu_in, in_mean, sizeof(float) * n->cfg.n_in, hipMemcpyHostToDevice));
     AVH_HIP(hipMemcpy(n->sd_in, in_std, sizeof(float) * n->cfg.n_in, hipMemcpyHostToDevice));
@@ -1298,13 +1298,13 @@ avh_status avh_mlp_set_normalization(avh_mlp* n, const float* in_mean, const flo
 // then b[out].
 avh_status avh_mlp_get_params(avh_mlp* n, int member, float* out) {
     if (!n || !out || member < 0 || member >= n->M) return fail(AVH_EINVAL, "bad argument");
-    AVH_HIP(hipSetDevice(n->ctx->device));
+    AVH_HIP(hipSetDevice(n->device));
     return read_packed(n, n->params + member * n->P, 1, out);
 }
 
 avh_status avh_mlp_set_params(avh_mlp* n, int member, const float* in) {
     if (!n || !in || member < 0 || member >= n->M) return fail(AVH_EINVAL, "bad argument");
-    AVH_HIP(hipSetDevice(n->ctx->device));
+    AVH_HIP(hipSetDevice(n->device));
     AVH_HIP(hipStreamSynchronize(n->stream));
     std::vector<float> h(n->P, 0.f);
     size_t o = 0;
@@ -1328,7 +1328,7 @@ avh_status avh_mlp_set_params(avh_mlp* n, int member, const float* in) {
 avh_status avh_mlp_gradients(avh_mlp* n, const float* X, const float* Y, int64_t rows, float* grads, float* loss) {
     if (!n || !X || !Y || !grads || !loss) return fail(AVH_EINVAL, "null argument");
     if (rows != n->B) return fail(AVH_EINVAL, "rows must equal the minibatch size");
-    AVH_HIP(hipSetDevice(n->ctx->device));
+    AVH_HIP(hipSetDevice(n->device));
     avh_status r = upload_data(n, X, Y, rows);
     if (r) return r;
     if ((r = ensure_idx(n, rows))) return r;
@@ -1351,7 +1351,7 @@ avh_status avh_mlp_gradients(avh_mlp* n, const float* X, const float* Y, int64_t
 // avh_mlp_gradients / training step (for step-by-step checks).
 avh_status avh_mlp_adam_step(avh_mlp* n, float lr) {
     if (!n) return fail(AVH_EINVAL, "null argument");
-    AVH_HIP(hipSetDevice(n->ctx->device));
+    AVH_HIP(hipSetDevice(n->device));
     avh_status r = adam_step(n, lr);
     if (r) return r;
     AVH_HIP(hipStreamSynchronize(n->stream));
@@ -1369,7 +1369,7 @@ avh_status avh_mlp_train(avh_mlp* n, const float* X, const float* Y, int64_t row
     if (!n || !X || !Y) return fail(AVH_EINVAL, "null argument");
     if (rows < n->B || epochs < 1) return fail(AVH_EINVAL, "need at least one minibatch and one epoch");
     if (rows > (1ll << 30)) return fail(AVH_EINVAL, "too many rows");
-    AVH_HIP(hipSetDevice(n->ctx->device));
+    AVH_HIP(hipSetDevice(n->device));
     avh_status r = upload_data(n, X, Y, rows);
     if (r) return r;
     if ((r = ensure_idx(n, rows * n->M))) return r;
@@ -1424,7 +1424,7 @@ avh_status avh_mlp_set_weight_decay(avh_mlp* n, float weight_decay) {
 avh_status avh_mlp_predict(avh_mlp* n, const float* X, int64_t rows, float* out) {
     if (!n || !X || !out) return fail(AVH_EINVAL, "null argument");
     if (rows < 1 || rows > (1ll << 30)) return fail(AVH_EINVAL, "bad row count");
-    AVH_HIP(hipSetDevice(n->ctx->device));
+    AVH_HIP(hipSetDevice(n->device));
     avh_status r = upload_data(n, X, nullptr, rows);
     if (r) return r;
     if (n->fused) return fused_predict(n, rows, out);

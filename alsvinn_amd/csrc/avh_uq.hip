@@ -437,7 +437,8 @@ BatchStats batch_stats_for(int eq) {
 }  // namespace
 
 struct avh_batch {
-    avh_ctx* ctx = nullptr;
+    int device = 0;
+    PinnedSlot slot;
     avh_config cfg{};
     int dim = 1, nv = 0;
     int ngroups = 0;
@@ -472,7 +473,7 @@ namespace {
 
 void free_batch(avh_batch* b) {
     if (!b) return;
-    (void)hipSetDevice(b->ctx->device);
+    (void)hipSetDevice(b->device);
     if (b->stream) (void)hipStreamSynchronize(b->stream);
     b->graph.reset();
     for (int i = 0; i < b->ngroups; ++i) {
@@ -491,7 +492,6 @@ void free_batch(avh_batch* b) {
         (void)hipFree(G.active_count);
     }
     (void)hipFree(b->work);
-    pinned_give(b->ctx, b->running);
     for (hipEvent_t e : b->passed)
         if (e) (void)hipEventDestroy(e);
     if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -790,7 +790,7 @@ avh_status avh_batch_create(avh_ctx* ctx, const avh_config* cfg, int ngroups, co
     AVH_HIP(hipSetDevice(ctx->device));
     auto b = new (std::nothrow) avh_batch;
     if (!b) return fail(AVH_ENOMEM, "host allocation failed");
-    b->ctx = ctx;
+    b->device = ctx->device;
     b->cfg = *cfg;
     b->dim = dim;
     b->nv = nv;
@@ -820,7 +820,7 @@ avh_status avh_batch_create(avh_ctx* ctx, const avh_config* cfg, int ngroups, co
         free_batch(b);
         return fail(AVH_EHIP, "hipStreamCreate failed");
     }
-    bool marks = (b->running = (int*)pinned_take(b->ctx)) != nullptr;
+    bool marks = (b->running = (int*)b->slot.take(ctx->pinned)) != nullptr;
     for (hipEvent_t& e : b->passed) marks = marks && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
     if (!marks) {
         free_batch(b);
@@ -879,7 +879,7 @@ avh_status avh_batch_add_fixed_interval_adjuster(avh_batch* b, double interval, 
     if (!b) return fail(AVH_EINVAL, "null argument");
     if (!(interval > 0)) return fail(AVH_EINVAL, "interval must be positive");
     if (b->proto.n_adj >= MAX_ADJ) return fail(AVH_EINVAL, "at most 4 adjusters");
-    AVH_HIP(hipSetDevice(b->ctx->device));
+    AVH_HIP(hipSetDevice(b->device));
     AVH_HIP(hipStreamSynchronize(b->stream));
     const int i = b->proto.n_adj++;
     b->proto.adj_interval[i] = interval;
@@ -913,7 +913,7 @@ avh_status avh_batch_set_state(avh_batch* b, int group, int sample, const double
     avh_status r = check_gs(b, group, sample);
     if (r) return r;
     if (!host_interior) return fail(AVH_EINVAL, "null argument");
-    AVH_HIP(hipSetDevice(b->ctx->device));
+    AVH_HIP(hipSetDevice(b->device));
     AVH_HIP(hipStreamSynchronize(b->stream));
     const GroupHost& G = b->g[group];
     const size_t n = (size_t)b->nv * G.ncells;
@@ -925,7 +925,7 @@ avh_status avh_batch_get_state(avh_batch* b, int group, int sample, double* host
     avh_status r = check_gs(b, group, sample);
     if (r) return r;
     if (!host_interior) return fail(AVH_EINVAL, "null argument");
-    AVH_HIP(hipSetDevice(b->ctx->device));
+    AVH_HIP(hipSetDevice(b->device));
     AVH_HIP(hipStreamSynchronize(b->stream));
     const GroupHost& G = b->g[group];
     const size_t n = (size_t)b->nv * G.ncells;
@@ -938,7 +938,7 @@ avh_status avh_batch_set_kh2d(avh_batch* b, int group, const double* host_interf
     if (r) return r;
     if (!host_interfaces) return fail(AVH_EINVAL, "null argument");
     if (b->cfg.equation != AVH_EQ_EULER2 || b->dim != 2) return fail(AVH_EINVAL, "KH fill needs euler2 on 2D grids");
-    AVH_HIP(hipSetDevice(b->ctx->device));
+    AVH_HIP(hipSetDevice(b->device));
     const GroupHost& G = b->g[group];
     const size_t bytes = (size_t)G.nsamples * 2 * G.n[0] * sizeof(double);
     double* d = nullptr;
@@ -981,7 +981,7 @@ static avh_status enqueue_until_stopped(avh_batch* b, int64_t n) {
 avh_status avh_batch_advance(avh_batch* b, int64_t max_steps, int chunk, int64_t* steps_done, int64_t* active_left) {
     if (!b) return fail(AVH_EINVAL, "null argument");
     if (chunk < 1) chunk = 1;
-    AVH_HIP(hipSetDevice(b->ctx->device));
+    AVH_HIP(hipSetDevice(b->device));
     if (b->stats_initial && !b->initial_done && b->nsaves > 0) {
         unsigned int nbs = 0;
         StatsParams S = stats_params(b, &nbs);
@@ -1023,7 +1023,7 @@ avh_status avh_batch_advance(avh_batch* b, int64_t max_steps, int chunk, int64_t
 
 avh_status avh_batch_set_graph_steps(avh_batch* b, int steps) {
     if (!b || steps < 0 || steps > 4096) return fail(AVH_EINVAL, "bad argument");
-    AVH_HIP(hipSetDevice(b->ctx->device));
+    AVH_HIP(hipSetDevice(b->device));
     AVH_HIP(hipStreamSynchronize(b->stream));
     b->graph.reset();
     b->graph_steps = steps;
@@ -1034,7 +1034,7 @@ avh_status avh_batch_violations(avh_batch* b, int group, int64_t* count, int64_t
     avh_status r = check_gs(b, group, 0);
     if (r) return r;
     if (!count || !first_sample) return fail(AVH_EINVAL, "null argument");
-    AVH_HIP(hipSetDevice(b->ctx->device));
+    AVH_HIP(hipSetDevice(b->device));
     AVH_HIP(hipStreamSynchronize(b->stream));
     const GroupHost& G = b->g[group];
     std::vector<Control> cs(G.nsamples);
@@ -1051,7 +1051,7 @@ avh_status avh_batch_violations(avh_batch* b, int group, int64_t* count, int64_t
 
 avh_status avh_batch_set_end_time(avh_batch* b, double t_end) {
     if (!b) return fail(AVH_EINVAL, "null argument");
-    AVH_HIP(hipSetDevice(b->ctx->device));
+    AVH_HIP(hipSetDevice(b->device));
     for (int i = 0; i < b->ngroups; ++i) {
         hipLaunchKernelGGL(set_end_time_kernel, dim3(1), dim3(256), 0, b->stream, b->g[i].ctrl, b->g[i].nsamples, t_end,
                            b->g[i].active_count);
@@ -1068,7 +1068,7 @@ avh_status avh_batch_kinetic_energy(avh_batch* b, int group, int component, doub
     if (!out) return fail(AVH_EINVAL, "null argument");
     if (b->cfg.equation == AVH_EQ_BURGERS || component < 0 || component >= b->nv - 2)
         return fail(AVH_EINVAL, "kinetic energy needs an euler equation and a velocity component < dimensions");
-    AVH_HIP(hipSetDevice(b->ctx->device));
+    AVH_HIP(hipSetDevice(b->device));
     const GroupHost& G = b->g[group];
     double dv = 1.0;
     for (int d = 0; d < 3; ++d)
@@ -1130,7 +1130,7 @@ avh_status avh_batch_structure_cube(avh_batch* b, int group, int var, int number
     if (number_of_h < 2 || number_of_h > 65535) return fail(AVH_EINVAL, "number_of_h must be in [2, 65535]");
     if (!(p > 0)) return fail(AVH_EINVAL, "p must be positive");
     if (G.nsamples > 65535) return fail(AVH_EINVAL, "structure functions: at most 65535 samples per group");
-    AVH_HIP(hipSetDevice(b->ctx->device));
+    AVH_HIP(hipSetDevice(b->device));
     const int nx = G.n[0], ny = G.n[1], nlags = number_of_h - 1;
     const bool two = b->dim == 2;
     const int cu = two ? ((nx + 63) / 64) * ((ny + 4 * SWEEP_ROWS - 1) / (4 * SWEEP_ROWS)) : (nx + 255) / 256;
@@ -1184,7 +1184,7 @@ avh_status avh_batch_structure_cube(avh_batch* b, int group, int var, int number
 avh_status avh_batch_set_tile_shape(avh_batch* b, int shape) {
     if (!b) return fail(AVH_EINVAL, "null argument");
     if (shape < -1 || shape >= num_shapes(b->dim)) return fail(AVH_EINVAL, "no such tile shape");
-    AVH_HIP(hipSetDevice(b->ctx->device));
+    AVH_HIP(hipSetDevice(b->device));
     AVH_HIP(hipStreamSynchronize(b->stream));
     b->graph.reset();
     b->shape = shape;
@@ -1193,13 +1193,13 @@ avh_status avh_batch_set_tile_shape(avh_batch* b, int shape) {
 
 avh_status avh_batch_autotune(avh_batch* b, int* best_shape, double* ms_per_shape, int* nshapes) {
     if (!b) return fail(AVH_EINVAL, "null argument");
-    AVH_HIP(hipSetDevice(b->ctx->device));
+    AVH_HIP(hipSetDevice(b->device));
     return batch_autotune(b, best_shape, ms_per_shape, nshapes);
 }
 
 avh_status avh_batch_time_step_kernels(avh_batch* b, int64_t steps, double* ms, int* kernels) {
     if (!b || !ms || !kernels || steps < 1 || steps > 100000) return fail(AVH_EINVAL, "bad argument");
-    AVH_HIP(hipSetDevice(b->ctx->device));
+    AVH_HIP(hipSetDevice(b->device));
     const int nk = batch_launches_per_step(b);
     avh_status r = batch_ensure_shape(b);
     if (r) return r;
@@ -1216,7 +1216,7 @@ avh_status avh_batch_get_progress(avh_batch* b, int group, int sample, avh_progr
     avh_status r = check_gs(b, group, sample);
     if (r) return r;
     if (!p) return fail(AVH_EINVAL, "null argument");
-    AVH_HIP(hipSetDevice(b->ctx->device));
+    AVH_HIP(hipSetDevice(b->device));
     AVH_HIP(hipStreamSynchronize(b->stream));
     Control c;
     AVH_HIP(hipMemcpy(&c, b->g[group].ctrl + sample, sizeof c, hipMemcpyDeviceToHost));
@@ -1234,7 +1234,7 @@ avh_status avh_batch_get_statistics(avh_batch* b, int group, int save, int primi
     if (r) return r;
     if (!mean || !variance || !count) return fail(AVH_EINVAL, "null argument");
     if (save < 0 || save >= b->nsaves) return fail(AVH_EINVAL, "no such statistics save");
-    AVH_HIP(hipSetDevice(b->ctx->device));
+    AVH_HIP(hipSetDevice(b->device));
     AVH_HIP(hipStreamSynchronize(b->stream));
     const GroupHost& G = b->g[group];
     const size_t n = (size_t)b->nv * G.ncells;

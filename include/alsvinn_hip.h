@@ -96,6 +96,8 @@ typedef struct avh_progress {
 
 const char* avh_last_error(void);
 
+/* Solvers, batches, statistics and networks may outlive the context they were
+ * created from: they and the context can be destroyed in any order. */
 avh_status avh_ctx_create(int device, avh_ctx** ctx);
 avh_status avh_ctx_destroy(avh_ctx* ctx);
 
