@@ -556,9 +556,8 @@ static avh_status enqueue_step(avh_solver* s, EventMarks* tm = nullptr) {
     return mark(s, tm);
 }
 
-static TuneKey tune_key(const avh_solver* s) {
-    return TuneKey(0, s->cfg.equation * 16 + s->cfg.reconstruction, s->cfg.flux, s->dim, s->cfg.n[0], s->cfg.n[1],
-                   s->cfg.n[2]);
+static TuneKey solver_key(const avh_config& c, int dim) {
+    return tune_key(TUNE_SOLVER, c, dim, {c.n[0], c.n[1], c.n[2]});
 }
 
 // Times every tile shape on the current state and keeps the fastest: the first
@@ -620,7 +619,7 @@ static avh_status autotune(avh_solver* s, int* best, double* ms, int* nshapes) {
     if ((r = push(s))) return r;
     if (s->shape != b) s->graph.reset();
     s->shape = b;
-    tune_store(tune_key(s), b);
+    tune_store(solver_key(s->cfg, s->dim), b, s->h.active != 0);
     if (best) *best = b;
     if (nshapes) *nshapes = ns;
     return AVH_OK;
@@ -629,7 +628,7 @@ static avh_status autotune(avh_solver* s, int* best, double* ms, int* nshapes) {
 static avh_status ensure_shape(avh_solver* s) {
     if (s->shape >= 0) return AVH_OK;
     int b;
-    if (tune_lookup(tune_key(s), &b)) {
+    if (tune_lookup(solver_key(s->cfg, s->dim), &b)) {
         s->shape = b;
         return AVH_OK;
     }
@@ -947,10 +946,7 @@ avh_status avh_step_noalloc(avh_ctx* ctx, const avh_config* cfg, double* state, 
     // one, else a fixed default (timing would need events)
     int shape = dim == 1 ? 0 : (dim == 2 ? 3 : 1);
     int tuned;
-    if (tune_lookup(TuneKey(0, cfg->equation * 16 + cfg->reconstruction, cfg->flux, dim, cfg->n[0], cfg->n[1],
-                            cfg->n[2]),
-                    &tuned))
-        shape = tuned;
+    if (tune_lookup(solver_key(*cfg, dim), &tuned)) shape = tuned;
     Control* ctrl = (Control*)sp;
     double* B = sp + NOALLOC_CTRL_DOUBLES;
     double* C = B + NOALLOC_MAX_VALUES;

@@ -3,16 +3,15 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
-#include <map>
 #include <memory>
 #include <mutex>
 #include <string>
-#include <tuple>
 #include <vector>
 
 #include "../../include/alsvinn_hip.h"
 #include "avh_pinned.hpp"
 #include "avh_stage_inst.hpp"
+#include "avh_tune.hpp"
 
 struct avh_ctx {
     int device;
@@ -180,34 +179,6 @@ avh_status enqueue_steps_graphed(StepGraph& G, int graph_steps, hipStream_t st, 
         if (r != AVH_OK) return r;
     }
     return AVH_OK;
-}
-
-// Autotuner cache: the tile shape chosen for a (equation, reconstruction,
-// flux, grid) of single solvers (kind 0) or batches (kind 1, grid = the
-// first group, n[2] = total samples), shared by every solver of the process.
-typedef std::tuple<int, int, int, int, long long, long long, long long> TuneKey;
-
-inline std::mutex& tune_mutex() {
-    static std::mutex m;
-    return m;
-}
-
-inline std::map<TuneKey, int>& tune_cache() {
-    static std::map<TuneKey, int> c;
-    return c;
-}
-
-inline bool tune_lookup(const TuneKey& k, int* shape) {
-    std::lock_guard<std::mutex> g(tune_mutex());
-    auto it = tune_cache().find(k);
-    if (it == tune_cache().end()) return false;
-    *shape = it->second;
-    return true;
-}
-
-inline void tune_store(const TuneKey& k, int shape) {
-    std::lock_guard<std::mutex> g(tune_mutex());
-    tune_cache()[k] = shape;
 }
 
 // Mean milliseconds of `reps` back-to-back calls of launch(), after one

@@ -593,11 +593,10 @@ StatsParams stats_params(const avh_batch* b, unsigned int* nblocks) {
     return S;
 }
 
-TuneKey batch_tune_key(const avh_batch* b) {
+TuneKey batch_key(const avh_batch* b) {
     long long total = 0;
     for (int i = 0; i < b->ngroups; ++i) total += b->g[i].nsamples;
-    return TuneKey(1, b->cfg.equation * 16 + b->cfg.reconstruction, b->cfg.flux, b->dim, b->g[0].n[0],
-                   b->g[0].n[1], total);
+    return tune_key(TUNE_BATCH, b->cfg, b->dim, {b->g[0].n[0], b->g[0].n[1], total});
 }
 
 // Times every tile shape over all samples with the first stage (flux-only if
@@ -661,7 +660,7 @@ avh_status batch_autotune(avh_batch* b, int* best, double* ms, int* nshapes) {
     if (r) return r;
     if (b->shape != bst) b->graph.reset();
     b->shape = bst;
-    tune_store(batch_tune_key(b), bst);
+    tune_store(batch_key(b), bst, active);
     if (best) *best = bst;
     if (nshapes) *nshapes = ns;
     return AVH_OK;
@@ -670,7 +669,7 @@ avh_status batch_autotune(avh_batch* b, int* best, double* ms, int* nshapes) {
 avh_status batch_ensure_shape(avh_batch* b) {
     if (b->shape >= 0) return AVH_OK;
     int s;
-    if (tune_lookup(batch_tune_key(b), &s)) {
+    if (tune_lookup(batch_key(b), &s)) {
         b->shape = s;
         return AVH_OK;
     }

@@ -182,20 +182,21 @@ avh_status avh_step_noalloc(avh_ctx* ctx, const avh_config* cfg, double* state, 
  * counterpart (set-up cost kept out of a timed or latency-bound loop). */
 avh_status avh_prepare_graph(avh_solver* solver);
 /* Tile shape of the fused stage kernel: -1 (default) lets the autotuner
- * pick on first use (cached per equation, reconstruction, flux and grid for
- * the process), 0..nshapes-1 fixes one (1D: 256 or 64 cells; 2D: 32x11 on 192
- * threads, 16x15 on 512, 16x7 on 256, 32x15 on 256 or 32x15 on 1024; 3D columns
- * marching over z-planes: 16x15 over 4 planes, 16x15, 17x14 and 14x17 over as
- * many as fill the compute units evenly, 16x15 over 16, 2 and 32).
+ * pick on first use (cached per equation, reconstruction, flux, integrator and
+ * grid for the process, unless the solver had stopped), 0..nshapes-1 fixes one
+ * (1D: 256 or 64 cells; 2D: 32x11 on 192 threads, 16x15 on 512, 16x7 on 256,
+ * 32x15 on 256 or 32x15 on 1024; 3D columns marching over z-planes: 16x15 over 4
+ * planes, 16x15, 17x14 and 14x17 over as many as fill the compute units evenly,
+ * 16x15 over 16, 2 and 32).
  * Results are identical for every shape.  Small 1D grids run whole steps in one
  * workgroup unless a shape is fixed.
  * No reference counterpart: the reference's CUDA kernels use fixed block
  * sizes (alsfvm/src/numflux/NumericalFluxCUDA.cu:330-414). */
 avh_status avh_set_tile_shape(avh_solver* solver, int shape);
-/* Time every tile shape on the solver's current state now (a flux-only
- * launch, and for RK3 the second stage on its output, into the solver's
- * scratch buffers; the solution and step state are unchanged) and select
- * the fastest.  ms_per_shape (may be NULL) receives *nshapes <= 8 timings. */
+/* Time every tile shape on the solver's current state now (the launches of a
+ * step, into the solver's scratch buffers, or of a solver that has stopped the
+ * first one; the solution and step state are unchanged) and select the
+ * fastest.  ms_per_shape (may be NULL) receives *nshapes <= 8 timings. */
 avh_status avh_autotune(avh_solver* solver, int* best_shape, double* ms_per_shape, int* nshapes);
 
 /* Run `steps` full time steps with a HIP event pair around every kernel
