@@ -1030,12 +1030,20 @@ avh_status avh_time_step_kernels(avh_solver* s, int64_t steps, double* ms, int* 
     if (!s || !ms || !kernels || steps < 1 || steps > 100000) return fail(AVH_EINVAL, "bad argument");
     avh_status r = use_device(s);
     if (r) return r;
+    EventMarks t;
+    if (line_steps(s)) {
+        // one launch holds many steps: a step's share of the launches of them all
+        if ((r = t.create(2)) || (r = mark(s, &t)) || (r = enqueue_steps(s, steps)) || (r = mark(s, &t))) return r;
+        if ((r = t.average(1, 1, ms))) return r;
+        ms[0] /= (double)steps;
+        *kernels = 1;
+        return AVH_OK;
+    }
     // launches per step: the stages, and forward euler's element-wise pass and
     // end-of-step kernel (the rk final stages end the step themselves)
     if ((r = ensure_shape(s))) return r;
     const bool two = s->cfg.integrator == AVH_INT_RUNGEKUTTA2 || pair_for(s->cfg, s->pair, s->dim, s->shape);
     const int nk = two ? 2 : 3;
-    EventMarks t;
     if ((r = t.create((size_t)steps * (nk + 1)))) return r;
     for (int64_t k = 0; k < steps; ++k)
         if ((r = enqueue_step(s, &t))) return r;

@@ -196,7 +196,8 @@ avh_status avh_set_tile_shape(avh_solver* solver, int shape);
 /* Time every tile shape on the solver's current state now (the launches of a
  * step, into the solver's scratch buffers, or of a solver that has stopped the
  * first one; the solution and step state are unchanged) and select the
- * fastest.  ms_per_shape (may be NULL) receives *nshapes <= 8 timings. */
+ * fastest.  On small 1D grids the shapes are those of the stage kernels, which
+ * steps take once one is fixed.  ms_per_shape (may be NULL) receives *nshapes <= 8 timings. */
 avh_status avh_autotune(avh_solver* solver, int* best_shape, double* ms_per_shape, int* nshapes);
 
 /* Run `steps` full time steps with a HIP event pair around every kernel
@@ -206,7 +207,9 @@ avh_status avh_autotune(avh_solver* solver, int* best_shape, double* ms_per_shap
  * k-th kernel of a step (k < *kernels_per_step <= 4), in launch order: the
  * stages, or forward euler's element-wise pass and end-of-step kernel (the
  * last RK2 / RK3 launch ends the step in its last workgroup; on small grids
- * RK3's last two stages are one launch). */
+ * RK3's last two stages are one launch).  On small 1D grids that run whole
+ * steps in one workgroup (no tile shape fixed) that kernel is the only one, and
+ * its duration is divided by the steps it ran. */
 avh_status avh_time_step_kernels(avh_solver* solver, int64_t steps, double* ms_per_launch,
                                  int* kernels_per_step);
 
