@@ -146,15 +146,29 @@ hipError_t launch_stage_k(const StageParams& P, hipStream_t stream) {
 // prologue; one alone leaves about a quarter of the pipe idle.
 // 128^3, 16x15 columns, us of a volume substep's launch at 8 / 13 / 16 / 32
 // planes and at the 19 this picks: 165 / 163 / 192 / 240 and 158.
+// A chunk past the box is the box, so longer ones are not tried (each try costs
+// a division, and a call over a small box is 31 us in all).
+// `thin`: one plane where even that gives each CU no more than one workgroup,
+// since what is left is a workgroup's chain.  us of a call of
+// avh_numerical_flux on boxes of 128^3 (64^3), euler3 weno2, with chunks of two
+// planes and more, and so: 2 cells in z 36.7 -> 33.0 (35.9 -> 31.5), in x
+// 45.3 -> 45.3 (38.6 -> 34.1), in y 41.4 -> 41.3 (36.5 -> 33.7), a 2x2 pencil
+// along x 35.8 -> 31.4, along z 36.6 -> 32.2, a 2x2x2 corner 35.1 -> 31.2; one
+// workgroup per 8x4x4 brick takes 38.0 (32.7), 49.2 (38.5), 41.1 (35.4), 31.8,
+// 39.1 and 31.7.  Not past one workgroup a CU: burgers eno2, 128x128x8 in 576
+// workgroups of one plane 33.3, in 288 of two 31.1.
 template <class K>
-int march_chunk(const int* n, long long* least = nullptr) {
-    const int CUS = 256;
-    int best = 1;
+int march_chunk(const int* n, bool thin = false, long long* least = nullptr) {
+    const unsigned int CUS = 256;
+    const unsigned int columns = K::tiles(n, n[2]);
+    const int longest = n[2] < 64 ? n[2] : 64;
+    const bool single = longest == 1 || (thin && (long long)columns * n[2] <= CUS);
+    int best = 0;
     long long cost = 0;
-    for (int lz = 2; lz <= 64; ++lz) {
-        const long long per_cu = (K::tiles(n, lz) + CUS - 1) / CUS;
+    for (int lz = single ? 1 : 2; lz <= (single ? 1 : longest); ++lz) {
+        const long long per_cu = (columns * (unsigned int)((n[2] + lz - 1) / lz) + CUS - 1) / CUS;
         const long long c = (2 * per_cu < 3 ? 3 : 2 * per_cu) * (lz + 1);
-        if (lz == 2 || c < cost) {
+        if (!best || c < cost) {
             best = lz;
             cost = c;
         }
@@ -243,10 +257,10 @@ struct VolumeKernel2 {
 };
 
 template <class K>
-hipError_t launch_volume_march_k(const StageParams& P, const VolumeParams& V, hipStream_t stream) {
+hipError_t launch_volume_march_k(const StageParams& P, const VolumeParams& V, int lz, hipStream_t stream) {
     StageParams Q = P;
-    Q.lz = march_chunk<K>(P.n);
-    hipLaunchKernelGGL(volume_march_kernel3<K>, dim3(K::tiles(P.n, Q.lz)), dim3(K::NT), 0, stream, Q, V);
+    Q.lz = lz;
+    hipLaunchKernelGGL(volume_march_kernel3<K>, dim3(K::tiles(P.n, lz)), dim3(K::NT), 0, stream, Q, V);
     return hipGetLastError();
 }
 
@@ -260,11 +274,9 @@ hipError_t launch_volume_march(const StageParams& P, const VolumeParams& V, hipS
     typedef MarchKernel3<EQ, RECON, FLUX, 17, 14, 256, MODE, true> B;
     typedef MarchKernel3<EQ, RECON, FLUX, 14, 17, 256, MODE, true> C;
     long long a, b, c;
-    march_chunk<A>(P.n, &a);
-    march_chunk<B>(P.n, &b);
-    march_chunk<C>(P.n, &c);
-    if (a <= b && a <= c) return launch_volume_march_k<A>(P, V, stream);
-    return b <= c ? launch_volume_march_k<B>(P, V, stream) : launch_volume_march_k<C>(P, V, stream);
+    const int la = march_chunk<A>(P.n, true, &a), lb = march_chunk<B>(P.n, true, &b), lc = march_chunk<C>(P.n, true, &c);
+    if (a <= b && a <= c) return launch_volume_march_k<A>(P, V, la, stream);
+    return b <= c ? launch_volume_march_k<B>(P, V, lb, stream) : launch_volume_march_k<C>(P, V, lc, stream);
 }
 
 template <class EQ, int RECON, class FLUX, int DIM>
