@@ -206,18 +206,39 @@ __device__ __forceinline__ int bc_value_index(int x, int n, int bc) {
 // boundary of the square of half-width h around it (2 points in 1D, 8h in
 // 2D), divided by the number of cells.
 //
-// 1D: block (x, y, z) sums 256 cells of sample z at lag y + 1.
+// One thread a cell: block (x, y, z) sums 256 cells of sample z at lag y + 1.
+// With periodic boundaries of a 2D grid one side of the ring is summed (see the
+// sweep below).  Serves 1D grids, and 2D ones as structure_sweeps says.
 template <int P>
-__global__ __launch_bounds__(256) void structure_line_kernel(const double* state, long long stride, int var, int nx,
-                                                             int bc, double p, double* partial) {
+__global__ __launch_bounds__(256) void structure_gather_kernel(const double* state, long long stride, int var, int nx,
+                                                               int ny, int dims, int bc, double p, double* partial) {
     const int h = blockIdx.y + 1;
-    const double* u = state + (long long)blockIdx.z * stride + (long long)var * nx;
-    const int c = blockIdx.x * 256 + threadIdx.x;
+    const long long ncells = (long long)nx * ny;
+    const double* u = state + (long long)blockIdx.z * stride + (long long)var * ncells;
+    const long long c = (long long)blockIdx.x * 256 + threadIdx.x;
     double acc = 0.0;
-    if (c < nx) {
+    if (c < ncells && dims == 1) {
         const double uc = u[c];
-        acc = add_power<P>(acc, uc - u[bc_value_index(c - h, nx, bc)], p);
-        acc = add_power<P>(acc, uc - u[bc_value_index(c + h, nx, bc)], p);
+        acc = add_power<P>(acc, uc - u[bc_value_index((int)c - h, nx, bc)], p);
+        acc = add_power<P>(acc, uc - u[bc_value_index((int)c + h, nx, bc)], p);
+    } else if (c < ncells) {
+        const double uc = u[c];
+        const int i = (int)(c % nx), j = (int)(c / nx);
+        const bool wrap = bc == AVH_BC_PERIODIC;
+        // count terms from cell k of a line of n on, s apart from one to the next
+        auto line = [&](const double* v, int k, int n, long long s, int count) {
+            int at = bc_value_index(k, n, bc);
+            for (int t = 0; t < count; ++t) {
+                acc = add_power<P>(acc, uc - v[at * s], p);
+                ++k;
+                if (wrap) at = at + 1 == n ? 0 : at + 1;
+                else at = k < 0 ? 0 : (k > n - 1 ? n - 1 : k);
+            }
+        };
+        for (int side = 0; side < (wrap ? 1 : 2); ++side) {
+            line(u + bc_value_index(side ? i - h : i + h, nx, bc), j - h + 1, ny, nx, 2 * h - 1);
+            line(u + (long long)bc_value_index(side ? j - h : j + h, ny, bc) * nx, i - h, nx, 1, 2 * h + 1);
+        }
     }
     const double sum = block_sum(acc);
     if (threadIdx.x == 0)
@@ -250,9 +271,9 @@ __global__ __launch_bounds__(256) void transpose_kernel(const double* state, lon
 // pair at +h seen from its other cell, so one side is swept and the finish
 // doubles it; with neumann boundaries both are.
 // Bound by the FP64 pipe (a subtraction and an FMA a pair for p = 2); the
-// loads, one per SWEEP_ROWS pairs, come from L1 and L2.  One thread per cell
-// gathering its ring with wrapped indices took 17.2 ms for 16 samples of
-// 256^2 and 62 lags; this takes 0.70 ms (60 % of the pipe).
+// loads, one per SWEEP_ROWS pairs, come from L1 and L2.  16 samples of 256^2
+// and 62 lags, periodic: 0.70 ms (60 % of the pipe), the gather of both sides
+// 17.2 ms.
 // Block = 64 columns x 4 * SWEEP_ROWS rows of one sample at one lag, of the
 // field (blockIdx.x < cu) or of its transpose; the longest lags start first.
 constexpr int SWEEP_ROWS = 8;
@@ -1092,15 +1113,40 @@ avh_status avh_batch_kinetic_energy(avh_batch* b, int group, int component, doub
     return AVH_OK;
 }
 
-static avh_status launch_structure_line(int pi, dim3 grid, hipStream_t st, const double* state, long long stride,
-                                        int var, int nx, int bc, double p, double* partial) {
+// blocks of a sweep of columns of nr cells, nc of them, and of its transpose
+static int sweep_blocks(int nc, int nr) { return ((nc + 63) / 64) * ((nr + 4 * SWEEP_ROWS - 1) / (4 * SWEEP_ROWS)); }
+
+// Whether a 2D structure function sweeps columns, or gathers a cell a thread.
+// The sweep saves loads and indices; it takes a transposed copy first, and
+// lanes and rows past the grid's edge are lost.  us of a call, gather / sweep:
+//   p = 2     1 lag     256^2 x 16 32 / 40, 1000x800 40 / 41, 17x300 x 3 26 / 31
+//             6 lags    256^2 x 16 82 / 62, 128^2 x 4 30 / 33, 17x300 x 3 29 / 33
+//             16 lags   128^2 x 4 46 / 36, 17x300 x 3 34 / 35, 16^2 31 / 32
+//             32 lags   256^2 x 16 975 / 247, 17x300 x 3 48 / 42, 16^2 36 / 34
+// so the gather takes calls of few lags and few pairs of cells.
+//   p = 2.5 is bound by the powers, whichever way the cells come: neumann
+//             62 lags   17x300 x 3 1565 / 3975, 130^2 x 8 11306 / 16474,
+//                       256^2 10760 (2 samples) / 9497
+//             8 lags    256^2 x 2 237 / 291, x 16 1645 / 1551, 1000x800 1296 / 1211
+// so there the sweep takes only grids that fill its lanes, in enough blocks.
+static bool structure_sweeps(bool general, int nx, int ny, int nsamples, int nlags) {
+    const long long cells = (long long)nx * ny;
+    if (!general) return nlags > 12 || cells * nsamples * (4 * nlags * (nlags + 1)) > (1ll << 24);
+    const int cu = sweep_blocks(nx, ny), ct = sweep_blocks(ny, nx);
+    const double slots = 64.0 * 4 * SWEEP_ROWS * (cu + ct);  // lanes times rows of the field's sweep and the transpose's
+    return nlags >= 8 && std::min(nx, ny) >= 128 && (long long)(cu + ct) * nlags * nsamples >= 2048 &&
+           2 * cells >= 0.92 * slots;
+}
+
+static avh_status launch_structure_gather(int pi, dim3 grid, hipStream_t st, const double* state, long long stride,
+                                        int var, int nx, int ny, int dims, int bc, double p, double* partial) {
     switch (pi) {
-    case 1: hipLaunchKernelGGL(structure_line_kernel<1>, grid, dim3(256), 0, st, state, stride, var, nx, bc, p, partial); break;
-    case 2: hipLaunchKernelGGL(structure_line_kernel<2>, grid, dim3(256), 0, st, state, stride, var, nx, bc, p, partial); break;
-    case 3: hipLaunchKernelGGL(structure_line_kernel<3>, grid, dim3(256), 0, st, state, stride, var, nx, bc, p, partial); break;
-    case 4: hipLaunchKernelGGL(structure_line_kernel<4>, grid, dim3(256), 0, st, state, stride, var, nx, bc, p, partial); break;
-    case 5: hipLaunchKernelGGL(structure_line_kernel<5>, grid, dim3(256), 0, st, state, stride, var, nx, bc, p, partial); break;
-    default: hipLaunchKernelGGL(structure_line_kernel<0>, grid, dim3(256), 0, st, state, stride, var, nx, bc, p, partial); break;
+    case 1: hipLaunchKernelGGL(structure_gather_kernel<1>, grid, dim3(256), 0, st, state, stride, var, nx, ny, dims, bc, p, partial); break;
+    case 2: hipLaunchKernelGGL(structure_gather_kernel<2>, grid, dim3(256), 0, st, state, stride, var, nx, ny, dims, bc, p, partial); break;
+    case 3: hipLaunchKernelGGL(structure_gather_kernel<3>, grid, dim3(256), 0, st, state, stride, var, nx, ny, dims, bc, p, partial); break;
+    case 4: hipLaunchKernelGGL(structure_gather_kernel<4>, grid, dim3(256), 0, st, state, stride, var, nx, ny, dims, bc, p, partial); break;
+    case 5: hipLaunchKernelGGL(structure_gather_kernel<5>, grid, dim3(256), 0, st, state, stride, var, nx, ny, dims, bc, p, partial); break;
+    default: hipLaunchKernelGGL(structure_gather_kernel<0>, grid, dim3(256), 0, st, state, stride, var, nx, ny, dims, bc, p, partial); break;
     }
     AVH_HIP(hipGetLastError());
     return AVH_OK;
@@ -1131,9 +1177,10 @@ avh_status avh_batch_structure_cube(avh_batch* b, int group, int var, int number
     if (G.nsamples > 65535) return fail(AVH_EINVAL, "structure functions: at most 65535 samples per group");
     AVH_HIP(hipSetDevice(b->device));
     const int nx = G.n[0], ny = G.n[1], nlags = number_of_h - 1;
-    const bool two = b->dim == 2;
-    const int cu = two ? ((nx + 63) / 64) * ((ny + 4 * SWEEP_ROWS - 1) / (4 * SWEEP_ROWS)) : (nx + 255) / 256;
-    const int ct = two ? ((ny + 63) / 64) * ((nx + 4 * SWEEP_ROWS - 1) / (4 * SWEEP_ROWS)) : 0;
+    const int pi = p == 1.0 ? 1 : p == 2.0 ? 2 : p == 3.0 ? 3 : p == 4.0 ? 4 : p == 5.0 ? 5 : 0;
+    const bool two = b->dim == 2 && structure_sweeps(pi == 0, nx, ny, G.nsamples, nlags);
+    const int cu = two ? sweep_blocks(nx, ny) : (int)((G.ncells + 255) / 256);
+    const int ct = two ? sweep_blocks(ny, nx) : 0;
     const size_t npart = (size_t)(cu + ct) * nlags;
     const size_t per = npart + (two ? (size_t)G.ncells : 0) + number_of_h;
     const int slab = slab_samples(per, G.nsamples);
@@ -1143,7 +1190,6 @@ avh_status avh_batch_structure_cube(avh_batch* b, int group, int var, int number
     double* const trans = part + npart * slab;
     double* const d = trans + (two ? (size_t)G.ncells * slab : 0);
     const long long stride = (long long)b->nv * G.ncells;
-    const int pi = p == 1.0 ? 1 : p == 2.0 ? 2 : p == 3.0 ? 3 : p == 4.0 ? 4 : p == 5.0 ? 5 : 0;
     for (int s0 = 0; s0 < G.nsamples; s0 += slab) {
         const int m = std::min(slab, G.nsamples - s0);
         const double* state = G.A + s0 * stride;
@@ -1165,11 +1211,11 @@ avh_status avh_batch_structure_cube(avh_batch* b, int group, int var, int number
             S.partial = part;
             r = launch_structure_sweep(pi, dim3(cu + ct, nlags, m), b->stream, S);
         } else {
-            r = launch_structure_line(pi, dim3(cu, nlags, m), b->stream, state, stride, var, nx, b->cfg.boundary, p,
-                                      part);
+            r = launch_structure_gather(pi, dim3(cu, nlags, m), b->stream, state, stride, var, nx, ny, b->dim,
+                                        b->cfg.boundary, p, part);
         }
         if (r) return r;
-        const double factor = two && b->cfg.boundary == AVH_BC_PERIODIC ? 2.0 : 1.0;
+        const double factor = b->dim == 2 && b->cfg.boundary == AVH_BC_PERIODIC ? 2.0 : 1.0;
         hipLaunchKernelGGL(structure_finish_kernel, dim3((m * number_of_h + 3) / 4), dim3(256), 0, b->stream, part,
                            cu + ct, number_of_h, m, (double)G.ncells, factor, d);
         AVH_HIP(hipGetLastError());
