@@ -27,6 +27,7 @@
 #include <cmath>
 #include <cstdint>
 #include <cstring>
+#include <memory>
 #include <new>
 #include <random>
 #include <vector>
@@ -1109,6 +1110,28 @@ avh_status read_packed(avh_mlp* n, const float* src, int count, float* host) {
     return AVH_OK;
 }
 
+// One member's parameters, copied as they are and packed by the host.  Less
+// than the launch of a pack kernel and its wait below HOST_PACK_MAX values (us
+// of get_params, on the device / here: 24 / 13 for 500 values, 30 / 20 for
+// 49e3, 41 / 35 for 116e3, 60 / 67 for 229e3).
+constexpr long long HOST_PACK_MAX = 1 << 17;
+avh_status read_member(avh_mlp* n, int member, float* host) {
+    std::unique_ptr<float[]> h(new (std::nothrow) float[(size_t)n->P]);
+    if (!h) return fail(AVH_ENOMEM, "host allocation failed");
+    AVH_HIP(hipStreamSynchronize(n->stream));
+    AVH_HIP(hipMemcpy(h.get(), n->params + member * n->P, sizeof(float) * n->P, hipMemcpyDeviceToHost));
+    for (int l = 0; l < n->nl; ++l) {
+        const LayerDesc& L = n->L[l];
+        const int fin = l == 0 ? n->cfg.n_in : n->cfg.width;
+        const int fout = l == n->nl - 1 ? n->cfg.n_out : n->cfg.width;
+        for (int o = 0; o < fout; ++o, host += fin)
+            std::memcpy(host, h.get() + L.w_off + (long long)o * L.nin, sizeof(float) * fin);
+        std::memcpy(host, h.get() + L.b_off, sizeof(float) * fout);
+        host += fout;
+    }
+    return AVH_OK;
+}
+
 // Outputs of every member for the first `rows` device rows, in data units,
 // slab by slab of at most PREDICT_SLAB rows (the outputs of a call then take
 // at most 16 MiB a member at 64 outputs).
@@ -1299,6 +1322,7 @@ avh_status avh_mlp_set_normalization(avh_mlp* n, const float* in_mean, const flo
 avh_status avh_mlp_get_params(avh_mlp* n, int member, float* out) {
     if (!n || !out || member < 0 || member >= n->M) return fail(AVH_EINVAL, "bad argument");
     AVH_HIP(hipSetDevice(n->device));
+    if (n->P < HOST_PACK_MAX) return read_member(n, member, out);
     return read_packed(n, n->params + member * n->P, 1, out);
 }
 
