@@ -280,8 +280,15 @@ __device__ __forceinline__ long long ghost_cell(const GhostCells& C, long long i
 
 // Every ghost cell takes the value of the interior cell the boundary map
 // assigns to it; interior cells are only read, so the order does not matter.
-// One variable a block (blockIdx.y), so that a thread pays one load's latency.
-__global__ __launch_bounds__(256) void volume_boundary_kernel(VolPtrs V, GhostCells C, int bc) {
+// TOGETHER: a thread copies every variable, which divides for its position
+// once; otherwise a block copies one (blockIdx.y), and a thread pays one load's
+// latency.  us of a call, five variables, together / one a block: 24x30x20 with
+// two ghost cells (20e3 of them) 14.9 / 13.5, 64^3 with three (88e3) 15.3 / 14.8,
+// 100x110x100 with three (203e3) 16.4 / 17.3, 400x400x5 with two (670e3)
+// 20.2 / 24.1, 1000x1000x4 with three 96 / 109.
+constexpr long long GHOSTS_TOGETHER = 1 << 17;
+template <bool TOGETHER>
+__global__ __launch_bounds__(256) void volume_boundary_kernel(VolPtrs V, GhostCells C, int nv, int bc) {
     for (long long j = (long long)blockIdx.x * 256 + threadIdx.x; j < C.all; j += (long long)gridDim.x * 256) {
         int x, y, z;
         const long long i = ghost_cell(C, j, x, y, z);
@@ -289,8 +296,12 @@ __global__ __launch_bounds__(256) void volume_boundary_kernel(VolPtrs V, GhostCe
         const int sy = V.g[1] ? bc_map(y, V.n[1], bc) : y;
         const int sz = V.g[2] ? bc_map(z, V.n[2], bc) : z;
         const long long si = ((long long)(sz + V.g[2]) * V.tot[1] + (sy + V.g[1])) * V.tot[0] + (sx + V.g[0]);
-        double* const a = V.v[blockIdx.y];
-        a[i] = a[si];
+        if constexpr (!TOGETHER) {
+            double* const a = V.v[blockIdx.y];
+            a[i] = a[si];
+        } else {
+            for (int v = 0; v < nv; ++v) V.v[v][i] = V.v[v][si];
+        }
     }
 }
 
@@ -541,8 +552,12 @@ avh_status avh_apply_boundary(avh_ctx* ctx, int boundary, avh_volume* volume, vo
     const hipStream_t st = (hipStream_t)stream;
     const GhostCells c = ghost_cells(volume->n, volume->ghosts);
     if (c.all > 0) {
-        hipLaunchKernelGGL(volume_boundary_kernel, dim3(grid_blocks(c.all), volume->nvars), dim3(256), 0, st,
-                           ptrs_of(volume), c, boundary);
+        if (c.all > GHOSTS_TOGETHER)
+            hipLaunchKernelGGL(volume_boundary_kernel<true>, dim3(grid_blocks(c.all)), dim3(256), 0, st,
+                               ptrs_of(volume), c, volume->nvars, boundary);
+        else
+            hipLaunchKernelGGL(volume_boundary_kernel<false>, dim3(grid_blocks(c.all), volume->nvars), dim3(256), 0, st,
+                               ptrs_of(volume), c, volume->nvars, boundary);
         AVH_HIP(hipGetLastError());
     }
     AVH_HIP(hipStreamSynchronize(st));
