@@ -758,9 +758,10 @@ struct avh_mlp {
     long long P = 0, WB = 0;
     float *params = nullptr, *m = nullptr, *v = nullptr, *grad = nullptr;
     uint16_t *wb = nullptr, *wtb = nullptr;
-    uint16_t *x0 = nullptr, *x0t = nullptr;
-    float* z = nullptr;        // [hidden][M][B][width]
-    uint16_t *a = nullptr, *at = nullptr;
+    uint16_t *x0t = nullptr, *at = nullptr;  // transposed inputs and activations
+    float* z = nullptr;        // [hidden][M][B][width] pre-activations, or gelu' of them (fused)
+    // of the layer-by-layer path alone
+    uint16_t *x0 = nullptr, *a = nullptr;
     float *yhat = nullptr, *yn = nullptr;
     uint16_t *dz[2] = {nullptr, nullptr}, *dzt[2] = {nullptr, nullptr};
     float *mu_in = nullptr, *sd_in = nullptr, *mu_out = nullptr, *sd_out = nullptr;
@@ -1218,17 +1219,9 @@ avh_status avh_mlp_create(avh_ctx* ctx, const avh_mlp_config* cfg, avh_mlp** out
     alloc((void**)&n->grad, sizeof(float) * M * P);
     alloc((void**)&n->wb, 2 * M * WB);
     alloc((void**)&n->wtb, 2 * M * WB);
-    alloc((void**)&n->x0, 2 * M * B * n->pin);
     alloc((void**)&n->x0t, 2 * M * B * n->pin);
     alloc((void**)&n->z, sizeof(float) * H * M * B * W);
-    alloc((void**)&n->a, 2 * H * M * B * W);
     alloc((void**)&n->at, 2 * H * M * B * W);
-    alloc((void**)&n->yhat, sizeof(float) * M * B * n->pout);
-    alloc((void**)&n->yn, sizeof(float) * M * B * n->pout);
-    for (int i = 0; i < 2; ++i) {
-        alloc((void**)&n->dz[i], 2 * M * dzw);
-        alloc((void**)&n->dzt[i], 2 * M * dzw);
-    }
     alloc((void**)&n->mu_in, sizeof(float) * cfg->n_in);
     alloc((void**)&n->sd_in, sizeof(float) * cfg->n_in);
     alloc((void**)&n->mu_out, sizeof(float) * cfg->n_out);
@@ -1237,6 +1230,15 @@ avh_status avh_mlp_create(avh_ctx* ctx, const avh_mlp_config* cfg, avh_mlp** out
     if (n->fused) {
         alloc((void**)&n->dztl, 2 * M * n->nl * dzw);
         alloc((void**)&n->loss_part, sizeof(float) * M * (B / ROWS));
+    } else {
+        alloc((void**)&n->x0, 2 * M * B * n->pin);
+        alloc((void**)&n->a, 2 * H * M * B * W);
+        alloc((void**)&n->yhat, sizeof(float) * M * B * n->pout);
+        alloc((void**)&n->yn, sizeof(float) * M * B * n->pout);
+        for (int i = 0; i < 2; ++i) {
+            alloc((void**)&n->dz[i], 2 * M * dzw);
+            alloc((void**)&n->dzt[i], 2 * M * dzw);
+        }
     }
     if (!ok) {
         free_mlp(n);
