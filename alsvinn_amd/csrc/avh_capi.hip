@@ -135,7 +135,7 @@ __device__ __forceinline__ double draw_double(unsigned long long r, int elo, int
     return __longlong_as_double((long long)(((unsigned long long)(e + 1023) << 52) | mant));
 }
 
-enum { ARITH_SQRT = 0, ARITH_DIV_RHO = 1, ARITH_DIV_WENO = 2, ARITH_DIV_ROE = 3, ARITH_FREXP = 4, ARITH_DIV_STAR = 5, ARITH_DIV_ONE = 6 };
+enum { ARITH_SQRT = 0, ARITH_DIV_RHO = 1, ARITH_DIV_WENO = 2, ARITH_DIV_ROE = 3, ARITH_FREXP = 4, ARITH_DIV_FLUX = 5, ARITH_DIV_ONE = 6 };
 
 // frexp exponent of a finite double from its bits: 0 for +-0; for normal x
 // the biased exponent - 1022; for subnormal x = mant * 2^-1074 the position
@@ -191,13 +191,25 @@ __global__ __launch_bounds__(256) void arith_selftest_kernel(int kind, unsigned 
             if (r1 & (1ull << 63)) a = -a;
             got = (double)frexp_exp(a);
             want = (double)frexp_exp_bits(a);
-        } else if (kind == ARITH_DIV_STAR) {
-            // HLL3's star quotients: denominators +-[2^-150, 2^150], nonzero
-            // numerators +-[2^-840, 2^600], each quotient within [2^-1000, 2^750]
-            b = draw_double(r1, -150, 150);
-            a = draw_double(r0, -840, 600);
-            if (r1 & (1ull << 62)) a = -a;
-            if (r1 & (1ull << 63)) b = -b;
+        } else if (kind == ARITH_DIV_FLUX) {
+            // the flux functions' quotients, each over the range its guards
+            // leave: HLL's over s_r - s_l (half of the draws), and HLL3's over
+            // -aa and over s_m - s_k (a quarter each; the last are nonzero and
+            // of either sign)
+            const unsigned long long r2 = splitmix64(r0 ^ r1);
+            const int which = (int)(r2 & 3ull);
+            if (which < 2) {
+                b = draw_double(r1, -100, 180);
+                a = (r0 & 1023ull) == 0 ? 0.0 : draw_double(r0, -701, 456);
+            } else if (which == 2) {
+                b = draw_double(r1, -150, 80);
+                a = (r0 & 1023ull) == 0 ? 0.0 : draw_double(r0, -919, 268);
+            } else {
+                b = draw_double(r1, -100, 150);
+                a = draw_double(r0, -800, 630);
+                if (r2 & 4ull) b = -b;
+            }
+            if (r2 & 8ull) a = -a;
             got = div_shared(a, b, div_recip(b));
             want = a / b;
         } else if (kind == ARITH_DIV_ONE) {

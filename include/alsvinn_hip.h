@@ -312,7 +312,10 @@ avh_status avh_substep(avh_ctx* ctx, const avh_config* cfg, const avh_volume* co
  * 2: WENO2 weight a0 / (a0 + a1), a0, a1 in [2^-400, 2^53];
  * 3: Roe quotient, denominators in [2^-50, 2^51]; 4: the binary exponent
  * the range checks read (v_frexp_exp_i32_f64) against the one the bits
- * give, on signed zeros, subnormals and normals.  Bounds are included.
+ * give, on signed zeros, subnormals and normals; 5: the quotients of HLL
+ * (denominators in [2^-100, 2^180], numerators 0 or +-[2^-701, 2^456]) and of
+ * HLL3 ([2^-150, 2^80], 0 or +-[2^-919, 2^268]; +-[2^-100, 2^150],
+ * +-[2^-800, 2^630]); 6: 1/d, d in [2^-53, 2^348].  Bounds are included.
  * mismatches = count of
  * differing results, first_bad[2] (may be NULL) = operands of one of them.
  * No reference counterpart (the reference divides and takes square roots
