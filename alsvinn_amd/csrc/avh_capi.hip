@@ -54,6 +54,7 @@ __global__ __launch_bounds__(256) void ew_kernel(const double* L, double* state,
     constexpr int NV = EQ::NV;
     const long long step = (long long)gridDim.x * blockDim.x;
     long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (!ctrl->active) return;  // step past the end: no-op
     // the first cell's values are in flight while dt is formed
     double l[NV], u[NV];
     if (i < nc) {
