@@ -1138,12 +1138,9 @@ avh_status avh_advance(avh_solver* s, double t_end, int64_t max_steps, int chunk
     seen.t_end = t_end;
     seen.pause_on_save = pause_on_save ? 1 : 0;
     recompute_active(seen);
-    if (max_steps <= 0 || !seen.active) {
-        if ((r = pull(s))) return r;
-    }
-    int64_t done = 0;
-    bool open = false;
-    if (max_steps > 0) {
+    const bool by_device = max_steps > 0 && seen.active;
+    bool open = true;
+    if (by_device) {
         hipLaunchKernelGGL(begin_run_kernel, dim3(1), dim3(64), 0, s->stream, s->ctrl, t_end, seen.pause_on_save,
                            s->pinned_steps());
         AVH_HIP(hipGetLastError());
@@ -1162,7 +1159,7 @@ avh_status avh_advance(avh_solver* s, double t_end, int64_t max_steps, int chunk
         const int64_t seen_steps = s->h.steps;
         if ((r = enqueue_steps(s, k))) return r;
         if ((r = pull(s))) return r;
-        const int64_t ran = s->h.steps - (first ? *s->pinned_steps() : seen_steps);
+        const int64_t ran = s->h.steps - (first && by_device ? *s->pinned_steps() : seen_steps);
         done += ran;
         if (ran < k) break;  // the device loop ended inside the chunk
         open = s->h.active;
