@@ -63,10 +63,15 @@ def kh_interfaces_many(n, params):
     """kh_interfaces for every row of params (samples, 40): (samples, 2, n).
     The same operations on blocks of samples that stay in the caches; what
     remains is the cosines (84 samples of 128 to 512 points: 17 ms one by one,
-    8 ms so; threads make it slower, as numpy's calls are short)."""
+    8 ms so; threads make it slower, as numpy's calls are short).  A lone sample
+    is taken by itself (us of setting one batch's interfaces, 64 points: 92, as a
+    block of one 109)."""
     params = np.asarray(params, dtype=np.float64)
-    x = midpoints(n)
     out = np.empty((params.shape[0], 2, n))
+    if params.shape[0] == 1:
+        out[0] = kh_interfaces(n, params[0])
+        return out
+    x = midpoints(n)
     rows = max(1, 4096 // n)
     for k in range(0, params.shape[0], rows):
         for side, (base, lo) in enumerate(((0.25, 10), (0.75, 0))):
