@@ -264,6 +264,28 @@ hipError_t launch_volume_march_k(const StageParams& P, const VolumeParams& V, in
     return hipGetLastError();
 }
 
+// Boxes at most NARROW_TX cells wide in x (a strip or a pencil beside a
+// neighbour): in 4x24 columns on 128 threads.  In 16x15 ones most lanes idle,
+// and the fifteen rows that a workgroup then loads, a cache line each and all at
+// once, are what it waits for.  As few planes as leave at most four workgroups a
+// CU, which is all of them at once.  us of a call of avh_numerical_flux, euler3
+// hll3, none / weno2 / eno3, one workgroup per 8x4x4 brick, in 16x15 columns and
+// so: a pencil along y of 128^3 31.0 / 36.0 / 33.5, 35.5 / 38.6 / 34.7 and
+// 30.7 / 31.2 / 32.6; a strip in x of 4x100x100 39.9 / 43.5 / - , 42.2 / 46.0 / -
+// and 35.0 / 36.9 / - , of 128^3 45.4 / 48.6 / 59.0, 41.3 / 45.2 / 47.6 and
+// 38.6 / 40.7 / 43.0, of 200x300x100 62.8 / 70.6 / 87.9, 51.7 / 59.2 / 63.6 and
+// 41.5 / 47.3 / 50.6.  Pencils along z lose past some 500 cells (2x2x900 34.9 /
+// 37.8 / 39.7, 38.7 / 41.0 / 43.0 and 40.3 / 42.0 / 43.9): a workgroup a plane, and
+// each reports its wave speeds.
+constexpr int NARROW_TX = 4;
+template <class K>
+int narrow_chunk(const int* n) {
+    const unsigned int most = 4 * 256;
+    const unsigned int columns = K::tiles(n, n[2]);
+    const unsigned int chunks = most / columns;  // along z
+    return chunks < 2 ? n[2] : (int)((n[2] + chunks - 1) / chunks);
+}
+
 // The columns whose launch the model finds shortest (a volume has no
 // autotuner): their workgroups do the same work a plane, so the costs compare.
 // us of an RK3 step through the volume interfaces, 16x15 alone and so: 97x83x61
@@ -273,6 +295,8 @@ hipError_t launch_volume_march(const StageParams& P, const VolumeParams& V, hipS
     typedef MarchKernel3<EQ, RECON, FLUX, 16, 15, 256, MODE, true> A;
     typedef MarchKernel3<EQ, RECON, FLUX, 17, 14, 256, MODE, true> B;
     typedef MarchKernel3<EQ, RECON, FLUX, 14, 17, 256, MODE, true> C;
+    typedef MarchKernel3<EQ, RECON, FLUX, NARROW_TX, 24, 128, MODE, true> D;
+    if (P.n[0] <= NARROW_TX) return launch_volume_march_k<D>(P, V, narrow_chunk<D>(P.n), stream);
     long long a, b, c;
     const int la = march_chunk<A>(P.n, true, &a), lb = march_chunk<B>(P.n, true, &b), lc = march_chunk<C>(P.n, true, &c);
     if (a <= b && a <= c) return launch_volume_march_k<A>(P, V, la, stream);
