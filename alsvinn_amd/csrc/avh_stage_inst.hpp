@@ -245,8 +245,15 @@ hipError_t launch_stage(const StageParams& P, int shape, hipStream_t stream) {
     }
 }
 
-// The reference-Volume kernels: 1D 256 cells, 2D 32x15, 3D columns.  P.mode is MODE_FLUX_ONLY, or MODE_RK3_3 for the
+// The reference-Volume kernels: 1D 256 cells, 2D 32x15 or 16x7, 3D columns.  P.mode is MODE_FLUX_ONLY, or MODE_RK3_3 for the
 // combination V describes.
+// 2D boxes of few 16x7 tiles take these: a workgroup's chain is then all there
+// is, and 32x15's threads march along two interfaces.  us of a call of
+// avh_numerical_flux, weno2 hll3, one interface at a time in 32x15 tiles, 32x15
+// so and 16x7: a strip of 2x200 cells 41.6 / 38.7 / 27.9, of 200x2 30.7 / 31.2 /
+// 27.2, 128^2 (152 tiles) 33.1 / 31.8 / 28.9, 200x150 (286) 33.4 / 31.8 / 30.3,
+// 200^2 (377) 33.6 / 32.1 / 31.4, 200x300 (559) 34.3 / 32.6 / 33.7.
+constexpr unsigned int VOLUME2_SMALL_TILES = 384;
 template <class EQ, int RECON, class FLUX>
 struct VolumeKernel1 {
     typedef StageKernel1<EQ, RECON, FLUX, 256, 256> type;
@@ -254,7 +261,14 @@ struct VolumeKernel1 {
 template <class EQ, int RECON, class FLUX>
 struct VolumeKernel2 {
     typedef TileKernel2<EQ, RECON, FLUX, 32, 15, 256> type;
+    typedef TileKernel2<EQ, RECON, FLUX, 16, 7, 256> small;  // both directions at once, one interface a thread
 };
+
+template <class K>
+hipError_t launch_volume_k(const StageParams& P, const VolumeParams& V, hipStream_t stream) {
+    hipLaunchKernelGGL(volume_stage_kernel<K>, dim3(K::tiles(P.n)), dim3(K::NTHREADS), 0, stream, P, V);
+    return hipGetLastError();
+}
 
 template <class K>
 hipError_t launch_volume_march_k(const StageParams& P, const VolumeParams& V, int lz, hipStream_t stream) {
@@ -311,9 +325,12 @@ hipError_t launch_volume_stage(const StageParams& P, const VolumeParams& V, hipS
         return launch_volume_march<EQ, RECON, FLUX, MODE_RK3_3>(P, V, stream);
     } else {
         typedef typename std::conditional<DIM == 1, VolumeKernel1<EQ, RECON, FLUX>,
-                                          VolumeKernel2<EQ, RECON, FLUX>>::type::type K;
-        hipLaunchKernelGGL(volume_stage_kernel<K>, dim3(K::tiles(P.n)), dim3(K::NTHREADS), 0, stream, P, V);
-        return hipGetLastError();
+                                          VolumeKernel2<EQ, RECON, FLUX>>::type Kernels;
+        if constexpr (DIM == 2) {
+            typedef typename Kernels::small S;
+            if (S::tiles(P.n) <= VOLUME2_SMALL_TILES) return launch_volume_k<S>(P, V, stream);
+        }
+        return launch_volume_k<typename Kernels::type>(P, V, stream);
     }
 }
 
