@@ -131,6 +131,11 @@ __device__ __forceinline__ void recon_faces_reg(const double (&u)[WZ][NV], const
 template <class EQ, int RECON, class FLUX, int TX, int TY, int NTH, int MODE_CT = -1, bool VOL = false>
 struct MarchKernel3 {
     static constexpr int NV = EQ::NV;
+    // Wavefronts a SIMD has to hold.  HLL3's first stage without reconstruction
+    // takes 183 registers with R(k) beside the window it equals and 173 without:
+    // two wavefronts; held to 168 it spills 5, and three run (first stage at
+    // 256^3 757 -> 717 us, 320^3 1465 -> 1385).
+    static constexpr int WAVES = RECON == RECON_NONE && MODE_CT == MODE_L ? 3 : 1;
     static constexpr int NC = TX * TY;  // columns: one per thread, threads past them work on the planes only
     static constexpr int NT = NTH;
     static_assert(NT >= NC && NT % 64 == 0, "one thread per column, whole wavefronts");
@@ -499,15 +504,17 @@ struct MarchKernel3 {
                     typedef typename OpsFor<FLUX::FAST>::type Ops;
                     double lz[NV];
                     bool ok = col_adm;
+                    // R(k); a cell itself where nothing is reconstructed
+                    const double* const behind = RECON == RECON_NONE ? w[HW - 1] : rprev;
                     recon_faces_reg<RECON, NV, WZ, Ops>(w, HW, rb, lz, rnext);
-                    typename EQ::All aL = EQ::template make_all_ops<Ops>(rprev, P.gamma, ok);
+                    typename EQ::All aL = EQ::template make_all_ops<Ops>(behind, P.gamma, ok);
                     typename EQ::All aR = EQ::template make_all_ops<Ops>(lz, P.gamma, ok);
                     double wz = FLUX::template flux_ops<Ops, 2, EQ>(aL, aR, P.gamma, fz, ok);
                     if (FLUX::FAST && !ok) {
                         // operands outside the guarded range: the plain path
                         recon_face_reg<RECON, NV, false, WZ>(w, HW, lz);
                         recon_face_reg<RECON, NV, true, WZ>(w, HW, rnext);
-                        aL = EQ::make_all(rprev, P.gamma);
+                        aL = EQ::make_all(behind, P.gamma);
                         aR = EQ::make_all(lz, P.gamma);
                         bool ok2 = true;
                         wz = FLUX::template flux_ops<PlainOps, 2, EQ>(aL, aR, P.gamma, fz, ok2);
@@ -620,7 +627,7 @@ struct MarchKernel3 {
 };
 
 template <class K>
-__global__ __launch_bounds__(256) void march_kernel3(StageParams P) {
+__global__ __launch_bounds__(256, K::WAVES) void march_kernel3(StageParams P) {
     K::run(P);
 }
 
