@@ -1133,7 +1133,9 @@ avh_status avh_advance(avh_solver* s, double t_end, int64_t max_steps, int chunk
     if (r) return r;
     // The device opens the run itself (begin_run_kernel), ahead of its steps,
     // unless the control block as last seen says that there is nothing to run:
-    // that may be out of date, so it decides only whether to look first.
+    // that may be out of date, so it decides only whether the host looks first
+    // and opens it (us of a call with nothing to run: 26.3; by the kernel and a
+    // second look 29.0).
     Control seen = s->h;
     seen.t_end = t_end;
     seen.pause_on_save = pause_on_save ? 1 : 0;
@@ -1144,16 +1146,17 @@ avh_status avh_advance(avh_solver* s, double t_end, int64_t max_steps, int chunk
         hipLaunchKernelGGL(begin_run_kernel, dim3(1), dim3(64), 0, s->stream, s->ctrl, t_end, seen.pause_on_save,
                            s->pinned_steps());
         AVH_HIP(hipGetLastError());
-        if (!seen.active) {
-            if ((r = pull(s))) return r;
+    } else {
+        if ((r = pull(s))) return r;
+        if (!s->h.violated) {
+            s->h.t_end = t_end;
+            s->h.pause_on_save = seen.pause_on_save;
+            recompute_active(s->h);
+            if ((r = push(s))) return r;
         }
-        open = seen.active || s->h.active;
-    } else if (!s->h.violated) {
-        s->h.t_end = t_end;
-        s->h.pause_on_save = seen.pause_on_save;
-        recompute_active(s->h);
-        if ((r = push(s))) return r;
+        open = s->h.active && !s->h.violated;
     }
+    int64_t done = 0;
     for (bool first = true; open && done < max_steps; first = false) {
         const int64_t k = (max_steps - done) < chunk ? (max_steps - done) : chunk;
         const int64_t seen_steps = s->h.steps;
