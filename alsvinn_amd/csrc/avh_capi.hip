@@ -64,7 +64,6 @@ __global__ __launch_bounds__(256) void ew_kernel(const double* L, double* state,
             u[v] = state[v * nc + i];
         }
     }
-    if (!ctrl->active) return;
     const double s = step_dt(ctrl) / ctrl->cell[0];
     bool bad = false;
     while (i < nc) {
