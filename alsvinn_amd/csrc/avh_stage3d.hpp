@@ -250,7 +250,7 @@ struct MarchKernel3 {
 
     // A FAST flux evaluates each interface with SharedOps and redoes those
     // whose operands leave the guarded range with PlainOps (as the 2D stage
-    // kernel's flux_pass); otherwise PlainOps throughout.
+    // kernel's flux_turn); otherwise PlainOps throughout.
     // `adm`: every cell of the plane tile is admitted to SharedOps.
     template <int DIR>
     __device__ __forceinline__ static void plane_pass(const double* sp, double* sf, int ox, int oy, const int* n,
