@@ -156,7 +156,7 @@ struct TileKernel2 {
         }
     }
 
-    __device__ static void run(const StageParams& P) { run_tile(P, tile_id_xcd(blockIdx.x, gridDim.x)); }
+    __device__ static void run(const StageParams& P) { run_tile<false, true>(P, tile_id_xcd(blockIdx.x, gridDim.x)); }
     __device__ static void run_volume(const StageParams& P, const VolumeParams& V) {
         run_tile<true>(P, tile_id_xcd(blockIdx.x, gridDim.x), &V);
     }
@@ -164,8 +164,11 @@ struct TileKernel2 {
     // VOL: the cells live in a reference Volume (V; MODE_FLUX_ONLY, or
     // MODE_RK3_3 for the combination V describes) and P.n is the extent of the
     // box the launch covers; otherwise in the interior-only buffers of P
-    // with the boundary map for the halo.
-    template <bool VOL = false>
+    // with the boundary map for the halo.  LOAD_FIRST: the launch's first
+    // workgroups, one a CU, issue their loads before the test whether the step
+    // runs at all (a single grid's steps nearly always do; of a batch's samples
+    // many may have ended).
+    template <bool VOL = false, bool LOAD_FIRST = false>
     __device__ static void run_tile(const StageParams& P, const unsigned int tile, const VolumeParams* V = nullptr) {
         __shared__ double su[NV * LT];
         __shared__ double sf[NV * NF];
@@ -175,11 +178,16 @@ struct TileKernel2 {
 
         Control* ctrl = P.ctrl;
         const int mode = MODE_CT >= 0 ? MODE_CT : P.mode;
-        // A step past the end is a no-op, and reads nothing: a run is launched
-        // in chunks, and most of its last one may lie past the end (2048^2, us
-        // of 48 such steps: 980 with the tile's loads issued ahead of this
-        // test, 493 so; the steps before the end are as fast).
-        if (!VOL && !ctrl->active && mode != MODE_FLUX_ONLY) return;
+        // A step past the end is a no-op.  A run is launched in chunks, and most
+        // of its last one may lie past the end, so all workgroups but the first
+        // read nothing then; those have nothing else to do while the test's
+        // answer travels.  us of 48 steps past the end, of 16 before it, every
+        // workgroup's loads ahead of the test / none / the first 256 so: 1024^2
+        // 397 / 264 / 307, 1958 / 1962 / 1947 (another card 2085 / 2110); 2048^2
+        // 980 / 495 / 506, 6972 / 6971 / 6933; 512^2 320 / 270 / 297, 885 / 888 /
+        // 881.
+        const bool early = LOAD_FIRST && blockIdx.x < 256;
+        if (!VOL && !early && !ctrl->active && mode != MODE_FLUX_ONLY) return;
 
         const int n0 = P.n[0], n1 = P.n[1];
         const int ntx = (n0 + TX - 1) / TX;
@@ -218,6 +226,7 @@ struct TileKernel2 {
 #pragma unroll
                 for (int v = 0; v < NV; ++v) s0[k][v] = soa_ld<OFF32>(P.u0, nc, v, sg[k]);
         }
+        if (!VOL && early && !ctrl->active && mode != MODE_FLUX_ONLY) return;
         // dt / dx, formed while the loads are in flight
         const double s = (mode == MODE_FLUX_ONLY || mode == MODE_L) ? 0.0
                          : VOL                                       ? V->s
