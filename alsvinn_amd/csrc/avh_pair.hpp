@@ -130,7 +130,6 @@ struct PairKernel {
         __shared__ double s_ws[3][NT / 64];
         __shared__ StepEnd s_end;
         Control* const ctrl = P.ctrl;
-        if (!ctrl->active) return;  // step past the end: no-op
         const int n0 = P.n[0], n1 = P.n[1];
         const long long nc = P.ncells;
         const unsigned int tile = tile_id_xcd(blockIdx.x, gridDim.x);
@@ -151,6 +150,7 @@ struct PairKernel {
                 u0[m][v] = P.u0[v * nc + gi];
             }
         }
+        if (!ctrl->active) return;  // step past the end: no-op
         const double s = stage_scale(P, ctrl, MODE_RK3_3, &s_end);
 
         // second stage

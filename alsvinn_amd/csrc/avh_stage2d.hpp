@@ -164,10 +164,10 @@ struct TileKernel2 {
     // VOL: the cells live in a reference Volume (V; MODE_FLUX_ONLY, or
     // MODE_RK3_3 for the combination V describes) and P.n is the extent of the
     // box the launch covers; otherwise in the interior-only buffers of P
-    // with the boundary map for the halo.  LOAD_FIRST: the launch's first
-    // workgroups, one a CU, issue their loads before the test whether the step
-    // runs at all (a single grid's steps nearly always do; of a batch's samples
-    // many may have ended).
+    // with the boundary map for the halo.  LOAD_FIRST: on
+    // grids that are not large the test whether the step runs at all comes after
+    // the tile's addresses (a single grid's steps nearly always do; of a batch's
+    // samples many may have ended).
     template <bool VOL = false, bool LOAD_FIRST = false>
     __device__ static void run_tile(const StageParams& P, const unsigned int tile, const VolumeParams* V = nullptr) {
         __shared__ double su[NV * LT];
@@ -179,16 +179,14 @@ struct TileKernel2 {
         Control* ctrl = P.ctrl;
         const int mode = MODE_CT >= 0 ? MODE_CT : P.mode;
         // A step past the end is a no-op.  A run is launched in chunks, and most
-        // of its last one may lie past the end, so all workgroups but the first
-        // read nothing then; those have nothing else to do while the test's
-        // answer travels.  us of 48 steps past the end, of 16 before it, every
-        // workgroup's loads ahead of the test / none / the first 256 so: 1024^2
-        // 397 / 264 / 307, 1958 / 1962 / 1947 (another card 2085 / 2110); 2048^2
-        // 980 / 495 / 506, 6972 / 6971 / 6933; 512^2 320 / 270 / 297, 885 / 888 /
-        // 881.
-        const bool early = LOAD_FIRST && blockIdx.x < 256;
-        if (!VOL && !early && !ctrl->active && mode != MODE_FLUX_ONLY) return;
-
+        // of its last one may lie past the end; on large grids the test comes first:
+        // 48 steps past the end of 2048^2 take 980 us with the addresses ahead of
+        // it and 495 so, a step before it 871 either way.  Up to some rounds of
+        // tiles the addresses ahead are worth more than they cost: at 1024^2 (2310
+        // tiles) 397 us against 264, but a step 130.1 us against 131.6 on one
+        // card, 122.4 both on another; at 1448^2 (4462) 595 and 340, steps alike.
+        // (The shapes that evaluate both directions at once are for small grids.)
+        if (!VOL && !(LOAD_FIRST && (DUAL || gridDim.x <= 4096)) && !ctrl->active && mode != MODE_FLUX_ONLY) return;
         const int n0 = P.n[0], n1 = P.n[1];
         const int ntx = (n0 + TX - 1) / TX;
         const int ox = (int)(tile % ntx) * TX, oy = (int)(tile / ntx) * TY;
@@ -226,7 +224,7 @@ struct TileKernel2 {
 #pragma unroll
                 for (int v = 0; v < NV; ++v) s0[k][v] = soa_ld<OFF32>(P.u0, nc, v, sg[k]);
         }
-        if (!VOL && early && !ctrl->active && mode != MODE_FLUX_ONLY) return;
+        if (!VOL && LOAD_FIRST && !ctrl->active && mode != MODE_FLUX_ONLY) return;
         // dt / dx, formed while the loads are in flight
         const double s = (mode == MODE_FLUX_ONLY || mode == MODE_L) ? 0.0
                          : VOL                                       ? V->s
