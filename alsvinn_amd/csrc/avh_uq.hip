@@ -1133,14 +1133,21 @@ static int sweep_blocks(int nc, int nr) { return ((nc + 63) / 64) * ((nr + 4 * S
 //             62 lags   17x300 x 3 1565 / 3975, 130^2 x 8 11306 / 16474,
 //                       256^2 10760 (2 samples) / 9497
 //             8 lags    256^2 x 2 237 / 291, x 16 1645 / 1551, 1000x800 1296 / 1211
-// so there the sweep takes only grids that fill its lanes, in enough blocks.
+//   and p = 1.5, periodic
+//             3 lags    256^2 x 16 181 / 197, x 64 621 / 607, 512^2 x 8 325 / 318
+//             6 lags    256^2 x 8 274 / 289, x 16 517 / 505, x 64 1975 / 1807
+//             8 lags    128^2 x 64 868 / 955, 256^2 x 2 135 / 161, x 8 442 / 442
+// so there the sweep takes only grids that fill its lanes, in enough blocks: more
+// of them where the lags are few.
 static bool structure_sweeps(bool general, int nx, int ny, int nsamples, int nlags) {
     const long long cells = (long long)nx * ny;
     if (!general) return nlags > 12 || cells * nsamples * (4 * nlags * (nlags + 1)) > (1ll << 24);
     const int cu = sweep_blocks(nx, ny), ct = sweep_blocks(ny, nx);
     const double slots = 64.0 * 4 * SWEEP_ROWS * (cu + ct);  // lanes times rows of the field's sweep and the transpose's
-    return nlags >= 8 && std::min(nx, ny) >= 128 && (long long)(cu + ct) * nlags * nsamples >= 2048 &&
-           2 * cells >= 0.92 * slots;
+    const long long blocks = (long long)(cu + ct) * nlags * nsamples;
+    const int n = std::min(nx, ny);
+    return 2 * cells >= 0.92 * slots &&
+           ((nlags >= 8 && n >= 128 && blocks >= 2048) || (nlags >= 3 && n > 128 && blocks >= 6144));
 }
 
 static avh_status launch_structure_gather(int pi, dim3 grid, hipStream_t st, const double* state, long long stride,
